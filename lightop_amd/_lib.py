@@ -105,6 +105,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 def lib() -> ctypes.CDLL:
@@ -122,6 +123,26 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def host():
+    """The native marshalling of the calls a serving loop makes on every step (csrc/host_binding.cpp), bound to
+    the library above.  Built with it, and as little optional."""
+    global _host
+    if _host is None:
+        handle = lib()
+        import torch  # noqa: F401  (its libraries are what the module links against)
+
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError(f"lightop_amd: the host binding cannot be loaded ({e}): build it with "
+                               "`python -m lightop_amd.build`") from e
+        mod.bind(*(ctypes.cast(getattr(handle, n), c_void_p).value for n in (
+            "lo_fused_experts_block_int8", "lo_fused_experts_channel_int8", "lo_fused_experts_workspace_bytes",
+            "lo_topk_softmax", "lo_moe_fused_gate", "lo_last_error")))
+        _host = mod
+    return _host
 
 
 def check(rc: int) -> None:

@@ -1,4 +1,5 @@
-"""Builds the HIP extension (lightop_amd/csrc/*.hip -> liblightop_mi355.so) for gfx950.
+"""Builds the HIP extension (lightop_amd/csrc/*.hip -> liblightop_mi355.so) for gfx950 and the host binding
+(csrc/host_binding.cpp -> lightop_amd/_host.so).
 
 Run as ``python -m lightop_amd.build``.  hipcc cross-compiles without a GPU, so the
 library is built ahead of time and shipped next to the sources; nothing is compiled
@@ -9,6 +10,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
@@ -57,5 +59,26 @@ def build_library(verbose: bool = False, extra_flags=(), out_path: str = LIB_PAT
     return out_path
 
 
+HOST_SRC = os.path.join(CSRC, "host_binding.cpp")
+HOST_PATH = os.path.join(os.path.dirname(CSRC), "_host.so")
+
+
+def build_host(out_path: str = HOST_PATH) -> str:
+    """Compile the native marshalling of the per-step calls: host code only, against torch's headers."""
+    import torch
+    from torch.utils import cpp_extension
+
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    includes = [f"-I{d}" for d in (*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"])]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *includes, HOST_SRC, "-o", out_path, f"-L{lib_dir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+           "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"the host binding does not compile:\n{res.stderr}")
+    return out_path
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_host())

@@ -13,6 +13,10 @@ from ..gemmopt import moe_gemm_w8a8
 from ..op import _act_dtype, _ids_dtype, _on_device, _require_cuda
 
 
+# forms of a whole-path call, as csrc/host_binding.cpp numbers them
+_FORM_BLOCK, _FORM_CHANNEL, _FORM_W4_GROUPS, _FORM_W4_CHANNEL = 0, 1, 2, 3
+
+
 def get_w8a8moe_json(m: int, E: int, n1: int, n2: int, k: int, use_int8_w8a8: bool,
                      block_shape: Optional[List[int]], topk: int,
                      global_num_experts: int = -1, preshuffled: bool = True,
@@ -408,6 +412,16 @@ def fused_experts_impl_int8(hidden_states: torch.Tensor,
     Unknown keyword arguments are ignored, as in the reference.
     """
     extra = _  # private knobs: lightop_amd_flags, lightop_amd_block_size_m, lightop_amd_workspace
+    if use_int8_w8a8 and not (extra or use_fp8_w8a8 or use_int8_w8a16 or use_int4_w4a16) and i_q is None:
+        form = _FORM_CHANNEL if per_channel_quant and block_shape is None else (
+            _FORM_BLOCK if not per_channel_quant and block_shape is not None and list(block_shape) == [128, 128] else None)
+        if form is not None and activation in ("silu", "gelu"):
+            out = (_lib._host or _lib.host()).fused_experts(
+                hidden_states, w1, w2, topk_weights, topk_ids, cache13, w1_scale, w2_scale, expert_map, shared_output,
+                form, inplace, apply_router_weight_on_input, global_num_experts, routed_scaling_factor,
+                _lib.LO_FUSED_ACT_GELU if activation == "gelu" else 0)
+            if out is not None:  # None: not an ordinary call (csrc/host_binding.cpp); checked and converted below
+                return out
     # Check constraints (int8.py:658-667).
     assert use_int8_w8a8 or use_fp8_w8a8
     assert hidden_states.shape[1] == w1.shape[2], "Hidden size mismatch"
@@ -509,6 +523,14 @@ def fused_experts_impl_w4a8(hidden_states: torch.Tensor,
     ``activation``: "silu" or "gelu"; the reduce is always performed.
     """
     extra = _
+    k_groups = block_shape is not None and list(block_shape) == [1, 128]
+    if not extra and (block_shape is None or (k_groups and w1_zp is None and w2_zp is None)) and activation in ("silu", "gelu"):
+        out = (_lib._host or _lib.host()).fused_experts(
+            hidden_states, w1, w2, topk_weights, topk_ids, cache13, w1_scale, w2_scale, expert_map, shared_output,
+            _FORM_W4_GROUPS if k_groups else _FORM_W4_CHANNEL, inplace, apply_router_weight_on_input, global_num_experts,
+            routed_scaling_factor, _lib.LO_FUSED_ACT_GELU if activation == "gelu" else 0)
+        if out is not None:
+            return out
     assert hidden_states.shape[1] == w1.shape[2] * 2, "Hidden size mismatch"  # w4a8.py:503
     assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
     assert hidden_states.is_contiguous(), "Hidden_states must be contiguous"
@@ -578,22 +600,6 @@ def _workspace_bytes_cached(M: int, top_k: int, H: int, I: int, num_experts: int
     return fused_experts_workspace_bytes(M, top_k, H, I, num_experts, 0)
 
 
-_ws_cache: Dict[Tuple[int, int], torch.Tensor] = {}
-
-
-def _cached_workspace(nbytes: int, device: torch.device, stream_key: int) -> torch.Tensor:
-    """The library's scratch for a whole-path call, kept per (device, stream) and grown on demand, so that a
-    serving loop does not allocate on every call (the reference keeps its own workspace, cache13, in a
-    process-wide cache the same way: vllm_compat/fused_moe_cache.py:19-24).  Calls on one stream run in
-    order, so they can share it; calls on different streams get workspaces of their own."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_key)
-    ws = _ws_cache.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _ws_cache[key] = ws
-    return ws
-
-
 def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, inplace, apply_router_weight_on_input,
                        global_num_experts, expert_map, w1_scale, w2_scale, routed_scaling_factor, shared_output,
                        I, flags, block_size_m, channel=False, workspace=None, prequant=None, chunk_size=None):
@@ -625,7 +631,9 @@ def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, i
     ws_bytes = _workspace_bytes_cached(M, top_k_num, H, I, global_num_experts)
     stream_handle = torch.cuda.current_stream(hidden_states.device).cuda_stream
     if workspace is None:
-        workspace = _cached_workspace(ws_bytes, hidden_states.device, stream_handle)
+        # kept per (device, stream) and grown on demand (the reference keeps its own workspace, cache13, in a
+        # process-wide cache the same way: vllm_compat/fused_moe_cache.py:19-24)
+        workspace = (_lib._host or _lib.host()).workspace(ws_bytes, hidden_states.device.index, stream_handle)
         ws_bytes = workspace.numel()
     else:  # the caller's own scratch (tests read the intermediates out of it afterwards)
         assert workspace.dtype == torch.uint8 and workspace.is_contiguous() and workspace.numel() >= ws_bytes

@@ -179,6 +179,9 @@ def topk_softmax(topk_weights: torch.Tensor, topk_indices: torch.Tensor,
     """Softmax top-k router into caller-allocated outputs (op.topk_softmax, export.cpp:546, :1437;
     topk_softmax_kernels.cu:1716-1790).  Winners in descending order, equal logits are won by
     the lower expert id; ``token_expert_indices[t, j] = j * num_tokens + t``."""
+    if (_lib._host or _lib.host()).topk_softmax(topk_weights, topk_indices, token_expert_indices, gating_output,
+                                                Is_renormalize):
+        return
     _require_cuda(topk_weights, topk_indices, token_expert_indices, gating_output)
     if gating_output.dim() != 2 or not gating_output.is_contiguous():
         raise RuntimeError("lightop_amd: gating_output must be a contiguous [num_tokens, num_experts] tensor")
@@ -204,6 +207,11 @@ def moe_fused_gate(input: torch.Tensor, bias: torch.Tensor, num_expert_group: in
                    apply_routed_scaling_factor_on_output: bool = True, output_indices_int64: bool = False):
     """Grouped sigmoid top-k with correction bias; returns ``[weights f32 [T, topk], indices [T, topk]]``
     (op.moe_fused_gate, export.cpp:566, :1508; moe_fused_gate.cu:1331-1530)."""
+    pair = (_lib._host or _lib.host()).fused_gate(input, bias, num_expert_group, topk_group, topk, n_share_experts_fusion,
+                                                  routed_scaling_factor, apply_routed_scaling_factor_on_output,
+                                                  output_indices_int64)
+    if pair is not None:
+        return pair
     _require_cuda(input, bias)
     if input.dim() != 2 or not input.is_contiguous():
         raise RuntimeError("lightop_amd: input must be a contiguous [num_tokens, num_experts] tensor")
