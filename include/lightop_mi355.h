@@ -317,8 +317,10 @@ typedef struct lo_moe_tile {
 
 /* kernel families (lo_moe_tile.kernel) */
 enum {
-  LO_KERNEL_WS = 0,      /* weight-streaming, no LDS in the K loop (token blocks of 16 / 32) */
-  LO_KERNEL_TILE = 1,    /* LDS-tiled, weights register-fed (row-major weights, 64 / 128 tokens) */
+  LO_KERNEL_WS = 0,      /* weight-streaming, no LDS in the K loop (token blocks of 16 / 32).  Row-major weights go
+                          * through one kernel that copies them into LDS at every block size; it is reported as WS up
+                          * to 32 tokens, TILE at 64, T128 at 128 and PC with per-channel scales, four waves each */
+  LO_KERNEL_TILE = 1,    /* LDS-tiled, weights register-fed (64 / 128 tokens) */
   LO_KERNEL_PC = 2,      /* per-channel LDS-tiled */
   LO_KERNEL_AS = 3,      /* activation-stationary second GEMM (short K) */
   LO_KERNEL_T128 = 4,    /* 128 tokens, both operands copied global -> LDS (pre-shuffled weights) */

@@ -1,5 +1,6 @@
 // Host side of the C ABI: error reporting, the gfx950 tile table and the whole-path
 // entry point that chains the stage kernels on one stream.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -212,9 +213,9 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   }
   if (per_expert <= 12.0) return 16;
   if (per_expert <= 24.0) return 32;
-  // Row-major block-form weights: 64-token LDS tiles, two workgroups per CU; their 128-token
-  // kernel is one phase-locked workgroup per CU and measured slower on every layer shape tried.
-  return 64;
+  // Row-major block-form weights, larger experts: 128-token tiles from 48 slots per expert on (64 / 128: Qwen3-235B-A22B-
+  // shaped layer at 1000 tokens 613 / 579 us, at 4096: 1330 / 1170; DeepSeek-V3 share at 4096: 540 / 510).
+  return H >= 4096 && per_expert > 48.0 && H / kGroup <= 128 && I / kGroup <= 128 ? 128 : 64;
 }
 
 // What the block-form whole-path call (int8 weights, or int4 weights with K-group scales) does with a
@@ -234,7 +235,7 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
   const bool block_size_m_auto = block_size_m == 0;
   if (block_size_m == 0 && dtype == LO_F32) // fp32 rows go through the weight-streaming kernel at every size
-    block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false);
+    block_size_m = std::min(pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false), 64);
   if (block_size_m == 0)
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false,
                                 !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true));
@@ -302,13 +303,14 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
   a.out_f16 = dtype == LO_F16 ? 1 : 0;
   a.out_f32 = dtype == LO_F32 ? 1 : 0;
   const int gflags = flags & ~(LO_FUSED_ACT_GELU | LO_FUSED_NO_DECODE_PATH | LO_FUSED_FORCE_DECODE_PATH);
+  auto rows = [&](bool fa) { return !(gflags & LO_GEMM_FORCE_STREAMING) && gemm_rows_supports(a, fa, bm); };
   if (gemm1) {
     a.N = 2 * I; a.K = H; a.a_rows = M;
-    describe_gemm_kernel(pick_gemm_kernel(a, fused, bm, gflags), fused, bm, gemm1);
+    describe_gemm_kernel(pick_gemm_kernel(a, fused, bm, gflags), fused, bm, rows(fused), gemm1);
   }
   if (gemm2) {
     a.N = H; a.K = I; a.a_rows = M * top_k;
-    describe_gemm_kernel(pick_gemm_kernel(a, false, bm, gflags), false, bm, gemm2);
+    describe_gemm_kernel(pick_gemm_kernel(a, false, bm, gflags), false, bm, rows(false), gemm2);
   }
   // a few tokens: the whole-path call serves the block form with its two-launch path
   if (decode) {

@@ -164,7 +164,7 @@ __device__ __forceinline__ void wave_store_32x64_bf16(int8_t *stg, const v4u16 (
 
 // Kernel a stage is served by, and its workgroup shape (gemm_api.hip).
 int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int block_size_m, int flags);
-void describe_gemm_kernel(int kernel, bool fused_act, int block_size_m, lo_moe_tile *t);
+void describe_gemm_kernel(int kernel, bool fused_act, int block_size_m, bool rows, lo_moe_tile *t);
 
 // Decode-size whole path in two launches (gemm_dec.hip): LO_ENOTSUP when it does not apply.
 // act: room for [M * top_k, I] bf16.  w4: packed int4 weights with K-group scales [E, K/128, N].
@@ -190,6 +190,9 @@ bool gemm_as_supports(const GemmArgs &a, bool fused_act, int block_size_m);
 // 128-token kernel, two four-wave workgroups per compute unit (gemm_t128.hip): pre-shuffled int8 weights.
 int launch_gemm_t128(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks, hipStream_t s);
 bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m);
+// Row-major int8 weights, block or per-channel scales (gemm_t128.hip): block_size_m 16, 32, 64 or 128.
+bool gemm_rows_supports(const GemmArgs &a, bool fused_act, int block_size_m);
+int launch_gemm_rows(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks, hipStream_t s);
 // W4A8 LDS-tiled kernel (gemm_w4.hip): block_size_m 64.
 int launch_gemm_w4_tile(const GemmArgs &a, bool fused_act, int flags, int64_t m_blocks, hipStream_t s);
 bool gemm_w4_tile_supports(const GemmArgs &a, bool fused_act, int block_size_m);

@@ -36,6 +36,10 @@ int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int bs, int flags) {
   if (a.out_f32) return LO_KERNEL_WS; // fp32 rows: the weight-streaming kernel's plain epilogue only
   if (bs == 160) return LO_KERNEL_T128; // 160-token blocks exist for that kernel only (the entry point checks)
   const bool tiled = !(flags & LO_GEMM_FORCE_STREAMING);
+  // Row-major int8 weights have one kernel (gemm_t128.hip, "row-major weights") at every block size; it is reported as what
+  // it stands in for: weight streaming up to 32 tokens, LDS tiles above.
+  if (tiled && gemm_rows_supports(a, fused_act, bs))
+    return bs <= 32 ? LO_KERNEL_WS : a.per_channel ? LO_KERNEL_PC : bs == 64 ? LO_KERNEL_TILE : LO_KERNEL_T128;
   if (a.w4 && a.per_channel) // the reference's own int4 form: 128-token LDS tiles, else streaming
     return tiled && gemm_t128_supports(a, fused_act, bs) ? LO_KERNEL_T128 : LO_KERNEL_WS;
   if (a.w4) { // int4 weights: 128- or 64-token LDS tiles, else streaming
@@ -54,9 +58,14 @@ int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int bs, int flags) {
 }
 
 // Workgroup shape of that kernel: wavefronts and weight rows per workgroup.
-void describe_gemm_kernel(int kernel, bool fused_act, int bs, lo_moe_tile *t) {
+void describe_gemm_kernel(int kernel, bool fused_act, int bs, bool rows, lo_moe_tile *t) {
   t->block_size_m = bs;
   t->kernel = kernel;
+  if (rows) { // row-major weights: four waves x 64 rows at every block size
+    t->waves = 4;
+    t->block_n = 256;
+    return;
+  }
   switch (kernel) {
   case LO_KERNEL_WS: { // gemm_ws.hip: launch_ws
     const int tm = bs / 16;
@@ -78,6 +87,8 @@ void describe_gemm_kernel(int kernel, bool fused_act, int bs, lo_moe_tile *t) {
 
 static int launch_gemm(const GemmArgs &a, bool fused_act, int bs, int flags, int64_t m_blocks,
                        hipStream_t s) {
+  if (!(flags & LO_GEMM_FORCE_STREAMING) && bs != 160 && gemm_rows_supports(a, fused_act, bs))
+    return launch_gemm_rows(a, fused_act, bs, flags, m_blocks, s);
   switch (pick_gemm_kernel(a, fused_act, bs, flags)) {
   case LO_KERNEL_T128: return launch_gemm_t128(a, fused_act, bs, flags, m_blocks, s);
   case LO_KERNEL_W4_TILE: return launch_gemm_w4_tile(a, fused_act, flags, m_blocks, s);

@@ -22,7 +22,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // knows how many memory operations follow each weight load and waits for exactly those; in the
 // general form the stores sit in a branch, the wait counts assume they did not happen, and after
 // every tile the wave waits for loads it has only just issued.
-template <int ORD, bool SHUF, int KBT = 0>
+template <int ORD, int KBT = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
                                                           int n_groups, int n_cnt, int sub_shift) {
@@ -113,15 +113,13 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   const brsrc rWs = make_rsrc(a.Ws + e * NB * KB, static_cast<uint32_t>(NB * KB * 4));
   // lane offsets inside tile nt0; a later tile and the K block go into the scalar offset
   int woff[2], wsoff[2];
-  const int wkstride = SHUF ? shuf_kb_stride(static_cast<int>(N / 16)) : kGroup;
-  const int wtstride = SHUF ? 16 * shuf_nb_stride(KB) : 256 * K; // 256 rows further
+  const int wkstride = shuf_kb_stride(static_cast<int>(N / 16));
+  const int wtstride = 16 * shuf_nb_stride(KB); // 256 rows further
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const int nr = nt0 * 256 + wr * 64 + rb * 32;
-    if constexpr (SHUF) // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
-      woff[rb] = (nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
-    else
-      woff[rb] = (nr + r) * K + c * 64;
+    // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
+    woff[rb] = (nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
     wsoff[rb] = (nr / kGroup) * KB * 4;
   }
 
@@ -143,7 +141,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) wreg[b][rb][ks] = bld16(rW, woff[rb], so + (SHUF ? ks * 512 : ks * 16));
+      for (int ks = 0; ks < 4; ++ks) wreg[b][rb][ks] = bld16(rW, woff[rb], so + ks * 512);
     const int ss = ((nt - nt0) * 2 * KB + kb) * 4;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) bsc[b][rb] = bld_f32(rWs, wsoff[rb], ss);
@@ -168,9 +166,9 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     for (int tb = 0; tb < 2; ++tb) {
       v4i bf[4];
       // the K bytes of k-step ks must be the ones the weight operand holds for it
-      const int8_t *src = sA + (tb * 32 + r) * pitch + kb * kGroup + (SHUF ? c * 16 : c * 64);
+      const int8_t *src = sA + (tb * 32 + r) * pitch + kb * kGroup + c * 16;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) bf[ks] = *reinterpret_cast<const v4i *>(src + (SHUF ? ks * 32 : ks * 16));
+      for (int ks = 0; ks < 4; ++ks) bf[ks] = *reinterpret_cast<const v4i *>(src + ks * 32);
       const float as = live ? sS[kb * kTileM + tb * 32 + r] : 0.0f; // a step past the end adds 0
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
@@ -285,7 +283,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
 static int64_t as_lds_bytes(int64_t K) { return 64 * (K + 16) + (K / kGroup) * 64 * 4 + 4 * 32 * kStgPitch; }
 
 bool gemm_as_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
-  if (fused_act || (block_size_m != 64 && block_size_m != 128)) return false;
+  if (fused_act || !a.w_shuffled || (block_size_m != 64 && block_size_m != 128)) return false;
   if (a.N % 64 != 0 || (reinterpret_cast<uintptr_t>(a.C) & 15) != 0) return false;
   if (as_lds_bytes(a.K) > 80 * 1024) return false; // two workgroups per CU
   // Pays off only when the launch is several rounds of workgroups deep even with half a
@@ -314,23 +312,17 @@ int launch_gemm_as(const GemmArgs &a0, int flags, int block_size_m, int64_t m_bl
   const size_t lds = static_cast<size_t>(as_lds_bytes(a.K));
   const dim3 g(static_cast<unsigned>(grid)), b(256);
   const int mbi = static_cast<int>(m_blocks), Gi = static_cast<int>(G);
-#define LO_AS_LAUNCH(FS, SH)                                                                          \
+#define LO_AS_LAUNCH(FS, KBT)                                                                         \
   do {                                                                                                \
-    if (a.K == 6 * kGroup) LO_AS_LAUNCH_K(FS, SH, 6);                                                 \
-    else LO_AS_LAUNCH_K(FS, SH, 0);                                                                   \
-  } while (0)
-#define LO_AS_LAUNCH_K(FS, SH, KBT)                                                                   \
-  do {                                                                                                \
-    auto kern = moe_gemm_as_kernel<FS, SH, KBT>;                                                      \
+    auto kern = moe_gemm_as_kernel<FS, KBT>;                                                          \
     static unsigned long long lds_done = 0; /* per instantiation: one bit per device */               \
     const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), 80 * 1024, &lds_done);  \
     if (rc_lds) return rc_lds;                                                                        \
     hipLaunchKernelGGL(kern, g, b, lds, s, a, mbi, Gi, n_groups, n_cnt, sub_shift);                   \
   } while (0)
-  if (a.w_shuffled) LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, true);
-  else LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, false);
+  if (a.K == 6 * kGroup) LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, 6);
+  else LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, 0);
 #undef LO_AS_LAUNCH
-#undef LO_AS_LAUNCH_K
   return check_launch("moe_gemm(activation-stationary)");
 }
 

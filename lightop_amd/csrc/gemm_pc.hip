@@ -25,9 +25,8 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kPcRow = 144; // LDS row pitch in bytes: 128 + 16 keeps ds_read_b128 conflict-free
 
-template <bool SHUF, int TB, bool STREAM>
+template <int TB, bool STREAM>
 __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks, int group_m) {
-  static_assert(!STREAM || SHUF, "streaming policy: pre-shuffled weights only");
   constexpr int kWAux = STREAM ? kCacheStream : kCacheDefault;
   constexpr int kTileM = 32 * TB;       // tokens per workgroup
   constexpr int kThrPerTok = 256 / kTileM; // threads that gather one token row
@@ -89,10 +88,8 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const int64_t nr = wave_active ? nrow[rb] : 0;
-    if constexpr (SHUF) // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
-      woff[rb] = static_cast<int>(nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
-    else
-      woff[rb] = static_cast<int>((nr + r) * K) + c * 64;
+    // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
+    woff[rb] = static_cast<int>(nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
   }
 
   using B0 = std::integral_constant<int, 0>;
@@ -127,8 +124,7 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        wreg[b][rb][ks] = SHUF ? bld16<kWAux>(rW, woff[rb], kc * wkstride + ks * 512)
-                               : bld16<kWAux>(rW, woff[rb], kc * kGroup + ks * 16);
+        wreg[b][rb][ks] = bld16<kWAux>(rW, woff[rb], kc * wkstride + ks * 512);
   };
   auto compute = [&](auto BUF) {
     constexpr int b = decltype(BUF)::value;
@@ -137,9 +133,9 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
     for (int tb = 0; tb < TB; ++tb) {
       v4i bf[4];
       // the K bytes of k-step ks must be the ones the weight operand holds for it
-      const int8_t *src = tile + (tb * 32 + r) * kPcRow + (SHUF ? c * 16 : c * 64);
+      const int8_t *src = tile + (tb * 32 + r) * kPcRow + c * 16;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) bf[ks] = *reinterpret_cast<const v4i *>(src + (SHUF ? ks * 32 : ks * 16));
+      for (int ks = 0; ks < 4; ++ks) bf[ks] = *reinterpret_cast<const v4i *>(src + ks * 32);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -204,19 +200,19 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
 
 // 128 tokens: 246 registers, two waves per SIMD.  64 tokens: 162 registers, so three workgroups
 // fit a compute unit and hide each other's barrier and memory waits better than two.
-template <bool SHUF, bool STREAM>
+template <bool STREAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_pc_kernel_128(const GemmArgs a, int m_blocks, int group_m) {
-  moe_gemm_pc_body<SHUF, 4, STREAM>(a, m_blocks, group_m);
+  moe_gemm_pc_body<4, STREAM>(a, m_blocks, group_m);
 }
-template <bool SHUF, bool STREAM>
+template <bool STREAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void moe_gemm_pc_kernel_64(const GemmArgs a, int m_blocks, int group_m) {
-  moe_gemm_pc_body<SHUF, 2, STREAM>(a, m_blocks, group_m);
+  moe_gemm_pc_body<2, STREAM>(a, m_blocks, group_m);
 }
 
 bool gemm_pc_supports(const GemmArgs &a, int block_size_m) {
-  return a.per_channel && (block_size_m == 64 || block_size_m == 128) && a.N % 64 == 0;
+  return a.per_channel && a.w_shuffled && (block_size_m == 64 || block_size_m == 128) && a.N % 64 == 0;
 }
 
 int launch_gemm_pc(const GemmArgs &a0, int block_size_m, int64_t m_blocks, hipStream_t s) {
@@ -232,16 +228,12 @@ int launch_gemm_pc(const GemmArgs &a0, int block_size_m, int64_t m_blocks, hipSt
   const int mbi = static_cast<int>(m_blocks), gi = static_cast<int>(G);
   // one token block per expert, by and large: up to 48 slots per expert on average with 64-token blocks
   // (as measured for the block form's 64-token kernel), half a block with 128-token blocks
-  // (pre-shuffled weights only: a 128-byte line of row-major weights serves several k-steps of a lane,
-  // and the hint would have it fetched again for each)
-  const bool stream = a.w_shuffled &&
-                      a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) *
+  const bool stream = a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) *
                                          (block_size_m == 64 ? 48 : 64);
 #define LO_PC_LAUNCH(KERN)                                                                    \
   do {                                                                                        \
-    if (stream) hipLaunchKernelGGL((KERN<true, true>), g, b, 0, s, a, mbi, gi);               \
-    else if (a.w_shuffled) hipLaunchKernelGGL((KERN<true, false>), g, b, 0, s, a, mbi, gi);   \
-    else hipLaunchKernelGGL((KERN<false, false>), g, b, 0, s, a, mbi, gi);                    \
+    if (stream) hipLaunchKernelGGL((KERN<true>), g, b, 0, s, a, mbi, gi);                     \
+    else hipLaunchKernelGGL((KERN<false>), g, b, 0, s, a, mbi, gi);                           \
   } while (0)
   if (block_size_m == 128) LO_PC_LAUNCH(moe_gemm_pc_kernel_128);
   else LO_PC_LAUNCH(moe_gemm_pc_kernel_64);

@@ -68,17 +68,19 @@ __device__ __forceinline__ void wait_copies_barrier() {
 // python/lightop/_lmslim_native/layers/fused_moe/w4a8.py:341-395): one scale per token row and one
 // per weight row, both applied in the epilogue, so the int32 sums run over the whole K inside the
 // MFMA accumulators and the K loop has no scale arithmetic at all.
-template <bool FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8, bool ROWS = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 4 : NTB == 2 ? 3 : 2, NTB == 1 ? 4 : NTB == 2 ? 3 : 2)))
 void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
-  static_assert(!PC || (!FUSED_ACT && ORD == kOrdSeparate && (W4 || NTB == 10)),
-                "per-channel scales: plain GEMM, int4 weights or 160-token tiles of int8 weights");
-  static_assert(NTB == 8 || (NTB == 10 && (PC || !W4)),
-                "160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales");
+  static_assert(!PC || (!FUSED_ACT && ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
+                "per-channel scales: plain GEMM, int4 weights, 160-token tiles of int8 weights or row-major ones");
+  static_assert(NTB == 8 || (NTB == 10 && (PC || !W4)) || ((NTB == 1 || NTB == 2 || NTB == 4) && ROWS),
+                "160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales; 16, 32 and 64 tokens: "
+                "row-major weights");
+  static_assert(!ROWS || (!W4 && NTB <= 8), "row-major weights: int8, up to 128 tokens");
   constexpr int T = 16 * NTB;        // tokens per workgroup
   constexpr int AST = T * kGroup;    // token rows of one K block
-  constexpr int APW = NTB / 2;       // 1 KB pieces (eight token rows) of a token stage that a wave copies
-  constexpr int RED = NTB == 8 ? kTRed : 0;
+  constexpr int APW = NTB == 1 ? 1 : NTB / 2;       // 1 KB pieces (eight token rows) of a token stage that a wave copies
+  constexpr int RED = NTB <= 8 ? 4 * T * 4 : 0;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t *const sA = smem + kTW;
   float *const sS = reinterpret_cast<float *>(smem + kTW + 2 * AST);
@@ -109,15 +111,16 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   constexpr bool kEarlyIds = !(FUSED_ACT && NTB == 10);
   const int32_t blocks_end = a.ntpp[0];
   const int e_raw = a.expert_ids[mb];
+  const int cw = NTB == 1 ? wave & 1 : wave; // 16 tokens are two pieces: the first two waves copy them
   int32_t lf_copy[APW];
   int32_t lf_v0 = 0, lf_v1 = 0, lf_v2 = 0, lf_scale = 0;
   auto load_ids = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < APW; ++j) lf_copy[j] = sorted[(wave * APW + j) * 8 + (lane >> 3)];
-    lf_v0 = sorted[lane];
-    lf_v1 = sorted[lane + 64];
+    for (int j = 0; j < APW; ++j) lf_copy[j] = sorted[(cw * APW + j) * 8 + (lane >> 3)];
+    lf_v0 = sorted[lane & (T - 1 < 63 ? T - 1 : 63)];
+    if constexpr (NTB >= 8) lf_v1 = sorted[lane + 64];
     if constexpr (NTB == 10) lf_v2 = sorted[128 + (lane & 31)];
-    lf_scale = sorted[NTB == 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
+    lf_scale = sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
   };
   if constexpr (kEarlyIds) load_ids();
   if (static_cast<int64_t>(mb) * T >= blocks_end) return;
@@ -162,7 +165,8 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   const brsrc rWs = make_rsrc(a.Ws + static_cast<int64_t>(e) * N * (PC ? 1 : KB), static_cast<uint32_t>(N * (PC ? 1 : KB) * 4));
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * (PC ? 1 : KB) * 4));
-  const int wkstride = W4 ? shuf_kb_stride(NBLK) / 2 : shuf_kb_stride(NBLK);
+  const int wkstride = ROWS ? kGroup : W4 ? shuf_kb_stride(NBLK) / 2 : shuf_kb_stride(NBLK);
+  const int wpstride = ROWS ? static_cast<int>(8 * K) : 1024; // second half of a 16-row block
   int wvoff[2][2]; // [step half][fragment]: the 2 KB block of 16 rows x 128 K, in lane order
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -172,7 +176,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if constexpr (FUSED_ACT) nb = (rf ? I / 16 : 0) + static_cast<int64_t>(nt) * 8 + wave * 2 + h;
       else nb = static_cast<int64_t>(nt) * 16 + wave * 4 + h * 2 + rf;
       if (nb >= NBLK) nb = 0; // rows past N: computed on block 0, never stored
-      wvoff[h][rf] = static_cast<int>(nb) * (W4 ? shuf_nb_stride(KB) / 2 : shuf_nb_stride(KB)) + lane * 16;
+      // row-major: a 1 KB piece is 128 bytes of eight rows, whole lines; slot lane & 7 of row lane >> 3 takes
+      // the row's 16-byte piece slot ^ row (as in the token stage)
+      if constexpr (ROWS) wvoff[h][rf] = static_cast<int>((nb * 16 + (lane >> 3)) * K) + (((lane & 7) ^ (lane >> 3)) * 16);
+      else wvoff[h][rf] = static_cast<int>(nb) * (W4 ? shuf_nb_stride(KB) / 2 : shuf_nb_stride(KB)) + lane * 16;
     }
   // W4: lane l copies the scale of row l of the wave's 64 (fused: 32 gate rows, then the 32 up rows)
   int wsvoff = 0;
@@ -199,13 +206,13 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   } else {
 #pragma unroll
     for (int p = 0; p < 8; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[p >> 2][(p >> 1) & 1], (p & 1) * 1024, 0,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[p >> 2][(p >> 1) & 1], (p & 1) * wpstride, 0,
                                                kWAux);
   }
   int avoff[5]; // 1 KB pieces wave*APW + j of a token stage, j < APW: eight token rows each
 #pragma unroll
   for (int j = 0; j < APW; ++j) {
-    const int t = (wave * APW + j) * 8 + (lane >> 3);
+    const int t = (cw * APW + j) * 8 + (lane >> 3);
     const int64_t lf = kEarlyIds ? lf_copy[j] : sorted[t];
     const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
     const int piece = (lane & 7) ^ (t & 7); // slot lane & 7 of row t holds piece slot ^ (t & 7)
@@ -223,7 +230,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if constexpr (NTB == 10) lf_v2 = sorted[128 + (lane & 31)];
     }
     const uint64_t v0 = __builtin_amdgcn_ballot_w64(lf_v0 < a.num_valid);
-    const uint64_t v1 = __builtin_amdgcn_ballot_w64(lf_v1 < a.num_valid);
+    const uint64_t v1 = NTB >= 8 ? __builtin_amdgcn_ballot_w64(lf_v1 < a.num_valid) : 0;
     int last = v1 ? 127 - __builtin_clzll(v1) : (v0 ? 63 - __builtin_clzll(v0) : 0);
     if constexpr (NTB == 10) {
       const uint64_t v2 = __builtin_amdgcn_ballot_w64(lane < 32 && lf_v2 < a.num_valid);
@@ -233,7 +240,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   }
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
-    const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB == 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
+    const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
     const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
     asoff = static_cast<int>(lrow * (PC ? 1 : KB) * 4);
     // The epilogues take the ids from LDS: a global load in each of their exec-masked blocks is a
@@ -267,11 +274,11 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       } else {
         const int h = p >> 2, rf = (p >> 1) & 1, kh = p & 1;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[h][rf],
-                                                 __builtin_amdgcn_readfirstlane(kc * wkstride) + kh * 1024, 0, kWAux);
+                                                 __builtin_amdgcn_readfirstlane(kc * wkstride) + kh * wpstride, 0, kWAux);
       }
-    } else {
+    } else if (p - 8 < APW && (NTB > 1 || wave < 2)) {
       const int j = p - 8;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, sA + (kb & 1) * AST + (wave * APW + j) * 1024, 16, avoff[j],
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, sA + (kb & 1) * AST + (cw * APW + j) * 1024, 16, avoff[j],
                                                __builtin_amdgcn_readfirstlane(kc) * kGroup, 0, 0);
     }
   };
@@ -289,6 +296,11 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   int alds[2];
 #pragma unroll
   for (int kh = 0; kh < 2; ++kh) alds[kh] = r * kGroup + (((4 * kh + q) ^ (r & 7)) * 16);
+
+  // weight fragment's k-half kh inside its 2 KB: lane order, or (row-major) rows of 128 bytes swizzled like the tokens
+  int wlds[2];
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh) wlds[kh] = ROWS ? alds[kh] : kh * 1024 + lane * 16;
 
   float acc[2][NTB][2][4]; // [step half][token fragment][fragment of the half][element]
 #pragma unroll
@@ -357,7 +369,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
         for (int rf = 0; rf < 2; ++rf)
 #pragma unroll
           for (int kh = 0; kh < 2; ++kh)
-            w[h][rf][kh] = *reinterpret_cast<const v4i *>(sWw + ((h * 2 + rf) * 2 + kh) * 1024 + lane * 16);
+            w[h][rf][kh] = *reinterpret_cast<const v4i *>(sWw + (h * 2 + rf) * 2048 + wlds[kh]);
     }
   };
   // Full tiles meet at the barrier two stages before the end of a K block instead of at its start:
@@ -371,7 +383,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     constexpr int nst_c = decltype(NST)::value; // stages of this variant: 4, 8, 12, 16 (or 20)
     constexpr int kFull = 2 * NTB;              // stages of a full tile
     constexpr int kE0 = kFull - 2, kE1 = kFull - 1;
-    constexpr bool kEarly = nst_c == kFull && !W4;
+    constexpr bool kEarly = nst_c == kFull && !W4 && NTB >= 8;
     const int8_t *ta = sA + (kb & 1) * AST;
     const float *ts = sS + (kb & 1) * T;
     v4i bf[2][2];
@@ -414,7 +426,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     // pipeline stage (tb, h): its MFMAs are issued, then the previous stage's fragments are folded
     // while the matrix pipe works; the operands of token fragment tb + 1 are requested in (tb, 0)
 #pragma unroll
-    for (int st = 0; st < kFull; ++st) {
+    for (int st = 0; st < (kFull < 4 ? 4 : kFull); ++st) {
       const int tb = st >> 1, h = st & 1;
       const int cur = tb & 1, nxt = cur ^ 1;
       if (nst_c >= 8 && st < 6) {
@@ -456,7 +468,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
           for (int rf = 0; rf < 2; ++rf)
 #pragma unroll
             for (int kh = 0; kh < 2; ++kh)
-              w[h][rf][kh] = *reinterpret_cast<const v4i *>(sWw + ((h * 2 + rf) * 2 + kh) * 1024 + lane * 16);
+              w[h][rf][kh] = *reinterpret_cast<const v4i *>(sWw + (h * 2 + rf) * 2048 + wlds[kh]);
           if (st == kE0) {
             const int8_t *tan = sA + ((kb + 1) & 1) * AST;
 #pragma unroll
@@ -504,7 +516,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   read_w();
 
   auto k_loop = [&](auto NST) __attribute__((always_inline)) {
-    if constexpr (decltype(NST)::value == 2 * NTB && !W4) {
+    if constexpr (decltype(NST)::value == 2 * NTB && !W4 && NTB >= 8) {
       wait_copies_barrier<0>(); // K block 0 is complete in LDS
       if (tid < T) sS[T + tid] = 1 < KB ? s_pending : 0.0f;
       s_pending = load_scale(2);
@@ -534,6 +546,13 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (nst > 16) k_loop(std::integral_constant<int, 20>{});
     else if (nst > 8) k_loop(std::integral_constant<int, 16>{});
     else k_loop(std::integral_constant<int, 8>{});
+  } else if constexpr (NTB == 1) {
+    k_loop(std::integral_constant<int, 2>{});
+  } else if constexpr (NTB == 2) {
+    k_loop(std::integral_constant<int, 4>{});
+  } else if constexpr (NTB == 4) {
+    if (nst > 4) k_loop(std::integral_constant<int, 8>{});
+    else k_loop(std::integral_constant<int, 4>{});
   } else {
     if (nst > 12) k_loop(std::integral_constant<int, 16>{});
     else if (nst > 8) k_loop(std::integral_constant<int, 12>{});
@@ -702,8 +721,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < T * 8 / 256; ++j) {
+    for (int j = 0; j < (T * 8 + 255) / 256; ++j) {
       const int id = tid + 256 * j, tok = id >> 3, piece = id & 7;
+      if (NTB == 1 && tok >= T) break;
       const int64_t ft = sIds[tok];
       if (ft < a.num_valid)
         *reinterpret_cast<v4i *>(a.A2q + ft * I + static_cast<int64_t>(nt) * kGroup + piece * 16) =
@@ -722,6 +742,82 @@ bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   if (a.per_channel && (!a.w4 || fused_act)) return false; // int8 per-channel weights have gemm_pc.hip
   if (!fused_act && a.N % 64 != 0) return false;
   return a.K / kGroup <= kTMaxKB;
+}
+
+#ifndef LO_DMA_SIZES
+#define LO_DMA_SIZES (16+32+64)
+#endif
+#ifndef LO_DMA_SHUF
+#define LO_DMA_SHUF (16)
+#endif
+// ---- row-major weights -----------------------------------------------------------------------------------
+// Weights as a checkpoint holds them, [E, N, K].  Loading an MFMA operand straight from global memory asks for 64 bytes
+// of each of 16 rows per instruction (32 of 32 rows with the 32x32 form): every 128-byte line is requested two to four
+// times over, and what of it is still in L1 by then is luck, the rows being a power of two apart.  Copied into LDS
+// instead, a request is eight whole lines, each once, and the operand reads then find their 16-byte pieces swizzled by
+// row as the tokens' are.  The data movement is otherwise that of the pre-shuffled form.  Measured (whole layer with its
+// router, us, register-fed kernels / this one): Qwen3-30B-A3B layer at 24 tokens 146 / 105, at 250: 211 / 131, at 8192: 857 /
+// 630; Qwen3-235B-A22B-shaped layer at 200 tokens 676 / 457; DeepSeek-V3 share at 64 tokens 302 / 213 - within a few
+// percent of the load-time layout.
+//
+// Tiles: 16, 32 or 64 tokens (four, three, two workgroups per compute unit) as the alignment blocks are.
+bool gemm_rows_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
+  if (a.w_shuffled || a.w4 || a.out_f32) return false;
+  if (block_size_m != 16 && block_size_m != 32 && block_size_m != 64 && block_size_m != 128) return false;
+  return (fused_act || a.N % 64 == 0) && (a.per_channel || a.K / kGroup <= kTMaxKB);
+}
+
+template <int NTB>
+static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, dim3 g, int mbi, int gi, hipStream_t s) {
+  constexpr int T = 16 * NTB;
+  constexpr int kLds = kTW + 2 * T * kGroup + 2 * T * 4 + 4 * T * 4 + kTBs + T * 4;
+#define LO_ROWS_LAUNCH2(ORD, FA, ST, PCV)                                                                       \
+  do {                                                                                                          \
+    static unsigned long long lds_done = 0; /* per instantiation: one bit per device */                         \
+    const auto kern = &moe_gemm_t128_kernel<FA, ORD, ST, false, PCV, NTB, true>;                                \
+    constexpr int bytes = kLds + (FA ? 2 * kSiluBandN * 2 : 0);                                                 \
+    const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), bytes, &lds_done);                \
+    if (rc_lds) return rc_lds;                                                                                  \
+    hipLaunchKernelGGL(kern, g, dim3(256), bytes, s, a, mbi, gi);                                               \
+  } while (0)
+#define LO_ROWS_LAUNCH(ORD, FA)                                                                                 \
+  do {                                                                                                          \
+    if (stream) LO_ROWS_LAUNCH2(ORD, FA, true, false);                                                          \
+    else LO_ROWS_LAUNCH2(ORD, FA, false, false);                                                                \
+  } while (0)
+  if (a.per_channel) { // one order only: the scales meet in the epilogue
+    if (stream) LO_ROWS_LAUNCH2(kOrdSeparate, false, true, true);
+    else LO_ROWS_LAUNCH2(kOrdSeparate, false, false, true);
+  } else if (fused_act) {
+    LO_ORD_DISPATCH(ord, LO_ROWS_LAUNCH, true);
+  } else {
+    LO_ORD_DISPATCH(ord, LO_ROWS_LAUNCH, false);
+  }
+#undef LO_ROWS_LAUNCH
+#undef LO_ROWS_LAUNCH2
+  return check_launch(a.per_channel ? "moe_gemm_w8a8(rows)" : fused_act ? "moe_gemm1_silu_quant(rows)" : "moe_gemm(rows)");
+}
+
+int launch_gemm_rows(const GemmArgs &a0, bool fused_act, int block_size_m, int flags, int64_t m_blocks, hipStream_t s) {
+  GemmArgs a = a0;
+  a.n_tiles = fused_act ? static_cast<int32_t>(a.N / 2 / kGroup) : static_cast<int32_t>((a.N + 255) / 256);
+  const int64_t experts = a.experts_routed > 0 ? a.experts_routed : 1;
+  // one token block per expert, by and large: the weights have one reader (as in gemm_tile.hip)
+  const bool stream = a.num_valid <= experts * 48;
+  int64_t G = a.num_valid / (experts * block_size_m);
+  G = G < 2 ? 2 : (G > 16 ? 16 : G);
+  const int64_t chunks = (m_blocks + G - 1) / G;
+  const int64_t grid = (chunks + 7) / 8 * (G * a.n_tiles) * 8;
+  LO_REQUIRE(grid < (1ll << 31), LO_EINVAL, "moe_gemm: grid too large");
+  const int ord = scale_order(flags);
+  const dim3 g(static_cast<unsigned>(grid));
+  const int mbi = static_cast<int>(m_blocks), gi = static_cast<int>(G);
+  switch (block_size_m) {
+  case 16: return launch_rows<1>(a, fused_act, ord, stream, g, mbi, gi, s);
+  case 32: return launch_rows<2>(a, fused_act, ord, stream, g, mbi, gi, s);
+  case 64: return launch_rows<4>(a, fused_act, ord, stream, g, mbi, gi, s);
+  default: return launch_rows<8>(a, fused_act, ord, stream, g, mbi, gi, s);
+  }
 }
 
 int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int flags, int64_t m_blocks,

@@ -32,15 +32,14 @@ constexpr int kTileRow = 144;    // LDS row pitch in bytes: 128 + 16 keeps ds_re
 // workgroup per CU; 1 -> 64-token tile, 4 waves, two workgroups per CU that are not
 // synchronised with each other, so one computes while the other waits at its barrier.
 //
-// STREAM (64-token tiles of pre-shuffled weights): an expert's weights are read by one token block,
+// STREAM (64-token tiles): an expert's weights are read by one token block,
 // by and large, and are loaded with the streaming cache policy (first GEMM of the Qwen3-30B-A3B
 // layer at 512 tokens 132 -> 74 us).  With several token blocks per expert the blocks share the
-// weights through L2 and the default policy is the faster one; with row-major weights, where a
-// 128-byte line serves several k-steps of a lane, the hint costs 50 %.
-template <bool FUSED_ACT, int ORD, bool SHUF, int WT, bool STREAM = false>
+// weights through L2 and the default policy is the faster one.
+template <bool FUSED_ACT, int ORD, int WT, bool STREAM = false>
 __global__ __launch_bounds__(256 * WT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
-  static_assert(!STREAM || (SHUF && WT == 1), "streaming policy: 64-token tiles of pre-shuffled weights");
+  static_assert(!STREAM || WT == 1, "streaming policy: 64-token tiles");
   constexpr int kWAux = STREAM ? kCacheStream : kCacheDefault;
   constexpr int kTileM = 64 * WT; // tokens per workgroup
   __shared__ __attribute__((aligned(16))) int8_t sA[2][kTileM * kTileRow];
@@ -124,10 +123,8 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const int64_t nr = wave_active ? nrow[rb] : 0;
-    if constexpr (SHUF) // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
-      woff[rb] = static_cast<int>(nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
-    else
-      woff[rb] = static_cast<int>((nr + r) * K) + c * 64;
+    // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
+    woff[rb] = static_cast<int>(nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
     wsrow[rb] = a.Ws + (static_cast<int64_t>(e) * NB + nr / kGroup) * KB;
   }
 
@@ -176,8 +173,7 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        wreg[b][rb][ks] = SHUF ? bld16<kWAux>(rW, woff[rb], kc * wkstride + ks * 512)
-                               : bld16(rW, woff[rb], kc * kGroup + ks * 16);
+        wreg[b][rb][ks] = bld16<kWAux>(rW, woff[rb], kc * wkstride + ks * 512);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) bsc[b][rb] = wsrow[rb][kc];
   };
@@ -203,10 +199,10 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     for (int tb = 0; tb < 2; ++tb) {
       v4i bf[4];
       // the K bytes of k-step ks must be the ones the weight operand holds for it
-      const int8_t *src = tile + (wt * 64 + tb * 32 + r) * kTileRow + (SHUF ? c * 16 : c * 64);
+      const int8_t *src = tile + (wt * 64 + tb * 32 + r) * kTileRow + c * 16;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        bf[ks] = *reinterpret_cast<const v4i *>(src + (SHUF ? ks * 32 : ks * 16));
+        bf[ks] = *reinterpret_cast<const v4i *>(src + ks * 32);
       const float as = sS[b][wt * 64 + tb * 32 + r];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
@@ -328,7 +324,7 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 }
 
 bool gemm_tile_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
-  if (block_size_m != 128 && block_size_m != 64) return false;
+  if ((block_size_m != 128 && block_size_m != 64) || !a.w_shuffled) return false;
   if (!fused_act && a.N % 64 != 0) return false;
   return true;
 }
@@ -347,27 +343,22 @@ int launch_gemm_tile(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   const int wt = block_size_m / 64;
   const dim3 g(static_cast<unsigned>(grid)), b(256 * wt);
   const int mbi = static_cast<int>(m_blocks);
-#define LO_TILE_LAUNCH2(FA, FS, SH)                                                             \
-  do {                                                                                          \
-    if (wt == 2) hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, SH, 2>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
-    else hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, SH, 1>), g, b, 0, s, a, mbi, static_cast<int>(G));         \
-  } while (0)
   // one token block per expert, by and large (measured up to 48 slots per expert on average: first GEMM
   // of the Qwen3-30B-A3B layer at 768 tokens 135 -> 88 us; at 64 the second GEMM loses more than
   // the first one gains)
-  const bool stream = a.w_shuffled && wt == 1 &&
-                      a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * 48;
+  const bool stream = wt == 1 && a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * 48;
 #define LO_TILE_LAUNCH(FS, FA)                         \
   do {                                                 \
     if (stream)                                        \
-      hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, true, 1, true>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
-    else if (a.w_shuffled) LO_TILE_LAUNCH2(FA, FS, true);   \
-    else LO_TILE_LAUNCH2(FA, FS, false);               \
+      hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 1, true>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
+    else if (wt == 2)                                  \
+      hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 2>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
+    else                                               \
+      hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 1>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
   } while (0)
   if (fused_act) LO_ORD_DISPATCH(ord, LO_TILE_LAUNCH, true);
   else LO_ORD_DISPATCH(ord, LO_TILE_LAUNCH, false);
 #undef LO_TILE_LAUNCH
-#undef LO_TILE_LAUNCH2
   return check_launch(fused_act ? "moe_gemm1_silu_quant(tile)" : "moe_gemm(tile)");
 }
 
