@@ -93,12 +93,11 @@ int lo_version(void);
 const char *lo_last_error(void);
 
 /*
- * Optional one-time set-up for the current device: builds the 128 KB bf16 SiLU table
- * that the fused GEMM epilogue looks activations up in and looks up the address of the
- * built-in scratch of lo_fused_experts_block_int8_noalloc.  The first fused-GEMM call on a
- * device does this by itself (and synchronises the stream once); call lo_init() first
- * when that first call would fall inside a HIP graph capture.  No counterpart in the
- * reference.
+ * Optional one-time set-up for the current device: builds the 128 KB bf16 SiLU table of
+ * lo_act_mul_group_quant and looks up the address of the built-in scratch of
+ * lo_fused_experts_block_int8_noalloc.  (The fused GEMM epilogues compute SiLU and need no
+ * table; GELU and fp16 rows build theirs on their first call, which must not be captured.)
+ * No counterpart in the reference.
  */
 int lo_init(lo_stream_t stream);
 

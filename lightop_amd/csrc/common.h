@@ -134,78 +134,56 @@ template <int DT> __device__ __forceinline__ uint16_t silu_mul(uint16_t g16, uin
   return from_f32<DT>(sg * to_f32<DT>(u16));
 }
 
-// Same with the SiLU taken from the per-device table.
-__device__ __forceinline__ uint16_t silu_mul_tab(const uint16_t *__restrict__ table, uint16_t g16, uint16_t u16) {
-  const float sg = bf16_to_f32(table[g16]);
-  return f32_to_bf16(sg * bf16_to_f32(u16));
-}
-
 // Any gated activation whose T(act(g)) sits in a 64K-entry table: act = T(T(act(g)) * u).
 template <int DT>
 __device__ __forceinline__ uint16_t act_mul_tab(const uint16_t *__restrict__ table, uint16_t g16, uint16_t u16) {
   return from_f32<DT>(to_f32<DT>(table[g16]) * to_f32<DT>(u16));
 }
 
-// bf16(silu(g)) has closed forms outside a narrow band of inputs: for |g| <= 0x3bb5 (about
-// 0.0055) it is bf16(g / 2), for g >= 0x40bf (about 5.97) it is g, for finite g <= 0xc2b2
-// (about -89) it is -0.  The band in between, 1788 patterns per sign, fits in LDS; NaN and
-// -inf go to the full table.  (The bounds come from the full table itself; a test drives
-// every finite bf16 gate through the kernels that use this.)
-constexpr int kSiluBandLo = 0x3bb6, kSiluBandN = 1788; // band = [lo, lo + n) on |g|
-// The band travels global -> registers early (kSiluBandPer values per thread of a 256-thread
-// workgroup) and registers -> LDS before the workgroup's first barrier.
-constexpr int kSiluBandPer = (2 * kSiluBandN + 255) / 256;
-__device__ __forceinline__ void silu_band_load(uint16_t (&regs)[kSiluBandPer], const uint16_t *__restrict__ table, int tid) {
-#pragma unroll
-  for (int j = 0; j < kSiluBandPer; ++j) {
-    int i = tid + 256 * j;
-    i = i < 2 * kSiluBandN ? i : 2 * kSiluBandN - 1;
-    const int sign = i >= kSiluBandN;
-    regs[j] = table[(sign ? 0x8000 : 0) + kSiluBandLo + (i - sign * kSiluBandN)];
-  }
-}
-__device__ __forceinline__ void silu_band_store(uint16_t *band, const uint16_t (&regs)[kSiluBandPer], int tid) {
-#pragma unroll
-  for (int j = 0; j < kSiluBandPer; ++j) {
-    const int i = tid + 256 * j;
-    if (i < 2 * kSiluBandN) band[i] = regs[j];
-  }
-}
-__device__ __forceinline__ uint16_t silu_mul_band(const uint16_t *band, const uint16_t *__restrict__ table,
-                                                  uint16_t g16, uint16_t u16) {
-  const uint32_t mag = g16 & 0x7fffu, neg = g16 >> 15;
-  const uint32_t bi = mag - kSiluBandLo;
-  uint16_t sg16;
-  if (bi < static_cast<uint32_t>(kSiluBandN)) {
-    sg16 = band[bi + neg * kSiluBandN];
-  } else if (mag < static_cast<uint32_t>(kSiluBandLo)) {
-    sg16 = f32_to_bf16(bf16_to_f32(g16) * 0.5f);
-  } else if (mag > 0x7f80u || g16 == 0xff80u) {
-    sg16 = table[g16]; // NaN, -inf
-  } else {
-    sg16 = neg ? static_cast<uint16_t>(0x8000u) : g16;
-  }
-  return f32_to_bf16(bf16_to_f32(sg16) * bf16_to_f32(u16));
+// ---- SiLU of bf16 gates on the transcendental unit ---------------------------------------------------------
+// Two floats rounded to bf16 by one instruction and widened again.
+typedef __bf16 v2bf16 __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void round_pair_bf16(float a, float b, float &ra, float &rb) {
+  const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf16));
+  ra = __uint_as_float(p << 16);
+  rb = __uint_as_float(p & 0xffff0000u);
 }
 
-// The same lookup as straight-line code, for epilogues that push dozens of unrelated values per
-// lane through it: lanes of a wave never agree on an arm, so per-value branches only add
-// exec-mask bookkeeping and keep the LDS reads from being issued back to back.  The three
-// common arms are computed and selected; NaN and -inf gates are NOT handled here: the caller
-// ORs silu_gate_special() over its values and, if any lane of the wave saw one, redoes the
-// values with silu_mul_band().
-__device__ __forceinline__ uint16_t silu_mul_band_common(const uint16_t *band, uint16_t g16, uint16_t u16) {
-  const uint32_t mag = g16 & 0x7fffu, neg = g16 >> 15;
-  const uint32_t bi = mag - kSiluBandLo; // wraps around below the band
-  const bool inside = bi < static_cast<uint32_t>(kSiluBandN);
-  const uint16_t in_band = band[(inside ? bi : 0u) + neg * kSiluBandN];
-  const uint16_t below = f32_to_bf16(bf16_to_f32(g16) * 0.5f);
-  const uint16_t above = neg ? static_cast<uint16_t>(0x8000u) : g16;
-  const uint16_t sg16 = inside ? in_band : (mag < static_cast<uint32_t>(kSiluBandLo) ? below : above);
-  return f32_to_bf16(bf16_to_f32(sg16) * bf16_to_f32(u16));
-}
-__device__ __forceinline__ bool silu_gate_special(uint16_t g16) {
-  return (g16 & 0x7fffu) > 0x7f80u || g16 == 0xff80u; // NaN, -inf
+// act[i] = bf16(bf16(silu(bf16(g[i]))) * bf16(u[i])) as floats, with bf16(silu(g)) bit for bit what silu_mul<LO_BF16>
+// computes: v_exp_f32 and v_rcp_f32 are good to an ulp of fp32, which is enough to round to bf16 correctly for every
+// bf16 gate from kSiluHwMin up, given 1 + 2^-23 for the one in the denominator (silu(5.9375) lies three fp32 ulps below
+// the middle between two bf16 numbers; the constant takes the quotient's error to the right side of it and moves no other
+// gate).  Below, the reciprocal of 1 + exp(-g) is denormal and flushed: a wave that holds such a gate (or -inf) redoes those
+// values the long way.  NaN gates give NaN.  A test drives every bf16 gate through it.
+//
+// 14 vector instructions per value, two of them transcendental, against about 36 for a table in LDS with its selects for
+// the closed forms outside of it (gather, index arithmetic and conversions one by one): whole Qwen3-30B-A3B layer at 8192
+// tokens 626 -> 607 us, at 2400: 264 -> 257, DeepSeek-V3 share at 4096: 558 -> 549.
+constexpr float kSiluHwMin = -87.25f;
+template <int N>
+__device__ __forceinline__ void silu_mul_bf16(const float (&g)[N], const float (&u)[N], float (&act)[N]) {
+  static_assert(N % 2 == 0, "values go in pairs");
+  float gb[N], lowest = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; i += 2) {
+    round_pair_bf16(g[i], g[i + 1], gb[i], gb[i + 1]);
+    lowest = fminf(fminf(gb[i], gb[i + 1]), lowest);
+    float s[2], ub[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float e = __builtin_amdgcn_exp2f(gb[i + j] * -1.44269504088896341f);
+      s[j] = gb[i + j] * __builtin_amdgcn_rcpf(1.00000011920928955078125f + e);
+    }
+    round_pair_bf16(s[0], s[1], s[0], s[1]);
+    round_pair_bf16(u[i], u[i + 1], ub[0], ub[1]);
+    round_pair_bf16(s[0] * ub[0], s[1] * ub[1], act[i], act[i + 1]);
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(lowest < kSiluHwMin) != 0, 0)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (gb[i] < kSiluHwMin) act[i] = bf16_to_f32(silu_mul<LO_BF16>(f32_to_bf16(gb[i]), f32_to_bf16(u[i])));
+  }
 }
 
 // q = (int8) trunc(clamp(v / s, -128, 127))
@@ -225,15 +203,14 @@ __device__ __forceinline__ int quant_one(float v, float s) {
 __device__ __forceinline__ int quant_one_rcp(float v, float s, float y) {
   const float q = v * y;
   const float rem = __builtin_fmaf(-q, s, v);
-  float t = __builtin_fmaf(rem, y, q);
-  t = fmaxf(t, -128.0f);
-  t = fminf(t, 127.0f);
-  return static_cast<int>(t);
+  // one instruction for the two ends; a NaN quotient becomes -128 as in quant_one (v_med3_f32 of a NaN is the minimum)
+  return static_cast<int>(__builtin_amdgcn_fmed3f(__builtin_fmaf(rem, y, q), -128.0f, 127.0f));
 }
 
 __device__ __forceinline__ uint32_t pack4_i8(int a, int b, int c, int d) {
-  return (static_cast<uint32_t>(a) & 0xffu) | ((static_cast<uint32_t>(b) & 0xffu) << 8) |
-         ((static_cast<uint32_t>(c) & 0xffu) << 16) | ((static_cast<uint32_t>(d) & 0xffu) << 24);
+  // byte 0 of each: v_perm_b32 selects 0-3 from its second operand, 4-7 from its first, 0x0c is zero
+  return __builtin_amdgcn_perm(static_cast<uint32_t>(b), static_cast<uint32_t>(a), 0x0c0c0400u) |
+         __builtin_amdgcn_perm(static_cast<uint32_t>(d), static_cast<uint32_t>(c), 0x04000c0cu);
 }
 
 // four elements of one row -> four packed int8; y = 1.0f / s

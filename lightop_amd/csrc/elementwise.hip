@@ -107,10 +107,18 @@ __global__ __launch_bounds__(256) void act_mul_group_quant_kernel(const uint16_t
 // no floor: a zero row gets scale 0 and multiplier 0).  One workgroup per row; a thread keeps
 // up to CH 8-value pieces of the row in registers between the amax pass and the rounding pass,
 // longer rows are read a second time.
-// ACT: 0 plain rows; 1 SiLU-and-mul first (the fused kernel above: no floor), bf16 only, through the
-// band of the SiLU table; 2 a gated activation from its full table first (`silu` being that table),
+// ACT: 0 plain rows; 1 SiLU-and-mul first (the fused kernel above: no floor), bf16 only, computed; 2 a gated activation from its full table first (`silu` being that table),
 // then per_token_quant_int8 with its floor (GELU: the two calls at int8.py:826-838 on the per-channel
-// branch); 3 as 2 without the floor (SiLU for fp16 rows, which have no band).
+// branch); 3 as 2 without the floor (SiLU for fp16 rows).
+__device__ __forceinline__ void silu_mul_bf16_raw(const v8u16 g16, const v8u16 u16, float (&act)[8]) {
+  float g[8], u[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    g[i] = bf16_to_f32(g16[i]);
+    u[i] = bf16_to_f32(u16[i]);
+  }
+  silu_mul_bf16<8>(g, u, act);
+}
 __device__ __forceinline__ int rne_i8(float v) {
   v = fminf(fmaxf(v, -128.0f), 127.0f);
   return static_cast<int>(__builtin_rintf(v)); // v_rndne_f32: ties to even
@@ -122,22 +130,15 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const uint16_t *__restri
                                                         float *__restrict__ s,
                                                         const int32_t *__restrict__ num_local_tokens, int32_t top_k,
                                                         const int32_t *__restrict__ row_ids) {
-  static_assert(ACT != 1 || DT == LO_BF16, "the SiLU band is a bf16 table");
+  static_assert(ACT != 1 || DT == LO_BF16, "SiLU is computed for bf16 rows");
   constexpr bool SILU = ACT == 1, GATED = ACT != 0, FLOOR = ACT == 0 || ACT == 2;
   __shared__ float sRed[4];
-  __shared__ uint16_t sSilu[SILU ? 2 * kSiluBandN : 2];
   const int tid = threadIdx.x;
   if (num_local_tokens) { // rows of padding tokens are left untouched
     const int64_t n = static_cast<int64_t>(num_local_tokens[0]) * top_k;
     rows = n < 0 ? 0 : (n < rows ? n : rows);
   }
   if (static_cast<int64_t>(blockIdx.x) >= rows) return;
-  if constexpr (SILU) {
-    uint16_t band_regs[kSiluBandPer];
-    silu_band_load(band_regs, silu, tid);
-    silu_band_store(sSilu, band_regs, tid);
-    __syncthreads();
-  }
   const int64_t in_stride = GATED ? 2 * C : C; // C = output columns
   const int pieces = static_cast<int>(C / 8);
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
@@ -147,10 +148,11 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const uint16_t *__restri
       const v8u16 a = *reinterpret_cast<const v8u16 *>(xr + p * 8);
       if constexpr (GATED) {
         const v8u16 u = *reinterpret_cast<const v8u16 *>(xr + C + p * 8);
+        if constexpr (SILU) {
+          silu_mul_bf16_raw(a, u, v);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if constexpr (SILU) v[i] = bf16_to_f32(silu_mul_band(sSilu, silu, a[i], u[i]));
-          else v[i] = to_f32<DT>(act_mul_tab<DT>(silu, a[i], u[i]));
+          for (int i = 0; i < 8; ++i) v[i] = to_f32<DT>(act_mul_tab<DT>(silu, a[i], u[i]));
         }
       } else {
 #pragma unroll
@@ -215,21 +217,14 @@ __global__ __launch_bounds__(256) void row_quant_wave_kernel(const uint16_t *__r
                                                              int8_t *__restrict__ q, float *__restrict__ s,
                                                              const int32_t *__restrict__ num_local_tokens,
                                                              int32_t top_k, const int32_t *__restrict__ row_ids) {
-  static_assert(ACT != 1 || DT == LO_BF16, "the SiLU band is a bf16 table");
+  static_assert(ACT != 1 || DT == LO_BF16, "SiLU is computed for bf16 rows");
   constexpr bool SILU = ACT == 1, GATED = ACT != 0, FLOOR = ACT == 0 || ACT == 2;
-  __shared__ uint16_t sSilu[SILU ? 2 * kSiluBandN : 2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (num_local_tokens) {
     const int64_t n = static_cast<int64_t>(num_local_tokens[0]) * top_k;
     rows = n < 0 ? 0 : (n < rows ? n : rows);
   }
   if (static_cast<int64_t>(blockIdx.x) * 4 >= rows) return;
-  if constexpr (SILU) {
-    uint16_t band_regs[kSiluBandPer];
-    silu_band_load(band_regs, silu, tid);
-    silu_band_store(sSilu, band_regs, tid);
-    __syncthreads();
-  }
   const int64_t in_stride = GATED ? 2 * C : C;
   const int pieces = static_cast<int>(C / 8);
   for (int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + wave; row < rows; row += static_cast<int64_t>(gridDim.x) * 4) {
@@ -248,10 +243,11 @@ __global__ __launch_bounds__(256) void row_quant_wave_kernel(const uint16_t *__r
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const bool live = lane + 64 * j < pieces;
+      if constexpr (SILU) silu_mul_bf16_raw(ga[j], up[j], v[j]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        if constexpr (SILU) v[j][i] = bf16_to_f32(silu_mul_band(sSilu, silu, ga[j][i], up[j][i]));
-        else if constexpr (GATED) v[j][i] = to_f32<DT>(act_mul_tab<DT>(silu, ga[j][i], up[j][i]));
+        if constexpr (SILU) {
+        } else if constexpr (GATED) v[j][i] = to_f32<DT>(act_mul_tab<DT>(silu, ga[j][i], up[j][i]));
         else v[j][i] = to_f32<DT>(ga[j][i]);
         amax = fmaxf(amax, live ? fabsf(v[j][i]) : 0.0f);
       }
@@ -475,8 +471,10 @@ int launch_act_mul_row_quant(const void *c1, int dtype, int act, int64_t rows, i
                              const int32_t *num_local_tokens, int32_t top_k, const int32_t *row_ids,
                              hipStream_t stream) {
   const uint16_t *table = nullptr;
-  int rc = act_table(stream, act, dtype, &table);
-  if (rc) return rc;
+  if (act != LO_ACT_SILU || dtype != LO_BF16) { // (SiLU of bf16 rows is computed)
+    const int rc = act_table(stream, act, dtype, &table);
+    if (rc) return rc;
+  }
   if (rows == 0) return LO_OK;
   const uint16_t *x = static_cast<const uint16_t *>(c1);
   if (dtype == LO_F16) {

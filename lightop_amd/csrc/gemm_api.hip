@@ -185,8 +185,6 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
   LO_REQUIRE(block_size_m != 160 || gemm_t128_supports(a, true, 160), LO_ENOTSUP,
              "moe_gemm1_silu_quant: 160-token blocks need int8 weights in the load-time layout "
              "(LO_GEMM_W_PRESHUFFLED) and K <= %d", kGroup * 128);
-  rc = silu_table(static_cast<hipStream_t>(stream), &a.silu);
-  if (rc) return rc;
   const int64_t mblocks = grid_m_blocks(sorted_cap, num_valid, block_size_m);
   LO_REQUIRE(mblocks * a.n_tiles < (1ll << 31), LO_EINVAL, "moe_gemm1_silu_quant: grid too large");
   if (mblocks == 0) return LO_OK;

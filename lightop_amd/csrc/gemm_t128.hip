@@ -42,13 +42,12 @@ constexpr int kTRed = 4 * kT * 4;             // [wave][token] amax exchange of 
 constexpr int kTMaxKB = 128;                  // K blocks whose weight-block scales fit the table below
 constexpr int kTBs = 2 * kTMaxKB * 4;         // [fragment][K block] weight-block scales of the tile
 constexpr int kTIds = kT * 4;                  // the tile's sorted ids, for the epilogues
-constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds + 2 * kSiluBandN * 2;
-// NTB = 10: 160 tokens per workgroup (plain epilogue only: no amax exchange, no SiLU band; int8 block
-// form, or int4 weights with per-channel scales, whose int32 accumulators need no fold registers), for layers
+constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds;
+// NTB = 10: 160 tokens per workgroup (int8 block form, or int4 weights with per-channel scales, whose int32 accumulators need no fold registers), for layers
 // whose experts see a few tokens more than 128: a remainder block is a second pass over the expert's
 // weights, and at that size the weights are what the stage streams.
 constexpr int kT160 = 160;
-constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + kTBs + kT160 * 4;
+constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + kT160 * 4;
 constexpr int kTPitch = 144;                  // staging pitch of the epilogues: 128 + 16
 
 // Wait until all but the newest `N` vector-memory operations of this wave are complete and its
@@ -80,22 +79,13 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   constexpr int T = 16 * NTB;        // tokens per workgroup
   constexpr int AST = T * kGroup;    // token rows of one K block
   constexpr int APW = NTB == 1 ? 1 : NTB / 2;       // 1 KB pieces (eight token rows) of a token stage that a wave copies
-  constexpr int RED = NTB <= 8 ? 4 * T * 4 : 0;
+  constexpr int RED = 4 * T * 4;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   int8_t *const sA = smem + kTW;
   float *const sS = reinterpret_cast<float *>(smem + kTW + 2 * AST);
-  // 160-token tiles have no room for the fused epilogue's amax exchange and SiLU band beside the stages
-  // (two workgroups per compute unit): there every wave copies the band into its own weight stage once its K
-  // loop is done, and its row of the exchange lies behind the band.
-  constexpr bool kLateBand = FUSED_ACT && NTB == 10;
-  static_assert(!kLateBand || 2 * kSiluBandN * 2 + 160 * 4 <= kTWStage, "band and amax row fit a weight stage");
-  auto red_row = [&](int w) __attribute__((always_inline)) { // [token] amax of wave w's 32 columns
-    if constexpr (kLateBand) return reinterpret_cast<float *>(smem + w * kTWStage + 2 * kSiluBandN * 2);
-    else return reinterpret_cast<float *>(smem + kTW + 2 * AST + 2 * T * 4) + w * T;
-  };
+  float *const sRed = reinterpret_cast<float *>(smem + kTW + 2 * AST + 2 * T * 4); // [wave][token] amax of its 32 columns
   float *const sBs = reinterpret_cast<float *>(smem + kTW + 2 * AST + 2 * T * 4 + RED);
   int32_t *const sIds = reinterpret_cast<int32_t *>(smem + kTW + 2 * AST + 2 * T * 4 + RED + kTBs);
-  uint16_t *const sSiluShared = reinterpret_cast<uint16_t *>(smem + kTW + 2 * AST + 2 * T * 4 + RED + kTBs + T * 4);
 
   int mb, nt;
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
@@ -152,9 +142,6 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     }
     return;
   }
-
-  uint16_t band_regs[kSiluBandPer];
-  if constexpr (FUSED_ACT && !kLateBand) silu_band_load(band_regs, a.silu, tid);
 
   // ---- what this wave copies -----------------------------------------------------------------------
   const int NBLK = static_cast<int>(N / 16);
@@ -511,7 +498,6 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   __builtin_amdgcn_sched_barrier(0);
   if (tid < T) sS[tid] = s_now;
   sBs[tid] = bs_mine;
-  if constexpr (FUSED_ACT && !kLateBand) silu_band_store(sSiluShared, band_regs, tid);
   wait_copies<0>();
   read_w();
 
@@ -626,24 +612,6 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       __builtin_amdgcn_wave_barrier();
     }
   } else {
-    const uint16_t *sSilu = sSiluShared;
-    if constexpr (kLateBand) {
-      // the band of the SiLU table (two runs of kSiluBandN entries, one per sign of the gate) straight into this
-      // wave's own weight stage, 256 bytes per copy
-      const brsrc rT = make_rsrc(a.silu, 65536 * 2);
-      constexpr int kRun = kSiluBandN * 2; // bytes per sign
-#pragma unroll
-      for (int sgn = 0; sgn < 2; ++sgn)
-#pragma unroll
-        for (int j = 0; j < (kRun + 255) / 256; ++j) {
-          int off = j * 256 + lane * 4;
-          off = off < kRun ? off : kRun - 4; // the last copy's surplus lanes repeat the run's last word
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rT, sWw + sgn * kRun + j * 256, 4,
-                                                   (sgn * 0x8000 + kSiluBandLo) * 2 + off, 0, 0, 0);
-        }
-      wait_copies<0>();
-      sSilu = reinterpret_cast<const uint16_t *>(sWw);
-    }
     // acc[h][tb][0] = gate, acc[h][tb][1] = up for activation columns nt*128 + wave*32 + 16h + 4q + i
     float actf[NTB][2][4];
     if (a.mul_routed) { // router weight on the first GEMM's output: rare, kept out of the main pass
@@ -659,29 +627,12 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
             for (int i = 0; i < 4; ++i) acc[h][tb][rf][i] = acc[h][tb][rf][i] * wgt;
       }
     }
-    // Token fragments are in use in pairs (nst is a multiple of four stages).  A pair shares one
-    // wave-uniform branch, so the LDS lookups of its two fragments are in flight together.
+    // Token fragments are in use in pairs (nst is a multiple of four stages): a pair shares one wave-uniform branch.
 #pragma unroll
     for (int tb = 0; tb < NTB; ++tb) {
       if (2 * (tb & ~1) >= nst) continue; // the same condition for both fragments of a pair
-      uint16_t g16[2][4], u16[2][4];
-      bool special = false;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          g16[h][i] = f32_to_bf16(acc[h][tb][0][i]);
-          u16[h][i] = f32_to_bf16(acc[h][tb][1][i]);
-          special |= silu_gate_special(g16[h][i]);
-          actf[tb][h][i] = bf16_to_f32(silu_mul_band_common(sSilu, g16[h][i], u16[h][i]));
-        }
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(special) != 0, 0)) { // a NaN or -inf gate in the wave
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            actf[tb][h][i] = bf16_to_f32(silu_mul_band(sSilu, a.silu, g16[h][i], u16[h][i]));
-      }
+      for (int h = 0; h < 2; ++h) silu_mul_bf16<4>(acc[h][tb][0], acc[h][tb][1], actf[tb][h]);
       float amax = 0.0f;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -689,7 +640,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
         for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(actf[tb][h][i]));
       amax = fmaxf(amax, __shfl_xor(amax, 16));
       amax = fmaxf(amax, __shfl_xor(amax, 32));
-      if (q == 0) red_row(wave)[tb * 16 + r] = amax;
+      if (q == 0) sRed[wave * T + tb * 16 + r] = amax;
     }
     __syncthreads(); // also: every wave is done with the token stages
     const int64_t G = I / kGroup;
@@ -701,7 +652,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
 #pragma unroll
     for (int tb = 0; tb < NTB; ++tb) {
       const int t = tb * 16 + r;
-      float amax = fmaxf(fmaxf(red_row(0)[t], red_row(1)[t]), fmaxf(red_row(2)[t], red_row(3)[t]));
+      float amax = fmaxf(fmaxf(sRed[t], sRed[T + t]), fmaxf(sRed[2 * T + t], sRed[3 * T + t]));
       amax = fmaxf(amax, 1e-10f);
       sc_all[tb] = amax / 127.0f;
       rsc_all[tb] = 1.0f / sc_all[tb];
@@ -775,10 +726,9 @@ static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, 
   do {                                                                                                          \
     static unsigned long long lds_done = 0; /* per instantiation: one bit per device */                         \
     const auto kern = &moe_gemm_t128_kernel<FA, ORD, ST, false, PCV, NTB, true>;                                \
-    constexpr int bytes = kLds + (FA ? 2 * kSiluBandN * 2 : 0);                                                 \
-    const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), bytes, &lds_done);                \
+    const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), kLds, &lds_done);                 \
     if (rc_lds) return rc_lds;                                                                                  \
-    hipLaunchKernelGGL(kern, g, dim3(256), bytes, s, a, mbi, gi);                                               \
+    hipLaunchKernelGGL(kern, g, dim3(256), kLds, s, a, mbi, gi);                                                \
   } while (0)
 #define LO_ROWS_LAUNCH(ORD, FA)                                                                                 \
   do {                                                                                                          \

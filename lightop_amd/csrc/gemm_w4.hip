@@ -41,7 +41,6 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   __shared__ __attribute__((aligned(16))) int8_t sA[2][kTileM * kW4Row];
   __shared__ float sS[2][kTileM];
   __shared__ float sRed[4][kTileM];
-  __shared__ uint16_t sSilu[FUSED_ACT ? 2 * kSiluBandN : 2];
   extern __shared__ __attribute__((aligned(16))) float sRowScale[]; // [K block][256 rows], already / 16
 
   int mb, nt;
@@ -89,9 +88,6 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     }
     return;
   }
-
-  uint16_t band_regs[kSiluBandPer];
-  if constexpr (FUSED_ACT) silu_band_load(band_regs, a.silu, tid);
 
   // cooperative gather role: thread -> (token, 32-byte quarter of the 128-byte K block)
   const int lt = tid >> 2, lq = tid & 3;
@@ -252,7 +248,6 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   __builtin_amdgcn_sched_barrier(0); // the first K block's requests go out ahead of the scales'
   copy_row_scales();
   store_act(B0{}, true);
-  if constexpr (FUSED_ACT) silu_band_store(sSilu, band_regs, tid);
   __syncthreads();
   for (int kb = 0; kb < KB; kb += 2) {
     load_act(B0{}, kb + 2);            // needed in two iterations
@@ -314,18 +309,17 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if (a.mul_routed && valid[tf]) w = a.topk_w[f[tf]];
       float amax = 0.0f;
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
+      for (int g = 0; g < 2; ++g) {
+        float gv[4], uv[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float gv = acc[g][tf][i], uv = acc[2 + g][tf][i];
-          if (a.mul_routed) {
-            gv = gv * w;
-            uv = uv * w;
-          }
-          const uint16_t act16 = silu_mul_band(sSilu, a.silu, f32_to_bf16(gv), f32_to_bf16(uv));
-          actf[tf][g][i] = bf16_to_f32(act16);
-          amax = fmaxf(amax, fabsf(actf[tf][g][i]));
+        for (int i = 0; i < 4; ++i) { // w = 1 leaves every value as it is
+          gv[i] = acc[g][tf][i] * w;
+          uv[i] = acc[2 + g][tf][i] * w;
         }
+        silu_mul_bf16<4>(gv, uv, actf[tf][g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(actf[tf][g][i]));
+      }
       amax = fmaxf(amax, __shfl_xor(amax, 16));
       amax = fmaxf(amax, __shfl_xor(amax, 32));
       if (q == 0) sRed[wr][tf * 16 + r] = amax;

@@ -405,17 +405,15 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
       float w = 1.0f;
       if (a.mul_routed && valid[j]) w = a.topk_w[f[j]];
       float amax = 0.0f;
+      float g[4], u[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float g = acc[0][j][i], u = acc[NW - 1][j][i];
-        if (a.mul_routed) {
-          g = g * w;
-          u = u * w;
-        }
-        const uint16_t act16 = silu_mul_tab(a.silu, f32_to_bf16(g), f32_to_bf16(u));
-        actf[j][i] = bf16_to_f32(act16);
-        amax = fmaxf(amax, fabsf(actf[j][i]));
+      for (int i = 0; i < 4; ++i) { // w = 1 leaves every value as it is
+        g[i] = acc[0][j][i] * w;
+        u[i] = acc[NW - 1][j][i] * w;
       }
+      silu_mul_bf16<4>(g, u, actf[j]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(actf[j][i]));
       amax = fmaxf(amax, __shfl_xor(amax, 16));
       amax = fmaxf(amax, __shfl_xor(amax, 32));
       if (c == 0) red[j][wave][r] = amax;
