@@ -296,7 +296,7 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
   a.num_valid = M * top_k;
   a.E = E_local > 0 ? E_local : num_experts;
   a.experts_routed = num_experts;
-  a.top_k = top_k;
+  set_top_k(a, top_k);
   a.w_shuffled = pre ? 1 : 0;
   a.w4 = (flags & LO_GEMM_W4) ? 1 : 0;
   a.per_channel = form == LO_FORM_CHANNEL ? 1 : 0;

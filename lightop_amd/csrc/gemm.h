@@ -30,6 +30,8 @@ struct GemmArgs {
   int64_t N;             // weight rows per expert (2I for the fused first GEMM)
   int64_t K;
   int32_t top_k;
+  uint32_t row_mul;      // slot -> token row without a division: __umulhi(2 * slot, row_mul) >> row_shift (set_top_k)
+  int32_t row_shift;
   int32_t n_tiles;       // workgroups along N
   int32_t E;             // experts held by W
   int32_t experts_routed; // experts the routing spreads the slots over (estimate, for tile order)
@@ -41,6 +43,22 @@ struct GemmArgs {
   int32_t out_f16;       // C holds IEEE half instead of bf16 (plain epilogues only)
   int32_t out_f32;       // C holds the fp32 sums themselves (block form, weight-streaming kernel only)
 };
+
+// Division of a slot id below 2^31 by top_k as a multiplication: with L = ceil(log2 d) and m = floor(2^(31+L) / d) + 1,
+// floor(n * m / 2^(31+L)) is the quotient for every n < 2^31 (m overshoots 2^(31+L) / d by less than 2^-31 of it), and m
+// fits 32 bits.  A 32-bit division is some twenty dependent instructions in front of a tile's first copies.
+inline void set_top_k(GemmArgs &a, int32_t d) {
+  int L = 0;
+  while ((1ll << L) < d) ++L;
+  a.top_k = d;
+  a.row_mul = static_cast<uint32_t>((1ull << (31 + L)) / static_cast<uint64_t>(d) + 1);
+  a.row_shift = L;
+}
+// Token row of a slot id of the sorted list (padding and ids out of range: row 0, whose values are never used).
+__device__ __forceinline__ int token_row(const GemmArgs &a, int64_t slot) {
+  const uint32_t row = __umulhi(2u * static_cast<uint32_t>(slot), a.row_mul) >> a.row_shift;
+  return slot < a.num_valid ? static_cast<int>(row) : 0;
+}
 
 // The 16-bit form a plain epilogue stores: bf16, or IEEE half when the caller's activations are fp16.
 // `body(cvt)` is run with the conversion of the output type; the choice is one wave-uniform branch

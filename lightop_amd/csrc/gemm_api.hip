@@ -129,7 +129,7 @@ extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const in
   GemmArgs a{};
   a.A = A; a.As = As; a.W = W; a.Ws = Ws; a.C = static_cast<uint16_t *>(C);
   a.topk_w = topk_w; a.sorted = sorted_ids; a.expert_ids = expert_ids; a.ntpp = num_tokens_post_pad;
-  a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows; a.num_valid = num_valid; a.N = N; a.K = K; a.top_k = top_k; a.mul_routed = mul_routed ? 1 : 0;
+  a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows; a.num_valid = num_valid; a.N = N; a.K = K; set_top_k(a, top_k); a.mul_routed = mul_routed ? 1 : 0;
   a.w_shuffled = (flags & LO_GEMM_W_PRESHUFFLED) ? 1 : 0;
   a.skip_nonlocal = (flags & LO_GEMM_SKIP_NONLOCAL) ? 1 : 0;
   a.w4 = (flags & LO_GEMM_W4) ? 1 : 0;
@@ -174,7 +174,7 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
   GemmArgs a{};
   a.A = A; a.As = As; a.W = W; a.Ws = Ws; a.A2q = A2q; a.A2s = A2s;
   a.topk_w = topk_w; a.sorted = sorted_ids; a.expert_ids = expert_ids; a.ntpp = num_tokens_post_pad;
-  a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows; a.num_valid = num_valid; a.N = 2 * I; a.K = K; a.top_k = top_k; a.mul_routed = mul_routed ? 1 : 0;
+  a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows; a.num_valid = num_valid; a.N = 2 * I; a.K = K; set_top_k(a, top_k); a.mul_routed = mul_routed ? 1 : 0;
   a.w_shuffled = (flags & LO_GEMM_W_PRESHUFFLED) ? 1 : 0;
   a.skip_nonlocal = (flags & LO_GEMM_SKIP_NONLOCAL) ? 1 : 0;
   a.w4 = (flags & LO_GEMM_W4) ? 1 : 0;
@@ -222,7 +222,7 @@ extern "C" int lo_moe_gemm_w8a8(const int8_t *A, const float *As, const int8_t *
   a.A = A; a.As = As; a.W = W; a.Ws = Ws; a.C = static_cast<uint16_t *>(C);
   a.topk_w = topk_w; a.sorted = sorted_ids; a.expert_ids = expert_ids; a.ntpp = num_tokens_post_pad;
   a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows;
-  a.num_valid = num_valid; a.N = N; a.K = K; a.top_k = top_k; a.mul_routed = mul_routed ? 1 : 0;
+  a.num_valid = num_valid; a.N = N; a.K = K; set_top_k(a, top_k); a.mul_routed = mul_routed ? 1 : 0;
   a.w_shuffled = (flags & LO_GEMM_W_PRESHUFFLED) ? 1 : 0;
   a.skip_nonlocal = (flags & LO_GEMM_SKIP_NONLOCAL) ? 1 : 0;
   a.per_channel = 1;

@@ -87,7 +87,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   {
     const int lt = tid >> 2, lq = tid & 3; // thread -> (token, every fourth 16-byte piece)
     const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
-    const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
+    const int64_t lrow = token_row(a, lf);
     const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
     const int aoff = static_cast<int>(lrow * K) + lq * 16;
     int8_t *dst = sA + lt * pitch + lq * 16;
@@ -102,7 +102,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     }
     const int st = tid & 63;
     const int64_t sf = a.sorted[static_cast<int64_t>(mb) * kTileM + st];
-    const int64_t srow = (sf < a.num_valid) ? sf / a.top_k : 0;
+    const int64_t srow = token_row(a, sf);
     for (int kb = tid >> 6; kb < KB; kb += 4) sS[kb * kTileM + st] = a.As[srow * KB + kb];
   }
 

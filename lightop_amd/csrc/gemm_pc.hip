@@ -76,7 +76,7 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
   // cooperative gather role: thread -> (token, run of kPieces 16-byte pieces of the 128-byte K block)
   const int lt = tid / kThrPerTok, lq = tid % kThrPerTok;
   const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
-  const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
+  const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const int aoff = static_cast<int>(lrow * K) + lq * (16 * kPieces);
   int8_t *const sdst0 = &sA[0][lt * kPcRow + lq * (16 * kPieces)];
@@ -179,7 +179,7 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
   for (int tb = 0; tb < TB; ++tb) {
     float ts = 0.0f;
     if (valid[tb]) {
-      ts = a.As[f[tb] / a.top_k];
+      ts = a.As[token_row(a, f[tb])];
       if (a.mul_routed) ts = a.topk_w[f[tb]] * ts;
     }
     v4u16 o[2][4];

@@ -201,7 +201,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   for (int j = 0; j < APW; ++j) {
     const int t = (cw * APW + j) * 8 + (lane >> 3);
     const int64_t lf = kEarlyIds ? lf_copy[j] : sorted[t];
-    const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
+    const int64_t lrow = token_row(a, lf);
     const int piece = (lane & 7) ^ (t & 7); // slot lane & 7 of row t holds piece slot ^ (t & 7)
     avoff[j] = static_cast<int>(lrow * K) + piece * 16;
   }
@@ -228,7 +228,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
     const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
-    const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
+    const int64_t lrow = token_row(a, lf);
     asoff = static_cast<int>(lrow * (PC ? 1 : KB) * 4);
     // The epilogues take the ids from LDS: a global load in each of their exec-masked blocks is a
     // full memory round trip that nothing overlaps.
@@ -563,7 +563,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
 #pragma unroll
       for (int tb = 0; tb < NTB; ++tb) {
         const int64_t ft = sIds[tb * 16 + r];
-        pas[tb] = bld_f32(rAs, static_cast<int>((ft < a.num_valid ? ft / a.top_k : 0) * 4), 0);
+        pas[tb] = bld_f32(rAs, static_cast<int>(token_row(a, ft) * 4), 0);
       }
     }
 #pragma unroll

@@ -102,7 +102,7 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // cooperative gather role: thread -> (token, 32-byte quarter of the 128-byte K block)
   const int lt = tid >> 2, lq = tid & 3;
   const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
-  const int64_t lrow = (lf < a.num_valid) ? lf / a.top_k : 0;
+  const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * KB * 4));
   const int aoff = static_cast<int>(lrow * K) + lq * 32;

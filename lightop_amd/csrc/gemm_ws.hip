@@ -87,7 +87,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   for (int j = 0; j < TM; ++j) {
     f[j] = a.sorted[static_cast<int64_t>(mb) * BM + j * 16 + r];
     valid[j] = f[j] < a.num_valid;
-    const int64_t row = valid[j] ? f[j] / a.top_k : 0;
+    const int64_t row = token_row(a, f[j]);
     aoff[j] = static_cast<int>(row * K) + c * 16;
     asoff[j] = static_cast<int>(row * (PC ? 1 : KB) * 4);
   }
