@@ -1,6 +1,5 @@
 // Host side of the C ABI: error reporting, the gfx950 tile table and the whole-path
 // entry point that chains the stage kernels on one stream.
-#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -213,9 +212,9 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   }
   if (per_expert <= 12.0) return 16;
   if (per_expert <= 24.0) return 32;
-  // Row-major block-form weights, larger experts: 128-token tiles from 48 slots per expert on (64 / 128: Qwen3-235B-A22B-
-  // shaped layer at 1000 tokens 613 / 579 us, at 4096: 1330 / 1170; DeepSeek-V3 share at 4096: 540 / 510).
-  return H >= 4096 && per_expert > 48.0 && H / kGroup <= 128 && I / kGroup <= 128 ? 128 : 64;
+  // Row-major block-form weights: 64-token tiles, three workgroups per CU (64 / 128, us: Qwen3-235B-A22B-shaped layer at
+  // 1000 tokens 575 / 576, at 4096: 1161 / 1163; DeepSeek-V3 share at 4096: 505 / 516; Qwen3-30B-A3B at 8192: 653 / 639).
+  return 64;
 }
 
 // What the block-form whole-path call (int8 weights, or int4 weights with K-group scales) does with a
@@ -235,7 +234,7 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
   const bool block_size_m_auto = block_size_m == 0;
   if (block_size_m == 0 && dtype == LO_F32) // fp32 rows go through the weight-streaming kernel at every size
-    block_size_m = std::min(pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false), 64);
+    block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false);
   if (block_size_m == 0)
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false,
                                 !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true));

@@ -30,6 +30,12 @@
 
 #include "gemm.h"
 
+#ifndef LO_EARLY10
+#define LO_EARLY10 20
+#endif
+#ifndef LO_EARLY
+#define LO_EARLY 12
+#endif
 namespace lo {
 
 constexpr int kT = 128;                       // tokens per workgroup
@@ -68,7 +74,7 @@ __device__ __forceinline__ void wait_copies_barrier() {
 // per weight row, both applied in the epilogue, so the int32 sums run over the whole K inside the
 // MFMA accumulators and the K loop has no scale arithmetic at all.
 template <bool FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8, bool ROWS = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 4 : NTB == 2 ? 3 : 2, NTB == 1 ? 4 : NTB == 2 ? 3 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 4 : NTB <= 4 ? 3 : 2, NTB == 1 ? 4 : NTB <= 4 ? 3 : 2)))
 void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   static_assert(!PC || (!FUSED_ACT && ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
                 "per-channel scales: plain GEMM, int4 weights, 160-token tiles of int8 weights or row-major ones");
@@ -206,10 +212,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     avoff[j] = static_cast<int>(lrow * K) + piece * 16;
   }
   // The alignment puts a block's valid tokens first, so a block of 128 is on average half a block
-  // of padding per expert: token fragments past the last valid token are skipped, in steps of
-  // 32 tokens (taken from the position of the last valid token, not from their number, so that
+  // of padding per expert: token fragments past the last valid token are skipped (taken from the position of the last valid token, not from their number, so that
   // a caller's own sorted ids with gaps are still computed in full).
-  int nst; // pipeline stages per K block: four per 32 tokens in use
+  int nst; // pipeline stages per K block: two per 16 tokens in use
   {
     if constexpr (!kEarlyIds) {
       lf_v0 = sorted[lane];
@@ -223,7 +228,8 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       const uint64_t v2 = __builtin_amdgcn_ballot_w64(lane < 32 && lf_v2 < a.num_valid);
       if (v2) last = 191 - __builtin_clzll(v2);
     }
-    nst = __builtin_amdgcn_readfirstlane(4 * ((last >> 5) + 1)); // the K loop comes in variants of 2, 4, 6, 8 (, 10) fragments
+    nst = __builtin_amdgcn_readfirstlane(2 * ((last >> 4) + 1)); // the K loop comes in variants by the number of fragments
+    if (NTB == 10 && a.coarse_fill && nst > 8 && nst < 16) nst = 16;
   }
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
@@ -363,14 +369,16 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // by then every copy for the next K block has had eight stages to land and nobody reads this K
   // block's token stage or scales any more, so the next block's first operands are read from LDS
   // under the last two stages and no wave stands waiting for LDS right after a barrier.
+  // (From twelve stages on, that is; with ten fragments of accumulators only the full variant, the others would spill.)
+  constexpr int kEarlyFrom = NTB == 10 && !PC ? 20 : 12;
   float s_pending;   // token scales on their way from global memory to sS
   v4i bf_first[2];   // first token fragment of the next K block
   float as_first = 0.0f;
   auto kblock = [&](auto NST, int kb) __attribute__((always_inline)) {
     constexpr int nst_c = decltype(NST)::value; // stages of this variant: 4, 8, 12, 16 (or 20)
     constexpr int kFull = 2 * NTB;              // stages of a full tile
-    constexpr int kE0 = kFull - 2, kE1 = kFull - 1;
-    constexpr bool kEarly = nst_c == kFull && !W4 && NTB >= 8;
+    constexpr int kE0 = nst_c - 2, kE1 = nst_c - 1;
+    constexpr bool kEarly = nst_c >= kEarlyFrom && !W4 && NTB >= 8;
     const int8_t *ta = sA + (kb & 1) * AST;
     const float *ts = sS + (kb & 1) * T;
     v4i bf[2][2];
@@ -502,7 +510,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   read_w();
 
   auto k_loop = [&](auto NST) __attribute__((always_inline)) {
-    if constexpr (decltype(NST)::value == 2 * NTB && !W4 && NTB >= 8) {
+    if constexpr (decltype(NST)::value >= kEarlyFrom && !W4 && NTB >= 8) {
       wait_copies_barrier<0>(); // K block 0 is complete in LDS
       if (tid < T) sS[T + tid] = 1 < KB ? s_pending : 0.0f;
       s_pending = load_scale(2);
@@ -525,25 +533,39 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     }
   };
   // one K loop per number of token fragments that hold valid tokens (wave-uniform choice)
-  if constexpr (NTB == 10) {
-    // three variants only (a block this size is chosen where experts fill it; a fourth one made the
-    // kernel spill): a tile in between runs the next larger one, whose surplus fragments compute on
-    // padding rows and are not stored
-    if (nst > 16) k_loop(std::integral_constant<int, 20>{});
-    else if (nst > 8) k_loop(std::integral_constant<int, 16>{});
+  // in steps of 16 tokens where the registers allow it: a 96-token block costs three quarters of a full one
+  if constexpr (NTB == 10 && PC) {
+    if (nst > 18) k_loop(std::integral_constant<int, 20>{});
+    else if (nst > 16) k_loop(std::integral_constant<int, 18>{});
+    else if (nst > 14) k_loop(std::integral_constant<int, 16>{});
+    else if (nst > 12) k_loop(std::integral_constant<int, 14>{});
+    else if (nst > 10) k_loop(std::integral_constant<int, 12>{});
+    else if (nst > 8) k_loop(std::integral_constant<int, 10>{});
     else k_loop(std::integral_constant<int, 8>{});
-  } else if constexpr (NTB == 1) {
-    k_loop(std::integral_constant<int, 2>{});
-  } else if constexpr (NTB == 2) {
-    k_loop(std::integral_constant<int, 4>{});
-  } else if constexpr (NTB == 4) {
-    if (nst > 4) k_loop(std::integral_constant<int, 8>{});
-    else k_loop(std::integral_constant<int, 4>{});
-  } else {
+  } else if constexpr (NTB == 10) {
+    if (nst > 16) k_loop(std::integral_constant<int, 20>{});
+    else if (nst > 12) k_loop(std::integral_constant<int, 16>{});
+    else if (nst > 8) k_loop(std::integral_constant<int, 12>{});
+    else k_loop(std::integral_constant<int, 8>{});
+  } else if constexpr (NTB == 8 && W4 && !PC) {
     if (nst > 12) k_loop(std::integral_constant<int, 16>{});
     else if (nst > 8) k_loop(std::integral_constant<int, 12>{});
     else if (nst > 4) k_loop(std::integral_constant<int, 8>{});
     else k_loop(std::integral_constant<int, 4>{});
+  } else if constexpr (NTB == 8) {
+    if (nst > 14) k_loop(std::integral_constant<int, 16>{});
+    else if (nst > 12) k_loop(std::integral_constant<int, 14>{});
+    else if (nst > 10) k_loop(std::integral_constant<int, 12>{});
+    else if (nst > 8) k_loop(std::integral_constant<int, 10>{});
+    else if (nst > 6) k_loop(std::integral_constant<int, 8>{});
+    else if (nst > 4) k_loop(std::integral_constant<int, 6>{});
+    else k_loop(std::integral_constant<int, 4>{});
+  } else if constexpr (NTB == 4) {
+    if (nst > 6) k_loop(std::integral_constant<int, 8>{});
+    else if (nst > 4) k_loop(std::integral_constant<int, 6>{});
+    else k_loop(std::integral_constant<int, 4>{});
+  } else {
+    k_loop(std::integral_constant<int, 2 * NTB>{});
   }
   wait_copies<0>(); // no copy may still be writing LDS when the epilogue reuses it or the wave ends
   if constexpr (!FUSED_ACT) {
@@ -627,7 +649,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
             for (int i = 0; i < 4; ++i) acc[h][tb][rf][i] = acc[h][tb][rf][i] * wgt;
       }
     }
-    // Token fragments are in use in pairs (nst is a multiple of four stages): a pair shares one wave-uniform branch.
+    // Token fragments go in pairs that share one wave-uniform branch (of the last pair's second one every value may be zero).
 #pragma unroll
     for (int tb = 0; tb < NTB; ++tb) {
       if (2 * (tb & ~1) >= nst) continue; // the same condition for both fragments of a pair
@@ -711,7 +733,9 @@ bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
 // 630; Qwen3-235B-A22B-shaped layer at 200 tokens 676 / 457; DeepSeek-V3 share at 64 tokens 302 / 213 - within a few
 // percent of the load-time layout.
 //
-// Tiles: 16, 32 or 64 tokens (four, three, two workgroups per compute unit) as the alignment blocks are.
+// Tiles: 16, 32, 64 or 128 tokens as the alignment blocks are, with four, three, three and two workgroups per compute unit
+// (64 tokens at 167 registers: three instead of two take the layer at 8192 tokens from 706 to 653 us, the DeepSeek-V3 share
+// at 4096 from 543 to 505).
 bool gemm_rows_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   if (a.w_shuffled || a.w4 || a.out_f32) return false;
   if (block_size_m != 16 && block_size_m != 32 && block_size_m != 64 && block_size_m != 128) return false;
@@ -809,6 +833,15 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     }                                                                                                           \
   } while (0)
   if (block_size_m == kT160) {
+    const int64_t experts = a.experts_routed > 0 ? a.experts_routed : 1;
+    // Tiles between one and two (two and three, ...) rounds of the 512 resident workgroups: if they take different times,
+    // the compute units that finish first take both workgroups of the last, partial round and the rest none.  Kept alike
+    // they finish together and the partial round spreads one workgroup to a compute unit: 1531 tokens of the
+    // Qwen3-30B-A3B layer (768 tiles) 194 us with the 96-token variant among them, 186 without.  In whole rounds the variant
+    // is worth what it leaves out (DeepSeek-V3 share, one round: 2600 tokens 366 -> 356 us, 3000: 385 -> 376).
+    const double rounds = static_cast<double>(a.E) * ((a.num_valid / experts + kT160 - 1) / kT160) * a.n_tiles / 512.0;
+    const double part = rounds - static_cast<int64_t>(rounds);
+    a.coarse_fill = rounds < 4.0 && part > 0.25 && part < 0.75;
     // chosen where an expert's tokens fill one block, so a weight byte has one reader: streaming hint
 #define LO_T160_LAUNCH(FS, FA)                                                                                  \
   do {                                                                                                          \
