@@ -251,7 +251,7 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
   plan->bs160 = bs160;
   // GELU and fp16 / fp32 activations have no fused epilogue
   plan->unfused = !fused_ok;
-  plan->try_decode = block_size_m_auto && pre && !plan->unfused && !(flags & LO_FUSED_NO_DECODE_PATH);
+  plan->try_decode = block_size_m_auto && pre && dtype != LO_F32 && !(flags & LO_FUSED_NO_DECODE_PATH);
   return LO_OK;
 }
 
@@ -285,9 +285,10 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
     flags = plan.flags;
     bm = plan.block_size_m;
     fused = !plan.unfused;
-    decode = plan.try_decode && M > 0 &&
-             decode_path_applies(M, top_k, H, I, num_experts, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0,
-                                 (flags & LO_GEMM_W4) != 0);
+    // (fp16 rows and GELU: the query describes the staged path)
+    decode = plan.try_decode && fused && M > 0 &&
+             decode_path_applies(M, top_k, H, I, E_local > 0 ? E_local : num_experts, num_experts,
+                                 (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, (flags & LO_GEMM_W4) != 0, false, false);
   }
   const bool pre = (flags & LO_GEMM_W_PRESHUFFLED) != 0;
   // the argument blocks the stage entry points would build for this problem
@@ -404,10 +405,9 @@ extern "C" int lo_fused_experts_block_int8(
   const bool unfused = plan.unfused;
   if (plan.try_decode) {
     // (cache3 is the front of the caller's cache13: the path keeps its bf16 activations [S, I] there)
-    const int rc2 = launch_decode_path(x, M, H, I, E, num_experts, top_k, w1, w1s, w2, w2s, topk_w, topk_ids, ids_dtype,
-                                       expert_map, apply_router_weight_on_input, routed_scaling_factor, shared_output,
-                                       cache3, out, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, (flags & LO_GEMM_W4) != 0,
-                                       flags, static_cast<hipStream_t>(stream));
+    const DecProblem d{x, dtype, M, H, I, E, num_experts, top_k, w1, w1s, w2, w2s, topk_w, topk_ids, ids_dtype, expert_map,
+                       apply_router_weight_on_input, routed_scaling_factor, shared_output, cache3, out, false};
+    const int rc2 = launch_decode_path(d, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, flags, static_cast<hipStream_t>(stream));
     if (rc2 != LO_ENOTSUP) return rc2;
   }
 
@@ -476,6 +476,9 @@ static int fused_experts_channel(
   LO_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, LO_EINVAL,
              "fused_experts(channel): workspace must be 256-byte aligned");
   if (M == 0) return LO_OK;
+  // a few tokens, weights in the load-time layout, rows not quantised by the caller: two launches
+  const bool try_decode = block_size_m == 0 && x && (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) &&
+                          !(flags & LO_FUSED_NO_DECODE_PATH);
   if (block_size_m == 0)
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_CHANNEL, true, (flags & LO_GEMM_W4) != 0,
                                 (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) && H / kGroup <= 128 &&
@@ -503,6 +506,12 @@ static int fused_experts_channel(
   uint8_t *mask = expert_map ? reinterpret_cast<uint8_t *>(ws + L.off[7]) : nullptr;
   const int64_t S = M * top_k;
 
+  if (try_decode) {
+    const DecProblem d{x, dtype, M, H, I, E, num_experts, top_k, w1, w1s, w2, w2s, topk_w, topk_ids, ids_dtype, expert_map,
+                       apply_router_weight_on_input, routed_scaling_factor, shared_output, cache13, out, true};
+    const int rc2 = launch_decode_path(d, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, flags, static_cast<hipStream_t>(stream));
+    if (rc2 != LO_ENOTSUP) return rc2;
+  }
   int rc = LO_OK;
   if (!x_q)
     rc = lo_per_token_quant_int8(x, dtype, M, H, reinterpret_cast<int8_t *>(ws + L.off[0]),

@@ -207,6 +207,12 @@ __device__ __forceinline__ int quant_one_rcp(float v, float s, float y) {
   return static_cast<int>(__builtin_amdgcn_fmed3f(__builtin_fmaf(rem, y, q), -128.0f, 127.0f));
 }
 
+// The per-token rule's rounding: to nearest, ties to even.
+__device__ __forceinline__ int rne_i8(float v) {
+  v = fminf(fmaxf(v, -128.0f), 127.0f);
+  return static_cast<int>(__builtin_rintf(v)); // v_rndne_f32
+}
+
 __device__ __forceinline__ uint32_t pack4_i8(int a, int b, int c, int d) {
   // byte 0 of each: v_perm_b32 selects 0-3 from its second operand, 4-7 from its first, 0x0c is zero
   return __builtin_amdgcn_perm(static_cast<uint32_t>(b), static_cast<uint32_t>(a), 0x0c0c0400u) |

@@ -119,10 +119,6 @@ __device__ __forceinline__ void silu_mul_bf16_raw(const v8u16 g16, const v8u16 u
   }
   silu_mul_bf16<8>(g, u, act);
 }
-__device__ __forceinline__ int rne_i8(float v) {
-  v = fminf(fmaxf(v, -128.0f), 127.0f);
-  return static_cast<int>(__builtin_rintf(v)); // v_rndne_f32: ties to even
-}
 
 template <int ACT, int CH, int DT>
 __global__ __launch_bounds__(256) void row_quant_kernel(const uint16_t *__restrict__ x, int64_t rows, int64_t C,

@@ -184,15 +184,32 @@ __device__ __forceinline__ void wave_store_32x64_bf16(int8_t *stg, const v4u16 (
 int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int block_size_m, int flags);
 void describe_gemm_kernel(int kernel, bool fused_act, int block_size_m, bool rows, lo_moe_tile *t);
 
-// Decode-size whole path in two launches (gemm_dec.hip): LO_ENOTSUP when it does not apply.
-// act: room for [M * top_k, I] bf16.  w4: packed int4 weights with K-group scales [E, K/128, N].
-bool decode_path_applies(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_t num_experts, bool force, bool w4);
+// Decode-size whole path in two launches (gemm_dec.hip): weights in the load-time layout, bf16 or fp16 rows.
+struct DecProblem {
+  const void *x;
+  int dtype;
+  int64_t M, H, I;
+  int32_t E, num_experts, top_k;
+  const int8_t *w1;
+  const float *w1s;
+  const int8_t *w2;
+  const float *w2s; // block scales, K-group scales [E, K/128, N] (LO_GEMM_W4) or, with `channel`, one scale per row
+  const float *topk_w;
+  const void *topk_ids;
+  int ids_dtype;
+  const int32_t *expert_map;
+  int mul_on_input;
+  float factor;
+  const void *shared_output;
+  void *act; // room for [M * top_k, I] 16-bit activations: the front of the caller's cache13
+  void *out;
+  bool channel;
+};
+// act_fits: `act` holds I values per slot whatever H is.  Whether the path is taken; LO_ENOTSUP from the launcher if not.
+bool decode_path_applies(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_t E, int32_t num_experts, bool force, bool w4,
+                         bool channel, bool act_fits);
 void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_waves);
-int launch_decode_path(const void *x, int64_t M, int64_t H, int64_t I, int32_t E, int32_t num_experts, int32_t top_k,
-                       const int8_t *w1, const float *w1s, const int8_t *w2, const float *w2s, const float *topk_w,
-                       const void *topk_ids, int ids_dtype, const int32_t *expert_map, int apply_router_weight_on_input,
-                       float factor, const void *shared_output, void *act, void *out, bool force, bool w4, int flags,
-                       hipStream_t stream);
+int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t stream);
 
 // Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
 int launch_gemm_ws(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks,

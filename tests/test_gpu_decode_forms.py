@@ -1,0 +1,57 @@
+"""The two-launch path for every form, row type and activation, bit for bit against the staged path: one to seven K blocks
+per wave, ranks that hold a part of the experts, experts with more slots than one pass multiplies, more experts hit than
+the grid has rows, shared-expert epilogue and router weight on the input."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+@pytest.mark.parametrize("form", ["block", "channel", "w4", "w4_channel"])
+@pytest.mark.parametrize("shape", ["one", "share", "seven", "wide", "crowded"])
+def test_forms(form, activation, dtype, shape):
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import (fused_experts_impl_int8, fused_experts_impl_w4a8, preshuffle_moe_scale_int4,
+                                 preshuffle_moe_weight, preshuffle_moe_weight_int4)
+
+    E, Eg, k, H, I, tokens = {"one": (8, 8, 2, 128, 128, (1, 3)), "share": (4, 32, 8, 1024, 896, (1, 5, 9)),
+                              "seven": (4, 4, 2, 3584, 256, (1, 2, 16)), "wide": (3, 3, 1, 2560, 2304, (1, 4)),
+                              "crowded": (3, 6, 3, 256, 128, (21, 50))}[shape]
+    dev = torch.device("cuda:0")
+    extra = {"quant": "channel"} if form.endswith("channel") else {}
+    if form.startswith("w4"):
+        extra["weight_bits"] = 4
+    layer = wl.MoeLayer(shape, E=E, E_global=Eg, top_k=k, H=H, I=I, routing="softmax", **extra)
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=3, device=dev)
+    kw = dict(w1_scale=w1s, w2_scale=w2s, activation=activation, global_num_experts=Eg,
+              block_shape=None if "channel" in form else [1, 128] if form == "w4" else [128, 128])
+    if form.startswith("w4"):
+        fn, w1, w2 = fused_experts_impl_w4a8, preshuffle_moe_weight_int4(w1), preshuffle_moe_weight_int4(w2)
+        if form == "w4":
+            kw.update(w1_scale=preshuffle_moe_scale_int4(w1s), w2_scale=preshuffle_moe_scale_int4(w2s))
+    else:
+        fn, w1, w2 = fused_experts_impl_int8, preshuffle_moe_weight(w1), preshuffle_moe_weight(w2)
+        kw.update(use_int8_w8a8=True, per_channel_quant=form == "channel")
+    for M in tokens:
+        print(f"[case] decode forms {form} {activation} {dtype} {shape} M={M}", flush=True)
+        x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, M, seed=M))
+        x = x.to(dtype)
+        x[M // 2] = 0
+        emap = None
+        if E != Eg:
+            emap = torch.full((Eg,), -1, dtype=torch.int32, device=dev)
+            emap[torch.randperm(Eg, generator=torch.Generator().manual_seed(1))[:E].to(dev)] = torch.arange(
+                E, dtype=torch.int32, device=dev)
+        outs = []
+        for flag in (_lib.LO_FUSED_NO_DECODE_PATH, _lib.LO_FUSED_FORCE_DECODE_PATH):
+            cache13 = torch.full((M * k * max(2 * I, H),), float("nan"), dtype=dtype, device=dev)
+            kx = dict(kw, shared_output=x + 1, routed_scaling_factor=2.5) if M % 2 else kw
+            outs.append(fn(x, w1, w2, tw, ids, cache13, expert_map=emap, lightop_amd_flags=flag,
+                           apply_router_weight_on_input=M == tokens[-1], **kx).cpu())
+            if flag == _lib.LO_FUSED_FORCE_DECODE_PATH:  # only this path leaves the activations at the front of the cache
+                act = cache13[: M * k * I].view(M * k, I).cpu()
+                here = ids.reshape(-1) if emap is None else emap[ids.reshape(-1).long()]
+                assert not torch.isnan(act[(here >= 0).cpu()].float()).any()
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16)), f"M={M}"
