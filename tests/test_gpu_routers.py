@@ -162,3 +162,24 @@ def test_router_argument_errors(dev):
         run_topk_softmax(torch.zeros(2, 16, device=dev), 17, True)
     with pytest.raises(RuntimeError):
         run_topk_softmax(torch.zeros(2, 2048, device=dev), 8, True)
+
+
+@pytest.mark.parametrize("T", [4095, 4096, 4099])
+@pytest.mark.parametrize("E,G,tg,k", [(16, 4, 1, 3), (100, 5, 2, 8), (128, 8, 4, 8), (256, 8, 4, 8)])
+def test_rows_per_wavefront_change_over(dev, oracle, T, E, G, tg, k):
+    """Either side of the row count from which four rows share a wavefront, with ties, rows of equal scores and a partial last
+    wavefront."""
+    from lightop_amd.moe import moe_fused_gate
+
+    say(f"routers T={T} E={E}")
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randint(-3, 4, (T, E), generator=g).float() * 0.5
+    x[1], x[-1] = 0.25, -0.5
+    for renorm in (True, False):
+        w, idx, _ = run_topk_softmax(x.to(dev), k, renorm, with_src=False)
+        rw, ridx, _ = oracle.topk_softmax(x, k, renorm)
+        assert torch.equal(idx, ridx) and torch.equal(w.view(torch.int32), rw.view(torch.int32))
+    bias = torch.randint(-2, 3, (E,), generator=g).float() * 0.25
+    w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, tg, k, 0, 2.5, False)
+    rw, ridx = oracle.moe_fused_gate(x, bias, G, tg, k, 0, 2.5, False)
+    assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
