@@ -128,10 +128,15 @@ __device__ __forceinline__ void moe_align_body(
     int e = base + tid;
     int c = 0;
     if (e < E) {
-      for (int w = 0; w < nw; ++w) {
-        int v = wcnt[w * E + e];
-        wcnt[w * E + e] = c; // tokens of expert e held by earlier waves
-        c += v;
+      for (int w = 0; w < nw; w += 4) { // (nw is 4, 8 or 16; four reads per LDS round trip)
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = wcnt[(w + u) * E + e];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          wcnt[(w + u) * E + e] = c; // tokens of expert e held by earlier waves
+          c += v[u];
+        }
       }
       total[e] = c;
     }
@@ -214,10 +219,9 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(
 }
 
 // Workgroup 0 aligns, the others quantise the activations: two independent stages, one launch.
-template <typename IdT>
+template <typename IdT, bool PER_ROW, int DT>
 __global__ __launch_bounds__(1024) void quant_align_kernel(
-    const uint16_t *__restrict__ x, int64_t groups, float eps, int8_t *__restrict__ q, float *__restrict__ qs,
-    const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
+    const QuantJob job, const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
     const int32_t *__restrict__ expert_map, int32_t *__restrict__ sorted, int64_t sorted_cap,
     int32_t *__restrict__ expert_ids, int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits,
     uint8_t *__restrict__ slot_mask) {
@@ -225,10 +229,7 @@ __global__ __launch_bounds__(1024) void quant_align_kernel(
     moe_align_body<IdT>(ids, numel, num_experts, bs, expert_map, 0, sorted, sorted_cap, expert_ids, expert_ids_cap,
                         ntpp, key_bits, slot_mask, nullptr, 1);
   } else {
-    const int per_block = blockDim.x >> 4; // groups a workgroup handles per pass
-    group_quant_body<LO_BF16>(x, groups, eps, q, qs,
-                              static_cast<int64_t>(blockIdx.x - 1) * per_block + (threadIdx.x >> 4),
-                              static_cast<int64_t>(gridDim.x - 1) * per_block, threadIdx.x & 15);
+    quant_job<PER_ROW, DT>(job, blockIdx.x - 1, gridDim.x - 1);
   }
 }
 
@@ -475,10 +476,9 @@ __global__ __launch_bounds__(256) void moe_align_scatter_kernel(
 // not depend on the alignment, and the scatter (a chain of dependent round trips on a few compute
 // units) costs nothing beside it.  The counting, which the scatter waits for, is a launch of its own
 // before this one.
-template <typename IdT>
+template <typename IdT, bool PER_ROW, int DT>
 __global__ __launch_bounds__(256) void quant_align_scatter_kernel(
-    const uint16_t *__restrict__ x, int64_t groups, float eps, int8_t *__restrict__ q, float *__restrict__ qs,
-    const IdT *__restrict__ ids, int64_t numel, int E, int bs, const int32_t *__restrict__ expert_map,
+    const QuantJob job, const IdT *__restrict__ ids, int64_t numel, int E, int bs, const int32_t *__restrict__ expert_map,
     int64_t chunk_slots, const int32_t *__restrict__ cnt, int32_t *__restrict__ sorted, int64_t sorted_cap,
     int32_t *__restrict__ expert_ids, int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits,
     int nchunks) {
@@ -486,9 +486,7 @@ __global__ __launch_bounds__(256) void quant_align_scatter_kernel(
     moe_align_scatter_body<IdT>(ids, numel, E, bs, expert_map, 0, chunk_slots, cnt, sorted, sorted_cap, expert_ids,
                                 expert_ids_cap, ntpp, key_bits, nullptr, 1, static_cast<int>(blockIdx.x), nchunks);
   } else {
-    group_quant_body<LO_BF16>(x, groups, eps, q, qs,
-                              static_cast<int64_t>(blockIdx.x - nchunks) * 16 + (threadIdx.x >> 4),
-                              static_cast<int64_t>(gridDim.x - nchunks) * 16, threadIdx.x & 15);
+    quant_job<PER_ROW, DT>(job, blockIdx.x - nchunks, gridDim.x - nchunks);
   }
 }
 
@@ -513,7 +511,20 @@ static void align_chunks(int64_t numel, int *nchunks, int64_t *chunk_slots) {
   *nchunks = static_cast<int>((numel + cs - 1) / cs);
 }
 
-int launch_quant_align(const void *x, int64_t M, int64_t H, float eps, int8_t *q, float *qs,
+// id type x quantisation x row type
+#define LO_QA_DISPATCH(LAUNCH)                            \
+  do {                                                    \
+    if (ids_dtype == LO_I32) LO_QA_BY_ROW(LAUNCH, int32_t); \
+    else LO_QA_BY_ROW(LAUNCH, int64_t);                   \
+  } while (0)
+#define LO_QA_BY_ROW(LAUNCH, IdT)                         \
+  do {                                                    \
+    if (per_row && f16) LAUNCH(IdT, true, LO_F16);        \
+    else if (per_row) LAUNCH(IdT, true, LO_BF16);         \
+    else if (f16) LAUNCH(IdT, false, LO_F16);             \
+    else LAUNCH(IdT, false, LO_BF16);                     \
+  } while (0)
+int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_t H, float eps, int8_t *q, float *qs,
                        const void *topk_ids, int ids_dtype, int64_t numel, int32_t num_experts,
                        int32_t block_size, const int32_t *expert_map, int32_t *sorted_ids, int64_t sorted_cap,
                        int32_t *expert_ids, int64_t expert_ids_cap, int32_t *num_tokens_post_pad,
@@ -523,6 +534,8 @@ int launch_quant_align(const void *x, int64_t M, int64_t H, float eps, int8_t *q
     return LO_ENOTSUP; // the multi-workgroup form needs its counters
   LO_REQUIRE(x && q && qs && topk_ids && sorted_ids && expert_ids && num_tokens_post_pad, LO_EINVAL,
              "quant_align: null pointer");
+  LO_REQUIRE((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(q) & 7) == 0, LO_EINVAL,
+             "quant_align: x must be 16-byte and q 8-byte aligned");
   LO_REQUIRE(H > 0 && H % kGroup == 0 && M >= 1 && numel >= 1 && num_experts >= 1 && num_experts <= 2048 &&
                  block_size >= 1,
              LO_EINVAL, "quant_align: bad shape");
@@ -532,6 +545,8 @@ int launch_quant_align(const void *x, int64_t M, int64_t H, float eps, int8_t *q
              "quant_align: alignment buffers too small");
   int key_bits = 1;
   while ((1 << key_bits) < num_experts) ++key_bits;
+  const QuantJob job{static_cast<const uint16_t *>(x), M, H, eps, q, qs};
+  const bool f16 = dtype == LO_F16;
   const int64_t groups = M * (H / kGroup);
   if (want > 0) { // many slots: counting, then the scatter beside the quantisation
     int nchunks;
@@ -540,47 +555,42 @@ int launch_quant_align(const void *x, int64_t M, int64_t H, float eps, int8_t *q
     int32_t *cnt = static_cast<int32_t *>(scratch);
     const size_t lds1 = static_cast<size_t>(num_experts) * 4;
     const size_t lds2 = (static_cast<size_t>(4 + 3) * num_experts + 1) * 4;
-    int64_t qb = (groups + 15) / 16;
+    int64_t qb = per_row ? M : (groups + 15) / 16;
     if (qb > 8192) qb = 8192;
     const dim3 grid2(static_cast<unsigned>(nchunks + qb));
-    if (ids_dtype == LO_I32) {
+#define LO_QA_SCATTER(IdT, PR, DT)                                                                                       \
+  hipLaunchKernelGGL((quant_align_scatter_kernel<IdT, PR, DT>), grid2, dim3(256), lds2, stream, job,                     \
+                     static_cast<const IdT *>(topk_ids), numel, num_experts, block_size, expert_map, cs, cnt, sorted_ids, \
+                     sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, nchunks)
+    if (ids_dtype == LO_I32)
       hipLaunchKernelGGL(moe_align_count_kernel<int32_t>, dim3(nchunks), dim3(256), lds1, stream,
                          static_cast<const int32_t *>(topk_ids), numel, num_experts, expert_map, 0, cs, cnt, slot_mask,
                          nullptr, 1, sorted_ids, sorted_cap);
-      hipLaunchKernelGGL(quant_align_scatter_kernel<int32_t>, grid2, dim3(256), lds2, stream,
-                         static_cast<const uint16_t *>(x), groups, eps, q, qs, static_cast<const int32_t *>(topk_ids),
-                         numel, num_experts, block_size, expert_map, cs, cnt, sorted_ids, sorted_cap, expert_ids,
-                         expert_ids_cap, num_tokens_post_pad, key_bits, nchunks);
-    } else {
+    else
       hipLaunchKernelGGL(moe_align_count_kernel<int64_t>, dim3(nchunks), dim3(256), lds1, stream,
                          static_cast<const int64_t *>(topk_ids), numel, num_experts, expert_map, 0, cs, cnt, slot_mask,
                          nullptr, 1, sorted_ids, sorted_cap);
-      hipLaunchKernelGGL(quant_align_scatter_kernel<int64_t>, grid2, dim3(256), lds2, stream,
-                         static_cast<const uint16_t *>(x), groups, eps, q, qs, static_cast<const int64_t *>(topk_ids),
-                         numel, num_experts, block_size, expert_map, cs, cnt, sorted_ids, sorted_cap, expert_ids,
-                         expert_ids_cap, num_tokens_post_pad, key_bits, nchunks);
-    }
+    LO_QA_DISPATCH(LO_QA_SCATTER);
+#undef LO_QA_SCATTER
     return check_launch("quant_align(multi)");
   }
   int nw;
   size_t lds_bytes;
   single_wg_shape(numel, sorted_cap, num_experts, &nw, &lds_bytes);
   const int per_block = nw * kWave / 16;
-  int64_t qblocks = (groups + per_block - 1) / per_block;
+  int64_t qblocks = per_row ? (M + nw / 4 - 1) / (nw / 4) : (groups + per_block - 1) / per_block;
   if (qblocks > 4096) qblocks = 4096;
   const dim3 grid(static_cast<unsigned>(1 + qblocks)), block(nw * kWave);
-  if (ids_dtype == LO_I32)
-    hipLaunchKernelGGL(quant_align_kernel<int32_t>, grid, block, lds_bytes, stream, static_cast<const uint16_t *>(x),
-                       groups, eps, q, qs, static_cast<const int32_t *>(topk_ids), numel, num_experts, block_size,
-                       expert_map, sorted_ids, sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits,
-                       slot_mask);
-  else
-    hipLaunchKernelGGL(quant_align_kernel<int64_t>, grid, block, lds_bytes, stream, static_cast<const uint16_t *>(x),
-                       groups, eps, q, qs, static_cast<const int64_t *>(topk_ids), numel, num_experts, block_size,
-                       expert_map, sorted_ids, sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits,
-                       slot_mask);
+#define LO_QA_ONE(IdT, PR, DT)                                                                                           \
+  hipLaunchKernelGGL((quant_align_kernel<IdT, PR, DT>), grid, block, lds_bytes, stream, job,                             \
+                     static_cast<const IdT *>(topk_ids), numel, num_experts, block_size, expert_map, sorted_ids,         \
+                     sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask)
+  LO_QA_DISPATCH(LO_QA_ONE);
+#undef LO_QA_ONE
   return check_launch("quant_align");
 }
+#undef LO_QA_DISPATCH
+#undef LO_QA_BY_ROW
 
 } // namespace lo
 

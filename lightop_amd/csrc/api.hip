@@ -411,12 +411,12 @@ extern "C" int lo_fused_experts_block_int8(
     if (rc2 != LO_ENOTSUP) return rc2;
   }
 
-  // the quantisation rides in the alignment's launch (bf16 rows)
-  int rc = dtype != LO_BF16 ? LO_ENOTSUP
-                            : launch_quant_align(x, M, H, 1e-10f, a1q, a1s, topk_ids, ids_dtype, S, num_experts,
-                                                 block_size_m, expert_map, sorted, L.sorted_cap, eids, L.blocks_cap,
-                                                 ntpp, mask, ws + L.off[8], L.align_scratch,
-                                                 static_cast<hipStream_t>(stream));
+  // the quantisation rides in the alignment's launch (16-bit rows)
+  int rc = dtype == LO_F32 ? LO_ENOTSUP
+                           : launch_quant_align(x, dtype, false, M, H, 1e-10f, a1q, a1s, topk_ids, ids_dtype, S, num_experts,
+                                                block_size_m, expert_map, sorted, L.sorted_cap, eids, L.blocks_cap,
+                                                ntpp, mask, ws + L.off[8], L.align_scratch,
+                                                static_cast<hipStream_t>(stream));
   if (rc == LO_ENOTSUP) {
     rc = lo_per_token_group_quant_int8(x, dtype, M, H, 1e-10f, a1q, a1s, stream);
     if (rc) return rc;
@@ -512,14 +512,16 @@ static int fused_experts_channel(
     const int rc2 = launch_decode_path(d, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, flags, static_cast<hipStream_t>(stream));
     if (rc2 != LO_ENOTSUP) return rc2;
   }
-  int rc = LO_OK;
+  int rc;
   if (!x_q)
-    rc = lo_per_token_quant_int8(x, dtype, M, H, reinterpret_cast<int8_t *>(ws + L.off[0]),
-                                 reinterpret_cast<float *>(ws + L.off[1]), stream);
-  if (rc) return rc;
-  rc = lo_moe_align_block_size_ws(topk_ids, ids_dtype, S, num_experts, block_size_m, expert_map, 0,
-                                  sorted, L.sorted_cap, eids, L.blocks_cap, ntpp, mask, ws + L.off[8],
-                                  L.align_scratch, stream);
+    rc = launch_quant_align(x, dtype, true, M, H, 1e-10f, reinterpret_cast<int8_t *>(ws + L.off[0]),
+                            reinterpret_cast<float *>(ws + L.off[1]), topk_ids, ids_dtype, S, num_experts, block_size_m,
+                            expert_map, sorted, L.sorted_cap, eids, L.blocks_cap, ntpp, mask, ws + L.off[8],
+                            L.align_scratch, static_cast<hipStream_t>(stream));
+  else
+    rc = lo_moe_align_block_size_ws(topk_ids, ids_dtype, S, num_experts, block_size_m, expert_map, 0,
+                                    sorted, L.sorted_cap, eids, L.blocks_cap, ntpp, mask, ws + L.off[8],
+                                    L.align_scratch, stream);
   if (rc) return rc;
   // rows of experts on other ranks are zero-filled here: the activation kernel reads every row
   const int gflags = flags & ~LO_FUSED_ACT_GELU;

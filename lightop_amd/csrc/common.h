@@ -258,12 +258,82 @@ __device__ __forceinline__ void group_quant_body(const uint16_t *__restrict__ x,
   }
 }
 
-// Group quant of x [M, H] and the routing alignment with the quantisation riding in the
-// alignment's (first) launch: they are independent, and at decode sizes a launch costs as much
+// per_token_quant_int8 (int8_utils.py:20-44: amax floored at 1e-10, s = amax / 127, q = rne(x * (127 / amax))): four
+// wavefronts per row, blockDim.x / 256 rows per workgroup and pass, pieces of up to 8192 values kept in registers between
+// the two steps.  Every wave of the workgroup makes the same number of passes.  red: 2 * 16 floats of LDS.
+template <int DT>
+__device__ __forceinline__ void row_quant_body(const uint16_t *__restrict__ x, int64_t rows, int64_t C,
+                                               int8_t *__restrict__ q, float *__restrict__ s, int64_t block,
+                                               int64_t nblocks, float *red) {
+  constexpr int CH = 4;
+  const int tid = threadIdx.x & 255, team = threadIdx.x >> 8, teams = blockDim.x >> 8;
+  const int pieces = static_cast<int>(C / 8);
+  int odd = 0; // two halves of `red` in turn: one barrier per pass
+  for (int64_t base = block * teams; base < rows; base += nblocks * teams, odd ^= 1) {
+    const int64_t row = base + team;
+    const uint16_t *xr = x + (row < rows ? row : base) * C;
+    v8u16 keep[CH];
+    float amax = 1e-10f;
+    auto widest = [&](const v8u16 raw) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(to_f32<DT>(raw[i])));
+    };
+#pragma unroll
+    for (int j = 0; j < CH; ++j) // (a thread past the row re-reads its start: the same maximum)
+      keep[j] = *reinterpret_cast<const v8u16 *>(xr + (tid + 256 * j < pieces ? tid + 256 * j : 0) * 8);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) widest(keep[j]);
+    for (int p = tid + 256 * CH; p < pieces; p += 256) widest(*reinterpret_cast<const v8u16 *>(xr + p * 8));
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
+    if ((threadIdx.x & 63) == 0) red[odd * 16 + (threadIdx.x >> 6)] = amax;
+    __syncthreads();
+    const float *const r4 = red + odd * 16 + team * 4;
+    amax = fmaxf(fmaxf(r4[0], r4[1]), fmaxf(r4[2], r4[3]));
+    if (row >= rows) continue;
+    const float inv = 127.0f / amax;
+    if (tid == 0) s[row] = amax / 127.0f;
+    auto emit = [&](int p, const v8u16 raw) __attribute__((always_inline)) {
+      int b[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) b[i] = rne_i8(to_f32<DT>(raw[i]) * inv);
+      *reinterpret_cast<v2i *>(q + row * C + p * 8) = v2i{static_cast<int>(pack4_i8(b[0], b[1], b[2], b[3])),
+                                                         static_cast<int>(pack4_i8(b[4], b[5], b[6], b[7]))};
+    };
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      if (tid + 256 * j < pieces) emit(tid + 256 * j, keep[j]);
+    for (int p = tid + 256 * CH; p < pieces; p += 256) emit(p, *reinterpret_cast<const v8u16 *>(xr + p * 8));
+  }
+}
+
+// The quantisation of the activations that rides in an alignment launch.
+struct QuantJob {
+  const uint16_t *x; // [M, H] bf16, or fp16
+  int64_t M, H;
+  float eps;         // floor of a group's maximum (rows: 1e-10)
+  int8_t *q;
+  float *s;          // [M, H/128], or [M] per row
+};
+// Workgroup `block` of `nblocks` that share the job (blockDim.x a multiple of 256).
+template <bool PER_ROW, int DT>
+__device__ __forceinline__ void quant_job(const QuantJob &j, int64_t block, int64_t nblocks) {
+  if constexpr (PER_ROW) {
+    __shared__ float red[32];
+    row_quant_body<DT>(j.x, j.M, j.H, j.q, j.s, block, nblocks, red);
+  } else {
+    const int per_block = blockDim.x >> 4; // groups a workgroup handles per pass
+    group_quant_body<DT>(j.x, j.M * (j.H / kGroup), j.eps, j.q, j.s, block * per_block + (threadIdx.x >> 4),
+                         nblocks * per_block, threadIdx.x & 15);
+  }
+}
+
+// The quantisation of x [M, H] (per group, or per row) and the routing alignment with the quantisation riding in the
+// alignment's (second) launch: they are independent, and at decode sizes a launch costs as much
 // as either.  scratch: the multi-workgroup alignment's counters (lo_moe_align_scratch_bytes);
 // returns LO_ENOTSUP when they are needed and missing - the caller then launches the two stages
 // separately.
-int launch_quant_align(const void *x, int64_t M, int64_t H, float eps, int8_t *q, float *s,
+int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_t H, float eps, int8_t *q, float *s,
                        const void *topk_ids, int ids_dtype, int64_t numel, int32_t num_experts,
                        int32_t block_size, const int32_t *expert_map, int32_t *sorted_ids, int64_t sorted_cap,
                        int32_t *expert_ids, int64_t expert_ids_cap, int32_t *num_tokens_post_pad,

@@ -296,24 +296,25 @@ static void launch_row_quant(const uint16_t *x, int64_t rows, int64_t C, const u
 // mask byte and every row is a round trip of its own).  A masked slot adds
 // +0.0f instead of being skipped, which is the same value: the sum starts at +0.0f and can
 // never become -0.0f.  TOPK = 0 keeps the run-time loop.
+// A workgroup takes 2048 columns of one token after the other (a flat index over all of them costs a 64-bit division in
+// front of the first load).
+constexpr int kSumThreads = 256;
 template <int DT, bool HAS_BIAS, int TOPK>
-__global__ __launch_bounds__(256) void moe_sum_kernel(const uint16_t *__restrict__ in,
+__global__ __launch_bounds__(kSumThreads) void moe_sum_kernel(const uint16_t *__restrict__ in,
                                                       uint16_t *__restrict__ out,
                                                       const uint16_t *__restrict__ bias,
                                                       const uint8_t *__restrict__ mask,
                                                       int64_t M, int topk, int64_t H,
                                                       float factor,
                                                       const int32_t *__restrict__ num_local_tokens) {
-  const int64_t vec_per_row = H / 8;
   // rows of padding tokens (t >= num_local_tokens[0]) are left untouched
   if (num_local_tokens) {
     const int64_t n = num_local_tokens[0];
-    M = n < 0 ? 0 : (n < M ? n : M);
+    M = n < M ? n : M;
   }
-  const int64_t total = M * vec_per_row;
-  for (int64_t v = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < total;
-       v += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t t = v / vec_per_row, c = (v % vec_per_row) * 8;
+  const int64_t c = (static_cast<int64_t>(blockIdx.y) * kSumThreads + threadIdx.x) * 8;
+  if (c >= H) return;
+  for (int64_t t = blockIdx.x; t < M; t += gridDim.x) {
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     const uint16_t *p = in + t * topk * H + c;
     if constexpr (TOPK > 0) {
@@ -638,17 +639,21 @@ extern "C" int lo_moe_sum(const void *in, void *out, const void *bias, const uin
     return launch_moe_sum_f32(static_cast<const float *>(in), static_cast<float *>(out),
                               static_cast<const float *>(bias), expert_mask, M, topk, H, factor, num_local_tokens,
                               static_cast<hipStream_t>(stream));
-  const int grid = grid_for(M * (H / 8), 256);
+  const int64_t cols = (H / 8 + kSumThreads - 1) / kSumThreads;
+  LO_REQUIRE(cols < 65536, LO_ENOTSUP, "moe_sum: rows of %lld values", (long long)H);
+  int64_t tokens = 4096 / cols; // sixteen workgroups per CU: what is resident, twice
+  tokens = tokens < 1 ? 1 : (tokens < M ? tokens : M);
+  const dim3 grid(static_cast<unsigned>(tokens), static_cast<unsigned>(cols));
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define LO_SUM_LAUNCH(DTV, HB, TK)                                                                   \
-  hipLaunchKernelGGL((moe_sum_kernel<DTV, HB, TK>), dim3(grid), dim3(256), 0, s,                    \
+  hipLaunchKernelGGL((moe_sum_kernel<DTV, HB, TK>), grid, dim3(kSumThreads), 0, s,                  \
                      static_cast<const uint16_t *>(in), static_cast<uint16_t *>(out),               \
                      static_cast<const uint16_t *>(bias), expert_mask, M, topk, H, factor, num_local_tokens)
 #define LO_SUM_PICK(TK)                                                                              \
   do {                                                                                               \
-    if (dtype == LO_F16) { /* fp16 rows: the run-time slot loop serves every width */               \
-      if (bias) LO_SUM_LAUNCH(LO_F16, true, 0);                                                      \
-      else LO_SUM_LAUNCH(LO_F16, false, 0);                                                          \
+    if (dtype == LO_F16) {                                                                           \
+      if (bias) LO_SUM_LAUNCH(LO_F16, true, TK);                                                     \
+      else LO_SUM_LAUNCH(LO_F16, false, TK);                                                         \
     } else if (bias) LO_SUM_LAUNCH(LO_BF16, true, TK);                                               \
     else LO_SUM_LAUNCH(LO_BF16, false, TK);                                                          \
   } while (0)
