@@ -249,8 +249,8 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
   plan->flags = flags;
   plan->block_size_m = block_size_m;
   plan->bs160 = bs160;
-  // GELU and fp16 / fp32 activations have no fused epilogue
-  plan->unfused = !fused_ok;
+  // fp32 rows have no fused epilogue; GELU and fp16 rows have one at some block sizes
+  plan->unfused = !fused_ok && (dtype == LO_F32 || !fused_table_supports(H, block_size_m, flags));
   plan->try_decode = block_size_m_auto && pre && dtype != LO_F32 && !(flags & LO_FUSED_NO_DECODE_PATH);
   return LO_OK;
 }
@@ -286,7 +286,7 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
     bm = plan.block_size_m;
     fused = !plan.unfused;
     // (fp16 rows and GELU: the query describes the staged path)
-    decode = plan.try_decode && fused && M > 0 &&
+    decode = plan.try_decode && dtype == LO_BF16 && !(flags & LO_FUSED_ACT_GELU) && M > 0 &&
              decode_path_applies(M, top_k, H, I, E_local > 0 ? E_local : num_experts, num_experts,
                                  (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, (flags & LO_GEMM_W4) != 0, false, false);
   }
@@ -435,9 +435,14 @@ extern "C" int lo_fused_experts_block_int8(
     rc = launch_act_mul_group_quant(cache3, dtype, gelu ? LO_ACT_GELU : LO_ACT_SILU, S, I, a2q, a2s, mask,
                                     static_cast<hipStream_t>(stream));
   } else {
-    rc = lo_moe_gemm1_silu_quant_block_int8(a1q, a1s, w1, w1s, a2q, a2s, dtype, topk_w, sorted, eids,
-                                            ntpp, L.sorted_cap, S, M, E, num_experts, I, H, top_k, block_size_m,
-                                            apply_router_weight_on_input, flags, stream);
+    const uint16_t *table = nullptr;
+    if (gelu || dtype == LO_F16)
+      rc = act_table(static_cast<hipStream_t>(stream), gelu ? LO_ACT_GELU : LO_ACT_SILU, dtype, &table);
+    if (rc) return rc;
+    rc = launch_gemm1_act_quant(a1q, a1s, w1, w1s, a2q, a2s, table ? kActTable : kActSiluBf16,
+                                dtype == LO_F16, table, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E, num_experts, I,
+                                H, top_k, block_size_m, apply_router_weight_on_input, flags & ~LO_FUSED_ACT_GELU,
+                                static_cast<hipStream_t>(stream));
   }
   if (rc) return rc;
   rc = lo_moe_gemm_block_int8(a2q, a2s, w2, w2s, cache3, dtype, topk_w, sorted, eids, ntpp,

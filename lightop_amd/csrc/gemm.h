@@ -41,9 +41,49 @@ struct GemmArgs {
   int32_t w4;            // W is packed int4 (load-time layout), Ws is [E, K/128, N]
   int32_t per_channel;   // As is [a_rows], Ws is [E, N]: scales applied once, after the whole-K int32 sum
   int32_t coarse_fill;   // 160-token tiles: round the token fragments in use up to 8
-  int32_t out_f16;       // C holds IEEE half instead of bf16 (plain epilogues only)
+  int32_t out_f16;       // C holds IEEE half instead of bf16; fused: the values between the stages are rounded to half
   int32_t out_f32;       // C holds the fp32 sums themselves (block form, weight-streaming kernel only)
+  int32_t fused;         // the fused epilogue's activation: kActSiluBf16 or kActTable (plain: 0)
+  const uint16_t *act_table; // kActTable: T(act(g)) of every 16-bit pattern g
 };
+
+// Gated activations of a fused first stage; the kernels' FUSED_ACT parameter, 0 being a plain GEMM.  SiLU of bf16 rows is
+// computed and comes in all three scale orders.  The others are looked up, 128 KB in L2: GELU, and SiLU of fp16 gates, which
+// the short forms of exp and reciprocal do not round right (the long way costs the epilogue more than the lookup: Qwen3-30B-A3B
+// layer at 8000 tokens 627 us against 618).  They exist in the default order, and in the kernels for 64 and 128 tokens and
+// for row-major weights; otherwise the first stage is a plain GEMM and an activation launch, which with the weight-streaming
+// kernel is as fast, its plain workgroups being finer (24 tokens: 100.0 plain, 101.1 fused).  Plain / fused, us:
+// Qwen3-30B-A3B layer, fp16 333 tokens 133.8 / 124.7, 4000: 399 / 375, 8000: 684 / 618; GELU 100: 117.6 / 114.3, 8001: 639 /
+// 598; DeepSeek-V3 share, fp16 2000: 326 / 314; Qwen3-235B-A22B-shaped layer, fp16 300: 434 / 409, row-major 492 / 468.
+constexpr int kActSiluBf16 = 1, kActTable = 2;
+// act[i] = T(T(act(T(g[i]))) * T(u[i])) as floats.
+template <int FUSED_ACT, int N>
+__device__ __forceinline__ void gated_act(const GemmArgs &a, const float (&g)[N], const float (&u)[N], float (&act)[N]) {
+  if constexpr (FUSED_ACT == kActSiluBf16) {
+    silu_mul_bf16<N>(g, u, act);
+  } else {
+    if (a.out_f16) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) act[i] = f16_to_f32(act_mul_tab<LO_F16>(a.act_table, f32_to_f16(g[i]), f32_to_f16(u[i])));
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) act[i] = bf16_to_f32(act_mul_tab<LO_BF16>(a.act_table, f32_to_bf16(g[i]), f32_to_bf16(u[i])));
+    }
+  }
+}
+// (K <= 16384: what the kernels with such an epilogue hold scales for)
+inline bool fused_table_supports(int64_t K, int block_size_m, int flags) {
+  if (flags & (LO_GEMM_SEPARATE_ORDER | LO_GEMM_FUSED_SCALE | LO_GEMM_FORCE_STREAMING)) return false;
+  if (K > 128 * kGroup) return false;
+  const bool rows = !(flags & (LO_GEMM_W_PRESHUFFLED | LO_GEMM_W4));
+  return block_size_m == 64 || block_size_m == 128 || (rows && (block_size_m == 16 || block_size_m == 32));
+}
+// Launcher macro MACRO(scale order, FUSED_ACT) for a fused first stage.
+#define LO_FUSED_DISPATCH(a, ord, MACRO)                                                \
+  do {                                                                                  \
+    if ((a).fused == ::lo::kActTable) MACRO(::lo::kOrdContract, ::lo::kActTable);  \
+    else LO_ORD_DISPATCH(ord, MACRO, ::lo::kActSiluBf16);                               \
+  } while (0)
 
 // Division of a slot id below 2^31 by top_k as a multiplication: with L = ceil(log2 d) and m = floor(2^(31+L) / d) + 1,
 // floor(n * m / 2^(31+L)) is the quotient for every n < 2^31 (m overshoots 2^(31+L) / d by less than 2^-31 of it), and m
@@ -212,6 +252,12 @@ void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_wa
 int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t stream);
 
 // Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
+// The fused first stage with a given activation (lo_moe_gemm1_silu_quant_block_int8 is this with kActSiluBf16).
+int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
+                           int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,
+                           const int32_t *expert_ids, const int32_t *num_tokens_post_pad, int64_t sorted_cap,
+                           int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts, int64_t I, int64_t K,
+                           int32_t top_k, int32_t block_size_m, int mul_routed, int flags, hipStream_t stream);
 int launch_gemm_ws(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks,
                    hipStream_t s);
 // LDS-tiled kernels (gemm_tile.hip): block_size_m 64 or 128, compute-bound regime.

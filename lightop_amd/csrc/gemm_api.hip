@@ -147,20 +147,18 @@ extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const in
   return launch_gemm(a, false, block_size_m, flags, mblocks, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int lo_moe_gemm1_silu_quant_block_int8(
-    const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
-    int c_dtype, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
-    const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows,
-    int32_t E, int32_t num_experts, int64_t I, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
-    int flags, lo_stream_t stream) {
-  using namespace lo;
+namespace lo {
+int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
+                           int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,
+                           const int32_t *expert_ids, const int32_t *num_tokens_post_pad, int64_t sorted_cap,
+                           int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts, int64_t I, int64_t K,
+                           int32_t top_k, int32_t block_size_m, int mul_routed, int flags, hipStream_t stream) {
   int rc = validate_common("moe_gemm1_silu_quant", A, As, W, Ws, sorted_ids, expert_ids,
                            num_tokens_post_pad, K, top_k, E, a_rows);
   if (rc) return rc;
   LO_REQUIRE(valid_block_m(block_size_m) || block_size_m == 160, LO_EINVAL,
              "moe_gemm1_silu_quant: block_size_m %d is not one of 16, 32, 64, 128 (or 160)", block_size_m);
   LO_REQUIRE(A2q && A2s, LO_EINVAL, "moe_gemm1_silu_quant: null output");
-  LO_REQUIRE(c_dtype == LO_BF16, LO_ENOTSUP, "moe_gemm1_silu_quant: only bf16 rounding is built");
   LO_REQUIRE(I > 0 && I % kGroup == 0, LO_EINVAL,
              "moe_gemm1_silu_quant: intermediate size (%lld) must be a multiple of 128", (long long)I);
   LO_REQUIRE(2 * I * K < (1ll << 31), LO_ENOTSUP, "moe_gemm1_silu_quant: one expert's weights exceed 2 GiB");
@@ -173,6 +171,7 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
   if (num_valid == 0) return LO_OK;
   GemmArgs a{};
   a.A = A; a.As = As; a.W = W; a.Ws = Ws; a.A2q = A2q; a.A2s = A2s;
+  a.fused = fused; a.act_table = act_table; a.out_f16 = f16 ? 1 : 0;
   a.topk_w = topk_w; a.sorted = sorted_ids; a.expert_ids = expert_ids; a.ntpp = num_tokens_post_pad;
   a.E = E; a.experts_routed = num_experts > E ? num_experts : E; a.a_rows = a_rows; a.num_valid = num_valid; a.N = 2 * I; a.K = K; set_top_k(a, top_k); a.mul_routed = mul_routed ? 1 : 0;
   a.w_shuffled = (flags & LO_GEMM_W_PRESHUFFLED) ? 1 : 0;
@@ -182,13 +181,29 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
              "moe_gemm1_silu_quant: int4 weights must be in the layout of lo_preshuffle_weight_int4 "
              "(LO_GEMM_W_PRESHUFFLED)");
   a.n_tiles = static_cast<int32_t>(I / kGroup);
-  LO_REQUIRE(block_size_m != 160 || gemm_t128_supports(a, true, 160), LO_ENOTSUP,
+  LO_REQUIRE(block_size_m != 160 || (fused == kActSiluBf16 && gemm_t128_supports(a, true, 160)), LO_ENOTSUP,
              "moe_gemm1_silu_quant: 160-token blocks need int8 weights in the load-time layout "
              "(LO_GEMM_W_PRESHUFFLED) and K <= %d", kGroup * 128);
+  LO_REQUIRE(fused == kActSiluBf16 || fused_table_supports(K, block_size_m, flags), LO_ENOTSUP,
+             "moe_gemm1_silu_quant: no looked-up activation at this block size or scale order");
   const int64_t mblocks = grid_m_blocks(sorted_cap, num_valid, block_size_m);
   LO_REQUIRE(mblocks * a.n_tiles < (1ll << 31), LO_EINVAL, "moe_gemm1_silu_quant: grid too large");
   if (mblocks == 0) return LO_OK;
-  return launch_gemm(a, true, block_size_m, flags, mblocks, static_cast<hipStream_t>(stream));
+  return launch_gemm(a, true, block_size_m, flags, mblocks, stream);
+}
+} // namespace lo
+
+extern "C" int lo_moe_gemm1_silu_quant_block_int8(
+    const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
+    int c_dtype, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
+    const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows,
+    int32_t E, int32_t num_experts, int64_t I, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
+    int flags, lo_stream_t stream) {
+  using namespace lo;
+  LO_REQUIRE(c_dtype == LO_BF16, LO_ENOTSUP, "moe_gemm1_silu_quant: only bf16 rounding is built");
+  return launch_gemm1_act_quant(A, As, W, Ws, A2q, A2s, kActSiluBf16, false, nullptr, topk_w, sorted_ids, expert_ids,
+                                num_tokens_post_pad, sorted_cap, num_valid, a_rows, E, num_experts, I, K, top_k,
+                                block_size_m, mul_routed, flags, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int lo_moe_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws,

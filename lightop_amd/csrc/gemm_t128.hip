@@ -73,7 +73,7 @@ __device__ __forceinline__ void wait_copies_barrier() {
 // python/lightop/_lmslim_native/layers/fused_moe/w4a8.py:341-395): one scale per token row and one
 // per weight row, both applied in the epilogue, so the int32 sums run over the whole K inside the
 // MFMA accumulators and the K loop has no scale arithmetic at all.
-template <bool FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8, bool ROWS = false>
+template <int FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8, bool ROWS = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 4 : NTB <= 4 ? 3 : 2, NTB == 1 ? 4 : NTB <= 4 ? 3 : 2)))
 void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   static_assert(!PC || (!FUSED_ACT && ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
@@ -654,7 +654,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     for (int tb = 0; tb < NTB; ++tb) {
       if (2 * (tb & ~1) >= nst) continue; // the same condition for both fragments of a pair
 #pragma unroll
-      for (int h = 0; h < 2; ++h) silu_mul_bf16<4>(acc[h][tb][0], acc[h][tb][1], actf[tb][h]);
+      for (int h = 0; h < 2; ++h) gated_act<FUSED_ACT, 4>(a, acc[h][tb][0], acc[h][tb][1], actf[tb][h]);
       float amax = 0.0f;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -763,9 +763,9 @@ static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, 
     if (stream) LO_ROWS_LAUNCH2(kOrdSeparate, false, true, true);
     else LO_ROWS_LAUNCH2(kOrdSeparate, false, false, true);
   } else if (fused_act) {
-    LO_ORD_DISPATCH(ord, LO_ROWS_LAUNCH, true);
+    LO_FUSED_DISPATCH(a, ord, LO_ROWS_LAUNCH);
   } else {
-    LO_ORD_DISPATCH(ord, LO_ROWS_LAUNCH, false);
+    LO_ORD_DISPATCH(ord, LO_ROWS_LAUNCH, 0);
   }
 #undef LO_ROWS_LAUNCH
 #undef LO_ROWS_LAUNCH2
@@ -865,9 +865,9 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
       if (rc_lds) return rc_lds;
       hipLaunchKernelGGL((moe_gemm_t128_kernel<false, kOrdSeparate, true, false, true, 10>), g, b, kTLds160, s, a, mbi, gi);
     } else if (fused_act) {
-      LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, true);
+      LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, kActSiluBf16);
     } else {
-      LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, false);
+      LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, 0);
     }
 #undef LO_T160_LAUNCH
     return check_launch(fused_act ? "moe_gemm1_silu_quant(t160)" : "moe_gemm(t160)");
@@ -878,9 +878,9 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     if (stream) LO_T128_LAUNCH_PC(true);
     else LO_T128_LAUNCH_PC(false);
   } else if (fused_act) {
-    LO_ORD_DISPATCH(ord, LO_T128_PICK, true);
+    LO_FUSED_DISPATCH(a, ord, LO_T128_PICK);
   } else {
-    LO_ORD_DISPATCH(ord, LO_T128_PICK, false);
+    LO_ORD_DISPATCH(ord, LO_T128_PICK, 0);
   }
 #undef LO_T128_PICK
 #undef LO_T128_LAUNCH_PC

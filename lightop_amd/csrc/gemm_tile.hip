@@ -36,7 +36,7 @@ constexpr int kTileRow = 144;    // LDS row pitch in bytes: 128 + 16 keeps ds_re
 // by and large, and are loaded with the streaming cache policy (first GEMM of the Qwen3-30B-A3B
 // layer at 512 tokens 132 -> 74 us).  With several token blocks per expert the blocks share the
 // weights through L2 and the default policy is the faster one.
-template <bool FUSED_ACT, int ORD, int WT, bool STREAM = false>
+template <int FUSED_ACT, int ORD, int WT, bool STREAM = false>
 __global__ __launch_bounds__(256 * WT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   static_assert(!STREAM || WT == 1, "streaming policy: 64-token tiles");
@@ -278,7 +278,7 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
           acc[tb][1][i] = acc[tb][1][i] * w;
         }
       }
-      silu_mul_bf16<16>(acc[tb][0], acc[tb][1], actf[tb]);
+      gated_act<FUSED_ACT, 16>(a, acc[tb][0], acc[tb][1], actf[tb]);
 #pragma unroll
       for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(actf[tb][i]));
       amax = fmaxf(amax, __shfl_xor(amax, 32));
@@ -348,8 +348,8 @@ int launch_gemm_tile(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     else                                               \
       hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 1>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
   } while (0)
-  if (fused_act) LO_ORD_DISPATCH(ord, LO_TILE_LAUNCH, true);
-  else LO_ORD_DISPATCH(ord, LO_TILE_LAUNCH, false);
+  if (fused_act) LO_FUSED_DISPATCH(a, ord, LO_TILE_LAUNCH);
+  else LO_ORD_DISPATCH(ord, LO_TILE_LAUNCH, 0);
 #undef LO_TILE_LAUNCH
   return check_launch(fused_act ? "moe_gemm1_silu_quant(tile)" : "moe_gemm(tile)");
 }

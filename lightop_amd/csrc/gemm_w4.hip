@@ -33,7 +33,7 @@ constexpr int kW4Row = 144; // LDS row pitch in bytes: 128 + 16 keeps ds_read_b1
 // loaded with the streaming cache policy (first GEMM of a 4096 x 1536 layer with 16 or 32 slots per
 // expert: 227 -> 180 us).  With several token blocks per expert the blocks share the weights through
 // L2 and the default policy is the faster one.
-template <bool FUSED_ACT, int ORD, bool STREAM>
+template <int FUSED_ACT, int ORD, bool STREAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   constexpr int kTileM = 64;
@@ -316,7 +316,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
           gv[i] = acc[g][tf][i] * w;
           uv[i] = acc[2 + g][tf][i] * w;
         }
-        silu_mul_bf16<4>(gv, uv, actf[tf][g]);
+        gated_act<FUSED_ACT, 4>(a, gv, uv, actf[tf][g]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(actf[tf][g][i]));
       }
@@ -390,8 +390,8 @@ int launch_gemm_w4_tile(const GemmArgs &a0, bool fused_act, int flags, int64_t m
     if (stream) LO_W4_TILE_LAUNCH(FA, FS, true); \
     else LO_W4_TILE_LAUNCH(FA, FS, false);   \
   } while (0)
-  if (fused_act) LO_ORD_DISPATCH(ord, LO_W4_TILE_PICK, true);
-  else LO_ORD_DISPATCH(ord, LO_W4_TILE_PICK, false);
+  if (fused_act) LO_FUSED_DISPATCH(a, ord, LO_W4_TILE_PICK);
+  else LO_ORD_DISPATCH(ord, LO_W4_TILE_PICK, 0);
 #undef LO_W4_TILE_PICK
 #undef LO_W4_TILE_LAUNCH
   return check_launch(fused_act ? "moe_gemm1_silu_quant(w4 tile)" : "moe_gemm(w4 tile)");

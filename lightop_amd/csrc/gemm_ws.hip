@@ -53,7 +53,7 @@ namespace lo {
 // python/lightop/_lmslim_native/layers/fused_moe/w4a8.py:341-395): the nibbles enter the sum as
 // int8(nibble << 4), the factor 16 stays in it, and C = bf16(((f32(d) [* topk_w[f]]) * As[row])
 // * Ws[e, n]).
-template <int TM, bool FUSED_ACT, int ORD, bool SHUF, int NWAVES, int PD, int RPW, bool W4 = false,
+template <int TM, int FUSED_ACT, int ORD, bool SHUF, int NWAVES, int PD, int RPW, bool W4 = false,
           bool PC = false>
 __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs a) {
   static_assert(!W4 || SHUF, "int4 weights exist in the load-time layout only");
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
         g[i] = acc[0][j][i] * w;
         u[i] = acc[NW - 1][j][i] * w;
       }
-      silu_mul_bf16<4>(g, u, actf[j]);
+      gated_act<FUSED_ACT, 4>(a, g, u, actf[j]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fabsf(actf[j][i]));
       amax = fmaxf(amax, __shfl_xor(amax, 16));
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   }
 }
 
-template <int TM, bool FUSED_ACT, int ORD>
+template <int TM, int FUSED_ACT, int ORD>
 static int launch_ws(const GemmArgs &a0, int64_t m_blocks, hipStream_t s) {
   constexpr int NWAVES = FUSED_ACT ? 8 : LO_WS_PLAIN_WAVES;
   // A plain-GEMM wave takes RPW consecutive 16-row fragments so that it streams a few
@@ -477,7 +477,7 @@ static int launch_ws(const GemmArgs &a0, int64_t m_blocks, hipStream_t s) {
   return LO_OK;
 }
 
-template <bool FUSED_ACT>
+template <int FUSED_ACT>
 static int dispatch_ws(const GemmArgs &a, int bs, int flags, int64_t m_blocks, hipStream_t s) {
   // per-channel scales are applied once, in the epilogue: one instantiation (tagged kOrdSeparate)
   const int ord = a.per_channel ? kOrdSeparate : scale_order(flags);
@@ -504,8 +504,8 @@ static int dispatch_ws(const GemmArgs &a, int bs, int flags, int64_t m_blocks, h
 
 int launch_gemm_ws(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks,
                    hipStream_t s) {
-  return fused_act ? dispatch_ws<true>(a, block_size_m, flags, m_blocks, s)
-                   : dispatch_ws<false>(a, block_size_m, flags, m_blocks, s);
+  return fused_act ? dispatch_ws<kActSiluBf16>(a, block_size_m, flags, m_blocks, s)
+                   : dispatch_ws<0>(a, block_size_m, flags, m_blocks, s);
 }
 
 } // namespace lo
