@@ -528,20 +528,29 @@ static int fused_experts_channel(
                                     sorted, L.sorted_cap, eids, L.blocks_cap, ntpp, mask, ws + L.off[8],
                                     L.align_scratch, stream);
   if (rc) return rc;
-  // rows of experts on other ranks are zero-filled here: the activation kernel reads every row
   const int gflags = flags & ~LO_FUSED_ACT_GELU;
-  rc = lo_moe_gemm_w8a8(a1q, a1s, w1, w1s, cache13, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
-                        num_experts, 2 * I, H, top_k, block_size_m, apply_router_weight_on_input, gflags, stream);
+  const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
+  const bool gated = gated_channel_supports(H, block_size_m, flags);
+  const uint16_t *table = nullptr;
+  if (gated && (gelu || dtype == LO_F16)) {
+    rc = act_table(static_cast<hipStream_t>(stream), gelu ? LO_ACT_GELU : LO_ACT_SILU, dtype, &table);
+    if (rc) return rc;
+  }
+  // rows of slots whose expert another rank holds are neither written by the first stage nor read by the quantisation
+  const int local_only = mask ? LO_GEMM_SKIP_NONLOCAL : 0;
+  rc = launch_gemm_w8a8(a1q, a1s, w1, w1s, cache13, dtype, !gated ? 0 : table ? kActTable : kActSiluBf16, table, topk_w,
+                        sorted, eids, ntpp, L.sorted_cap, S, M, E, num_experts, 2 * I, H, top_k, block_size_m,
+                        apply_router_weight_on_input, gflags | local_only, static_cast<hipStream_t>(stream));
   if (rc) return rc;
-  if (flags & LO_FUSED_ACT_GELU) // gelu_and_mul, then per_token_quant_int8 with its floor (int8.py:826-838)
-    rc = launch_act_mul_row_quant(cache13, dtype, LO_ACT_GELU, S, I, a2q, a2s, nullptr, 1, nullptr,
-                                  static_cast<hipStream_t>(stream));
-  else
-    rc = lo_fuse_silu_mul_quant(cache13, dtype, S, I, a2q, a2s, nullptr, 1, stream);
+  if (gated)
+    rc = launch_act_rows_quant(cache13, dtype, gelu, S, I, a2q, a2s, mask, static_cast<hipStream_t>(stream));
+  else // GELU: gelu_and_mul, then per_token_quant_int8 with its floor (int8.py:826-838)
+    rc = launch_act_mul_row_quant(cache13, dtype, gelu ? LO_ACT_GELU : LO_ACT_SILU, S, I, a2q, a2s, nullptr, 1, nullptr,
+                                  mask, static_cast<hipStream_t>(stream));
   if (rc) return rc;
   rc = lo_moe_gemm_w8a8(a2q, a2s, w2, w2s, cache13, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, S, E,
                         num_experts, H, I, 1, block_size_m, !apply_router_weight_on_input,
-                        gflags | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), stream);
+                        gflags | local_only, stream);
   if (rc) return rc;
   return lo_moe_sum(cache13, out, shared_output, mask, dtype, M, top_k, H, routed_scaling_factor, nullptr,
                     stream);

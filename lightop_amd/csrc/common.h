@@ -55,7 +55,11 @@ int launch_moe_sum_f32(const float *in, float *out, const float *bias, const uin
                        int64_t H, float factor, const int32_t *num_local_tokens, hipStream_t stream);
 int launch_act_mul_row_quant(const void *c1, int dtype, int act, int64_t rows, int64_t I, int8_t *q, float *s,
                              const int32_t *num_local_tokens, int32_t top_k, const int32_t *row_ids,
-                             hipStream_t stream);
+                             const uint8_t *row_mask, hipStream_t stream);
+
+// The per-token quantisation alone, of activations [rows, I] that a gated first stage left; floored as above.
+int launch_act_rows_quant(const void *act, int dtype, bool floored, int64_t rows, int64_t I, int8_t *q, float *s,
+                          const uint8_t *row_mask, hipStream_t stream);
 
 // Raises a kernel's dynamic-LDS limit once per device instead of on every launch (kernels that use
 // more than the default 64 KB).  `done` is the call site's own static flag set, one bit per device.

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void act_mul_group_quant_kernel(const uint16_t
 // longer rows are read a second time.
 // ACT: 0 plain rows; 1 SiLU-and-mul first (the fused kernel above: no floor), bf16 only, computed; 2 a gated activation from its full table first (`silu` being that table),
 // then per_token_quant_int8 with its floor (GELU: the two calls at int8.py:826-838 on the per-channel
-// branch); 3 as 2 without the floor (SiLU for fp16 rows).
+// branch); 3 as 2 without the floor (SiLU for fp16 rows); 4 plain rows without the floor (behind SiLU-and-mul elsewhere).
 __device__ __forceinline__ void silu_mul_bf16_raw(const v8u16 g16, const v8u16 u16, float (&act)[8]) {
   float g[8], u[8];
 #pragma unroll
@@ -125,9 +125,10 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const uint16_t *__restri
                                                         const uint16_t *__restrict__ silu, int8_t *__restrict__ q,
                                                         float *__restrict__ s,
                                                         const int32_t *__restrict__ num_local_tokens, int32_t top_k,
-                                                        const int32_t *__restrict__ row_ids) {
+                                                        const int32_t *__restrict__ row_ids,
+                                                        const uint8_t *__restrict__ row_mask) {
   static_assert(ACT != 1 || DT == LO_BF16, "SiLU is computed for bf16 rows");
-  constexpr bool SILU = ACT == 1, GATED = ACT != 0, FLOOR = ACT == 0 || ACT == 2;
+  constexpr bool SILU = ACT == 1, GATED = ACT != 0 && ACT != 4, FLOOR = ACT == 0 || ACT == 2;
   __shared__ float sRed[4];
   const int tid = threadIdx.x;
   if (num_local_tokens) { // rows of padding tokens are left untouched
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(256) void row_quant_kernel(const uint16_t *__restri
   const int64_t in_stride = GATED ? 2 * C : C; // C = output columns
   const int pieces = static_cast<int>(C / 8);
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
-    if (row_ids && row_ids[row] == -1) continue; // a row of an expert held elsewhere: left untouched
+    if ((row_ids && row_ids[row] == -1) || (row_mask && !row_mask[row])) continue; // of an expert held elsewhere: left untouched
     const uint16_t *xr = x + row * in_stride;
     auto piece = [&](int p, float (&v)[8]) {
       const v8u16 a = *reinterpret_cast<const v8u16 *>(xr + p * 8);
@@ -212,9 +213,10 @@ __global__ __launch_bounds__(256) void row_quant_wave_kernel(const uint16_t *__r
                                                              const uint16_t *__restrict__ silu,
                                                              int8_t *__restrict__ q, float *__restrict__ s,
                                                              const int32_t *__restrict__ num_local_tokens,
-                                                             int32_t top_k, const int32_t *__restrict__ row_ids) {
+                                                             int32_t top_k, const int32_t *__restrict__ row_ids,
+                                                        const uint8_t *__restrict__ row_mask) {
   static_assert(ACT != 1 || DT == LO_BF16, "SiLU is computed for bf16 rows");
-  constexpr bool SILU = ACT == 1, GATED = ACT != 0, FLOOR = ACT == 0 || ACT == 2;
+  constexpr bool SILU = ACT == 1, GATED = ACT != 0 && ACT != 4, FLOOR = ACT == 0 || ACT == 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (num_local_tokens) {
     const int64_t n = static_cast<int64_t>(num_local_tokens[0]) * top_k;
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(256) void row_quant_wave_kernel(const uint16_t *__r
   const int64_t in_stride = GATED ? 2 * C : C;
   const int pieces = static_cast<int>(C / 8);
   for (int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + wave; row < rows; row += static_cast<int64_t>(gridDim.x) * 4) {
-    if (row_ids && row_ids[row] == -1) continue; // a row of an expert held elsewhere: left untouched
+    if ((row_ids && row_ids[row] == -1) || (row_mask && !row_mask[row])) continue; // of an expert held elsewhere: left untouched
     const uint16_t *xr = x + row * in_stride;
     v8u16 ga[CH], up[CH];
 #pragma unroll
@@ -272,20 +274,20 @@ __global__ __launch_bounds__(256) void row_quant_wave_kernel(const uint16_t *__r
 
 template <int ACT, int DT = LO_BF16>
 static void launch_row_quant(const uint16_t *x, int64_t rows, int64_t C, const uint16_t *silu, int8_t *q, float *s,
-                             const int32_t *nlt, int32_t top_k, const int32_t *row_ids, hipStream_t st) {
+                             const int32_t *nlt, int32_t top_k, const int32_t *row_ids, hipStream_t st, const uint8_t *row_mask = nullptr) {
   const int pieces = static_cast<int>(C / 8);
   if (pieces <= 256 && rows >= 4) {
     int64_t grid = (rows + 3) / 4;
     if (grid > 256 * 32) grid = 256 * 32;
     const dim3 g(static_cast<unsigned>(grid)), b(256);
-    if (pieces <= 64) hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 1, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids);
-    else if (pieces <= 128) hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 2, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids);
-    else hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 4, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids);
+    if (pieces <= 64) hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 1, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids, row_mask);
+    else if (pieces <= 128) hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 2, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids, row_mask);
+    else hipLaunchKernelGGL((row_quant_wave_kernel<ACT, 4, DT>), g, b, 0, st, x, rows, C, silu, q, s, nlt, top_k, row_ids, row_mask);
     return;
   }
   const unsigned grid = static_cast<unsigned>(rows < 65536 ? rows : 65536);
-  hipLaunchKernelGGL((row_quant_kernel<ACT, ACT ? 2 : 4, DT>), dim3(grid), dim3(256), 0, st, x, rows, C, silu, q, s, nlt,
-                     top_k, row_ids);
+  hipLaunchKernelGGL((row_quant_kernel<ACT, ACT && ACT != 4 ? 2 : 4, DT>), dim3(grid), dim3(256), 0, st, x, rows, C, silu, q, s, nlt,
+                     top_k, row_ids, row_mask);
 }
 
 // ---- moe_sum -------------------------------------------------------------------
@@ -466,7 +468,7 @@ int launch_act_mul_group_quant(const void *c1, int dtype, int act, int64_t rows,
 // per_token_quant_int8 with its floor.
 int launch_act_mul_row_quant(const void *c1, int dtype, int act, int64_t rows, int64_t I, int8_t *q, float *s,
                              const int32_t *num_local_tokens, int32_t top_k, const int32_t *row_ids,
-                             hipStream_t stream) {
+                             const uint8_t *row_mask, hipStream_t stream) {
   const uint16_t *table = nullptr;
   if (act != LO_ACT_SILU || dtype != LO_BF16) { // (SiLU of bf16 rows is computed)
     const int rc = act_table(stream, act, dtype, &table);
@@ -475,13 +477,26 @@ int launch_act_mul_row_quant(const void *c1, int dtype, int act, int64_t rows, i
   if (rows == 0) return LO_OK;
   const uint16_t *x = static_cast<const uint16_t *>(c1);
   if (dtype == LO_F16) {
-    if (act == LO_ACT_GELU) launch_row_quant<2, LO_F16>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream);
-    else launch_row_quant<3, LO_F16>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream);
+    if (act == LO_ACT_GELU) launch_row_quant<2, LO_F16>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream, row_mask);
+    else launch_row_quant<3, LO_F16>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream, row_mask);
   } else {
-    if (act == LO_ACT_GELU) launch_row_quant<2>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream);
-    else launch_row_quant<1>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream);
+    if (act == LO_ACT_GELU) launch_row_quant<2>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream, row_mask);
+    else launch_row_quant<1>(x, rows, I, table, q, s, num_local_tokens, top_k, row_ids, stream, row_mask);
   }
   return check_launch("act_mul_row_quant");
+}
+
+int launch_act_rows_quant(const void *act, int dtype, bool floored, int64_t rows, int64_t I, int8_t *q, float *s,
+                          const uint8_t *row_mask, hipStream_t stream) {
+  if (rows == 0) return LO_OK;
+  const uint16_t *x = static_cast<const uint16_t *>(act);
+#define LO_ACT_ROWS(ACT, DT) launch_row_quant<ACT, DT>(x, rows, I, nullptr, q, s, nullptr, 1, nullptr, stream, row_mask)
+  if (dtype == LO_F16 && floored) LO_ACT_ROWS(0, LO_F16);
+  else if (dtype == LO_F16) LO_ACT_ROWS(4, LO_F16);
+  else if (floored) LO_ACT_ROWS(0, LO_BF16);
+  else LO_ACT_ROWS(4, LO_BF16);
+#undef LO_ACT_ROWS
+  return check_launch("act_rows_quant");
 }
 
 int silu_table(hipStream_t stream, const uint16_t **out) {
@@ -701,7 +716,7 @@ extern "C" int lo_fuse_silu_mul_quant_ids(const void *c1, int dtype, int64_t row
              LO_EINVAL, "fuse_silu_mul_quant: input must be 16-byte and q 8-byte aligned");
   if (rows == 0) return LO_OK;
   return launch_act_mul_row_quant(c1, dtype, LO_ACT_SILU, rows, I, q, s, num_local_tokens, top_k, row_expert_ids,
-                                  static_cast<hipStream_t>(stream));
+                                  nullptr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int lo_fuse_silu_mul_quant(const void *c1, int dtype, int64_t rows, int64_t I, int8_t *q, float *s,

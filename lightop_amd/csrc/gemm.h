@@ -78,6 +78,23 @@ inline bool fused_table_supports(int64_t K, int block_size_m, int flags) {
   const bool rows = !(flags & (LO_GEMM_W_PRESHUFFLED | LO_GEMM_W4));
   return block_size_m == 64 || block_size_m == 128 || (rows && (block_size_m == 16 || block_size_m == 32));
 }
+// Per-channel scales: a first stage that ends with the gated activation in 16 bits, C [num_valid, I], instead of gate and up
+// (the row's quantisation follows in its own launch either way).  From 64 tokens on, where the kernels are not the
+// weight-streaming one.  Plain / gated, whole path, us: Qwen3-30B-A3B-shaped layer at 300 tokens 127.7 / 124.0, at 700:
+// 147.6 / 141.0, at 8000: 555 / 525, fp16 608 / 572; int4 at 300 tokens of the Qwen3-235B-A22B-shaped layer 252 / 245, at 6000:
+// 1100 / 1061.
+inline bool gated_channel_supports(int64_t K, int block_size_m, int flags) {
+  if (flags & LO_GEMM_FORCE_STREAMING) return false;
+  if (flags & LO_GEMM_W4) return block_size_m >= 128 && K <= 128 * kGroup;
+  return block_size_m >= 64;
+}
+// Launcher macro MACRO(FUSED_ACT) of a per-channel GEMM.
+#define LO_GATED_DISPATCH(a, fused_act, MACRO)                        \
+  do {                                                                \
+    if (!(fused_act)) MACRO(0);                                       \
+    else if ((a).fused == ::lo::kActTable) MACRO(::lo::kActTable);    \
+    else MACRO(::lo::kActSiluBf16);                                   \
+  } while (0)
 // Launcher macro MACRO(scale order, FUSED_ACT) for a fused first stage.
 #define LO_FUSED_DISPATCH(a, ord, MACRO)                                                \
   do {                                                                                  \
@@ -252,6 +269,12 @@ void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_wa
 int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t stream);
 
 // Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
+// lo_moe_gemm_w8a8, and with `fused` its gated form (N = 2I, C [num_valid, I]).
+int launch_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype, int fused,
+                     const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
+                     const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
+                     int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
+                     int flags, hipStream_t stream);
 // The fused first stage with a given activation (lo_moe_gemm1_silu_quant_block_int8 is this with kActSiluBf16).
 int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
                            int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,
@@ -278,7 +301,7 @@ int launch_gemm_rows(const GemmArgs &a, bool fused_act, int block_size_m, int fl
 int launch_gemm_w4_tile(const GemmArgs &a, bool fused_act, int flags, int64_t m_blocks, hipStream_t s);
 bool gemm_w4_tile_supports(const GemmArgs &a, bool fused_act, int block_size_m);
 // Per-channel LDS-tiled kernel (gemm_pc.hip): block_size_m 64 or 128.
-int launch_gemm_pc(const GemmArgs &a, int block_size_m, int64_t m_blocks, hipStream_t s);
+int launch_gemm_pc(const GemmArgs &a, bool fused_act, int block_size_m, int64_t m_blocks, hipStream_t s);
 bool gemm_pc_supports(const GemmArgs &a, int block_size_m);
 
 } // namespace lo

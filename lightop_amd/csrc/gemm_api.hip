@@ -92,7 +92,7 @@ static int launch_gemm(const GemmArgs &a, bool fused_act, int bs, int flags, int
   switch (pick_gemm_kernel(a, fused_act, bs, flags)) {
   case LO_KERNEL_T128: return launch_gemm_t128(a, fused_act, bs, flags, m_blocks, s);
   case LO_KERNEL_W4_TILE: return launch_gemm_w4_tile(a, fused_act, flags, m_blocks, s);
-  case LO_KERNEL_PC: return launch_gemm_pc(a, bs, m_blocks, s);
+  case LO_KERNEL_PC: return launch_gemm_pc(a, fused_act, bs, m_blocks, s);
   case LO_KERNEL_AS: return launch_gemm_as(a, flags, bs, m_blocks, s);
   case LO_KERNEL_TILE: return launch_gemm_tile(a, fused_act, bs, flags, m_blocks, s);
   default: return launch_gemm_ws(a, fused_act, bs, flags, m_blocks, s);
@@ -206,13 +206,12 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
                                 block_size_m, mul_routed, flags, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int lo_moe_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws,
-                                void *C, int c_dtype, const float *topk_w, const int32_t *sorted_ids,
-                                const int32_t *expert_ids, const int32_t *num_tokens_post_pad,
-                                int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
-                                int32_t num_experts, int64_t N, int64_t K, int32_t top_k,
-                                int32_t block_size_m, int mul_routed, int flags, lo_stream_t stream) {
-  using namespace lo;
+namespace lo {
+int launch_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype, int fused,
+                     const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
+                     const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
+                     int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
+                     int flags, hipStream_t stream) {
   int rc = validate_common("moe_gemm_w8a8", A, As, W, Ws, sorted_ids, expert_ids, num_tokens_post_pad, K,
                            top_k, E, a_rows);
   if (rc) return rc;
@@ -241,14 +240,28 @@ extern "C" int lo_moe_gemm_w8a8(const int8_t *A, const float *As, const int8_t *
   a.w_shuffled = (flags & LO_GEMM_W_PRESHUFFLED) ? 1 : 0;
   a.skip_nonlocal = (flags & LO_GEMM_SKIP_NONLOCAL) ? 1 : 0;
   a.per_channel = 1;
+  a.fused = fused; a.act_table = act_table;
   a.out_f16 = c_dtype == LO_F16 ? 1 : 0;
   a.w4 = (flags & LO_GEMM_W4) ? 1 : 0;
   a.n_tiles = static_cast<int32_t>((N + 63) / 64);
-  LO_REQUIRE(block_size_m != 160 || gemm_t128_supports(a, false, 160), LO_ENOTSUP,
+  LO_REQUIRE(!fused || (N % (2 * kGroup) == 0 && gated_channel_supports(K, block_size_m, flags)), LO_ENOTSUP,
+             "moe_gemm_w8a8: no gated form at this block size");
+  LO_REQUIRE(block_size_m != 160 || gemm_t128_supports(a, fused != 0, 160), LO_ENOTSUP,
              "moe_gemm_w8a8: 160-token blocks need N a multiple of 64 and K <= %d", kGroup * 128);
   const int64_t mblocks = grid_m_blocks(sorted_cap, num_valid, block_size_m);
   LO_REQUIRE(mblocks * a.n_tiles < (1ll << 30), LO_EINVAL, "moe_gemm_w8a8: grid too large");
   if (mblocks == 0) return LO_OK;
-  return launch_gemm(a, false, block_size_m, flags & ~(LO_GEMM_FUSED_SCALE | LO_GEMM_SEPARATE_ORDER), mblocks,
-                     static_cast<hipStream_t>(stream));
+  return launch_gemm(a, fused != 0, block_size_m, flags & ~(LO_GEMM_FUSED_SCALE | LO_GEMM_SEPARATE_ORDER), mblocks, stream);
+}
+} // namespace lo
+
+extern "C" int lo_moe_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws,
+                                void *C, int c_dtype, const float *topk_w, const int32_t *sorted_ids,
+                                const int32_t *expert_ids, const int32_t *num_tokens_post_pad,
+                                int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
+                                int32_t num_experts, int64_t N, int64_t K, int32_t top_k,
+                                int32_t block_size_m, int mul_routed, int flags, lo_stream_t stream) {
+  return lo::launch_gemm_w8a8(A, As, W, Ws, C, c_dtype, 0, nullptr, topk_w, sorted_ids, expert_ids, num_tokens_post_pad,
+                              sorted_cap, num_valid, a_rows, E, num_experts, N, K, top_k, block_size_m, mul_routed, flags,
+                              static_cast<hipStream_t>(stream));
 }

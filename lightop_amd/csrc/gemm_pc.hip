@@ -25,7 +25,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kPcRow = 144; // LDS row pitch in bytes: 128 + 16 keeps ds_read_b128 conflict-free
 
-template <int TB, bool STREAM>
+template <int TB, bool STREAM, int FUSED_ACT>
 __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks, int group_m) {
   constexpr int kWAux = STREAM ? kCacheStream : kCacheDefault;
   constexpr int kTileM = 32 * TB;       // tokens per workgroup
@@ -54,11 +54,13 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
     f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 32 + r];
     valid[tb] = f[tb] < a.num_valid;
   }
+  const int64_t I = N / 2; // gated: 32 gate rows per wave and the matching 32 up rows
   int64_t nrow[2];
-  nrow[0] = static_cast<int64_t>(nt) * 256 + wr * 64;
-  nrow[1] = nrow[0] + 32;
-  const bool wave_active = nrow[0] < N; // N % 64 == 0 is checked on the host
+  nrow[0] = FUSED_ACT ? static_cast<int64_t>(nt) * kGroup + wr * 32 : static_cast<int64_t>(nt) * 256 + wr * 64;
+  nrow[1] = nrow[0] + (FUSED_ACT ? I : 32);
+  const bool wave_active = FUSED_ACT || nrow[0] < N; // N % 64 == 0 is checked on the host
 
+  if (FUSED_ACT && e < 0) return; // nothing of these rows is read
   if (e < 0) { // expert of another rank: its rows are defined to be zero
     if (wave_active && (!a.skip_nonlocal || e_oob)) {
 #pragma unroll
@@ -182,6 +184,35 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
       ts = a.As[token_row(a, f[tb])];
       if (a.mul_routed) ts = a.topk_w[f[tb]] * ts;
     }
+    if constexpr (FUSED_ACT) {
+      // the gated activation in 16 bits (its quantisation needs the whole row): a 32-token x 32-column piece per wave
+      float gu[2][16], act[16];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) gu[rb][i] = (static_cast<float>(acc[tb][rb][i]) * ts) * bs4[rb][i >> 2][i & 3];
+      gated_act<FUSED_ACT, 16>(a, gu[0], gu[1], act);
+      with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v4u16 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = cvt(act[4 * q + i]);
+          *reinterpret_cast<v4u16 *>(stg + r * kStgPitch + (8 * q + 4 * c) * 2) = o;
+        }
+      });
+      __builtin_amdgcn_wave_barrier();
+      const int slot = valid[tb] ? static_cast<int>(f[tb]) : -1;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int tok = (lane >> 2) + 16 * j;
+        const v4i v = *reinterpret_cast<const v4i *>(stg + tok * kStgPitch + (lane & 3) * 16);
+        const int ft = __shfl(slot, tok);
+        if (ft >= 0) *reinterpret_cast<v4i *>(a.C + static_cast<int64_t>(ft) * I + nrow[0] + (lane & 3) * 8) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
     v4u16 o[2][4];
     with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
@@ -200,24 +231,24 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
 
 // 128 tokens: 246 registers, two waves per SIMD.  64 tokens: 162 registers, so three workgroups
 // fit a compute unit and hide each other's barrier and memory waits better than two.
-template <bool STREAM>
+template <bool STREAM, int FUSED_ACT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_pc_kernel_128(const GemmArgs a, int m_blocks, int group_m) {
-  moe_gemm_pc_body<4, STREAM>(a, m_blocks, group_m);
+  moe_gemm_pc_body<4, STREAM, FUSED_ACT>(a, m_blocks, group_m);
 }
-template <bool STREAM>
+template <bool STREAM, int FUSED_ACT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void moe_gemm_pc_kernel_64(const GemmArgs a, int m_blocks, int group_m) {
-  moe_gemm_pc_body<2, STREAM>(a, m_blocks, group_m);
+  moe_gemm_pc_body<2, STREAM, FUSED_ACT>(a, m_blocks, group_m);
 }
 
 bool gemm_pc_supports(const GemmArgs &a, int block_size_m) {
   return a.per_channel && a.w_shuffled && (block_size_m == 64 || block_size_m == 128) && a.N % 64 == 0;
 }
 
-int launch_gemm_pc(const GemmArgs &a0, int block_size_m, int64_t m_blocks, hipStream_t s) {
+int launch_gemm_pc(const GemmArgs &a0, bool fused_act, int block_size_m, int64_t m_blocks, hipStream_t s) {
   GemmArgs a = a0;
-  a.n_tiles = static_cast<int32_t>((a.N + 255) / 256);
+  a.n_tiles = fused_act ? static_cast<int32_t>(a.N / 2 / kGroup) : static_cast<int32_t>((a.N + 255) / 256);
   // every chunk of G token blocks owns G * n_tiles consecutive slots on one XCD
   int64_t G = a.num_valid / (static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * block_size_m);
   G = G < 2 ? 2 : (G > 16 ? 16 : G);
@@ -230,13 +261,17 @@ int launch_gemm_pc(const GemmArgs &a0, int block_size_m, int64_t m_blocks, hipSt
   // (as measured for the block form's 64-token kernel), half a block with 128-token blocks
   const bool stream = a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) *
                                          (block_size_m == 64 ? 48 : 64);
-#define LO_PC_LAUNCH(KERN)                                                                    \
-  do {                                                                                        \
-    if (stream) hipLaunchKernelGGL((KERN<true>), g, b, 0, s, a, mbi, gi);                     \
-    else hipLaunchKernelGGL((KERN<false>), g, b, 0, s, a, mbi, gi);                           \
+#define LO_PC_LAUNCH(FA)                                                                                             \
+  do {                                                                                                               \
+    if (block_size_m == 128) {                                                                                       \
+      if (stream) hipLaunchKernelGGL((moe_gemm_pc_kernel_128<true, FA>), g, b, 0, s, a, mbi, gi);                    \
+      else hipLaunchKernelGGL((moe_gemm_pc_kernel_128<false, FA>), g, b, 0, s, a, mbi, gi);                          \
+    } else {                                                                                                         \
+      if (stream) hipLaunchKernelGGL((moe_gemm_pc_kernel_64<true, FA>), g, b, 0, s, a, mbi, gi);                     \
+      else hipLaunchKernelGGL((moe_gemm_pc_kernel_64<false, FA>), g, b, 0, s, a, mbi, gi);                           \
+    }                                                                                                                \
   } while (0)
-  if (block_size_m == 128) LO_PC_LAUNCH(moe_gemm_pc_kernel_128);
-  else LO_PC_LAUNCH(moe_gemm_pc_kernel_64);
+  LO_GATED_DISPATCH(a, fused_act, LO_PC_LAUNCH);
 #undef LO_PC_LAUNCH
   return check_launch("moe_gemm_w8a8(tile)");
 }

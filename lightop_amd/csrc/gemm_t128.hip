@@ -76,8 +76,8 @@ __device__ __forceinline__ void wait_copies_barrier() {
 template <int FUSED_ACT, int ORD, bool STREAM, bool W4, bool PC = false, int NTB = 8, bool ROWS = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 4 : NTB <= 4 ? 3 : 2, NTB == 1 ? 4 : NTB <= 4 ? 3 : 2)))
 void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
-  static_assert(!PC || (!FUSED_ACT && ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
-                "per-channel scales: plain GEMM, int4 weights, 160-token tiles of int8 weights or row-major ones");
+  static_assert(!PC || (ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
+                "per-channel scales: int4 weights, 160-token tiles of int8 weights or row-major ones");
   static_assert(NTB == 8 || (NTB == 10 && (PC || !W4)) || ((NTB == 1 || NTB == 2 || NTB == 4) && ROWS),
                 "160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales; 16, 32 and 64 tokens: "
                 "row-major weights");
@@ -633,6 +633,53 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       }
       __builtin_amdgcn_wave_barrier();
     }
+  } else if constexpr (PC) {
+    // The gated activation of a per-channel first stage, in 16 bits: its quantisation needs the whole row.  Gate and up meet
+    // here, so that half as much is written and read back as with a plain first stage, and by a launch without the activation.
+    int8_t *stg = sWw;
+    v4f pbs[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int rf = 0; rf < 2; ++rf)
+        pbs[h][rf] = __builtin_bit_cast(v4f, bld16(rWs, static_cast<int>(((rf ? I : 0) + nrow0 + h * 16 + 4 * q) * 4), 0));
+    float pas[NTB];
+#pragma unroll
+    for (int tb = 0; tb < NTB; ++tb) pas[tb] = bld_f32(rAs, static_cast<int>(token_row(a, sIds[tb * 16 + r]) * 4), 0);
+#pragma unroll
+    for (int tb = 0; tb < NTB; ++tb) {
+      if (2 * tb >= nst) continue;
+      const int64_t ft = sIds[tb * 16 + r];
+      const bool valid = ft < a.num_valid;
+      float wgt = 1.0f;
+      if (a.mul_routed && valid) wgt = a.topk_w[ft];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float gu[2][4], act[4];
+#pragma unroll
+        for (int rf = 0; rf < 2; ++rf)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) { // the orders of the plain epilogue above; a weight of one changes nothing
+            float v = static_cast<float>(acci[h][tb][rf][i]);
+            if constexpr (W4) v = (v * wgt) * pas[tb];
+            else v = v * (wgt * pas[tb]);
+            gu[rf][i] = v * pbs[h][rf][i];
+          }
+        gated_act<FUSED_ACT, 4>(a, gu[0], gu[1], act);
+        v4u16 o;
+        with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = cvt(act[i]);
+        });
+        *reinterpret_cast<v4u16 *>(stg + r * kTPitch + (h * 16 + 4 * q) * 2) = o;
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int slot = valid ? static_cast<int>(ft) : -1, tok = lane >> 2;
+      const v4i v = *reinterpret_cast<const v4i *>(stg + tok * kTPitch + (lane & 3) * 16);
+      const int fs = __shfl(slot, tok);
+      if (fs >= 0) *reinterpret_cast<v4i *>(a.C + static_cast<int64_t>(fs) * I + nrow0 + (lane & 3) * 8) = v;
+      __builtin_amdgcn_wave_barrier();
+    }
   } else {
     // acc[h][tb][0] = gate, acc[h][tb][1] = up for activation columns nt*128 + wave*32 + 16h + 4q + i
     float actf[NTB][2][4];
@@ -708,11 +755,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
 bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   if (block_size_m == kT160) { // 160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales
     if (!a.w_shuffled || a.K / kGroup > kTMaxKB) return false;
-    if (fused_act) return !a.per_channel && !a.w4;
-    return (a.per_channel || !a.w4) && a.N % 64 == 0;
+    return (a.per_channel || !a.w4) && (fused_act || a.N % 64 == 0);
   }
   if (block_size_m != 128 || !a.w_shuffled) return false;
-  if (a.per_channel && (!a.w4 || fused_act)) return false; // int8 per-channel weights have gemm_pc.hip
+  if (a.per_channel && !a.w4) return false; // int8 per-channel weights have gemm_pc.hip
   if (!fused_act && a.N % 64 != 0) return false;
   return a.K / kGroup <= kTMaxKB;
 }
@@ -760,8 +806,13 @@ static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, 
     else LO_ROWS_LAUNCH2(ORD, FA, false, false);                                                                \
   } while (0)
   if (a.per_channel) { // one order only: the scales meet in the epilogue
-    if (stream) LO_ROWS_LAUNCH2(kOrdSeparate, false, true, true);
-    else LO_ROWS_LAUNCH2(kOrdSeparate, false, false, true);
+#define LO_ROWS_LAUNCH_PC(FA)                                           \
+  do {                                                                  \
+    if (stream) LO_ROWS_LAUNCH2(kOrdSeparate, FA, true, true);          \
+    else LO_ROWS_LAUNCH2(kOrdSeparate, FA, false, true);                \
+  } while (0)
+    LO_GATED_DISPATCH(a, fused_act, LO_ROWS_LAUNCH_PC);
+#undef LO_ROWS_LAUNCH_PC
   } else if (fused_act) {
     LO_FUSED_DISPATCH(a, ord, LO_ROWS_LAUNCH);
   } else {
@@ -814,13 +865,23 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     if (rc_lds) return rc_lds;                                                                                  \
     hipLaunchKernelGGL((moe_gemm_t128_kernel<FA, FS, ST, W>), g, b, kTLds, s, a, mbi, gi);                      \
   } while (0)
-#define LO_T128_LAUNCH_PC(ST)                                                                                   \
+#define LO_T128_LAUNCH_PC2(FA, ST, W, NTB, LDS)                                                                 \
   do {                                                                                                          \
     static unsigned long long lds_done = 0;                                                                     \
-    const int rc_lds = reserve_lds_once(                                                                        \
-        reinterpret_cast<const void *>(&moe_gemm_t128_kernel<false, kOrdSeparate, ST, true, true>), kTLds, &lds_done); \
+    const auto kern = &moe_gemm_t128_kernel<FA, kOrdSeparate, ST, W, true, NTB>;                                \
+    const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), LDS, &lds_done);                  \
     if (rc_lds) return rc_lds;                                                                                  \
-    hipLaunchKernelGGL((moe_gemm_t128_kernel<false, kOrdSeparate, ST, true, true>), g, b, kTLds, s, a, mbi, gi);       \
+    hipLaunchKernelGGL(kern, g, b, LDS, s, a, mbi, gi);                                                         \
+  } while (0)
+#define LO_T128_LAUNCH_PC(FA)                                                                                   \
+  do {                                                                                                          \
+    if (stream) LO_T128_LAUNCH_PC2(FA, true, true, 8, kTLds);                                                   \
+    else LO_T128_LAUNCH_PC2(FA, false, true, 8, kTLds);                                                         \
+  } while (0)
+#define LO_T160_LAUNCH_PC(FA)                                                                                   \
+  do {                                                                                                          \
+    if (a.w4) LO_T128_LAUNCH_PC2(FA, true, true, 10, kTLds160);                                                 \
+    else LO_T128_LAUNCH_PC2(FA, true, false, 10, kTLds160);                                                     \
   } while (0)
 #define LO_T128_PICK(FS, FA)                                                                                    \
   do {                                                                                                          \
@@ -852,18 +913,8 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     if (rc_lds) return rc_lds;                                                                                  \
     hipLaunchKernelGGL((moe_gemm_t128_kernel<FA, FS, true, false, false, 10>), g, b, kTLds160, s, a, mbi, gi);  \
   } while (0)
-    if (a.per_channel && a.w4) {
-      static unsigned long long lds_done = 0;
-      const int rc_lds = reserve_lds_once(
-          reinterpret_cast<const void *>(&moe_gemm_t128_kernel<false, kOrdSeparate, true, true, true, 10>), kTLds160, &lds_done);
-      if (rc_lds) return rc_lds;
-      hipLaunchKernelGGL((moe_gemm_t128_kernel<false, kOrdSeparate, true, true, true, 10>), g, b, kTLds160, s, a, mbi, gi);
-    } else if (a.per_channel) {
-      static unsigned long long lds_done = 0;
-      const int rc_lds = reserve_lds_once(
-          reinterpret_cast<const void *>(&moe_gemm_t128_kernel<false, kOrdSeparate, true, false, true, 10>), kTLds160, &lds_done);
-      if (rc_lds) return rc_lds;
-      hipLaunchKernelGGL((moe_gemm_t128_kernel<false, kOrdSeparate, true, false, true, 10>), g, b, kTLds160, s, a, mbi, gi);
+    if (a.per_channel) {
+      LO_GATED_DISPATCH(a, fused_act, LO_T160_LAUNCH_PC);
     } else if (fused_act) {
       LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, kActSiluBf16);
     } else {
@@ -875,15 +926,16 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   // one token block per expert, by and large: the slots spread over the routed experts fill half a block
   const bool stream = a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * (kT / 2);
   if (a.per_channel) {
-    if (stream) LO_T128_LAUNCH_PC(true);
-    else LO_T128_LAUNCH_PC(false);
+    LO_GATED_DISPATCH(a, fused_act, LO_T128_LAUNCH_PC);
   } else if (fused_act) {
     LO_FUSED_DISPATCH(a, ord, LO_T128_PICK);
   } else {
     LO_ORD_DISPATCH(ord, LO_T128_PICK, 0);
   }
 #undef LO_T128_PICK
+#undef LO_T160_LAUNCH_PC
 #undef LO_T128_LAUNCH_PC
+#undef LO_T128_LAUNCH_PC2
 #undef LO_T128_LAUNCH
   return check_launch(fused_act ? "moe_gemm1_silu_quant(t128)" : "moe_gemm(t128)");
 }
