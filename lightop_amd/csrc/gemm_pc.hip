@@ -34,12 +34,21 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
   __shared__ __attribute__((aligned(16))) int8_t sA[2][kTileM * kPcRow];
 
   int mb, nt;
+  const int E = start_args(a);
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
-  if (static_cast<int64_t>(mb) * kTileM >= a.ntpp[0]) return;
+  const int32_t blocks_end = a.ntpp[0];
+  const int e_raw = a.expert_ids[mb];
+  int32_t ids[TB];
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) ids[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 32 + (threadIdx.x & 31)];
+  const int32_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + threadIdx.x / kThrPerTok];
+  int slots = ids[0];
+#pragma unroll
+  for (int j = 1; j < TB; ++j) slots &= ids[j];
+  if (block_unused(mb * kTileM, blocks_end, e_raw, slots & lf)) return;
   // An expert_map entry outside the weight tensor is treated like an expert of another rank, but its
   // rows are always zero-filled: the slot mask of the alignment counts such a slot as local.
-  const int e_raw = a.expert_ids[mb];
-  const bool e_oob = e_raw >= a.E;
+  const bool e_oob = e_raw >= E;
   const int e = e_oob ? -1 : e_raw;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wr = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of the tile
@@ -51,7 +60,7 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
   bool valid[TB];
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) {
-    f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 32 + r];
+    f[tb] = ids[tb];
     valid[tb] = f[tb] < a.num_valid;
   }
   const int64_t I = N / 2; // gated: 32 gate rows per wave and the matching 32 up rows
@@ -77,7 +86,6 @@ __device__ __forceinline__ void moe_gemm_pc_body(const GemmArgs &a, int m_blocks
 
   // cooperative gather role: thread -> (token, run of kPieces 16-byte pieces of the 128-byte K block)
   const int lt = tid / kThrPerTok, lq = tid % kThrPerTok;
-  const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
   const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const int aoff = static_cast<int>(lrow * K) + lq * (16 * kPieces);

@@ -47,12 +47,19 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   __shared__ float sRed[WT][2][4][32];
 
   int mb, nt;
+  const int E = start_args(a);
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
-  if (static_cast<int64_t>(mb) * kTileM >= a.ntpp[0]) return;
+  const int32_t blocks_end = a.ntpp[0];
+  const int e_raw = a.expert_ids[mb];
+  int32_t ids[2];
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb)
+    ids[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + (threadIdx.x >> 8) * 64 + tb * 32 + (threadIdx.x & 31)];
+  const int32_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + (threadIdx.x >> 2)];
+  if (block_unused(mb * kTileM, blocks_end, e_raw, ids[0] & ids[1] & lf)) return;
   // An expert_map entry outside the weight tensor is treated like an expert of another rank, but its
   // rows are always zero-filled: the slot mask of the alignment counts such a slot as local.
-  const int e_raw = a.expert_ids[mb];
-  const bool e_oob = e_raw >= a.E;
+  const bool e_oob = e_raw >= E;
   const int e = e_oob ? -1 : e_raw;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform: scalar address math
@@ -68,7 +75,7 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   bool valid[2];
 #pragma unroll
   for (int tb = 0; tb < 2; ++tb) {
-    f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + wt * 64 + tb * 32 + r];
+    f[tb] = ids[tb];
     valid[tb] = f[tb] < a.num_valid;
   }
 
@@ -101,7 +108,6 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 
   // cooperative gather role: thread -> (token, 32-byte quarter of the 128-byte K block)
   const int lt = tid >> 2, lq = tid & 3;
-  const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
   const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * KB * 4));

@@ -44,12 +44,18 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   extern __shared__ __attribute__((aligned(16))) float sRowScale[]; // [K block][256 rows], already / 16
 
   int mb, nt;
+  const int E = start_args(a);
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
-  if (static_cast<int64_t>(mb) * kTileM >= a.ntpp[0]) return;
+  const int32_t blocks_end = a.ntpp[0];
+  const int e_raw = a.expert_ids[mb];
+  int32_t ids[4];
+#pragma unroll
+  for (int tf = 0; tf < 4; ++tf) ids[tf] = a.sorted[static_cast<int64_t>(mb) * kTileM + tf * 16 + (threadIdx.x & 15)];
+  const int32_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + (threadIdx.x >> 2)];
+  if (block_unused(mb * kTileM, blocks_end, e_raw, ids[0] & ids[1] & ids[2] & ids[3] & lf)) return;
   // An expert_map entry outside the weight tensor is treated like an expert of another rank, but its
   // rows are always zero-filled: the slot mask of the alignment counts such a slot as local.
-  const int e_raw = a.expert_ids[mb];
-  const bool e_oob = e_raw >= a.E;
+  const bool e_oob = e_raw >= E;
   const int e = e_oob ? -1 : e_raw;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wr = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of the tile
@@ -63,7 +69,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   bool valid[4];
 #pragma unroll
   for (int tf = 0; tf < 4; ++tf) {
-    f[tf] = a.sorted[static_cast<int64_t>(mb) * kTileM + tf * 16 + r];
+    f[tf] = ids[tf];
     valid[tf] = f[tf] < a.num_valid;
   }
 
@@ -91,7 +97,6 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 
   // cooperative gather role: thread -> (token, 32-byte quarter of the 128-byte K block)
   const int lt = tid >> 2, lq = tid & 3;
-  const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
   const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * KB * 4));

@@ -65,13 +65,21 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   // With at most 32 tokens per block an expert's weights are read by one pass only:
   // mark those loads as streaming so that they do not displace the activations in L2.
   constexpr int WAUX = (TM <= LO_WS_STREAM_TM) ? kCacheStream : kCacheDefault;
+  const int E = start_args(a);
   const int bid = blockIdx.x;
   const int mb = bid / a.n_tiles, nt = bid - mb * a.n_tiles;
-  if (static_cast<int64_t>(mb) * BM >= a.ntpp[0]) return;
+  const int32_t blocks_end = a.ntpp[0];
+  const int e_raw = a.expert_ids[mb];
+  int32_t ids[TM];
+#pragma unroll
+  for (int j = 0; j < TM; ++j) ids[j] = a.sorted[static_cast<int64_t>(mb) * BM + j * 16 + (threadIdx.x & 15)];
+  int slots = ids[0];
+#pragma unroll
+  for (int j = 1; j < TM; ++j) slots &= ids[j];
+  if (block_unused(mb * BM, blocks_end, e_raw, slots)) return;
   // An expert_map entry outside the weight tensor is treated like an expert of another rank, but its
   // rows are always zero-filled: the slot mask of the alignment counts such a slot as local.
-  const int e_raw = a.expert_ids[mb];
-  const bool e_oob = e_raw >= a.E;
+  const bool e_oob = e_raw >= E;
   const int e = e_oob ? -1 : e_raw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform: scalar address math
@@ -85,7 +93,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   int aoff[TM], asoff[TM]; // byte offsets of the token's row in A and As
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
-    f[j] = a.sorted[static_cast<int64_t>(mb) * BM + j * 16 + r];
+    f[j] = ids[j];
     valid[j] = f[j] < a.num_valid;
     const int64_t row = token_row(a, f[j]);
     aoff[j] = static_cast<int>(row * K) + c * 16;
