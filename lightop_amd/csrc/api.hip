@@ -306,11 +306,11 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
   auto rows = [&](bool fa) { return !(gflags & LO_GEMM_FORCE_STREAMING) && gemm_rows_supports(a, fa, bm); };
   if (gemm1) {
     a.N = 2 * I; a.K = H; a.a_rows = M;
-    describe_gemm_kernel(pick_gemm_kernel(a, fused, bm, gflags), fused, bm, rows(fused), gemm1);
+    describe_gemm_kernel(pick_gemm_kernel(a, fused, bm, gflags), fused, bm, rows(fused), a, gemm1);
   }
   if (gemm2) {
     a.N = H; a.K = I; a.a_rows = M * top_k;
-    describe_gemm_kernel(pick_gemm_kernel(a, false, bm, gflags), false, bm, rows(false), gemm2);
+    describe_gemm_kernel(pick_gemm_kernel(a, false, bm, gflags), false, bm, rows(false), a, gemm2);
   }
   // a few tokens: the whole-path call serves the block form with its two-launch path
   if (decode) {

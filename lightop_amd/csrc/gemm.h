@@ -2,15 +2,6 @@
 #pragma once
 #include "common.h"
 
-// Shape of the plain (not fused) weight-streaming workgroup: waves, and 16-row fragments per wave
-// at token blocks of 16 or 32 (gemm_ws.hip; the tile query reports the same numbers).
-#ifndef LO_WS_PLAIN_WAVES
-#define LO_WS_PLAIN_WAVES 4
-#endif
-#ifndef LO_WS_RPW
-#define LO_WS_RPW 4
-#endif
-
 namespace lo {
 
 struct GemmArgs {
@@ -118,6 +109,20 @@ __device__ __forceinline__ bool block_unused(int32_t first, int32_t blocks_end, 
   constexpr int kNever = -2147483647 - 1;
   __builtin_amdgcn_sched_barrier(0); // all of the loads before the first wait
   return (first >= blocks_end) | ((expert == kNever) & (__builtin_amdgcn_readfirstlane(slots) == kNever));
+}
+
+// Shape of the plain (not fused) weight-streaming workgroup: waves, and 16-row fragments per wave (gemm_ws.hip; the tile
+// query reports the same numbers).  Two fragments rather than four: what a stage cannot fill with whole rounds of resident
+// workgroups it loses, and a workgroup of half the bytes halves that.  us with four / two, one pass of the layer: per-channel
+// Qwen3-30B-A3B layer at 20 tokens 96.6 / 90.7, per-channel DeepSeek-V3 share at 40: 180 / 169.5, int4 per-channel at 38: 190.5 /
+// 185, block form, Qwen3-30B-A3B layer at 32 tokens 101.6 / 99.0 (one fragment with three or four K blocks in flight: 3 to
+// 14 % slower).  Four for the block form's long outputs, which have tiles enough (DeepSeek-V3, 28 per expert), and for int4
+// weights with K-group scales, whose workgroups fill their scale table first (60 tokens 231.6 with four, 234.7 with two).
+constexpr int kWsPlainWaves = 4;
+inline int ws_plain_fragments(const GemmArgs &a, int token_fragments) {
+  if (token_fragments > 2) return token_fragments == 4 ? 2 : 1;
+  if (a.per_channel) return 2;
+  return a.w4 || a.N > 4096 ? 4 : 2;
 }
 
 // Division of a slot id below 2^31 by top_k as a multiplication: with L = ceil(log2 d) and m = floor(2^(31+L) / d) + 1,
@@ -257,7 +262,7 @@ __device__ __forceinline__ void wave_store_32x64_bf16(int8_t *stg, const v4u16 (
 
 // Kernel a stage is served by, and its workgroup shape (gemm_api.hip).
 int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int block_size_m, int flags);
-void describe_gemm_kernel(int kernel, bool fused_act, int block_size_m, bool rows, lo_moe_tile *t);
+void describe_gemm_kernel(int kernel, bool fused_act, int block_size_m, bool rows, const GemmArgs &a, lo_moe_tile *t);
 
 // Decode-size whole path in two launches (gemm_dec.hip): weights in the load-time layout, bf16 or fp16 rows.
 struct DecProblem {

@@ -58,7 +58,7 @@ int pick_gemm_kernel(const GemmArgs &a, bool fused_act, int bs, int flags) {
 }
 
 // Workgroup shape of that kernel: wavefronts and weight rows per workgroup.
-void describe_gemm_kernel(int kernel, bool fused_act, int bs, bool rows, lo_moe_tile *t) {
+void describe_gemm_kernel(int kernel, bool fused_act, int bs, bool rows, const GemmArgs &a, lo_moe_tile *t) {
   t->block_size_m = bs;
   t->kernel = kernel;
   if (rows) { // row-major weights: four waves x 64 rows at every block size
@@ -68,10 +68,8 @@ void describe_gemm_kernel(int kernel, bool fused_act, int bs, bool rows, lo_moe_
   }
   switch (kernel) {
   case LO_KERNEL_WS: { // gemm_ws.hip: launch_ws
-    const int tm = bs / 16;
-    const int rpw = tm <= 2 ? LO_WS_RPW : (tm == 4 ? 2 : 1);
-    t->waves = fused_act ? 8 : LO_WS_PLAIN_WAVES;
-    t->block_n = fused_act ? 256 : 16 * LO_WS_PLAIN_WAVES * rpw;
+    t->waves = fused_act ? 8 : kWsPlainWaves;
+    t->block_n = fused_act ? 256 : 16 * kWsPlainWaves * ws_plain_fragments(a, bs / 16);
     break;
   }
   case LO_KERNEL_TILE:

@@ -20,16 +20,6 @@
 // barrier in the main loop and keeps PD K-blocks of loads in flight per wave.
 #include "gemm.h"
 
-#ifndef LO_WS_STREAM_TM
-#define LO_WS_STREAM_TM 2
-#endif
-#ifndef LO_WS_PD_SMALL
-#define LO_WS_PD_SMALL 4
-#endif
-#ifndef LO_WS_PD_PLAIN
-#define LO_WS_PD_PLAIN 2
-#endif
-
 namespace lo {
 
 //
@@ -64,7 +54,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   constexpr int NW = FUSED_ACT ? 2 : RPW;
   // With at most 32 tokens per block an expert's weights are read by one pass only:
   // mark those loads as streaming so that they do not displace the activations in L2.
-  constexpr int WAUX = (TM <= LO_WS_STREAM_TM) ? kCacheStream : kCacheDefault;
+  constexpr int WAUX = (TM <= 2) ? kCacheStream : kCacheDefault;
   const int E = start_args(a);
   const int bid = blockIdx.x;
   const int mb = bid / a.n_tiles, nt = bid - mb * a.n_tiles;
@@ -443,14 +433,9 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   }
 }
 
-template <int TM, int FUSED_ACT, int ORD>
-static int launch_ws(const GemmArgs &a0, int64_t m_blocks, hipStream_t s) {
-  constexpr int NWAVES = FUSED_ACT ? 8 : LO_WS_PLAIN_WAVES;
-  // A plain-GEMM wave takes RPW consecutive 16-row fragments so that it streams a few
-  // hundred KB even when K is short; the ring depth shrinks as the fragments multiply.
-  constexpr int RPW = FUSED_ACT ? 2 : (TM <= 2 ? LO_WS_RPW : (TM == 4 ? 2 : 1));
-  constexpr int PD = FUSED_ACT ? ((TM <= 2) ? LO_WS_PD_SMALL : (TM == 4 ? 2 : 1))
-                               : ((TM <= 2) ? LO_WS_PD_PLAIN : (TM == 4 ? 2 : 1));
+template <int TM, int FUSED_ACT, int ORD, int RPW, int PD>
+static int launch_ws_rows(const GemmArgs &a0, int64_t m_blocks, hipStream_t s) {
+  constexpr int NWAVES = FUSED_ACT ? 8 : kWsPlainWaves;
   GemmArgs a = a0;
   if (!FUSED_ACT) a.n_tiles = static_cast<int32_t>((a.N + 16 * NWAVES * RPW - 1) / (16 * NWAVES * RPW));
   const dim3 grid(static_cast<unsigned>(m_blocks * a.n_tiles)), block(NWAVES * 64);
@@ -483,6 +468,21 @@ static int launch_ws(const GemmArgs &a0, int64_t m_blocks, hipStream_t s) {
   else
     hipLaunchKernelGGL((moe_gemm_ws_kernel<TM, FUSED_ACT, ORD, false, NWAVES, PD, RPW>), grid, block, 0, s, a);
   return LO_OK;
+}
+
+template <int TM, int FUSED_ACT, int ORD>
+static int launch_ws(const GemmArgs &a, int64_t m_blocks, hipStream_t s) {
+  // Two K blocks in flight per wave: the registers this leaves free hold another workgroup on the compute unit, three of
+  // them fused instead of two with a ring of four, which is worth more while K is short (fused with four / three / two, us:
+  // 24 tokens of the Qwen3-30B-A3B layer 99.4 / 100.6 / 97.5, at 40: 107.4 / 108.7 / 105.3; 60 tokens of int4 weights with
+  // K-group scales, K 4096: 236 / 236 / 231.6; 16 tokens of the DeepSeek-V3 share, K 7168: 112.0 / - / 112.8).
+  if constexpr (TM == 8) return launch_ws_rows<TM, FUSED_ACT, ORD, FUSED_ACT ? 2 : 1, 1>(a, m_blocks, s);
+  else if constexpr (TM == 4) return launch_ws_rows<TM, FUSED_ACT, ORD, 2, 2>(a, m_blocks, s);
+  else if constexpr (FUSED_ACT)
+    return a.K > 4096 ? launch_ws_rows<TM, FUSED_ACT, ORD, 2, 4>(a, m_blocks, s)
+                      : launch_ws_rows<TM, FUSED_ACT, ORD, 2, 2>(a, m_blocks, s);
+  else return ws_plain_fragments(a, TM) == 4 ? launch_ws_rows<TM, 0, ORD, 4, 2>(a, m_blocks, s)
+                                             : launch_ws_rows<TM, 0, ORD, 2, 2>(a, m_blocks, s);
 }
 
 template <int FUSED_ACT>
