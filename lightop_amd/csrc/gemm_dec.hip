@@ -271,12 +271,10 @@ __device__ __forceinline__ void dec_gemm1_body(const DecArgs &a) {
         }
       }
       // ---- requests in the order of need: token rows, weight scales, the first weights ------------------
-      if (a.M > 1) {
-        load_row(slot[0] / a.top_k, raw[0]);
+      if (a.M > 1) load_row(slot[0] / a.top_k, raw[0]);
 #pragma unroll
-        for (int i = 1; i < kDecTP; ++i)
-          if (i < nc) load_row(slot[i] / a.top_k, raw[i]);
-      }
+      for (int i = 1; i < kDecTP; ++i) // (one token as well: several of its slots may be this expert's)
+        if (i < nc) load_row(slot[i] / a.top_k, raw[i]);
       // block scales of the wave's K range: lanes 0..7 the gate rows', lanes 8..15 the up rows'; PC: the channel scales of
       // the last wave's columns, one gate and one up row per lane
       float bs_l = 0.0f, bs_u = 0.0f;
