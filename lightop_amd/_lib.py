@@ -160,3 +160,13 @@ def stream_of(t) -> c_void_p:
     import torch
 
     return c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+
+
+def capture_id(stream: int) -> int:
+    """Number of the capture under way on a stream, 0 if there is none (hipStreamGetCaptureInfo of the HIP runtime that
+    the library is linked against)."""
+    status, number = c_int(0), ctypes.c_ulonglong(0)
+    rc = lib().hipStreamGetCaptureInfo(c_void_p(stream), ctypes.byref(status), ctypes.byref(number))
+    if rc != 0:
+        raise RuntimeError(f"lightop_amd: hipStreamGetCaptureInfo: error {rc}")
+    return int(number.value)

@@ -4,8 +4,8 @@
 // checks on fifteen tensors, ctypes conversions, stream and workspace look-ups) took 25-27 us of host time and set
 // the pace of the loop.  Here the ordinary call - tensors of the expected types, contiguous, on the current device,
 // one chunk - is checked, given its workspace and launched natively.  Anything else (a conversion to make, several
-// chunks, a tuning file, an argument to refuse) is declined by returning None, and the Python code beside it does what it
-// always did, error messages included: nothing is decided in two places.
+// chunks, a tuning file, a stream being captured, an argument to refuse) is declined by returning None, and the Python
+// code beside it does what it always did, error messages included: nothing is decided in two places.
 //
 // The kernels' entry points are the C ABI of include/lightop_mi355.h, handed over by address (the library is the one
 // `lightop_amd._lib` has loaded, whichever file that is).
@@ -69,8 +69,9 @@ int64_t chunk_size() {
 // The library's scratch for a whole-path call, one per (device, stream) and grown on demand, so that a serving loop
 // does not allocate on every call.  Calls on one stream run in order and can share it; calls on different streams get
 // workspaces of their own.  At most kMaxWorkspaces are kept: beyond that the one that was used longest ago goes back to the
-// caching allocator (it was allocated on its own stream, so its memory is reused in that stream's order).  All under the
-// interpreter lock.
+// caching allocator (it was allocated on its own stream, so its memory is reused in that stream's order), as does one that
+// a larger call outgrows.  A graph would keep the address of such memory, so none of it is ever captured: calls on a stream
+// that is being captured are declined, and get scratch that lives as long as the graph.  All under the interpreter lock.
 struct Workspace {
   int device;
   hipStream_t stream;
@@ -112,6 +113,15 @@ PyObject *raise(int rc) {
   const char *msg = g_last_error ? g_last_error() : nullptr;
   PyErr_Format(PyExc_RuntimeError, "lightop_amd: %s (code %d)", msg && *msg ? msg : "error", rc);
   return nullptr;
+}
+
+// Whether work put on the stream goes into a graph (the legacy default stream cannot be captured).
+bool capturing(hipStream_t stream) {
+  if (!stream) return false;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
 }
 
 int device_now() {
@@ -205,6 +215,7 @@ PyObject *fused_experts(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const int64_t bytes = g_ws_bytes(M, static_cast<int32_t>(k), H, I, static_cast<int32_t>(experts), 0);
   if (bytes < 0) return raise(static_cast<int>(bytes));
   const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
+  if (capturing(stream)) Py_RETURN_NONE;
   const at::Tensor &ws = workspace_for(bytes, dev, stream);
   const uintptr_t base = reinterpret_cast<uintptr_t>(ws.data_ptr());
   const uintptr_t aligned = (base + 255) / 256 * 256;
@@ -307,17 +318,6 @@ PyObject *fused_gate(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   LO_CATCH
 }
 
-// workspace(bytes, device, stream) -> uint8 tensor, for the calls that Python marshals itself.
-PyObject *workspace(PyObject *, PyObject *args) {
-  long long bytes;
-  int device;
-  unsigned long long stream;
-  if (!PyArg_ParseTuple(args, "LiK", &bytes, &device, &stream)) return nullptr;
-  LO_TRY
-  return THPVariable_Wrap(at::Tensor(workspace_for(bytes, device, reinterpret_cast<hipStream_t>(stream))));
-  LO_CATCH
-}
-
 // bind(lo_fused_experts_block_int8, lo_fused_experts_channel_int8, lo_fused_experts_workspace_bytes, lo_topk_softmax,
 //      lo_moe_fused_gate, lo_last_error): addresses of the library's functions.
 PyObject *bind(PyObject *, PyObject *args) {
@@ -334,7 +334,6 @@ PyObject *bind(PyObject *, PyObject *args) {
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
-    {"workspace", workspace, METH_VARARGS, nullptr},
     {"fused_experts", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(fused_experts)), METH_FASTCALL, nullptr},
     {"topk_softmax", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(topk_softmax)), METH_FASTCALL, nullptr},
     {"fused_gate", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(fused_gate)), METH_FASTCALL, nullptr},

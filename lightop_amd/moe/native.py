@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import threading
 from typing import Any, Dict, List, Optional, Tuple
 
 import torch
@@ -600,6 +601,46 @@ def _workspace_bytes_cached(M: int, top_k: int, H: int, I: int, num_experts: int
     return fused_experts_workspace_bytes(M, top_k, H, I, num_experts, 0)
 
 
+_capture_lock = threading.Lock()
+_capture_seen: Tuple[Tuple[int, int], bool] = ((-1, 0), False)  # ((device, capture id), whether the graph owns what it allocates)
+_capture_kept: Dict[Tuple[int, int], List[torch.Tensor]] = {}
+
+
+def _scratch(nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
+    """Scratch of one call that is marshalled here: from the caching allocator, back to it when the call's launches are
+    queued, and reused in the stream's order.
+
+    A captured call's scratch has to outlive the call, since every replay writes to it.  ``torch.cuda.graph`` sees to
+    that: what is allocated under it comes from memory that belongs to the graph (and to the graphs that share its pool)
+    until the graph is gone.  A capture that the allocator knows nothing of, begun with hipStreamBeginCapture on
+    an external stream, has no such memory: its scratch is kept for good, one piece per (device, stream) and the ones it
+    outgrew."""
+    def new():
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+    if not torch.cuda.is_current_stream_capturing():
+        return new()
+    global _capture_seen
+    with _capture_lock:
+        at = (device.index, _lib.capture_id(stream))
+        if _capture_seen[0] != at:  # once per capture: a snapshot lists every block of the process
+            _capture_seen = (at, _in_graph_pool(new()))
+        if _capture_seen[1]:
+            return new()
+        kept = _capture_kept.setdefault((device.index, stream), [])
+        if not kept or kept[-1].numel() < nbytes:
+            kept.append(new())
+        return kept[-1]
+
+
+def _in_graph_pool(t: torch.Tensor) -> bool:
+    """Whether the allocator took ``t`` from a private pool, as it does under ``torch.cuda.graph``."""
+    for seg in torch.cuda.memory_snapshot():
+        if seg["device"] == t.device.index and seg["address"] <= t.data_ptr() < seg["address"] + seg["total_size"]:
+            return tuple(seg["segment_pool_id"]) != (0, 0)
+    return False
+
+
 def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, inplace, apply_router_weight_on_input,
                        global_num_experts, expert_map, w1_scale, w2_scale, routed_scaling_factor, shared_output,
                        I, flags, block_size_m, channel=False, workspace=None, prequant=None, chunk_size=None):
@@ -631,9 +672,8 @@ def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, i
     ws_bytes = _workspace_bytes_cached(M, top_k_num, H, I, global_num_experts)
     stream_handle = torch.cuda.current_stream(hidden_states.device).cuda_stream
     if workspace is None:
-        # kept per (device, stream) and grown on demand (the reference keeps its own workspace, cache13, in a
-        # process-wide cache the same way: vllm_compat/fused_moe_cache.py:19-24)
-        workspace = (_lib._host or _lib.host()).workspace(ws_bytes, hidden_states.device.index, stream_handle)
+        with _on_device(hidden_states):
+            workspace = _scratch(ws_bytes, hidden_states.device, stream_handle)
         ws_bytes = workspace.numel()
     else:  # the caller's own scratch (tests read the intermediates out of it afterwards)
         assert workspace.dtype == torch.uint8 and workspace.is_contiguous() and workspace.numel() >= ws_bytes

@@ -1,7 +1,10 @@
 """The whole path recorded into a HIP graph: every replay must reproduce the eager result.
 
-The entry points allocate nothing and never synchronise, so a caller may capture them.
+The C entry points allocate nothing and never synchronise, and what the Python ones allocate under a capture lives as long
+as the graph, so a caller may capture them.
 The replays are separated by eager work and synchronisations of the program itself."""
+import ctypes
+
 import pytest
 import torch
 
@@ -56,3 +59,77 @@ def test_graph_replays_match_eager(M, form):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay {rep} differs"
+
+
+class HipGraph:
+    """A graph recorded with the runtime's own calls on a stream of the program's, which torch's allocator does not
+    know to be capturing into a graph."""
+
+    def __init__(self, stream, fn):
+        from lightop_amd import _lib
+
+        hip = _lib.lib()  # (symbols of the HIP runtime it is linked against)
+        self.hip, self.exec, graph = hip, ctypes.c_void_p(), ctypes.c_void_p()
+        self.check(hip.hipStreamBeginCapture(ctypes.c_void_p(stream.cuda_stream), 2))  # relaxed
+        with torch.cuda.stream(stream):
+            self.out = fn()
+        self.check(hip.hipStreamEndCapture(ctypes.c_void_p(stream.cuda_stream), ctypes.byref(graph)))
+        self.check(hip.hipGraphInstantiate(ctypes.byref(self.exec), graph, None, None, ctypes.c_size_t(0)))
+
+    @staticmethod
+    def check(rc):
+        assert rc == 0, f"HIP error {rc}"
+
+    def replay(self):
+        self.check(self.hip.hipGraphLaunch(self.exec, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+
+
+@pytest.mark.parametrize("capture", ["torch", "runtime"])
+def test_replays_write_to_no_memory_of_others(capture, monkeypatch):
+    """A graph's scratch stays the graph's: after a warm-up and a capture on one stream, larger calls there and calls on
+    more streams than workspaces are kept for, the memory that stream then gets from the allocator survives replays."""
+    from lightop_amd import workloads as wl
+    from lightop_amd.moe import fused_experts_impl_int8, native, preshuffle_moe_weight
+
+    dev, layer, M = torch.device("cuda:0"), wl.TINY, 48
+    print(f"[case] graph scratch {capture}", flush=True)
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=0, device=dev)
+    w1, w2 = preshuffle_moe_weight(w1), preshuffle_moe_weight(w2)
+    args = {m: tuple(t.to(dev) for t in wl.make_inputs(layer, m, seed=m)) for m in (M, 4096)}
+    cache13 = torch.empty(4096 * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
+
+    def run(m=M):
+        x, tw, ids = args[m]
+        return fused_experts_impl_int8(x, w1, w2, tw, ids, cache13, use_int8_w8a8=True, w1_scale=w1s, w2_scale=w2s,
+                                       block_shape=[128, 128])
+
+    monkeypatch.setattr(native, "_capture_kept", {})
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        eager = run().clone()
+    torch.cuda.synchronize()
+    if capture == "torch":
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            out = run()
+    else:
+        g = HipGraph(side, run)
+        out = g.out
+    assert list(native._capture_kept) == ([(0, side.cuda_stream)] if capture == "runtime" else [])  # torch's graphs own theirs
+    torch.cuda.synchronize()
+    for stream in [torch.cuda.Stream() for _ in range(20)] + [side]:
+        with torch.cuda.stream(stream):
+            for m in (M, 4096):
+                run(m)
+        torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        canaries = [torch.full((n,), 0x5A, dtype=torch.uint8, device=dev) for n in (1 << 20, 2 << 20, 16 << 20) for _ in range(8)]
+    for rep in range(4):
+        out.zero_()
+        cache13.fill_(float(rep))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay {rep} differs"
+        assert all(bool((c == 0x5A).all()) for c in canaries), f"replay {rep} wrote to memory of others"
