@@ -5,7 +5,8 @@
 // the pace of the loop.  Here the ordinary call - tensors of the expected types, contiguous, on the current device,
 // one chunk - is checked, given its workspace and launched natively.  Anything else (a conversion to make, several
 // chunks, a tuning file, a stream being captured, an argument to refuse) is declined by returning None, and the Python
-// code beside it does what it always did, error messages included: nothing is decided in two places.
+// code beside it does what it always did, error messages included: nothing is decided in two places.  What torch throws in
+// here reaches Python as torch's own exception types (an allocation that fails is torch.OutOfMemoryError).
 //
 // The kernels' entry points are the C ABI of include/lightop_mi355.h, handed over by address (the library is the one
 // `lightop_amd._lib` has loaded, whichever file that is).
@@ -14,6 +15,7 @@
 #include <ATen/Functions.h>
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cerrno>
@@ -129,14 +131,6 @@ int device_now() {
   return hipGetDevice(&d) == hipSuccess ? d : -1;
 }
 
-#define LO_TRY try {
-#define LO_CATCH                                       \
-  }                                                    \
-  catch (const std::exception &e) {                    \
-    PyErr_SetString(PyExc_RuntimeError, e.what());     \
-    return nullptr;                                    \
-  }
-
 int dtype_code(at::ScalarType t) {
   switch (t) {
   case at::kBFloat16: return LO_BF16;
@@ -168,7 +162,7 @@ PyObject *fused_experts(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const double factor = PyFloat_AsDouble(args[14]);
   long flags = PyLong_AsLong(args[15]);
   if (inplace < 0 || mul_on_input < 0 || PyErr_Occurred()) return nullptr;
-  LO_TRY
+  HANDLE_TH_ERRORS
   const at::Tensor &x = *t[0], &w1 = *t[1], &w2 = *t[2], &tw = *t[3], &ids = *t[4], &cache = *t[5], &s1 = *t[6], &s2 = *t[7];
   if (!x.is_cuda() || x.get_device() != device_now()) Py_RETURN_NONE;
   const int dev = x.get_device();
@@ -235,7 +229,7 @@ PyObject *fused_experts(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     return args[0];
   }
   return THPVariable_Wrap(std::move(out));
-  LO_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // topk_softmax(weights, indices, source_rows, gating, renormalize) -> True, or None: not an ordinary call.
@@ -248,7 +242,7 @@ PyObject *topk_softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!w || !idx || !g || (args[2] != Py_None && !(src = tensor_of(args[2])))) Py_RETURN_NONE;
   const int renorm = PyObject_IsTrue(args[4]);
   if (renorm < 0) return nullptr;
-  LO_TRY
+  HANDLE_TH_ERRORS
   if (!g->is_cuda() || g->get_device() != device_now()) Py_RETURN_NONE;
   const int dev = g->get_device();
   if (!plain(*g, dev) || !plain(*w, dev) || !plain(*idx, dev) || (src && !plain(*src, dev))) Py_RETURN_NONE;
@@ -266,7 +260,7 @@ PyObject *topk_softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                                 c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
   if (rc < 0) return raise(rc);
   Py_RETURN_TRUE;
-  LO_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // fused_gate(input, bias, groups, topk_group, topk, n_share, factor, factor_on_output, int64_indices)
@@ -289,7 +283,7 @@ PyObject *fused_gate(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const double factor = PyFloat_AsDouble(args[6]);
   const int on_output = PyObject_IsTrue(args[7]), i64 = PyObject_IsTrue(args[8]);
   if (on_output < 0 || i64 < 0 || PyErr_Occurred()) return nullptr;
-  LO_TRY
+  HANDLE_TH_ERRORS
   if (!x->is_cuda() || x->get_device() != device_now()) Py_RETURN_NONE;
   const int dev = x->get_device();
   if (!plain(*x, dev) || !plain(*b, dev) || x->dim() != 2 || b->dim() != 1 || b->numel() != x->size(1)) Py_RETURN_NONE;
@@ -315,7 +309,7 @@ PyObject *fused_gate(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   PyList_SET_ITEM(pair, 0, pw);
   PyList_SET_ITEM(pair, 1, pi);
   return pair;
-  LO_CATCH
+  END_HANDLE_TH_ERRORS
 }
 
 // bind(lo_fused_experts_block_int8, lo_fused_experts_channel_int8, lo_fused_experts_workspace_bytes, lo_topk_softmax,

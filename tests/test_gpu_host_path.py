@@ -102,3 +102,44 @@ def test_routers(dtype, renorm):
         moe_fused_gate(g, bias.cpu(), 8, 4, k, 0, 2.5)
     with pytest.raises(RuntimeError, match="topk_group"):
         moe_fused_gate(g, bias, 8, 9, k, 0, 2.5)
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_out_of_memory_keeps_its_type(warm):
+    """A call whose output or workspace does not fit raises torch's own out-of-memory error, as the allocation in Python
+    does, and works again once there is room.  ``warm``: the stream has a smaller workspace that has to grow."""
+    from lightop_amd import workloads as wl
+    from lightop_amd.moe import fused_experts_impl_int8
+
+    dev, M = torch.device("cuda:0"), 16384
+    print(f"[case] out of memory warm={warm}", flush=True)
+    layer, weights, kw = _layer("block", dev)
+    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, M, seed=3))
+    cache13 = torch.empty(M * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
+
+    def run(m, inplace):
+        return fused_experts_impl_int8(x[:m].clone() if inplace else x[:m], *weights, tw[:m], ids[:m], cache13, inplace=inplace,
+                                       use_int8_w8a8=True, block_shape=[128, 128], **kw)
+
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        if warm:
+            run(64, False)
+        held = x.clone()  # what an in-place call works on
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(dev).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+        try:
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                run(M, False)
+            with pytest.raises(torch.cuda.OutOfMemoryError):  # the workspace alone
+                fused_experts_impl_int8(held, *weights, tw, ids, cache13, inplace=True, use_int8_w8a8=True,
+                                        block_shape=[128, 128], **kw)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.equal(held, x)
+        got = run(M, False)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), run(M, True).view(torch.int16))
