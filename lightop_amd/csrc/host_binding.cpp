@@ -21,6 +21,8 @@
 #include <cerrno>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "../../include/lightop_mi355.h"
@@ -70,14 +72,20 @@ int64_t chunk_size() {
 // ---- workspaces ----------------------------------------------------------------------------------------
 // The library's scratch for a whole-path call, one per (device, stream) and grown on demand, so that a serving loop
 // does not allocate on every call.  Calls on one stream run in order and can share it; calls on different streams get
-// workspaces of their own.  At most kMaxWorkspaces are kept: beyond that the one that was used longest ago goes back to the
+// workspaces of their own, and of several threads on one stream only one queues its launches at a time, so that
+// a workspace holds one call's intermediates from the first launch to the last.  At most kMaxWorkspaces are kept: beyond that the one that was used longest ago goes back to the
 // caching allocator (it was allocated on its own stream, so its memory is reused in that stream's order), as does one that
 // a larger call outgrows.  A graph would keep the address of such memory, so none of it is ever captured: calls on a stream
-// that is being captured are declined, and get scratch that lives as long as the graph.  All under the interpreter lock.
+// that is being captured are declined, and get scratch that lives as long as the graph.  The table is touched under the interpreter lock only; a call holds a
+// reference to its workspace while it is without that lock.
+struct Scratch {
+  at::Tensor buf;
+  std::mutex busy; // held while a call's launches are queued
+};
 struct Workspace {
   int device;
   hipStream_t stream;
-  at::Tensor buf;
+  std::shared_ptr<Scratch> scratch;
 };
 constexpr size_t kMaxWorkspaces = 16;
 std::vector<Workspace> &workspaces() { // most recently used first; never destroyed (the allocator may be gone by then)
@@ -85,12 +93,14 @@ std::vector<Workspace> &workspaces() { // most recently used first; never destro
   return *v;
 }
 
-at::Tensor new_workspace(int64_t bytes, int device) {
-  return at::empty({std::max<int64_t>(bytes, 1 << 20)},
-                   at::TensorOptions().dtype(at::kByte).device(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device))));
+std::shared_ptr<Scratch> new_workspace(int64_t bytes, int device) {
+  auto s = std::make_shared<Scratch>();
+  s->buf = at::empty({std::max<int64_t>(bytes, 1 << 20)},
+                     at::TensorOptions().dtype(at::kByte).device(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device))));
+  return s;
 }
 
-const at::Tensor &workspace_for(int64_t bytes, int device, hipStream_t stream) {
+std::shared_ptr<Scratch> workspace_for(int64_t bytes, int device, hipStream_t stream) {
   auto &all = workspaces();
   size_t i = 0;
   while (i < all.size() && !(all[i].device == device && all[i].stream == stream)) ++i;
@@ -98,17 +108,31 @@ const at::Tensor &workspace_for(int64_t bytes, int device, hipStream_t stream) {
     if (all.size() >= kMaxWorkspaces) all.pop_back();
     all.push_back({device, stream, new_workspace(bytes, device)});
     i = all.size() - 1;
-  } else if (all[i].buf.numel() < bytes) {
-    all[i].buf = at::Tensor(); // back to the allocator first: the larger one may take its place
+  } else if (all[i].scratch->buf.numel() < bytes) {
+    all[i].scratch.reset(); // back to the allocator first: the larger one may take its place
     try {
-      all[i].buf = new_workspace(bytes, device);
+      all[i].scratch = new_workspace(bytes, device);
     } catch (...) {
       all.erase(all.begin() + static_cast<std::ptrdiff_t>(i));
       throw;
     }
   }
   for (; i > 0; --i) std::swap(all[i], all[i - 1]);
-  return all[0].buf;
+  return all[0].scratch;
+}
+
+// Calls `entry` without the interpreter lock, as ctypes does: a launch waits while the stream's queue is full, the first
+// call of an activation waits for its table, and Python threads, or a callback on the stream, may have to run until then.
+// The arguments are plain values, taken from the tensors before the lock is let go.
+struct NoGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+template <typename F, typename... A> int launch(std::mutex *busy, F entry, A... args) {
+  const NoGil nogil;
+  std::unique_lock<std::mutex> lock; // taken without the interpreter lock, whose holder may be waiting for it
+  if (busy) lock = std::unique_lock<std::mutex>(*busy);
+  return entry(args...);
 }
 
 PyObject *raise(int rc) {
@@ -210,19 +234,19 @@ PyObject *fused_experts(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (bytes < 0) return raise(static_cast<int>(bytes));
   const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
   if (capturing(stream)) Py_RETURN_NONE;
-  const at::Tensor &ws = workspace_for(bytes, dev, stream);
-  const uintptr_t base = reinterpret_cast<uintptr_t>(ws.data_ptr());
+  const std::shared_ptr<Scratch> ws = workspace_for(bytes, dev, stream);
+  const uintptr_t base = reinterpret_cast<uintptr_t>(ws->buf.data_ptr());
   const uintptr_t aligned = (base + 255) / 256 * 256;
   at::Tensor out = inplace ? x : at::empty(x.sizes(), x.options().requires_grad(false));
 
   const auto entry = channel ? g_channel : g_block;
-  const int rc = entry(x.data_ptr(), dtype, M, H, I, static_cast<int32_t>(E), static_cast<int32_t>(experts),
-                       static_cast<int32_t>(k), static_cast<const int8_t *>(w1.data_ptr()), s1.data_ptr<float>(),
-                       static_cast<const int8_t *>(w2.data_ptr()), s2.data_ptr<float>(), tw.data_ptr<float>(), ids.data_ptr(),
-                       ids64 ? LO_I64 : LO_I32, t[8] ? t[8]->data_ptr<int32_t>() : nullptr, mul_on_input,
-                       static_cast<float>(factor), t[9] ? t[9]->data_ptr() : nullptr, cache.data_ptr(), out.data_ptr(),
-                       reinterpret_cast<void *>(aligned), ws.numel() - static_cast<int64_t>(aligned - base), 0,
-                       static_cast<int>(flags), stream);
+  const int rc = launch(&ws->busy, entry, x.data_ptr(), dtype, M, H, I, static_cast<int32_t>(E), static_cast<int32_t>(experts),
+                        static_cast<int32_t>(k), static_cast<const int8_t *>(w1.data_ptr()), s1.data_ptr<float>(),
+                        static_cast<const int8_t *>(w2.data_ptr()), s2.data_ptr<float>(), tw.data_ptr<float>(), ids.data_ptr(),
+                        ids64 ? LO_I64 : LO_I32, t[8] ? t[8]->data_ptr<int32_t>() : nullptr, mul_on_input,
+                        static_cast<float>(factor), t[9] ? t[9]->data_ptr() : nullptr, cache.data_ptr(), out.data_ptr(),
+                        reinterpret_cast<void *>(aligned), ws->buf.numel() - static_cast<int64_t>(aligned - base), 0,
+                        static_cast<int>(flags), stream);
   if (rc < 0) return raise(rc);
   if (inplace) {
     Py_INCREF(args[0]);
@@ -254,10 +278,9 @@ PyObject *topk_softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!i64 && idx->scalar_type() != at::kInt) Py_RETURN_NONE;
   if (src && (src->scalar_type() != at::kInt || src->numel() != T * k)) Py_RETURN_NONE;
   if (E > INT32_MAX || k > INT32_MAX) Py_RETURN_NONE;
-  const int rc = g_topk_softmax(g->data_ptr(), dtype, T, static_cast<int32_t>(E), static_cast<int32_t>(k), renorm,
-                                w->data_ptr<float>(), idx->data_ptr(), i64 ? LO_I64 : LO_I32,
-                                src ? src->data_ptr<int32_t>() : nullptr,
-                                c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
+  const int rc = launch(nullptr, g_topk_softmax, g->data_ptr(), dtype, T, static_cast<int32_t>(E), static_cast<int32_t>(k), renorm,
+                        w->data_ptr<float>(), idx->data_ptr(), i64 ? LO_I64 : LO_I32, src ? src->data_ptr<int32_t>() : nullptr,
+                        c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
   if (rc < 0) return raise(rc);
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -293,8 +316,8 @@ PyObject *fused_gate(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const auto opts = x->options().requires_grad(false);
   at::Tensor weights = at::empty({T, topk}, opts.dtype(at::kFloat));
   at::Tensor indices = at::empty({T, topk}, opts.dtype(i64 ? at::kLong : at::kInt));
-  const int rc = g_gate(x->data_ptr(), dt, b->data_ptr(), bt, T, static_cast<int32_t>(x->size(1)), static_cast<int32_t>(v[0]),
-                        static_cast<int32_t>(v[1]), static_cast<int32_t>(v[2]), static_cast<int32_t>(v[3]), factor, on_output,
+  const int rc = launch(nullptr, g_gate, x->data_ptr(), dt, b->data_ptr(), bt, T, static_cast<int32_t>(x->size(1)),
+                        static_cast<int32_t>(v[0]), static_cast<int32_t>(v[1]), static_cast<int32_t>(v[2]), static_cast<int32_t>(v[3]), factor, on_output,
                         weights.data_ptr<float>(), indices.data_ptr(), i64 ? LO_I64 : LO_I32,
                         c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
   if (rc < 0) return raise(rc);

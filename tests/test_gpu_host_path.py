@@ -1,5 +1,10 @@
 """The native marshalling of the whole-path call and of the routers (csrc/host_binding.cpp) against the Python
-marshalling beside it, bit for bit: the ordinary calls it takes, and the ones it has to leave to Python."""
+marshalling beside it, bit for bit: the ordinary calls it takes, and the ones it has to leave to Python; threads and errors."""
+import ctypes
+import subprocess
+import threading
+import time
+
 import pytest
 import torch
 
@@ -143,3 +148,92 @@ def test_out_of_memory_keeps_its_type(warm):
         got = run(M, False)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), run(M, True).view(torch.int16))
+
+
+STUB = """
+#include <unistd.h>
+volatile int entered, let_go;
+int stub(void) {
+  entered = 1;
+  for (int i = 0; i < 5000 && !let_go; ++i) usleep(1000);
+  return let_go ? 0 : -1;
+}
+const char *message(void) { return "no other thread ran during the call"; }
+"""
+
+
+@pytest.mark.parametrize("entry", ["block", "channel", "topk_softmax", "fused_gate"])
+def test_other_threads_run_during_a_launch(entry, tmp_path):
+    """A launch may wait (for room in the queue, for a table), and what it waits for may need the interpreter: in the place
+    of the library's function, one that returns when another Python thread has run, or after five seconds."""
+    from lightop_amd import _lib, workloads as wl
+
+    dev = torch.device("cuda:0")
+    print(f"[case] threads during a launch {entry}", flush=True)
+    (tmp_path / "stub.c").write_text(STUB)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "stub.so"), str(tmp_path / "stub.c")], check=True)
+    stub = ctypes.CDLL(str(tmp_path / "stub.so"))
+    entered, let_go = ctypes.c_int.in_dll(stub, "entered"), ctypes.c_int.in_dll(stub, "let_go")
+    layer, weights, kw = _layer("channel" if entry == "channel" else "block", dev)
+    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, 4, seed=3))
+    cache13 = torch.empty(4 * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
+    g, bias = torch.randn(4, 64, device=dev), torch.zeros(64, device=dev)
+
+    def other():
+        for _ in range(20000):
+            if entered.value:
+                let_go.value = 1
+                return
+            time.sleep(0.0005)
+
+    host, real = _lib.host(), _lib.lib()
+    address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value  # noqa: E731
+    thread = threading.Thread(target=other)
+    thread.start()
+    try:
+        host.bind(*[address(stub.stub)] * 2, address(real.lo_fused_experts_workspace_bytes), *[address(stub.stub)] * 2,
+                  address(stub.message))
+        if entry == "topk_softmax":
+            out = host.topk_softmax(torch.empty(4, 6, device=dev), torch.empty(4, 6, dtype=torch.int32, device=dev), None, g, True)
+        elif entry == "fused_gate":
+            out = host.fused_gate(g, bias, 8, 4, 6, 0, 2.5, False, False)
+        else:
+            out = host.fused_experts(x, *weights, tw, ids, cache13, kw["w1_scale"], kw["w2_scale"], None, None,
+                                     int(entry == "channel"), False, False, -1, 1.0, 0)
+        assert out is not None and let_go.value == 1
+    finally:
+        _lib._host = None
+        _lib.host()  # the library's own functions again
+        thread.join()
+
+
+@pytest.mark.parametrize("form", ["block", "channel"])
+def test_threads_share_a_stream(form):
+    """Two threads that queue calls of different sizes on one stream: neither's launches come between the other's, whose
+    intermediates are in the same workspace."""
+    from lightop_amd import workloads as wl
+    from lightop_amd.moe import fused_experts_impl_int8
+
+    dev = torch.device("cuda:0")
+    print(f"[case] threads on one stream {form}", flush=True)
+    layer, weights, kw = _layer(form, dev)
+    kw.update(use_int8_w8a8=True, per_channel_quant=form == "channel", block_shape=None if form == "channel" else [128, 128])
+    sizes = (300, 77)
+    inputs = [tuple(t.to(dev) for t in wl.make_inputs(layer, m, seed=m)) for m in sizes]
+    caches = [torch.empty(m * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev) for m in sizes]
+
+    def call(i):
+        x, tw, ids = inputs[i]
+        return fused_experts_impl_int8(x, *weights, tw, ids, caches[i], **kw)
+
+    want = [call(i).clone() for i in (0, 1)]
+    torch.cuda.synchronize()
+    got = [[], []]
+    threads = [threading.Thread(target=lambda i=i: got[i].extend(call(i) for _ in range(200))) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        assert len(got[i]) == 200 and all(torch.equal(o.view(torch.int16), want[i].view(torch.int16)) for o in got[i])
