@@ -217,18 +217,18 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   return 64;
 }
 
-// What the block-form whole-path call (int8 weights, or int4 weights with K-group scales) does with a
-// problem: the token-block size and which launches follow.  One function for the call itself, for its
+// What a whole-path call does with a problem: the token-block size and which launches follow.  One function per entry
+// point (block scales, which packed int4 with K-group scales share; per-channel scales) for the call itself, for its
 // no-allocation variant's space check and for the tile query, so that the three cannot drift apart.
-struct BlockPlan {
-  int flags;            // the caller's flags, LO_GEMM_W4 implying LO_GEMM_W_PRESHUFFLED
+struct PathPlan {
+  int flags;            // the caller's flags, LO_GEMM_W4 implying LO_GEMM_W_PRESHUFFLED in the block form
   int32_t block_size_m; // the caller's, or the table's pick when the caller passed 0
-  bool bs160;           // 160-token blocks of the direct-to-LDS kernel
-  bool unfused;         // the first GEMM writes [S, 2I] and one launch applies the activation and quantises
-  bool try_decode;      // the two-launch path is attempted first (it may still decline by size)
+  bool fused;           // the first GEMM ends with the activation (block form: and its quantisation); else it writes [S, 2I]
+                        // and one launch applies the activation and quantises
+  bool try_decode;      // the two-launch path is attempted first (decode_path_applies has the last word)
 };
 static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts, int32_t top_k, int64_t H, int64_t I,
-                           int32_t block_size_m, BlockPlan *plan) {
+                           int32_t block_size_m, PathPlan *plan) {
   if (flags & LO_GEMM_W4) flags |= LO_GEMM_W_PRESHUFFLED; // packed int4 exists in the load-time layout only
   const bool w4 = (flags & LO_GEMM_W4) != 0, pre = (flags & LO_GEMM_W_PRESHUFFLED) != 0;
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
@@ -240,18 +240,35 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
                                 !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true));
   // 160: the 160-token form of the direct-to-LDS kernel (int8 block form, load-time layout) for both GEMMs; bf16
   // rows with SiLU take its fused first stage, fp16 rows and GELU the plain one and the activation launch
-  const bool fused_ok = dtype == LO_BF16 && !gelu;
-  const bool bs160 = block_size_m == 160 && pre && !w4 && dtype != LO_F32 && blocks_of_160_fit(H, I, fused_ok);
+  const bool silu_bf16 = dtype == LO_BF16 && !gelu;
+  const bool bs160 = block_size_m == 160 && pre && !w4 && dtype != LO_F32 && blocks_of_160_fit(H, I, silu_bf16);
   LO_REQUIRE(block_size_m == 16 || block_size_m == 32 || block_size_m == 64 || block_size_m == 128 || bs160,
              LO_EINVAL,
              "fused_experts: block_size_m %d is not one of 16, 32, 64, 128 (160: int8 weights in the load-time "
              "layout and 16-bit rows; with fp16 rows or GELU 2I <= H as well)", block_size_m);
   plan->flags = flags;
   plan->block_size_m = block_size_m;
-  plan->bs160 = bs160;
   // fp32 rows have no fused epilogue; GELU and fp16 rows have one at some block sizes
-  plan->unfused = !fused_ok && (dtype == LO_F32 || !fused_table_supports(H, block_size_m, flags));
+  plan->fused = silu_bf16 || (dtype != LO_F32 && fused_table_supports(H, block_size_m, flags));
   plan->try_decode = block_size_m_auto && pre && dtype != LO_F32 && !(flags & LO_FUSED_NO_DECODE_PATH);
+  return LO_OK;
+}
+// own_rows: the activations are quantised by the call, not by the caller.
+static int plan_channel_path(int flags, int64_t M, int32_t num_experts, int32_t top_k, int64_t H, int64_t I,
+                             int32_t block_size_m, bool own_rows, PathPlan *plan) {
+  const bool pre = (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) != 0;
+  const bool fits160 = pre && H / kGroup <= 128 && I / kGroup <= 128; // the direct-to-LDS kernel with 160 tokens
+  plan->try_decode = block_size_m == 0 && own_rows && pre && !(flags & LO_FUSED_NO_DECODE_PATH);
+  if (block_size_m == 0)
+    block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_CHANNEL, true, (flags & LO_GEMM_W4) != 0, fits160);
+  LO_REQUIRE(block_size_m == 16 || block_size_m == 32 || block_size_m == 64 || block_size_m == 128 ||
+                 (block_size_m == 160 && fits160),
+             LO_EINVAL,
+             "fused_experts(channel): block_size_m %d is not one of 16, 32, 64, 128 (160: weights in the load-time "
+             "layout)", block_size_m);
+  plan->flags = flags;
+  plan->block_size_m = block_size_m;
+  plan->fused = gated_channel_supports(H, block_size_m, flags);
   return LO_OK;
 }
 
@@ -271,48 +288,41 @@ extern "C" int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t bl
              "moe_tile_query: bad problem size");
   LO_REQUIRE(dtype == LO_BF16 || dtype == LO_F16 || dtype == LO_F32, LO_EINVAL, "moe_tile_query: unknown dtype %d", dtype);
   if (form == LO_FORM_W4) flags |= LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED;
-  int32_t bm = block_size_m;
-  bool fused = false, decode = false;
-  if (form == LO_FORM_CHANNEL) {
-    const bool pre = (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) != 0;
-    if (bm == 0)
-      bm = pick_block_m(M, num_experts, top_k, H, I, form, true, (flags & LO_GEMM_W4) != 0,
-                        pre && H / kGroup <= 128 && I / kGroup <= 128);
-  } else {
-    BlockPlan plan;
-    const int rc = plan_block_path(dtype, flags, M, num_experts, top_k, H, I, block_size_m, &plan);
-    if (rc) return rc;
-    flags = plan.flags;
-    bm = plan.block_size_m;
-    fused = !plan.unfused;
-    // (fp16 rows and GELU: the query describes the staged path)
-    decode = plan.try_decode && dtype == LO_BF16 && !(flags & LO_FUSED_ACT_GELU) && M > 0 &&
-             decode_path_applies(M, top_k, H, I, E_local > 0 ? E_local : num_experts, num_experts,
-                                 (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, (flags & LO_GEMM_W4) != 0, false, false);
-  }
+  const int32_t E = E_local > 0 ? E_local : num_experts;
+  const bool channel = form == LO_FORM_CHANNEL;
+  PathPlan plan;
+  const int rc = channel ? plan_channel_path(flags, M, num_experts, top_k, H, I, block_size_m, true, &plan)
+                         : plan_block_path(dtype, flags, M, num_experts, top_k, H, I, block_size_m, &plan);
+  if (rc) return rc;
+  flags = plan.flags;
+  const int32_t bm = plan.block_size_m;
+  DecProblem dec{};
+  dec.dtype = dtype; dec.M = M; dec.H = H; dec.I = I; dec.E = E; dec.num_experts = num_experts; dec.top_k = top_k;
+  dec.channel = channel;
+  const bool decode = plan.try_decode && decode_path_applies(dec, flags);
   const bool pre = (flags & LO_GEMM_W_PRESHUFFLED) != 0;
   // the argument blocks the stage entry points would build for this problem
   GemmArgs a{};
   a.num_valid = M * top_k;
-  a.E = E_local > 0 ? E_local : num_experts;
+  a.E = E;
   a.experts_routed = num_experts;
   set_top_k(a, top_k);
   a.w_shuffled = pre ? 1 : 0;
   a.w4 = (flags & LO_GEMM_W4) ? 1 : 0;
-  a.per_channel = form == LO_FORM_CHANNEL ? 1 : 0;
+  a.per_channel = channel ? 1 : 0;
   a.out_f16 = dtype == LO_F16 ? 1 : 0;
   a.out_f32 = dtype == LO_F32 ? 1 : 0;
   const int gflags = flags & ~(LO_FUSED_ACT_GELU | LO_FUSED_NO_DECODE_PATH | LO_FUSED_FORCE_DECODE_PATH);
   auto rows = [&](bool fa) { return !(gflags & LO_GEMM_FORCE_STREAMING) && gemm_rows_supports(a, fa, bm); };
   if (gemm1) {
     a.N = 2 * I; a.K = H; a.a_rows = M;
-    describe_gemm_kernel(pick_gemm_kernel(a, fused, bm, gflags), fused, bm, rows(fused), a, gemm1);
+    describe_gemm_kernel(pick_gemm_kernel(a, plan.fused, bm, gflags), plan.fused, bm, rows(plan.fused), a, gemm1);
   }
   if (gemm2) {
     a.N = H; a.K = I; a.a_rows = M * top_k;
     describe_gemm_kernel(pick_gemm_kernel(a, false, bm, gflags), false, bm, rows(false), a, gemm2);
   }
-  // a few tokens: the whole-path call serves the block form with its two-launch path
+  // a few tokens: the whole-path calls serve them with the two-launch path
   if (decode) {
     int w1 = 0, w2 = 0;
     decode_path_waves(top_k, H, &w1, &w2);
@@ -378,7 +388,7 @@ extern "C" int lo_fused_experts_block_int8(
   LO_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, LO_EINVAL,
              "fused_experts: workspace must be 256-byte aligned");
   if (M == 0) return LO_OK;
-  BlockPlan plan;
+  PathPlan plan;
   const int rc_plan = plan_block_path(dtype, flags, M, num_experts, top_k, H, I, block_size_m, &plan);
   if (rc_plan) return rc_plan;
   flags = plan.flags;
@@ -402,12 +412,11 @@ extern "C" int lo_fused_experts_block_int8(
   // Decode sizes: routing, quantisation, both GEMMs and the reduction in two launches (in the default scale
   // order, or the one of LO_GEMM_SEPARATE_ORDER; LO_GEMM_FUSED_SCALE buys nothing there and gets the default).
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
-  const bool unfused = plan.unfused;
   if (plan.try_decode) {
     // (cache3 is the front of the caller's cache13: the path keeps its bf16 activations [S, I] there)
     const DecProblem d{x, dtype, M, H, I, E, num_experts, top_k, w1, w1s, w2, w2s, topk_w, topk_ids, ids_dtype, expert_map,
                        apply_router_weight_on_input, routed_scaling_factor, shared_output, cache3, out, false};
-    const int rc2 = launch_decode_path(d, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, flags, static_cast<hipStream_t>(stream));
+    const int rc2 = launch_decode_path(d, flags, static_cast<hipStream_t>(stream));
     if (rc2 != LO_ENOTSUP) return rc2;
   }
 
@@ -425,7 +434,7 @@ extern "C" int lo_fused_experts_block_int8(
                                     L.align_scratch, stream);
   }
   if (rc) return rc;
-  if (unfused) {
+  if (!plan.fused) {
     // rows of slots whose expert another rank holds are neither written by the first GEMM nor read by
     // the activation launch (the slot mask of the alignment says which)
     rc = lo_moe_gemm_block_int8(a1q, a1s, w1, w1s, cache3, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
@@ -481,20 +490,10 @@ static int fused_experts_channel(
   LO_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, LO_EINVAL,
              "fused_experts(channel): workspace must be 256-byte aligned");
   if (M == 0) return LO_OK;
-  // a few tokens, weights in the load-time layout, rows not quantised by the caller: two launches
-  const bool try_decode = block_size_m == 0 && x && (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) &&
-                          !(flags & LO_FUSED_NO_DECODE_PATH);
-  if (block_size_m == 0)
-    block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_CHANNEL, true, (flags & LO_GEMM_W4) != 0,
-                                (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) && H / kGroup <= 128 &&
-                                    I / kGroup <= 128);
-  // 160: the 160-token form of the direct-to-LDS kernel (weights in the load-time layout)
-  const bool bs160 = block_size_m == 160 && (flags & (LO_GEMM_W4 | LO_GEMM_W_PRESHUFFLED)) && H / kGroup <= 128 &&
-                     I / kGroup <= 128;
-  LO_REQUIRE(block_size_m == 16 || block_size_m == 32 || block_size_m == 64 || block_size_m == 128 || bs160,
-             LO_EINVAL,
-             "fused_experts(channel): block_size_m %d is not one of 16, 32, 64, 128 (160: weights in the load-time "
-             "layout)", block_size_m);
+  PathPlan plan;
+  const int rc_plan = plan_channel_path(flags, M, num_experts, top_k, H, I, block_size_m, x != nullptr, &plan);
+  if (rc_plan) return rc_plan;
+  block_size_m = plan.block_size_m;
   // the block layout is roomy enough: its scale segments hold one float per 128 values
   const WsLayout L = ws_layout(M, top_k, H, I, num_experts, block_size_m);
   LO_REQUIRE(workspace_bytes >= L.total, LO_ENOSPC,
@@ -511,10 +510,10 @@ static int fused_experts_channel(
   uint8_t *mask = expert_map ? reinterpret_cast<uint8_t *>(ws + L.off[7]) : nullptr;
   const int64_t S = M * top_k;
 
-  if (try_decode) {
+  if (plan.try_decode) {
     const DecProblem d{x, dtype, M, H, I, E, num_experts, top_k, w1, w1s, w2, w2s, topk_w, topk_ids, ids_dtype, expert_map,
                        apply_router_weight_on_input, routed_scaling_factor, shared_output, cache13, out, true};
-    const int rc2 = launch_decode_path(d, (flags & LO_FUSED_FORCE_DECODE_PATH) != 0, flags, static_cast<hipStream_t>(stream));
+    const int rc2 = launch_decode_path(d, flags, static_cast<hipStream_t>(stream));
     if (rc2 != LO_ENOTSUP) return rc2;
   }
   int rc;
@@ -530,7 +529,7 @@ static int fused_experts_channel(
   if (rc) return rc;
   const int gflags = flags & ~LO_FUSED_ACT_GELU;
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
-  const bool gated = gated_channel_supports(H, block_size_m, flags);
+  const bool gated = plan.fused;
   const uint16_t *table = nullptr;
   if (gated && (gelu || dtype == LO_F16)) {
     rc = act_table(static_cast<hipStream_t>(stream), gelu ? LO_ACT_GELU : LO_ACT_SILU, dtype, &table);
@@ -638,7 +637,7 @@ extern "C" int lo_fused_experts_block_int8_noalloc(
   LO_REQUIRE(dtype == LO_BF16 || dtype == LO_F16 || (dtype == LO_F32 && !(flags & LO_GEMM_W4)), LO_ENOTSUP,
              "fused_experts(noalloc): activations are bf16, fp16 or (int8 weights) fp32");
   // the block size the workspace form will resolve to (same function, same arguments), for the space check
-  BlockPlan plan;
+  PathPlan plan;
   const int rc_plan = plan_block_path(dtype, flags, M, num_experts, top_k, H, I, block_size_m, &plan);
   if (rc_plan) return rc_plan;
   const int32_t block_size_m_arg = block_size_m;

@@ -285,11 +285,10 @@ struct DecProblem {
   void *out;
   bool channel;
 };
-// act_fits: `act` holds I values per slot whatever H is.  Whether the path is taken; LO_ENOTSUP from the launcher if not.
-bool decode_path_applies(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_t E, int32_t num_experts, bool force, bool w4,
-                         bool channel, bool act_fits);
+// Whether the path is taken: by sizes, element type and flags alone, so that the tile query asks with the pointers null.
+bool decode_path_applies(const DecProblem &d, int flags);
 void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_waves);
-int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t stream);
+int launch_decode_path(const DecProblem &d, int flags, hipStream_t stream); // LO_ENOTSUP if it is not
 
 // Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
 // lo_moe_gemm_w8a8, and with `fused` its gated form (N = 2I, C [num_valid, I]).

@@ -690,14 +690,42 @@ static int decode_max_slots() {
   return v;
 }
 
-bool decode_path_applies(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_t E, int32_t num_experts, bool force, bool w4,
-                         bool channel, bool act_fits) {
-  const int64_t S = M * top_k;
-  if (S > kDecMaxSlots || top_k > 64) return false;
-  if (H % kGroup || I % kGroup || 2 * I * H >= (1ll << 31)) return false;
-  if ((!act_fits && I > H) || I / kGroup > kDecMaxKB2) return false; // the activations [S, I] live in the caller's buffer
-  if (pick_waves(static_cast<int>(H / kGroup)) == 0) return false;
-  if (force) return true;
+// Column pieces per workgroup of the second kernel, and the dynamic LDS of both kernels.
+static int decode_path_nrb2(const DecProblem &d, int W2) {
+  // A rank that holds a fraction of the experts serves that fraction of a token's slots: its workgroups of the second kernel
+  // take as many more 16-column pieces, so that their waves have work, while the grid still covers the chip (one token of
+  // a 32/256 rank, 7168 wide: 10.0 us with one piece, 15.7 with eight; four tokens: 27.1 with one, 19.8 with eight).
+  int nrb2 = 1;
+  while (nrb2 < 8 && static_cast<int64_t>(nrb2) * 2 * d.E <= d.num_experts && d.H / 16 * d.M / (2 * nrb2) >= 384) nrb2 *= 2;
+  while (nrb2 * 16 > 64 * W2) nrb2 /= 2;
+  return nrb2;
+}
+static void decode_path_lds(const DecProblem &d, bool w4, size_t *l1, size_t *l2) {
+  const int64_t S = d.M * d.top_k;
+  const size_t KB1 = static_cast<size_t>(d.H / kGroup), KB2 = static_cast<size_t>(d.I / kGroup);
+  int w1, w2;
+  decode_path_waves(d.top_k, d.H, &w1, &w2);
+  const size_t W1 = static_cast<size_t>(w1), W2 = static_cast<size_t>(w2);
+  const size_t list = S > 64 ? static_cast<size_t>((S + 3) & ~int64_t(3)) * 4 : 0;
+  *l1 = (d.channel ? W1 * 512 : KB1 * (128 + (w4 ? 32 : 2)) * 4) + W1 * kDecTP * 4 + list + 16 +
+        W1 * kDecTP * kDecMaxKBw * 4 + W1 * kDecTP * (KB1 / W1 * kGroup + 16);
+  *l2 = ((static_cast<size_t>(decode_path_nrb2(d, w2)) * d.top_k * 32 + 15) & ~size_t(15)) +
+        ((W2 * KB2 * 4 + 15) & ~size_t(15)) + W2 * static_cast<size_t>(d.I);
+}
+
+bool decode_path_applies(const DecProblem &d, int flags) {
+  const bool w4 = (flags & LO_GEMM_W4) != 0;
+  const int64_t S = d.M * d.top_k;
+  if (d.dtype != LO_BF16 && d.dtype != LO_F16) return false;
+  if (d.M < 1 || S > kDecMaxSlots || d.top_k > 64) return false;
+  if (d.H % kGroup || d.I % kGroup || 2 * d.I * d.H >= (1ll << 31)) return false;
+  // the activations [S, I] live in the caller's buffer: [S, max(2I, H)], or [S, H] for bf16 rows with SiLU in the block form
+  if (!d.channel && !(flags & LO_FUSED_ACT_GELU) && d.dtype == LO_BF16 && d.I > d.H) return false;
+  if (d.I / kGroup > kDecMaxKB2 || pick_waves(static_cast<int>(d.H / kGroup)) == 0) return false;
+  size_t l1, l2;
+  decode_path_lds(d, w4, &l1, &l2);
+  if (l1 > 64 * 1024 || l2 > 64 * 1024) return false;
+  if (flags & LO_FUSED_FORCE_DECODE_PATH) return true;
   const int forced = decode_max_slots();
   if (forced >= 0) return S <= forced;
   // Where the two launches and the staged path with its weight-streaming kernels cross (us, two launches / staged):
@@ -705,10 +733,10 @@ bool decode_path_applies(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_t
   // int8, longer K: DeepSeek-V3's 32-expert share 72 / 82 at 4 tokens and 96 / 90 at 8, all 256 experts 81 / 87 at 1 token and
   // 120 / 113 at 2, so what counts are the slots on this rank;
   // int4: per-channel scales 70 / 72 at 32 slots and 122 / 108 at 64, K groups 31 / 41 at 8 and 50 / 48 at 16.
-  if (w4) return S <= (channel ? 32 : 16);
-  const int KB = static_cast<int>(H / kGroup);
+  if (w4) return S <= (d.channel ? 32 : 16);
+  const int KB = static_cast<int>(d.H / kGroup);
   if (KB / pick_waves(KB) <= 4) return S <= 64;
-  return S <= 32 && S * E <= static_cast<int64_t>(8) * num_experts;
+  return S <= 32 && S * d.E <= static_cast<int64_t>(8) * d.num_experts;
 }
 
 void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_waves) {
@@ -717,11 +745,9 @@ void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_wa
 }
 
 // Whole path in two launches; LO_ENOTSUP when the problem is not a decode-size one this file serves.
-int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t stream) {
+int launch_decode_path(const DecProblem &d, int flags, hipStream_t stream) {
   const bool w4 = (flags & LO_GEMM_W4) != 0, gelu = (flags & LO_FUSED_ACT_GELU) != 0;
-  const bool act_fits = d.channel || gelu || d.dtype == LO_F16; // the caller's buffer holds [S, max(2I, H)] then
-  if (d.dtype != LO_BF16 && d.dtype != LO_F16) return LO_ENOTSUP;
-  if (!decode_path_applies(d.M, d.top_k, d.H, d.I, d.E, d.num_experts, force, w4, d.channel, act_fits)) return LO_ENOTSUP;
+  if (!decode_path_applies(d, flags)) return LO_ENOTSUP;
   const int64_t S = d.M * d.top_k;
   const int KB1 = static_cast<int>(d.H / kGroup), KB2 = static_cast<int>(d.I / kGroup);
   int W1, W2;
@@ -745,13 +771,7 @@ int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t s
     const int rc = act_table(stream, LO_ACT_GELU, d.dtype, &a.table);
     if (rc) return rc;
   }
-  // A rank that holds a fraction of the experts serves that fraction of a token's slots: its workgroups of the second kernel
-  // take as many more 16-column pieces, so that their waves have work, while the grid still covers the chip (one token of
-  // a 32/256 rank, 7168 wide: 10.0 us with one piece, 15.7 with eight; four tokens: 27.1 with one, 19.8 with eight).
-  a.nrb2 = 1;
-  while (a.nrb2 < 8 && static_cast<int64_t>(a.nrb2) * 2 * d.E <= d.num_experts && d.H / 16 * d.M / (2 * a.nrb2) >= 384)
-    a.nrb2 *= 2;
-  while (a.nrb2 * 16 > 64 * W2) a.nrb2 /= 2;
+  a.nrb2 = decode_path_nrb2(d, W2);
   // workgroups along the distinct experts: what the batch can hit here, some to spare; more are served in rounds
   int64_t hits = S;
   if (S <= 64) {
@@ -761,13 +781,8 @@ int launch_decode_path(const DecProblem &d, bool force, int flags, hipStream_t s
     hits = hits < d.E ? hits : d.E;
   }
 
-  const size_t list = S > 64 ? static_cast<size_t>((S + 3) & ~int64_t(3)) * 4 : 0;
-  const size_t l1 = (d.channel ? static_cast<size_t>(W1) * 512 : static_cast<size_t>(KB1) * (128 + (w4 ? 32 : 2)) * 4) +
-                    static_cast<size_t>(W1) * kDecTP * 4 + list + 16 + static_cast<size_t>(W1) * kDecTP * kDecMaxKBw * 4 +
-                    static_cast<size_t>(W1) * kDecTP * (a.kbw * kGroup + 16);
-  const size_t l2 = ((static_cast<size_t>(a.nrb2) * d.top_k * 32 + 15) & ~size_t(15)) +
-                    ((static_cast<size_t>(W2) * KB2 * 4 + 15) & ~size_t(15)) + static_cast<size_t>(W2) * d.I;
-  if (l1 > 64 * 1024 || l2 > 64 * 1024) return LO_ENOTSUP;
+  size_t l1, l2;
+  decode_path_lds(d, w4, &l1, &l2);
   const dim3 g1(static_cast<unsigned>(d.I / 16), static_cast<unsigned>(hits));
   const dim3 g2(static_cast<unsigned>(d.H / 16 / a.nrb2), static_cast<unsigned>(d.M));
 #define LO_DEC_LAUNCH(W4V, PCV, DTV)                                                                             \

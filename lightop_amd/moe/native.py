@@ -35,8 +35,9 @@ def get_w8a8moe_json(m: int, E: int, n1: int, n2: int, k: int, use_int8_w8a8: bo
     keep the reference's keys; ``kernel`` / ``num_warps`` / ``BLOCK_SIZE_N`` describe the kernel the
     whole-path call launches for that block size, ``source`` says where the block size came from.
     ``preshuffled``: the weights are in the load-time layout of ``preshuffle_moe_weight`` (the table
-    differs for row-major weights); ``dtype`` / ``activation``: rows other than bfloat16 and GELU take the
-    path without the fused epilogue."""
+    differs for row-major weights); ``dtype`` / ``activation``: float16 rows and GELU have a fused first stage at
+    64- and 128-token blocks only, float32 rows none at all, and 160-token blocks are picked for bfloat16 rows with
+    SiLU only (any 16-bit rows with ``block_shape=None``)."""
     del use_int8_w8a8
     from . import tile_files
 

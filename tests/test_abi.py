@@ -161,8 +161,9 @@ def test_tile_query_names_the_kernel_that_is_launched(lib):
     assert q(_lib.LO_FORM_CHANNEL, pre, 4096, *qwen) == 0 and t1.block_size_m == 128  # int8 weights: no second window
     assert q(_lib.LO_FORM_CHANNEL, pre, 2048, *qwen) == 0 and (t1.block_size_m, t1.kernel) == (160, _lib.LO_KERNEL_T128)
     assert q(_lib.LO_FORM_CHANNEL, 0, 2048, *qwen) == 0 and t1.block_size_m == 128  # row-major weights: no such form
-    assert q(_lib.LO_FORM_W4, 0, 2, *dsv3) == 0 and t1.kernel == _lib.LO_KERNEL_DEC  # int4: up to 16 slots
-    assert q(_lib.LO_FORM_W4, 0, 4, *dsv3) == 0 and t1.kernel == _lib.LO_KERNEL_WS
+    assert q(_lib.LO_FORM_W4, 0, 2, *qwen) == 0 and t1.kernel == _lib.LO_KERNEL_DEC  # int4: up to 16 slots
+    assert q(_lib.LO_FORM_W4, 0, 4, *qwen) == 0 and t1.kernel == _lib.LO_KERNEL_WS
+    assert q(_lib.LO_FORM_W4, 0, 2, *dsv3) == 0 and t1.kernel == _lib.LO_KERNEL_WS  # its first kernel's LDS does not fit
     assert q(_lib.LO_FORM_W4, 0, 512, *dsv3) == 0 and t1.kernel == _lib.LO_KERNEL_W4_TILE
     assert q(_lib.LO_FORM_W4, 0, 8192, *dsv3) == 0 and t1.kernel == _lib.LO_KERNEL_T128
     # the convenience query is the block form with the load-time layout
@@ -243,11 +244,21 @@ def test_tile_query_path_follows_element_type_activation_and_block_size(lib):
             want = q(_lib.LO_FORM_BLOCK, pre, _lib.LO_BF16, 0, M, shape)
             assert lib.lo_moe_tile_query_form(_lib.LO_FORM_BLOCK, pre, M, *shape, t1, t2) == 0
             assert ((t1.block_size_m, t1.kernel), (t2.block_size_m, t2.kernel)) == want
-    # one token: bf16 + SiLU takes the two-launch path; GELU and fp16 rows have no fused epilogue and never do
-    assert q(_lib.LO_FORM_BLOCK, pre, _lib.LO_BF16, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_DEC
-    assert q(_lib.LO_FORM_BLOCK, pre | _lib.LO_FUSED_ACT_GELU, _lib.LO_BF16, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_WS
-    assert q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F16, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_WS
-    # the plain first GEMM of those paths has the plain workgroup shape (four waves), not the fused one (eight)
+    # one token: the two-launch path, whatever the form, the 16-bit type and the activation; row-major weights never
+    for form, flags in ((_lib.LO_FORM_BLOCK, pre), (_lib.LO_FORM_CHANNEL, pre), (_lib.LO_FORM_CHANNEL, pre | _lib.LO_GEMM_W4),
+                        (_lib.LO_FORM_W4, 0)):
+        for act in (0, _lib.LO_FUSED_ACT_GELU):
+            for dtype in (_lib.LO_BF16, _lib.LO_F16):
+                assert q(form, flags | act, dtype, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_DEC, (form, flags, act, dtype)
+                assert q(form, flags | act | _lib.LO_FUSED_NO_DECODE_PATH, dtype, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_WS
+    assert q(_lib.LO_FORM_CHANNEL, 0, _lib.LO_BF16, 0, 1, qwen)[0][1] == _lib.LO_KERNEL_WS
+    # what the launcher refuses for want of LDS is not reported either
+    # (K-group scales of 56 K blocks beside the products of as many)
+    force = _lib.LO_FUSED_FORCE_DECODE_PATH
+    assert q(_lib.LO_FORM_W4, force, _lib.LO_BF16, 0, 1, dsv3)[0][1] == _lib.LO_KERNEL_WS
+    assert q(_lib.LO_FORM_BLOCK, pre | force, _lib.LO_BF16, 0, 64, dsv3)[0][1] == _lib.LO_KERNEL_DEC
+    # the plain first GEMM that GELU and fp16 rows have with the weight-streaming kernel has the plain workgroup shape (four waves), not the
+    # fused one (eight)
     q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F16, 0, 16, dsv3)
     assert (t1.kernel, t1.waves) == (_lib.LO_KERNEL_WS, 4)
     q(_lib.LO_FORM_BLOCK, pre, _lib.LO_BF16, 0, 16, dsv3)
@@ -270,6 +281,6 @@ def test_tile_query_path_follows_element_type_activation_and_block_size(lib):
     assert lib.lo_moe_tile_query_path(_lib.LO_FORM_BLOCK, pre, _lib.LO_BF16, 48, 64, *qwen, t1, t2) < 0
     assert lib.lo_moe_tile_query_path(_lib.LO_FORM_BLOCK, pre, 9, 0, 64, *qwen, t1, t2) < 0
     # int4 weights imply the load-time layout in the whole-path call, at every size
-    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, dsv3)[0][1] == _lib.LO_KERNEL_DEC
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, qwen)[0][1] == _lib.LO_KERNEL_DEC
     assert q(_lib.LO_FORM_BLOCK, _lib.LO_GEMM_W4, _lib.LO_BF16, 0, 2048, dsv3) == \
         q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2048, dsv3)

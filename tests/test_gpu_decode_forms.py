@@ -108,3 +108,29 @@ def test_one_token_with_a_repeated_expert(form, H, dtype, routing):
         outs.append(run(x, tw, ids, cache13, expert_map=emap, lightop_amd_flags=flag).cpu())
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+@pytest.mark.parametrize("form", ["block", "channel", "w4", "w4_channel"])
+def test_tile_query_names_the_path_that_is_taken(form, activation, dtype):
+    """On both sides of every form's line between the two-launch path, which leaves the workspace alone, and the
+    staged path, which does not."""
+    from lightop_amd import workloads as wl
+    from lightop_amd.moe import get_w8a8moe_json
+
+    dev, k, (E, H, I) = torch.device("cuda:0"), 8, (16, 1024, 256)
+    layer, run = make_layer(form, activation, "query", E, E, k, H, I)
+    block_shape = None if "channel" in form else [1, 128] if form == "w4" else [128, 128]
+    taken = []
+    for M in (1, 2, 3, 4, 5, 8, 9):
+        print(f"[case] tile query {form} {activation} {dtype} M={M}", flush=True)
+        x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, M, seed=M))
+        cache13 = torch.empty(M * k * max(2 * I, H), dtype=dtype, device=dev)
+        ws = torch.full((1 << 20,), 0xA5, dtype=torch.uint8, device=dev)
+        run(x.to(dtype), tw, ids, cache13, lightop_amd_workspace=ws)
+        kernel = get_w8a8moe_json(M, E, 2 * I, H, I, True, block_shape, k, E, int4=form.startswith("w4"), dtype=dtype,
+                                  activation=activation)[0]["kernel_name"]
+        taken.append(bool((ws == 0xA5).all()))
+        assert taken[-1] == kernel.startswith("dec_"), (M, kernel)
+    assert taken[0] and not taken[-1]
