@@ -187,8 +187,6 @@ __device__ __forceinline__ float fold_elem(int d, float sc, float as, float bs, 
     else MACRO(::lo::kOrdFusedScale, __VA_ARGS__);                         \
   } while (0)
 
-__device__ __forceinline__ v4i ld16(const int8_t *p) { return *reinterpret_cast<const v4i *>(p); }
-
 // Buffer addressing: a wave-uniform 128-bit resource (base, extent) + one 32-bit lane
 // offset + one scalar offset.  The K loop then advances a scalar only, no per-lane 64-bit
 // address arithmetic, and a read past the extent returns zero instead of faulting.
@@ -290,7 +288,6 @@ bool decode_path_applies(const DecProblem &d, int flags);
 void decode_path_waves(int32_t top_k, int64_t H, int *gemm1_waves, int *gemm2_waves);
 int launch_decode_path(const DecProblem &d, int flags, hipStream_t stream); // LO_ENOTSUP if it is not
 
-// Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
 // lo_moe_gemm_w8a8, and with `fused` its gated form (N = 2I, C [num_valid, I]).
 int launch_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype, int fused,
                      const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
@@ -303,6 +300,7 @@ int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, co
                            const int32_t *expert_ids, const int32_t *num_tokens_post_pad, int64_t sorted_cap,
                            int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts, int64_t I, int64_t K,
                            int32_t top_k, int32_t block_size_m, int mul_routed, int flags, hipStream_t stream);
+// Weight-streaming kernels (gemm_ws.hip): block_size_m in {16, 32, 64, 128}.
 int launch_gemm_ws(const GemmArgs &a, bool fused_act, int block_size_m, int flags, int64_t m_blocks,
                    hipStream_t s);
 // LDS-tiled kernels (gemm_tile.hip): block_size_m 64 or 128, compute-bound regime.

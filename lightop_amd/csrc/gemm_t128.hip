@@ -30,12 +30,6 @@
 
 #include "gemm.h"
 
-#ifndef LO_EARLY10
-#define LO_EARLY10 20
-#endif
-#ifndef LO_EARLY
-#define LO_EARLY 12
-#endif
 namespace lo {
 
 constexpr int kT = 128;                       // tokens per workgroup
@@ -763,12 +757,6 @@ bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   return a.K / kGroup <= kTMaxKB;
 }
 
-#ifndef LO_DMA_SIZES
-#define LO_DMA_SIZES (16+32+64)
-#endif
-#ifndef LO_DMA_SHUF
-#define LO_DMA_SHUF (16)
-#endif
 // ---- row-major weights -----------------------------------------------------------------------------------
 // Weights as a checkpoint holds them, [E, N, K].  Loading an MFMA operand straight from global memory asks for 64 bytes
 // of each of 16 rows per instruction (32 of 32 rows with the 32x32 form): every 128-byte line is requested two to four
