@@ -3,6 +3,8 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
@@ -125,19 +127,44 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def binding_key() -> str:
+    """What the host binding has to be built for: it uses torch's C++ types, whose layout belongs to one version."""
+    import torch
+
+    return f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
+class _NoHost:
+    """In the binding's place where it cannot be used: declines every call, which Python then marshals for the same
+    library."""
+
+    @staticmethod
+    def _decline(*args):
+        return None
+
+    fused_experts = topk_softmax = fused_gate = _decline
+
+
 def host():
     """The native marshalling of the calls a serving loop makes on every step (csrc/host_binding.cpp), bound to
-    the library above.  Built with it, and as little optional."""
+    the library above.  Where it is missing or was built for another torch or Python, the calls are marshalled in Python
+    instead, as every other call is; that costs host time and nothing else, and a warning says so once."""
     global _host
     if _host is None:
         handle = lib()
-        import torch  # noqa: F401  (its libraries are what the module links against)
-
+        key, problem = binding_key(), ""
         try:
             from . import _host as mod
-        except ImportError as e:
-            raise RuntimeError(f"lightop_amd: the host binding cannot be loaded ({e}): build it with "
-                               "`python -m lightop_amd.build`") from e
+
+            if mod.built_for != key:
+                problem = f"it was built for {mod.built_for}, this is {key}"
+        except (ImportError, AttributeError) as e:
+            problem = str(e)
+        if problem:
+            warnings.warn(f"lightop_amd: the host binding cannot be used ({problem}): a call takes about 10 us more of host "
+                          "time; build it with `python -m lightop_amd.build`", RuntimeWarning, stacklevel=3)
+            _host = _NoHost()
+            return _host
         mod.bind(*(ctypes.cast(getattr(handle, n), c_void_p).value for n in (
             "lo_fused_experts_block_int8", "lo_fused_experts_channel_int8", "lo_fused_experts_workspace_bytes",
             "lo_topk_softmax", "lo_moe_fused_gate", "lo_last_error")))

@@ -68,10 +68,12 @@ def build_host(out_path: str = HOST_PATH) -> str:
     import torch
     from torch.utils import cpp_extension
 
+    from ._lib import binding_key
+
     lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
     includes = [f"-I{d}" for d in (*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"])]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           *includes, HOST_SRC, "-o", out_path, f"-L{lib_dir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+           f'-DLO_BUILT_FOR="{binding_key()}"', *includes, HOST_SRC, "-o", out_path, f"-L{lib_dir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
            "-lc10", "-lc10_hip"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

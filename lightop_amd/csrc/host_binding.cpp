@@ -44,12 +44,13 @@ const at::Tensor *tensor_of(PyObject *o) {
   return &THPVariable_Unpack(o);
 }
 
-// Whether the tensor object carries a true attribute `name` (an entry of its instance dictionary).
+// Whether the tensor object carries a true attribute `name` (an entry of its instance dictionary: asking for an attribute
+// that is not there would raise and clear an exception on every call with row-major weights).
 bool flag_of(PyObject *o, PyObject *name) {
-  PyObject **d = _PyObject_GetDictPtr(o);
-  if (!d || !*d) return false;
-  PyObject *v = PyDict_GetItemWithError(*d, name);
+  PyObject *d = PyObject_GenericGetDict(o, nullptr);
+  PyObject *v = d ? PyDict_GetItemWithError(d, name) : nullptr;
   const int is = v ? PyObject_IsTrue(v) : 0;
+  Py_XDECREF(d);
   if (PyErr_Occurred()) PyErr_Clear();
   return is == 1;
 }
@@ -364,5 +365,10 @@ PyMODINIT_FUNC PyInit__host(void) {
   s_int4 = PyUnicode_InternFromString("lo_int4");
   s_kmajor = PyUnicode_InternFromString("lo_kmajor");
   if (!s_preshuffled || !s_int4 || !s_kmajor) return nullptr;
-  return PyModule_Create(&module);
+  PyObject *m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", LO_BUILT_FOR) < 0) { // checked before the first call
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

@@ -237,3 +237,25 @@ def test_threads_share_a_stream(form):
     torch.cuda.synchronize()
     for i in (0, 1):
         assert len(got[i]) == 200 and all(torch.equal(o.view(torch.int16), want[i].view(torch.int16)) for o in got[i])
+
+
+def test_without_the_binding(monkeypatch):
+    """The routers and the whole path with the Python marshalling alone."""
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import fused_experts_impl_int8, moe_fused_gate, topk_softmax
+
+    dev = torch.device("cuda:0")
+    layer, weights, kw = _layer("block", dev)
+    x, _, _ = (t.to(dev) for t in wl.make_inputs(layer, 21, seed=3))
+    logits = torch.randn(21, layer.E, device=dev)
+    cache13 = torch.empty(21 * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
+    outs = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(_lib, "_host", _lib._NoHost())
+        w, ids = torch.empty(21, layer.top_k, device=dev), torch.empty(21, layer.top_k, dtype=torch.int32, device=dev)
+        topk_softmax(w, ids, None, logits, True)
+        gw, gi = moe_fused_gate(logits, torch.zeros(layer.E, device=dev), 2, 1, 2, 0, 2.5)
+        out = fused_experts_impl_int8(x, *weights, w, ids, cache13, use_int8_w8a8=True, block_shape=[128, 128], **kw)
+        outs.append((w, ids, gw, gi, out.view(torch.int16)))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))

@@ -421,3 +421,30 @@ def test_expert_ids_must_cover_the_blocks_the_grid_reaches():
     _check_block_extents(sorted_ids, torch.zeros(3, dtype=torch.int32), 128, 3)        # at most one block per slot
     with pytest.raises(ValueError, match="span 7 blocks"):
         _check_block_extents(sorted_ids, torch.zeros(6, dtype=torch.int32), 128, 10_000)
+
+
+@pytest.mark.parametrize("problem", ["another torch", "older binding", "missing"])
+def test_calls_go_through_python_without_a_usable_binding(problem, monkeypatch):
+    """A host binding that is missing, or built for another torch, is not used: one warning, and every call is declined,
+    so that Python marshals it."""
+    import sys
+
+    import lightop_amd
+    from lightop_amd import _lib
+
+    monkeypatch.setattr(_lib, "_host", None)
+    if problem == "missing":
+        monkeypatch.setitem(sys.modules, "lightop_amd._host", None)
+        monkeypatch.delattr(lightop_amd, "_host", raising=False)
+    else:
+        from lightop_amd import _host
+
+        assert _host.built_for == _lib.binding_key()  # the one that is there is this torch's
+        if problem == "another torch":
+            monkeypatch.setattr(_host, "built_for", "torch 2.9.1+rocm6.4, Python 3.10")
+        else:
+            monkeypatch.delattr(_host, "built_for")
+    with pytest.warns(RuntimeWarning, match="host binding"):
+        host = _lib.host()
+    assert _lib.host() is host
+    assert host.topk_softmax(*range(5)) is None and host.fused_gate(*range(9)) is None and host.fused_experts(*range(16)) is None
