@@ -882,15 +882,17 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     }                                                                                                           \
   } while (0)
   if (block_size_m == kT160) {
-    const int64_t experts = a.experts_routed > 0 ? a.experts_routed : 1;
-    // Tiles between one and two (two and three, ...) rounds of the 512 resident workgroups: if they take different times,
-    // the compute units that finish first take both workgroups of the last, partial round and the rest none.  Kept alike
-    // they finish together and the partial round spreads one workgroup to a compute unit: 1531 tokens of the
-    // Qwen3-30B-A3B layer (768 tiles) 194 us with the 96-token variant among them, 186 without.  In whole rounds the variant
-    // is worth what it leaves out (DeepSeek-V3 share, one round: 2600 tokens 366 -> 356 us, 3000: 385 -> 376).
-    const double rounds = static_cast<double>(a.E) * ((a.num_valid / experts + kT160 - 1) / kT160) * a.n_tiles / 512.0;
-    const double part = rounds - static_cast<int64_t>(rounds);
-    a.coarse_fill = rounds < 4.0 && part > 0.25 && part < 0.75;
+    // Tiles for one or two rounds of the 512 resident workgroups and almost half a round more: if they take different
+    // times, the compute units that finish first take both workgroups of the half round and the rest none.  Kept alike they
+    // finish together, and the half round is one workgroup to a compute unit.  Whole layer, us, fragments as they are / rounded
+    // up to 8: Qwen3-30B-A3B layer (1.5 rounds of first-stage tiles) at 75 slots per expert 181 / 186, at 84: 191 / 185, at
+    // 92: 197 / 184, at 108: 205 / 195, at 118: 203 / 203; 62 experts of 4096 x 1536 (1.45) at 72: 279 / 289, at 84: 290 / 282, at
+    // 92: 302 / 283.  It costs time where the last round is fuller (130 experts of 2048 x 768, 1.52 rounds, at 92: 209 / 215)
+    // or shorter (128 of 2048 x 640, 1.25, at 88: 172 / 183), with a longer K (48 of 7168 x 2048, 1.5, at 88: 453 / 469) and with
+    // per-channel scales (the first layer at 92: 196 / 198).
+    const double slots = static_cast<double>(a.num_valid) / (a.experts_routed > 0 ? a.experts_routed : 1);
+    const double rounds = static_cast<double>(a.E) * a.n_tiles / 512.0, part = rounds - static_cast<int>(rounds); // (a block an expert)
+    a.coarse_fill = !a.per_channel && a.K <= 4096 && slots >= 84.0 && rounds >= 1.0 && rounds < 3.0 && part >= 0.4 && part <= 0.5;
     // chosen where an expert's tokens fill one block, so a weight byte has one reader: streaming hint
 #define LO_T160_LAUNCH(FS, FA)                                                                                  \
   do {                                                                                                          \

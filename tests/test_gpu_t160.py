@@ -292,6 +292,24 @@ def test_whole_path_tiny_bit_exact(dev, oracle, M, with_map):
         assert torch.equal(out.cpu().view(torch.int16), ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("slots", [83, 84, 118])
+@pytest.mark.parametrize("order", ["contract", "separate"])
+def test_fragments_rounded_up(dev, slots, order):
+    """A first stage of one and a half rounds, on both sides of the slots per expert from which its tiles round the
+    fragments in use up to eight (and where most use that many), against 128-token blocks, which never do."""
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import preshuffle_moe_weight
+
+    say(f"fragments rounded up, {slots} slots per expert {order}")
+    layer = wl.MoeLayer("half-round", E=48, E_global=48, top_k=4, H=256, I=2048, routing="softmax")
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=3, device=dev)
+    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, 12 * slots, seed=slots))
+    wd = (preshuffle_moe_weight(w1), preshuffle_moe_weight(w2), w1s, w2s)
+    flags = {} if order == "contract" else {"lightop_amd_flags": _lib.LO_GEMM_SEPARATE_ORDER}
+    got, want = (_run(layer, wd, x, tw, ids, None, dev, bs, **flags) for bs in (160, 128))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_whole_path_rejects_160_where_it_does_not_apply(dev):
     from lightop_amd import workloads as wl
 
