@@ -426,15 +426,25 @@ __global__ __launch_bounds__(256) void moe_fused_gate16_kernel(const void *__res
 }
 
 // Rows from which the 16-lane kernels are used: below, a row per wavefront finishes sooner, since there are wavefront
-// slots to spare (128 experts, us with a wavefront / a quarter per row: 3.7 / 4.8 at 333 rows, 4.0 / 4.8 at 1531,
-// 4.7 / 4.6 at 4096, 7.3 / 4.7 at 8192).
-constexpr int64_t kRows16From = 4096;
+// slots to spare; above, a quarter of a wavefront per row leaves fewer instructions to issue.  The more experts, the longer
+// a quarter's chain and the later the line.  us, a wavefront / a quarter per row:
+//   softmax, 64 experts:  bf16 2048 rows 3.57 / 3.82, 2560: 3.99 / 3.83, 4096: 4.61 / 3.87
+//            128 experts: bf16 3072 rows 4.35 / 4.68, 3584: 4.87 / 4.68, 8192: 7.11 / 5.10
+//            256 experts: bf16 5120 rows 6.42 / 7.07, 5632: 7.04 / 7.10, 7168: 7.68 / 7.16; fp32 4096: 5.41 / 5.67, 4608: 6.11 / 5.96
+//   gate,    32 experts:  fp32 3072 rows 4.85 / 4.87, 4096: 5.30 / 4.88
+//            64 experts:  fp32 4096 rows 5.59 / 5.76, 5120: 6.20 / 6.00
+//            128 experts: fp32 6144 rows 7.54 / 8.21, 7168: 8.25 / 8.25, 8192: 8.94 / 8.27
+//            256 experts: fp32 8192 rows 11.5 / 13.2 (16 scores per lane): never
+template <int VPT, int DT> constexpr int64_t softmax_rows16_from() {
+  return VPT == 1 ? 2560 : VPT == 2 ? 3584 : DT == LO_F32 ? 4608 : 5632;
+}
+static int64_t gate_rows16_from(int E) { return E <= 32 ? 4096 : E <= 64 ? 4608 : 7168; }
 
 template <int VPT, int DT> static void launch_topk_softmax(const void *g, int64_t T, int E, int k, int renorm,
                                                            float *w, void *idx, int idx_dtype, int32_t *src,
                                                            hipStream_t s) {
   if constexpr (VPT <= 4) { // up to 256 experts
-    if (T >= kRows16From && k <= 16) {
+    if (T >= softmax_rows16_from<VPT, DT>() && k <= 16) {
       const dim3 grid16(static_cast<unsigned>((T + 15) / 16)), block16(256);
       if (idx_dtype == LO_I64)
         hipLaunchKernelGGL((topk_softmax16_kernel<4 * VPT, DT, int64_t>), grid16, block16, 0, s, g, T, E, k, renorm, w,
@@ -459,9 +469,8 @@ static void launch_gate(const void *x, const void *b, int64_t T, int E, int G, i
                         float scale, float *w, void *idx, int idx_dtype, hipStream_t s) {
   GateGroups gg{G, E / G, 4, static_cast<uint32_t>(((1u << 20) + E / G - 1) / (E / G))};
   while ((G << gg.lsh) > 64) --gg.lsh;
-  if constexpr (VPT <= 4) { // up to 256 experts
-    // (256 experts: 16 scores per lane make every selection round longer than the 64-lane kernel's: 14.8 us against 13 at 8192 rows)
-    if (T >= kRows16From && topk <= 16 && G <= 16 && VPT <= 2) {
+  if constexpr (VPT <= 2) { // up to 128 experts
+    if (T >= gate_rows16_from(E) && topk <= 16 && G <= 16) {
       while ((G << gg.lsh) > 16) --gg.lsh;
       const dim3 grid16(static_cast<unsigned>((T + 15) / 16)), block16(256);
       if (idx_dtype == LO_I64)

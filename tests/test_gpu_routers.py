@@ -90,7 +90,7 @@ GATE16_CONFIGS = [(128, 8, 4, 8, 0), (64, 4, 2, 6, 0), (96, 2, 1, 7, 1), (128, 2
 
 
 @pytest.mark.parametrize("E,G,tg,topk,nshare", GATE16_CONFIGS)
-@pytest.mark.parametrize("T", [65, 1000, 4096])
+@pytest.mark.parametrize("T", [65, 1000, 4096, 7201])
 @pytest.mark.parametrize("ties", [False, True])
 def test_moe_fused_gate_16_lane_rows_merge_groups_across_lanes(dev, oracle, E, G, tg, topk, nshare, T, ties):
     from lightop_amd.moe import moe_fused_gate
@@ -167,8 +167,8 @@ def test_router_argument_errors(dev):
 @pytest.mark.parametrize("T", [4095, 4096, 4099])
 @pytest.mark.parametrize("E,G,tg,k", [(16, 4, 1, 3), (100, 5, 2, 8), (128, 8, 4, 8), (256, 8, 4, 8)])
 def test_rows_per_wavefront_change_over(dev, oracle, T, E, G, tg, k):
-    """Either side of the row count from which four rows share a wavefront, with ties, rows of equal scores and a partial last
-    wavefront."""
+    """Both kernels at a few thousand rows (which one serves a case depends on its experts), with ties, rows of equal scores
+    and a partial last wavefront."""
     from lightop_amd.moe import moe_fused_gate
 
     say(f"routers T={T} E={E}")
@@ -183,3 +183,25 @@ def test_rows_per_wavefront_change_over(dev, oracle, T, E, G, tg, k):
     w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, tg, k, 0, 2.5, False)
     rw, ridx = oracle.moe_fused_gate(x, bias, G, tg, k, 0, 2.5, False)
     assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
+
+
+@pytest.mark.parametrize("E,G,k,dtype,lines", [(32, 4, 4, torch.float32, (2560, 4096)), (60, 4, 8, torch.bfloat16, (2560, 4608)),
+                                               (128, 8, 8, torch.float16, (3584, 7168)), (160, 8, 6, torch.float32, (4608, 7168)),
+                                               (256, 8, 8, torch.bfloat16, (5632, 7168))])
+def test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtype, lines):
+    """Row counts around the one from which four rows share a wavefront: it differs by the number of experts, by the type
+    (softmax) and between softmax and gate."""
+    from lightop_amd.moe import moe_fused_gate
+
+    for T in sorted(line + d for line in lines for d in (-1, 0, 3)):
+        say(f"routers T={T} E={E} {dtype}")
+        g = torch.Generator().manual_seed(T + E)
+        x = (torch.randint(-3, 4, (T, E), generator=g).float() * 0.5).to(dtype)
+        x[1], x[-1] = 0.25, -0.5
+        w, idx, _ = run_topk_softmax(x.to(dev), k, True, with_src=False)
+        rw, ridx, _ = oracle.topk_softmax(x, k, True)
+        assert torch.equal(idx, ridx) and torch.equal(w.view(torch.int32), rw.view(torch.int32))
+        bias = (torch.randint(-2, 3, (E,), generator=g).float() * 0.25).to(dtype)
+        w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, 2, k, 0, 2.5, False)
+        rw, ridx = oracle.moe_fused_gate(x, bias, G, 2, k, 0, 2.5, False)
+        assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
