@@ -732,8 +732,14 @@ bool decode_path_applies(const DecProblem &d, int flags) {
   // int8, at most four K blocks per wave: Qwen3 30B 57.6 / 69.5 and 235B 190 / 190 at 64 slots;
   // int8, longer K: DeepSeek-V3's 32-expert share 72 / 82 at 4 tokens and 96 / 90 at 8, all 256 experts 81 / 87 at 1 token and
   // 120 / 113 at 2, so what counts are the slots on this rank;
-  // int4: per-channel scales 70 / 72 at 32 slots and 122 / 108 at 64, K groups 31 / 41 at 8 and 50 / 48 at 16.
-  if (w4) return S <= (d.channel ? 32 : 16);
+  // int4, per-channel scales: 70 / 72 at 32 slots and 122 / 108 at 64;
+  // int4, K groups: experts of 2048 x 768 20 / 32 at 16 slots, 4096 x 768 28 / 39, 4096 x 1536 40 / 43 at 12 and 48 / 44 at 16,
+  // 4096 x 3584 65 / 51 at 14; with fp16 rows or GELU, whose staged path has a launch more, 4096 x 1536 48 / 48 at 16.
+  if (w4 && d.channel) return S <= 32;
+  if (w4) {
+    const bool large = d.H * d.I >= 4096ll * 1536, fused_stage = d.dtype == LO_BF16 && !(flags & LO_FUSED_ACT_GELU);
+    return S <= (large && fused_stage ? 12 : 16);
+  }
   const int KB = static_cast<int>(d.H / kGroup);
   if (KB / pick_waves(KB) <= 4) return S <= 64;
   return S <= 32 && S * d.E <= static_cast<int64_t>(8) * d.num_experts;

@@ -257,6 +257,14 @@ def test_tile_query_path_follows_element_type_activation_and_block_size(lib):
     force = _lib.LO_FUSED_FORCE_DECODE_PATH
     assert q(_lib.LO_FORM_W4, force, _lib.LO_BF16, 0, 1, dsv3)[0][1] == _lib.LO_KERNEL_WS
     assert q(_lib.LO_FORM_BLOCK, pre | force, _lib.LO_BF16, 0, 64, dsv3)[0][1] == _lib.LO_KERNEL_DEC
+    # K-group int4: sixteen slots, twelve where an expert is large and the staged path has its fused first stage
+    large, twelve = (128, 128, 8, 4096, 1536), (128, 128, 4, 4096, 1536)
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, qwen)[0][1] == _lib.LO_KERNEL_DEC
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, (128, 128, 8, 4096, 768))[0][1] == _lib.LO_KERNEL_DEC
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, large)[0][1] == _lib.LO_KERNEL_WS
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 3, twelve)[0][1] == _lib.LO_KERNEL_DEC
+    assert q(_lib.LO_FORM_W4, 0, _lib.LO_F16, 0, 2, large)[0][1] == _lib.LO_KERNEL_DEC
+    assert q(_lib.LO_FORM_W4, _lib.LO_FUSED_ACT_GELU, _lib.LO_BF16, 0, 2, large)[0][1] == _lib.LO_KERNEL_DEC
     # the plain first GEMM that GELU and fp16 rows have with the weight-streaming kernel has the plain workgroup shape (four waves), not the
     # fused one (eight)
     q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F16, 0, 16, dsv3)
