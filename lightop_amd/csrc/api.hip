@@ -102,7 +102,7 @@ static bool blocks_of_160_fit(int64_t H, int64_t I, bool fused) {
 // thresholds below were measured on one layer of each class with `python -m lightop_amd.tune`.
 static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64_t H, int64_t I,
                             int form = LO_FORM_BLOCK, bool preshuffled = true, bool int4_channel = false,
-                            bool allow160 = false) {
+                            bool allow160 = false, bool copied_rows = false) {
   const double per_expert = static_cast<double>(M) * top_k / (num_experts > 0 ? num_experts : 1);
   // Packed int4 weights with per-channel scales: the 128-token kernel has no scale arithmetic in
   // its K loop and skips the padded part of a block, so it takes over as soon as an expert sees more
@@ -210,11 +210,23 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
     if (allow160 && per_expert >= 72.0 && per_expert < (H >= 4096 ? 140.0 : 152.0)) return 160;
     return (H >= 4096 || per_expert >= 48.0) ? 128 : 64;
   }
+  // Row-major block-form weights, copied into LDS at every block size: 64-token tiles run three workgroups to a compute
+  // unit, 128-token ones halve the passes over an expert's weights, except where its tokens spill a few rows into a second
+  // block of 128.  Whole path, us, 16 / 32 / 64: Qwen3-30B-A3B layer at 128 tokens (8 slots per expert) 115 / 118 / 118, at 160:
+  // 128 / 118 / 119, at 320: - / 126 / 127, at 384: - / 141 / 130; DeepSeek-V3 share at 256 231 / 235 / 237, at 320: 295 / 238 /
+  // 239; Qwen3-235B-A22B-shaped layer at 384 - / 494 / 473.  64 / 128 in the same layers' order, at 48 slots per expert 155 /
+  // 158, 280 / 290, 547 / 539, at 60: 175 / 171, 384 / 319, 600 / 569, at 90: 195 / 194, 416 / 356, 651 / 607, at 104: 220 / 216,
+  // 455 / 441, 686 / 670 (64 experts of 2048 x 1408: 187 / 197), at 128: 239 / 246, 501 / 537, 801 / 775, at 150: 262 / 275,
+  // 560 / 579, 899 / 898, at 176: 290 / 286, 615 / 572, 965 / 931, at 512: 668 / 647, 1564 / 1394, 2263 / 2115.
+  if (copied_rows) {
+    if (per_expert <= 9.0) return 16;
+    if (per_expert <= 20.0) return 32;
+    return per_expert < 58.0 || (per_expert >= 96.0 && per_expert < 176.0) ? 64 : 128;
+  }
+  // The weight-streaming kernel whatever the layout: fp32 rows, or LO_GEMM_FORCE_STREAMING with row-major weights (and the
+  // register-fed tiles, for row-major rows too long for the LDS tables)
   if (per_expert <= 12.0) return 16;
-  if (per_expert <= 24.0) return 32;
-  // Row-major block-form weights: 64-token tiles, three workgroups per CU (64 / 128, us: Qwen3-235B-A22B-shaped layer at
-  // 1000 tokens 575 / 576, at 4096: 1161 / 1163; DeepSeek-V3 share at 4096: 505 / 516; Qwen3-30B-A3B at 8192: 653 / 639).
-  return 64;
+  return per_expert <= 24.0 ? 32 : 64;
 }
 
 // What a whole-path call does with a problem: the token-block size and which launches follow.  One function per entry
@@ -237,7 +249,8 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false);
   if (block_size_m == 0)
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false,
-                                !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true));
+                                !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true),
+                                !pre && !(flags & LO_GEMM_FORCE_STREAMING) && H / kGroup <= 128 && I / kGroup <= 128);
   // 160: the 160-token form of the direct-to-LDS kernel (int8 block form, load-time layout) for both GEMMs; bf16
   // rows with SiLU take its fused first stage, fp16 rows and GELU the plain one and the activation launch
   const bool silu_bf16 = dtype == LO_BF16 && !gelu;
@@ -640,9 +653,13 @@ extern "C" int lo_fused_experts_block_int8_noalloc(
   PathPlan plan;
   const int rc_plan = plan_block_path(dtype, flags, M, num_experts, top_k, H, I, block_size_m, &plan);
   if (rc_plan) return rc_plan;
-  const int32_t block_size_m_arg = block_size_m;
-  block_size_m = plan.block_size_m;
-  const int64_t need = ws_layout(M, top_k, H, I, num_experts, block_size_m).total;
+  int32_t block_size_m_arg = block_size_m;
+  int64_t need = ws_layout(M, top_k, H, I, num_experts, plan.block_size_m).total;
+  // row-major weights, the table's pick of 128 and a scratch that 64-token blocks, which pad less, still fit
+  if (need > kScratchBytes && block_size_m == 0 && plan.block_size_m == 128 && !(plan.flags & LO_GEMM_W_PRESHUFFLED)) {
+    block_size_m_arg = 64;
+    need = ws_layout(M, top_k, H, I, num_experts, 64).total;
+  }
   LO_REQUIRE(need <= kScratchBytes, LO_ENOSPC,
              "fused_experts(noalloc): this problem needs %lld bytes of scratch, the built-in scratch holds %lld; "
              "use lo_fused_experts_block_int8 with a caller workspace",

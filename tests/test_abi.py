@@ -137,10 +137,14 @@ def test_tile_query_names_the_kernel_that_is_launched(lib):
     assert t2.kernel == _lib.LO_KERNEL_AS
     assert q(_lib.LO_FORM_BLOCK, pre, 4096, *dsv3) == 0
     assert t1.kernel == _lib.LO_KERNEL_T128 and t2.kernel == _lib.LO_KERNEL_T128  # K = 2048: too long to stay in LDS
-    # row-major weights: 64-token register-fed tiles, and a different block size than the load-time layout
-    assert q(_lib.LO_FORM_BLOCK, 0, 8192, *qwen) == 0
+    # row-major weights: lines of their own
+    assert q(_lib.LO_FORM_BLOCK, 0, 2048, *qwen) == 0
     assert (t1.block_size_m, t1.kernel, t1.waves) == (64, _lib.LO_KERNEL_TILE, 4)
     assert q(_lib.LO_FORM_BLOCK, 0, 256, *qwen) == 0 and t1.block_size_m == 32 and t1.kernel == _lib.LO_KERNEL_WS
+    for M, want in ((144, 16), (145, 32), (320, 32), (336, 64), (912, 64), (928, 128), (1520, 128), (1536, 64), (2800, 64),
+                    (2816, 128), (8192, 128)):
+        assert q(_lib.LO_FORM_BLOCK, 0, M, *qwen) == 0 and t1.block_size_m == want == t2.block_size_m, M
+    assert (t1.kernel, t1.waves, t1.block_n) == (_lib.LO_KERNEL_T128, 4, 256)
     assert q(_lib.LO_FORM_BLOCK, pre, 256, *qwen) == 0 and (t1.block_size_m, t1.kernel) == (64, _lib.LO_KERNEL_TILE)
     assert q(_lib.LO_FORM_BLOCK, pre, 256, *dsv3) == 0 and (t1.block_size_m, t1.kernel) == (128, _lib.LO_KERNEL_T128)
     # forced streaming is honoured
@@ -276,11 +280,12 @@ def test_tile_query_path_follows_element_type_activation_and_block_size(lib):
     assert q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F16, 0, 2048, qwen)[0][0] == 64
     assert q(_lib.LO_FORM_BLOCK, pre | _lib.LO_FUSED_ACT_GELU, _lib.LO_BF16, 0, 2048, qwen)[0][0] == 64
     assert q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F16, 160, 2048, qwen)[0] == (160, _lib.LO_KERNEL_T128)  # on request
-    # fp32 rows: the row-major table and the weight-streaming kernel at every size, whatever the layout
-    for M in (1, 512, 8192):
+    # fp32 rows: the weight-streaming kernel at every size, whatever the layout, and the lines that kernel has when it is
+    # forced on row-major weights
+    for M, want in ((1, 16), (192, 16), (200, 32), (384, 32), (512, 64), (8192, 64)):
         a, b = q(_lib.LO_FORM_BLOCK, pre, _lib.LO_F32, 0, M, qwen)
-        assert a[1] == _lib.LO_KERNEL_WS == b[1]
-        assert a[0] == q(_lib.LO_FORM_BLOCK, 0, _lib.LO_BF16, 0, M, qwen)[0][0]
+        assert a == (want, _lib.LO_KERNEL_WS) == b
+        assert a == q(_lib.LO_FORM_BLOCK, _lib.LO_GEMM_FORCE_STREAMING, _lib.LO_BF16, 0, M, qwen)[0]
     assert lib.lo_moe_tile_query_path(_lib.LO_FORM_BLOCK, pre, _lib.LO_F32, 160, 2048, *qwen, t1, t2) < 0  # refused, as the call does
     # a caller's block size (for instance from a tuning file) is described as it would be launched, and
     # switches the two-launch path off, as it does in the call

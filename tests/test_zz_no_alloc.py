@@ -89,3 +89,23 @@ def test_noalloc_entry_point_refuses_what_does_not_fit(dev):
                                                  _p(None), 0, ctypes.c_float(1.0), _p(None), p, p, 128, 0,
                                                  ctypes.c_void_p(0))
     assert rc == -2 and b"built-in scratch holds" in lib.lo_last_error()
+
+
+def test_noalloc_row_major_weights_at_the_scratch_limit(dev):
+    """A problem that 64-token blocks fit into the built-in scratch and the 128-token ones of the table's pick do not: still
+    served, with the former; one that neither fits is refused."""
+    from lightop_amd import _lib, workloads as wl
+
+    lib = _lib.lib()
+    layer = wl.MoeLayer("many-experts", E=512, E_global=512, top_k=8, H=256, I=128, routing="softmax")
+    shape = (layer.top_k, layer.H, layer.I, layer.E)
+    fits = lambda M, bs: lib.lo_fused_experts_workspace_bytes(M, *shape, bs) - 256 <= _lib.LO_NOALLOC_SCRATCH_BYTES  # noqa: E731
+    M = max(m for m in range(15000, 30000) if fits(m, 64))
+    assert not fits(M, 128) and fits(M - 400, 128)
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=0, device=dev, gen_device="cuda")
+    for m in (M, M - 400):
+        say(f"noalloc row-major M={m}")
+        a, b = call_both(dev, layer, m, 3, (w1, w2, w1s, w2s), 0, 0)
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    with pytest.raises(RuntimeError, match="built-in scratch holds"):
+        call_both(dev, layer, M + 1, 3, (w1, w2, w1s, w2s), 0, 0)
