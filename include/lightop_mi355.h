@@ -28,9 +28,10 @@ enum {
   LO_ENOTSUP = -4   /* valid request that this build has no kernel for */
 };
 
-/* activation element types.  fp16 rows go the same way as bf16 ones except that no kernel fuses the gated
- * activation for them: the first GEMM writes [S, 2I] in fp16 and one launch applies the activation and
- * quantises (as with LO_FUSED_ACT_GELU), and the two-launch path is not taken.  LO_F32 (besides router
+/* activation element types.  fp16 rows go the same way as bf16 ones except that their gated activation is
+ * looked up (as with LO_FUSED_ACT_GELU) and that the first GEMM ends with it in fewer cases: in the default
+ * scale order, with block sizes of 64 and 128 (16 to 128 with row-major weights); otherwise it writes [S, 2I]
+ * in fp16 and one launch applies the activation and quantises.  LO_F32 (besides router
  * inputs): the block form with int8 weights and its stages (lo_per_token_group_quant_int8,
  * lo_moe_gemm_block_int8, lo_silu_and_mul, lo_gelu_and_mul, lo_act_mul_group_quant, lo_moe_sum); nothing
  * between the stages is rounded to 16 bits then (compute_type tl.float32, int8.py:689-696), and the GEMMs
@@ -76,16 +77,16 @@ enum {
    * the high nibble, :341, :375-377) is the one lo_preshuffle_weight_int4 reads.  Served by
    * an LDS-tiled kernel at block_size_m 64 and by the weight-streaming kernels otherwise. */
   LO_GEMM_W4 = 32,
-  /* whole-path calls only.  With block_size_m = 0 and weights in the load-time layout the block
-   * form serves small batches (few routed slots per expert) with a two-launch path that needs no
+  /* whole-path calls only.  With block_size_m = 0 and weights in the load-time layout small batches (few
+   * routed slots per expert) of 16-bit rows are served, in every form, with a two-launch path that needs no
    * alignment, no quantised copy of x and no per-slot output rows; same results bit for bit.
    * NO_DECODE_PATH: never take it.  FORCE_DECODE_PATH: take it whenever it can serve the problem
-   * (at most 512 routed slots), whatever the size heuristic says. */
+   * (at most 512 routed slots, its LDS), whatever the size heuristic says. */
   LO_FUSED_NO_DECODE_PATH = 64,
   LO_FUSED_FORCE_DECODE_PATH = 128,
   /* whole-path calls only: activation="gelu" (int8.py:825-838, w4a8.py:602-605) instead of SiLU.
-   * No fused epilogue exists for it: the first GEMM writes bf16 [S, 2I], one launch applies
-   * GELU-and-mul and quantises, so cache3 / cache13 must hold S * max(2I, H) elements. */
+   * The activation is looked up, in the first GEMM's epilogue where fp16 rows have one too (above), else by
+   * a launch of its own on the first GEMM's [S, 2I], so cache3 / cache13 must hold S * max(2I, H) elements. */
   LO_FUSED_ACT_GELU = 256
 };
 
@@ -306,9 +307,9 @@ int lo_preshuffle_weight_int8(const int8_t *src, int8_t *dst, int32_t E, int64_t
  * configs/w8a8/MOE_BLOCKINT8[128,128]_*.json.
  */
 typedef struct lo_moe_tile {
-  int32_t block_size_m; /* 16, 32, 64, 128 or 160 (160: int8 weights in the load-time layout; bf16 rows with
-                         * SiLU keep the fused first stage, fp16 rows and GELU take the plain stage
-                         * followed by lo_act_mul_group_quant, as they do with every block size) */
+  int32_t block_size_m; /* 16, 32, 64, 128 or 160 (160: int8 weights in the load-time layout; in the block form
+                         * bf16 rows with SiLU keep the fused first stage, fp16 rows and GELU take the plain
+                         * stage followed by lo_act_mul_group_quant) */
   int32_t kernel;       /* LO_KERNEL_*: the kernel the stage entry points launch for this problem */
   int32_t waves;        /* wavefronts per workgroup of that kernel */
   int32_t block_n;      /* weight rows per workgroup of that kernel */
@@ -326,7 +327,7 @@ enum {
   LO_KERNEL_W4_TILE = 5, /* packed-int4 LDS-tiled, 64 tokens */
   LO_KERNEL_DEC = 6      /* the whole-path call's two-launch path for a few tokens (weights in the load-time
                           * layout, block_size_m = 0): 16 weight rows per workgroup, the waves of the first
-                          * kernel split K, those of the second take one routed slot each.  The stage entry
+                          * kernel split K, those of the second share out a token's slots.  The stage entry
                           * points have no such kernel: given the reported block_size_m they launch
                           * LO_KERNEL_WS. */
 };
@@ -350,7 +351,8 @@ int lo_moe_tile_query_form(int form, int flags, int64_t M, int32_t E_local, int3
  * vllm_compat/w8a8_get_cache_json.py:133-174).  flags may carry LO_FUSED_ACT_GELU and the decode-path
  * flags as well.  The whole-path calls resolve block size, fused / plain first stage and the two-launch
  * path through the very function this query reports from.  lo_moe_tile_query_form is this call with
- * LO_BF16 and block_size_m = 0. */
+ * LO_BF16 and block_size_m = 0.  The per-channel call with rows the caller has quantised
+ * (lo_fused_experts_channel_int8_prequant) never takes the two-launch path. */
 int lo_moe_tile_query_path(int form, int flags, int dtype, int32_t block_size_m, int64_t M, int32_t E_local,
                            int32_t num_experts, int32_t top_k, int64_t H, int64_t I, lo_moe_tile *gemm1,
                            lo_moe_tile *gemm2);
@@ -380,7 +382,7 @@ int lo_measure_mfma_issue_rate(int valu_per_mfma, int random_operands, int iters
  *   w1s [E, 2I/128, H/128], w2s [E, H/128, I/128]
  *   topk_w [M, top_k] f32;  topk_ids [M, top_k] int32/int64;  expert_map [num_experts] or NULL
  *   cache3 [M*top_k, H] act dtype: the caller's cache13 workspace (second GEMM's output); with fp16
- *   rows or LO_FUSED_ACT_GELU it also receives the first GEMM's output: [M*top_k, max(2I, H)]
+ *   rows or LO_FUSED_ACT_GELU it may also receive the first GEMM's output: [M*top_k, max(2I, H)]
  *   shared_output [M, H] or NULL;  out [M, H]
  *   workspace: lo_fused_experts_workspace_bytes(...) bytes of device memory, 256-byte aligned
  *   block_size_m: 0 = take it from the tile table (lo_fused_experts_workspace_bytes(.., 0) is

@@ -85,7 +85,7 @@ static WsLayout ws_layout(int64_t M, int32_t top_k, int64_t H, int64_t I, int32_
   return L;
 }
 
-// 160-token blocks: both K extents have to fit the kernel's scale table (128 K blocks); where the first GEMM
+// 160-token blocks: both K extents have to fit the kernel's scale table (128 K blocks); where the first GEMM of this size
 // is not fused with the activation (fp16 rows, GELU) its 16-bit output [S, 2I] has to fit the caller's [S, H]
 // buffer as well.
 static bool blocks_of_160_fit(int64_t H, int64_t I, bool fused) {
@@ -223,8 +223,8 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
     if (per_expert <= 20.0) return 32;
     return per_expert < 58.0 || (per_expert >= 96.0 && per_expert < 176.0) ? 64 : 128;
   }
-  // The weight-streaming kernel whatever the layout: fp32 rows, or LO_GEMM_FORCE_STREAMING with row-major weights (and the
-  // register-fed tiles, for row-major rows too long for the LDS tables)
+  // The weight-streaming kernel at every size: fp32 rows; row-major weights with LO_GEMM_FORCE_STREAMING, or with rows too
+  // long for the scale table in LDS
   if (per_expert <= 12.0) return 16;
   return per_expert <= 24.0 ? 32 : 64;
 }

@@ -163,7 +163,7 @@ __device__ __forceinline__ void round_pair_bf16(float a, float b, float &ra, flo
 //
 // 14 vector instructions per value, two of them transcendental, against about 36 for a table in LDS with its selects for
 // the closed forms outside of it (gather, index arithmetic and conversions one by one): whole Qwen3-30B-A3B layer at 8192
-// tokens 626 -> 607 us, at 2400: 264 -> 257, DeepSeek-V3 share at 4096: 558 -> 549.
+// tokens 626 -> 607 us, at 2400: 264 -> 257; around 1 % on the DeepSeek-V3 share at 4096, within what two runs differ by.
 constexpr float kSiluHwMin = -87.25f;
 template <int N>
 __device__ __forceinline__ void silu_mul_bf16(const float (&g)[N], const float (&u)[N], float (&act)[N]) {

@@ -359,10 +359,8 @@ __global__ __launch_bounds__(kSumThreads) void moe_sum_kernel(const uint16_t *__
 }
 
 // ---- SiLU table ------------------------------------------------------------------
-// bf16(silu(g)) for every bf16 pattern g (128 KB, stays in L2).  The GEMM epilogues look
-// the activation up instead of spending ~45 vector instructions per element on
-// exp / divide / round; the entries are produced by exactly those instructions, once
-// per device.
+// bf16(silu(g)) for every bf16 pattern g (128 KB, stays in L2), for lo_act_mul_group_quant; the GEMM epilogues and the
+// other launches compute it.  The entries are produced by exp / divide / round, once per device.
 __device__ uint16_t g_silu_bf16_table[65536];
 
 __global__ __launch_bounds__(256) void silu_table_init_kernel(uint16_t *table) {
@@ -443,7 +441,7 @@ int act_table(hipStream_t stream, int act, int dtype, const uint16_t **out) {
   return LO_OK;
 }
 
-// The launch between the GEMMs where no fused epilogue exists (GELU; fp16 activations): the gated
+// The launch between the GEMMs where the first one's epilogue does not end with the activation: the gated
 // activation from its table and the quantisation of the form in one pass over c1 [rows, 2I].
 int launch_act_mul_group_quant(const void *c1, int dtype, int act, int64_t rows, int64_t I, int8_t *q, float *s,
                                const uint8_t *row_mask, hipStream_t stream) {

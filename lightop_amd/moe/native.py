@@ -401,12 +401,12 @@ def fused_experts_impl_int8(hidden_states: torch.Tensor,
     Same signature as the reference (int8.py:628-656).  This build implements the branches
     ``use_int8_w8a8=True, block_shape=[128, 128]`` and ``use_int8_w8a8=True,
     per_channel_quant=True, block_shape=None`` (one scale per token and per weight row,
-    ``w1_scale`` [E, 2I, 1], ``w2_scale`` [E, H, 1]) with ``activation="silu"`` or ``"gelu"`` (the
-    latter without the fused epilogue: one more launch and a bf16 round trip of [S, 2I]); every other
-    combination raises.  ``hidden_states`` is bfloat16, float16 or, in the block form, float32 (float16 and
-    float32 rows take the path without the fused epilogue as well; every value between the stages is rounded
-    to float16, or not at all, as the reference's compute_type does, int8.py:689-696; float32 rows go
-    through the weight-streaming kernel at every size); float32 with per-channel scales raises.
+    ``w1_scale`` [E, 2I, 1], ``w2_scale`` [E, H, 1]) with ``activation="silu"`` or ``"gelu"``; every other
+    combination raises.  ``hidden_states`` is bfloat16, float16 or, in the block form, float32 (every value between
+    the stages is rounded to float16, or not at all, as the reference's compute_type does, int8.py:689-696; float32
+    rows go through the weight-streaming kernel at every size, with a launch for the activation between the GEMMs);
+    float32 with per-channel scales raises.  GELU, and SiLU of float16 rows, are looked up: in the first GEMM's
+    epilogue with 64- and 128-token blocks, else in a launch of their own and a round trip of [S, 2I].
     ``cache13`` is the caller's workspace (dtype of ``hidden_states``,
     at least ``min(M, CHUNK) * topk * max(2I, H)`` elements); its first ``M*topk*H``
     elements receive the second GEMM's per-slot output.  The top-k reduction is always

@@ -356,8 +356,8 @@ def test_gemm1_silu_quant_bit_exact(dev, oracle, M, k, E, Eg, I, K, bs, order):
 
 @pytest.mark.parametrize("bs", [16, 64, 128])
 def test_gemm1_epilogue_every_finite_bf16_gate(dev, oracle, bs):
-    """Every bf16 value below 1e18 in magnitude as the gate of the fused epilogue (SiLU table, its LDS band and the
-    closed forms outside the band): token t's group scale is the t-th bf16 pattern and the single
+    """Every bf16 value below 1e18 in magnitude as the gate of the fused epilogue (SiLU computed, and its long way for gates
+    whose reciprocal is denormal): token t's group scale is the t-th bf16 pattern and the single
     non-zero product of its row is 1, so gate = up = that value."""
     from lightop_amd.moe import invoke_fused_moe_gemm1_silu_quant, moe_align_block_size
 

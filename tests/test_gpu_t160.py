@@ -125,8 +125,7 @@ def test_160_token_blocks_need_the_load_time_layout(dev):
                          [(c, k) for k in (128, 256, 1024) for c in (40, 136, 160)])
 def test_gemm1_fused_160_token_blocks_fill_levels(dev, oracle, count, K):
     """The first stage with its fused epilogue on blocks of 160 holding 1 ... 160 valid tokens, in both bit-exact
-    scale orders, with and without the router weight: int8 activations and group scales against the oracle.
-    (The SiLU band and the amax exchange of this form live in the waves' weight stages after the K loop.)"""
+    scale orders, with and without the router weight: int8 activations and group scales against the oracle."""
     from lightop_amd import _lib
     from lightop_amd.moe import invoke_fused_moe_gemm1_silu_quant, moe_align_block_size, preshuffle_moe_weight
 
@@ -174,7 +173,7 @@ def test_gemm1_fused_160_bit_exact_with_expert_map(dev, oracle, M, k, E, Eg, I, 
 
 def test_gemm1_fused_160_every_finite_bf16_gate_and_special_gates(dev, oracle):
     """Every bf16 value below 1e18 in magnitude as the gate of the 160-token form's fused epilogue, then rows with
-    NaN and infinite gates next to ordinary rows (they leave the fast lookup by a wave-wide vote)."""
+    NaN and infinite gates next to ordinary rows (some of which take a wave the long way)."""
     from lightop_amd.moe import invoke_fused_moe_gemm1_silu_quant, moe_align_block_size, preshuffle_moe_weight
 
     say("fused first stage bs=160 over all bf16 gates")
