@@ -635,10 +635,14 @@ def _scratch(nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
 
 
 def _in_graph_pool(t: torch.Tensor) -> bool:
-    """Whether the allocator took ``t`` from a private pool, as it does under ``torch.cuda.graph``."""
-    for seg in torch.cuda.memory_snapshot():
-        if seg["device"] == t.device.index and seg["address"] <= t.data_ptr() < seg["address"] + seg["total_size"]:
-            return tuple(seg["segment_pool_id"]) != (0, 0)
+    """Whether the allocator took ``t`` from a private pool, as it does under ``torch.cuda.graph``.  False where it cannot
+    say: what is kept without need costs memory, what is not kept would be written to by replays."""
+    try:
+        for seg in torch.cuda.memory_snapshot():
+            if seg["device"] == t.device.index and seg["address"] <= t.data_ptr() < seg["address"] + seg["total_size"]:
+                return tuple(seg["segment_pool_id"]) != (0, 0)
+    except (RuntimeError, KeyError):  # another allocator behind torch's, another layout of its snapshot
+        pass
     return False
 
 

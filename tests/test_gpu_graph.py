@@ -84,7 +84,7 @@ class HipGraph:
         self.check(self.hip.hipGraphLaunch(self.exec, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
 
 
-@pytest.mark.parametrize("capture", ["torch", "runtime"])
+@pytest.mark.parametrize("capture", ["torch", "torch without snapshots", "runtime"])
 def test_replays_write_to_no_memory_of_others(capture, monkeypatch):
     """A graph's scratch stays the graph's: after a warm-up and a capture on one stream, larger calls there and calls on
     more streams than workspaces are kept for, the memory that stream then gets from the allocator survives replays."""
@@ -109,14 +109,19 @@ def test_replays_write_to_no_memory_of_others(capture, monkeypatch):
     with torch.cuda.stream(side):
         eager = run().clone()
     torch.cuda.synchronize()
-    if capture == "torch":
+    if capture == "torch without snapshots":
+        def refuse():
+            raise RuntimeError("snapshots are not supported")
+
+        monkeypatch.setattr(torch.cuda, "memory_snapshot", refuse)
+    if capture != "runtime":
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, stream=side):
             out = run()
     else:
         g = HipGraph(side, run)
         out = g.out
-    assert list(native._capture_kept) == ([(0, side.cuda_stream)] if capture == "runtime" else [])  # torch's graphs own theirs
+    assert list(native._capture_kept) == ([] if capture == "torch" else [(0, side.cuda_stream)])  # torch's graphs own theirs
     torch.cuda.synchronize()
     for stream in [torch.cuda.Stream() for _ in range(20)] + [side]:
         with torch.cuda.stream(stream):
