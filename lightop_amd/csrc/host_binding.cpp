@@ -70,15 +70,24 @@ int64_t chunk_size() {
   return 16 * 1024;
 }
 
+// Blocking work (allocations, which may wait for the GPU when memory is short; launches, which wait while the stream's queue
+// is full and, for the first call of an activation, for its table) is done without the interpreter lock, as torch and ctypes
+// do it: Python threads, or a callback on the stream, may have to run until it is through.  What it needs of the tensors is
+// taken from them before.
+struct NoGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // ---- workspaces ----------------------------------------------------------------------------------------
 // The library's scratch for a whole-path call, one per (device, stream) and grown on demand, so that a serving loop
 // does not allocate on every call.  Calls on one stream run in order and can share it; calls on different streams get
 // workspaces of their own, and of several threads on one stream only one queues its launches at a time, so that
-// a workspace holds one call's intermediates from the first launch to the last.  At most kMaxWorkspaces are kept: beyond that the one that was used longest ago goes back to the
-// caching allocator (it was allocated on its own stream, so its memory is reused in that stream's order), as does one that
-// a larger call outgrows.  A graph would keep the address of such memory, so none of it is ever captured: calls on a stream
-// that is being captured are declined, and get scratch that lives as long as the graph.  The table is touched under the interpreter lock only; a call holds a
-// reference to its workspace while it is without that lock.
+// a workspace holds one call's intermediates from the first launch to the last.  At most kMaxWorkspaces are kept: beyond
+// that the one that was used longest ago goes back to the caching allocator (it was allocated on its own stream, so its
+// memory is reused in that stream's order), as does one that a larger call outgrows.  A graph would keep the address of
+// such memory, so none of it is ever captured: calls on a stream that is being captured are declined, and get scratch that
+// lives as long as the graph.  The locks are taken without the interpreter lock, whose holder may be waiting for them.
 struct Scratch {
   at::Tensor buf;
   std::mutex busy; // held while a call's launches are queued
@@ -102,6 +111,8 @@ std::shared_ptr<Scratch> new_workspace(int64_t bytes, int device) {
 }
 
 std::shared_ptr<Scratch> workspace_for(int64_t bytes, int device, hipStream_t stream) {
+  static std::mutex table;
+  const std::lock_guard<std::mutex> lock(table);
   auto &all = workspaces();
   size_t i = 0;
   while (i < all.size() && !(all[i].device == device && all[i].stream == stream)) ++i;
@@ -120,20 +131,6 @@ std::shared_ptr<Scratch> workspace_for(int64_t bytes, int device, hipStream_t st
   }
   for (; i > 0; --i) std::swap(all[i], all[i - 1]);
   return all[0].scratch;
-}
-
-// Calls `entry` without the interpreter lock, as ctypes does: a launch waits while the stream's queue is full, the first
-// call of an activation waits for its table, and Python threads, or a callback on the stream, may have to run until then.
-// The arguments are plain values, taken from the tensors before the lock is let go.
-struct NoGil {
-  PyThreadState *state = PyEval_SaveThread();
-  ~NoGil() { PyEval_RestoreThread(state); }
-};
-template <typename F, typename... A> int launch(std::mutex *busy, F entry, A... args) {
-  const NoGil nogil;
-  std::unique_lock<std::mutex> lock; // taken without the interpreter lock, whose holder may be waiting for it
-  if (busy) lock = std::unique_lock<std::mutex>(*busy);
-  return entry(args...);
 }
 
 PyObject *raise(int rc) {
@@ -235,19 +232,28 @@ PyObject *fused_experts(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (bytes < 0) return raise(static_cast<int>(bytes));
   const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
   if (capturing(stream)) Py_RETURN_NONE;
-  const std::shared_ptr<Scratch> ws = workspace_for(bytes, dev, stream);
-  const uintptr_t base = reinterpret_cast<uintptr_t>(ws->buf.data_ptr());
-  const uintptr_t aligned = (base + 255) / 256 * 256;
-  at::Tensor out = inplace ? x : at::empty(x.sizes(), x.options().requires_grad(false));
-
   const auto entry = channel ? g_channel : g_block;
-  const int rc = launch(&ws->busy, entry, x.data_ptr(), dtype, M, H, I, static_cast<int32_t>(E), static_cast<int32_t>(experts),
-                        static_cast<int32_t>(k), static_cast<const int8_t *>(w1.data_ptr()), s1.data_ptr<float>(),
-                        static_cast<const int8_t *>(w2.data_ptr()), s2.data_ptr<float>(), tw.data_ptr<float>(), ids.data_ptr(),
-                        ids64 ? LO_I64 : LO_I32, t[8] ? t[8]->data_ptr<int32_t>() : nullptr, mul_on_input,
-                        static_cast<float>(factor), t[9] ? t[9]->data_ptr() : nullptr, cache.data_ptr(), out.data_ptr(),
-                        reinterpret_cast<void *>(aligned), ws->buf.numel() - static_cast<int64_t>(aligned - base), 0,
-                        static_cast<int>(flags), stream);
+  const auto sizes = x.sizes().vec();
+  const auto options = x.options().requires_grad(false);
+  const auto call = [=, xp = x.data_ptr(), w1p = static_cast<const int8_t *>(w1.data_ptr()), s1p = s1.data_ptr<float>(),
+                     w2p = static_cast<const int8_t *>(w2.data_ptr()), s2p = s2.data_ptr<float>(), twp = tw.data_ptr<float>(),
+                     idp = ids.data_ptr(), map = t[8] ? t[8]->data_ptr<int32_t>() : nullptr,
+                     shared = t[9] ? t[9]->data_ptr() : nullptr, cp = cache.data_ptr()](void *dst, const at::Tensor &ws) { // dst null: in place
+    const uintptr_t base = reinterpret_cast<uintptr_t>(ws.data_ptr()), aligned = (base + 255) / 256 * 256;
+    return entry(xp, dtype, M, H, I, static_cast<int32_t>(E), static_cast<int32_t>(experts), static_cast<int32_t>(k), w1p, s1p,
+                 w2p, s2p, twp, idp, ids64 ? LO_I64 : LO_I32, map, mul_on_input, static_cast<float>(factor), shared, cp, dst ? dst : xp,
+                 reinterpret_cast<void *>(aligned), ws.numel() - static_cast<int64_t>(aligned - base), 0,
+                 static_cast<int>(flags), stream);
+  };
+  at::Tensor out;
+  int rc;
+  {
+    const NoGil nogil;
+    const std::shared_ptr<Scratch> ws = workspace_for(bytes, dev, stream);
+    if (!inplace) out = at::empty(sizes, options);
+    const std::lock_guard<std::mutex> lock(ws->busy);
+    rc = call(inplace ? nullptr : out.data_ptr(), ws->buf);
+  }
   if (rc < 0) return raise(rc);
   if (inplace) {
     Py_INCREF(args[0]);
@@ -279,9 +285,17 @@ PyObject *topk_softmax(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!i64 && idx->scalar_type() != at::kInt) Py_RETURN_NONE;
   if (src && (src->scalar_type() != at::kInt || src->numel() != T * k)) Py_RETURN_NONE;
   if (E > INT32_MAX || k > INT32_MAX) Py_RETURN_NONE;
-  const int rc = launch(nullptr, g_topk_softmax, g->data_ptr(), dtype, T, static_cast<int32_t>(E), static_cast<int32_t>(k), renorm,
-                        w->data_ptr<float>(), idx->data_ptr(), i64 ? LO_I64 : LO_I32, src ? src->data_ptr<int32_t>() : nullptr,
-                        c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
+  const void *gp = g->data_ptr();
+  float *const wp = w->data_ptr<float>();
+  void *const ip = idx->data_ptr();
+  int32_t *const sp = src ? src->data_ptr<int32_t>() : nullptr;
+  int rc;
+  {
+    const NoGil nogil;
+    rc = g_topk_softmax(gp, dtype, T, static_cast<int32_t>(E), static_cast<int32_t>(k), renorm, wp, ip, i64 ? LO_I64 : LO_I32, sp,
+                        stream);
+  }
   if (rc < 0) return raise(rc);
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -313,14 +327,20 @@ PyObject *fused_gate(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (!plain(*x, dev) || !plain(*b, dev) || x->dim() != 2 || b->dim() != 1 || b->numel() != x->size(1)) Py_RETURN_NONE;
   const int dt = dtype_code(x->scalar_type()), bt = dtype_code(b->scalar_type());
   if (dt < 0 || bt < 0 || x->size(1) > INT32_MAX) Py_RETURN_NONE;
-  const int64_t T = x->size(0), topk = v[2];
+  const int64_t T = x->size(0), E = x->size(1), topk = v[2];
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
+  const void *xp = x->data_ptr(), *bp = b->data_ptr();
   const auto opts = x->options().requires_grad(false);
-  at::Tensor weights = at::empty({T, topk}, opts.dtype(at::kFloat));
-  at::Tensor indices = at::empty({T, topk}, opts.dtype(i64 ? at::kLong : at::kInt));
-  const int rc = launch(nullptr, g_gate, x->data_ptr(), dt, b->data_ptr(), bt, T, static_cast<int32_t>(x->size(1)),
-                        static_cast<int32_t>(v[0]), static_cast<int32_t>(v[1]), static_cast<int32_t>(v[2]), static_cast<int32_t>(v[3]), factor, on_output,
-                        weights.data_ptr<float>(), indices.data_ptr(), i64 ? LO_I64 : LO_I32,
-                        c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
+  at::Tensor weights, indices;
+  int rc;
+  {
+    const NoGil nogil;
+    weights = at::empty({T, topk}, opts.dtype(at::kFloat));
+    indices = at::empty({T, topk}, opts.dtype(i64 ? at::kLong : at::kInt));
+    rc = g_gate(xp, dt, bp, bt, T, static_cast<int32_t>(E), static_cast<int32_t>(v[0]), static_cast<int32_t>(v[1]),
+                static_cast<int32_t>(v[2]), static_cast<int32_t>(v[3]), factor, on_output, weights.data_ptr<float>(),
+                indices.data_ptr(), i64 ? LO_I64 : LO_I32, stream);
+  }
   if (rc < 0) return raise(rc);
   PyObject *pw = THPVariable_Wrap(std::move(weights)), *pi = THPVariable_Wrap(std::move(indices));
   PyObject *pair = PyList_New(2);

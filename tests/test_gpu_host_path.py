@@ -207,6 +207,74 @@ def test_other_threads_run_during_a_launch(entry, tmp_path):
         thread.join()
 
 
+ALLOCATOR = """
+#include <stddef.h>
+#include <sys/types.h>
+#include <unistd.h>
+int (*real_malloc)(void **, size_t);
+int (*real_free)(void *);
+volatile int entered, let_go, waited_in_vain;
+void *take(ssize_t bytes, int device, void *stream) {
+  void *p = NULL;
+  entered = 1;
+  for (int i = 0; i < 5000 && !let_go; ++i) usleep(1000);
+  waited_in_vain |= !let_go;
+  return real_malloc(&p, (size_t)bytes) ? NULL : p;
+}
+void give(void *p, ssize_t bytes, int device, void *stream) { real_free(p); }
+"""
+
+
+@pytest.mark.parametrize("entry", ["block", "fused_gate"])
+def test_other_threads_run_during_an_allocation(entry, tmp_path):
+    """Short of memory an allocation waits for the GPU, and what that waits for may need the interpreter: outputs come from
+    an allocator that returns when another Python thread has run, or after five seconds."""
+    from lightop_amd import _lib, workloads as wl
+
+    dev = torch.device("cuda:0")
+    print(f"[case] threads during an allocation {entry}", flush=True)
+    (tmp_path / "stub.c").write_text(ALLOCATOR)
+    path = str(tmp_path / "stub.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", path, str(tmp_path / "stub.c")], check=True)
+    stub, host, hip = ctypes.CDLL(path), _lib.host(), _lib.lib()
+    for name, fn in (("real_malloc", hip.hipMalloc), ("real_free", hip.hipFree)):
+        ctypes.c_void_p.in_dll(stub, name).value = ctypes.cast(fn, ctypes.c_void_p).value
+    entered, let_go, in_vain = (ctypes.c_int.in_dll(stub, n) for n in ("entered", "let_go", "waited_in_vain"))
+    layer, weights, kw = _layer("block", dev)
+    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, 4, seed=3))
+    cache13 = torch.empty(4 * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
+    g, bias = torch.randn(4, 64, device=dev), torch.zeros(64, device=dev)
+
+    def call():
+        if entry == "fused_gate":
+            return host.fused_gate(g, bias, 8, 4, 6, 0, 2.5, False, False)[0]
+        return host.fused_experts(x, *weights, tw, ids, cache13, kw["w1_scale"], kw["w2_scale"], None, None, 0, False, False, -1,
+                                  1.0, 0)
+
+    def other():
+        for _ in range(20000):
+            if entered.value:
+                let_go.value = 1
+                return
+            time.sleep(0.0005)
+
+    want = call()  # (the workspace is there from now on)
+    allocator = torch.cuda.memory.CUDAPluggableAllocator(path, "take", "give")
+    pool = torch.cuda.MemPool(allocator.allocator())
+    thread = threading.Thread(target=other)
+    thread.start()
+    try:
+        with torch.cuda.use_mem_pool(pool):
+            got = call()
+    finally:
+        entered.value = 1
+        thread.join()
+    torch.cuda.synchronize()
+    same = torch.equal(got, want)
+    del got, pool  # the pool gives its memory back through the allocator, which it does not keep alive
+    assert same and not in_vain.value
+
+
 @pytest.mark.parametrize("form", ["block", "channel"])
 def test_threads_share_a_stream(form):
     """Two threads that queue calls of different sizes on one stream: neither's launches come between the other's, whose
