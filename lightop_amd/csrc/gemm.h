@@ -178,6 +178,31 @@ __device__ __forceinline__ float fold_elem(int d, float sc, float as, float bs, 
     return acc + t;
   }
 }
+// The contracted fold without a conversion: two vector instructions per element, and bit for bit the three of fold_elem.
+// The MFMA chain starts from the integer 2^23 instead of 0, so that the K block's sum d leaves it as the integer 2^23 + d.
+// Read as a float, an integer of up to 24 bits is that integer times 2^-149: below 2^23 it is a denormal, from there on a
+// normal number of the first binade, and both have the same spacing.  So with A = a_s * 2^85
+//     fma(m, A, -2^-126 * A)  =  round(((2^23 + d) - 2^23) * a_s * 2^-64)  =  round(d * a_s) * 2^-64,
+// the subtraction being exact inside the fused operation because 2^-126 * A is, and
+//     fma(that, b_s * 2^64, acc)
+// is the second step of the contracted order.  (A bias that is no power of two, as the usual 1.5 * 2^23, has a rounded product
+// with a_s.)  |d| < 2^23 for any K block of int8 operands: 128 * 2^14 = 2^21.  v_fma_f32 takes denormals at full rate.
+// It holds while nothing on the way leaves the normal range: |a_s| zero or in [2^-62, 2^43), |b_s| below 2^64.  The
+// quantisation's scales lie between 2^-41 and the largest 16-bit value / 127, so that only rows of more than 10^15, weight
+// scales of 10^19, or a caller's own scales ever leave it; kernels fold a tile that holds such a scale the long way.
+constexpr int kFoldBias = 0x00800000;
+__device__ __forceinline__ float fold_token_scale(float as) { return as * 0x1p85f; }
+__device__ __forceinline__ float fold_weight_scale(float bs) { return bs * 0x1p64f; }
+__device__ __forceinline__ bool fold_token_scale_ok(float as) {
+  const float v = fabsf(as);
+  return v == 0.0f || (v >= 0x1p-62f && v < 0x1p43f); // (a NaN is refused)
+}
+__device__ __forceinline__ bool fold_weight_scale_ok(float bs) { return fabsf(bs) < 0x1p64f; }
+// m: the biased sum; as, bs: scales that went through the two functions above; as_bias = fold_bias(as).
+__device__ __forceinline__ float fold_bias(float as) { return as * -0x1p-126f; }
+__device__ __forceinline__ float fold_biased(int m, float as, float as_bias, float bs, float acc) {
+  return __builtin_fmaf(__builtin_fmaf(__builtin_bit_cast(float, m), as, as_bias), bs, acc);
+}
 // Three-way dispatch of a launcher macro on the order: LO_ORD_DISPATCH(ord, MACRO, args...) expands to
 // MACRO(order constant, args...).
 #define LO_ORD_DISPATCH(ord, MACRO, ...)                                   \

@@ -42,12 +42,13 @@ constexpr int kTRed = 4 * kT * 4;             // [wave][token] amax exchange of 
 constexpr int kTMaxKB = 128;                  // K blocks whose weight-block scales fit the table below
 constexpr int kTBs = 2 * kTMaxKB * 4;         // [fragment][K block] weight-block scales of the tile
 constexpr int kTIds = kT * 4;                  // the tile's sorted ids, for the epilogues
-constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds;
+constexpr int kTFlag = 16;                    // [wave]: it met a scale that the biased fold does not take
+constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds + kTFlag;
 // NTB = 10: 160 tokens per workgroup (int8 block form, or int4 weights with per-channel scales, whose int32 accumulators need no fold registers), for layers
 // whose experts see a few tokens more than 128: a remainder block is a second pass over the expert's
 // weights, and at that size the weights are what the stage streams.
 constexpr int kT160 = 160;
-constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + kT160 * 4;
+constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + kT160 * 4 + kTFlag;
 constexpr int kTPitch = 144;                  // staging pitch of the epilogues: 128 + 16
 
 // Wait until all but the newest `N` vector-memory operations of this wave are complete and its
@@ -87,11 +88,18 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   float *const sBs = reinterpret_cast<float *>(smem + kTW + 2 * AST + 2 * T * 4 + RED);
   int32_t *const sIds = reinterpret_cast<int32_t *>(smem + kTW + 2 * AST + 2 * T * 4 + RED + kTBs);
 
+  int32_t *const sFlag = sIds + T;
+  // The contracted order folds without a conversion (fold_biased): 2 vector instructions an element and K block instead of 3,
+  // where they were issued in 83 % of a SIMD's cycles.  Layer with its router, us, before / after: full DeepSeek-V3 layer, 8192
+  // tokens 4828 / 4531, Qwen3-30B-A3B layer, 8192: 603.8 / 578.9, DeepSeek-V3 share, 4096: 539 / 525, int4 with K-group scales,
+  // 2048: 629 / 594.  A tile that meets a scale outside of its range is done again with the conversion.
+  constexpr bool kBiased = ORD == kOrdContract && !PC;
+
   int mb, nt;
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of the tile
-  const int r = lane & 15, q = lane >> 4;
+  int r = lane & 15, q = lane >> 4;
   const int32_t *const sorted = a.sorted + static_cast<int64_t>(mb) * T;
   // Everything the tile's start-up reads from memory by its block index alone is requested here, in one go:
   // the number of blocks in use, the block's expert and the sorted ids this thread needs (token rows it
@@ -154,7 +162,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * (PC ? 1 : KB) * 4));
   const int wkstride = ROWS ? kGroup : W4 ? shuf_kb_stride(NBLK) / 2 : shuf_kb_stride(NBLK);
   const int wpstride = ROWS ? static_cast<int>(8 * K) : 1024; // second half of a 16-row block
-  int wvoff[2][2]; // [step half][fragment]: the 2 KB block of 16 rows x 128 K, in lane order
+  int wsoff[2][2]; // [step half][fragment]: the 2 KB block of 16 rows x 128 K (wave-uniform)
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -163,11 +171,12 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if constexpr (FUSED_ACT) nb = (rf ? I / 16 : 0) + static_cast<int64_t>(nt) * 8 + wave * 2 + h;
       else nb = static_cast<int64_t>(nt) * 16 + wave * 4 + h * 2 + rf;
       if (nb >= NBLK) nb = 0; // rows past N: computed on block 0, never stored
-      // row-major: a 1 KB piece is 128 bytes of eight rows, whole lines; slot lane & 7 of row lane >> 3 takes
-      // the row's 16-byte piece slot ^ row (as in the token stage)
-      if constexpr (ROWS) wvoff[h][rf] = static_cast<int>((nb * 16 + (lane >> 3)) * K) + (((lane & 7) ^ (lane >> 3)) * 16);
-      else wvoff[h][rf] = static_cast<int>(nb) * (W4 ? shuf_nb_stride(KB) / 2 : shuf_nb_stride(KB)) + lane * 16;
+      if constexpr (ROWS) wsoff[h][rf] = static_cast<int>(nb * 16 * K);
+      else wsoff[h][rf] = static_cast<int>(nb) * (W4 ? shuf_nb_stride(KB) / 2 : shuf_nb_stride(KB));
     }
+  // the lane's part of it: in lane order, or, row-major, a 1 KB piece is 128 bytes of eight rows, whole lines; slot lane & 7
+  // of row lane >> 3 takes the row's 16-byte piece slot ^ row (as in the token stage)
+  const int wvoff = ROWS ? static_cast<int>((lane >> 3) * K) + (((lane & 7) ^ (lane >> 3)) * 16) : lane * 16;
   // W4: lane l copies the scale of row l of the wave's 64 (fused: 32 gate rows, then the 32 up rows)
   int wsvoff = 0;
   if constexpr (W4) {
@@ -185,25 +194,28 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // The first K block's weights depend on the expert only: they are requested before the token
   // ids are read, so that the two dependent round trips of the tile's start-up overlap.
   int8_t *const sWw = smem + wave * kTWStage; // int8: [row half][fragment][k half] x 1 KB; W4: [row half][fragment] x 1 KB, row scales
-  if constexpr (W4) {
+  auto copy_w0 = [&]() __attribute__((always_inline)) {
+    if constexpr (W4) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[p >> 1][p & 1], 0, 0, kWAux);
-    if constexpr (!PC) __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, sWw + 4096, 4, wsvoff, 0, 0, kWAux);
-  } else {
+      for (int p = 0; p < 4; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff, wsoff[p >> 1][p & 1], 0, kWAux);
+      if constexpr (!PC) __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, sWw + 4096, 4, wsvoff, 0, 0, kWAux);
+    } else {
 #pragma unroll
-    for (int p = 0; p < 8; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[p >> 2][(p >> 1) & 1], (p & 1) * wpstride, 0,
-                                               kWAux);
-  }
+      for (int p = 0; p < 8; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff, wsoff[p >> 2][(p >> 1) & 1] + (p & 1) * wpstride, 0,
+                                                 kWAux);
+    }
+  };
+  copy_w0();
   int avoff[5]; // 1 KB pieces wave*APW + j of a token stage, j < APW: eight token rows each
 #pragma unroll
   for (int j = 0; j < APW; ++j) {
     const int t = (cw * APW + j) * 8 + (lane >> 3);
     const int64_t lf = kEarlyIds ? lf_copy[j] : sorted[t];
-    const int64_t lrow = token_row(a, lf);
     const int piece = (lane & 7) ^ (t & 7); // slot lane & 7 of row t holds piece slot ^ (t & 7)
-    avoff[j] = static_cast<int>(lrow * K) + piece * 16;
+    // (the move leaves one register: an offset that stays the lower half of a 64-bit multiply-add keeps two through the K loop)
+    asm("v_mov_b32 %0, %1" : "=v"(avoff[j]) : "v"(token_row(a, lf) * static_cast<int>(K) + piece * 16));
   }
   // The alignment puts a block's valid tokens first, so a block of 128 is on average half a block
   // of padding per expert: token fragments past the last valid token are skipped (taken from the position of the last valid token, not from their number, so that
@@ -228,8 +240,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
     const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
-    const int64_t lrow = token_row(a, lf);
-    asoff = static_cast<int>(lrow * (PC ? 1 : KB) * 4);
+    asoff = token_row(a, lf) * (PC ? 1 : KB) * 4;
     // The epilogues take the ids from LDS: a global load in each of their exec-masked blocks is a
     // full memory round trip that nothing overlaps.
     if (tid < T) sIds[tid] = static_cast<int32_t>(lf);
@@ -237,13 +248,13 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // weight-block scales of the tile: table row 0 / 1 = gate / up block (fused), or the first / second
   // 128 rows of the tile (plain: waves 0, 1 / waves 2, 3).  Thread t fetches entry (t >> 7, t & 127).
   const int NB = static_cast<int>((N + kGroup - 1) / kGroup);
-  float bs_mine = 0.0f;
-  {
+  auto load_bs = [&]() __attribute__((always_inline)) {
     const int which = tid >> 7, kbi = tid & (kTMaxKB - 1);
     int64_t nblk = FUSED_ACT ? (which ? I / kGroup : 0) + nt : static_cast<int64_t>(nt) * 2 + which;
     if (nblk >= NB) nblk = 0;
-    if (!W4 && !PC && kbi < KB) bs_mine = a.Ws[(static_cast<int64_t>(e) * NB + nblk) * KB + kbi];
-  }
+    return !W4 && !PC && kbi < KB ? a.Ws[(static_cast<int64_t>(e) * NB + nblk) * KB + kbi] : 0.0f;
+  };
+  float bs_mine = load_bs();
   const float *const sBs0 = sBs + (FUSED_ACT ? 0 : (wave >> 1) * kTMaxKB);
   const float *const sBs1 = sBs + (FUSED_ACT ? kTMaxKB : (wave >> 1) * kTMaxKB);
 
@@ -253,15 +264,15 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (p < 8) {
       if constexpr (W4) { // four weight pieces, the row scales, three empty slots
         if (p < 4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[p >> 1][p & 1],
-                                                   __builtin_amdgcn_readfirstlane(kc * wkstride), 0, kWAux);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff,
+                                                   __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[p >> 1][p & 1], 0, kWAux);
         else if (p == 4 && !PC)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, sWw + 4096, 4, wsvoff,
                                                    __builtin_amdgcn_readfirstlane(kc) * static_cast<int>(N) * 4, 0, kWAux);
       } else {
         const int h = p >> 2, rf = (p >> 1) & 1, kh = p & 1;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff[h][rf],
-                                                 __builtin_amdgcn_readfirstlane(kc * wkstride) + kh * wpstride, 0, kWAux);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff,
+                                                 __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[h][rf] + kh * wpstride, 0, kWAux);
       }
     } else if (p - 8 < APW && (NTB > 1 || wave < 2)) {
       const int j = p - 8;
@@ -310,25 +321,32 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // scale, which read_w() multiplies by 1/16 once per K block (a power of two: (f32(d) * a_s) * (b_s / 16)
   // is bit for bit (f32(d / 16) * a_s) * b_s unless b_s lies below 2^-122 or the product above 2^124).
   // One scale per weight row: bs4[i] for row 4q + i.
-  auto fold4 = [&](const v4i &d, float as, const v4f &bs4, float *dst) __attribute__((always_inline)) {
+  auto fold4 = [&](auto BIASED, const v4i &d, float as, float as_bias, const v4f &bs4, float *dst) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) // bs4 already holds scale / 16
-      dst[i] = fold_elem<ORD>(d[i], ORD == kOrdFusedScale ? as * bs4[i] : 0.0f, as, bs4[i], dst[i]);
+      if constexpr (decltype(BIASED)::value) dst[i] = fold_biased(d[i], as, as_bias, bs4[i], dst[i]);
+      else dst[i] = fold_elem<ORD>(d[i], ORD == kOrdFusedScale ? as * bs4[i] : 0.0f, as, bs4[i], dst[i]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(dst[i])); // keep the fold here
   };
-  auto fold = [&](const v4i &d, float sc, float as, float bs, float *dst) __attribute__((always_inline)) {
+  auto fold = [&](auto BIASED, const v4i &d, float sc, float as, float as_bias, float bs, float *dst) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = fold_elem<ORD>(d[i], sc, as, bs, dst[i]);
+    for (int i = 0; i < 4; ++i)
+      if constexpr (decltype(BIASED)::value) dst[i] = fold_biased(d[i], as, as_bias, bs, dst[i]);
+      else dst[i] = fold_elem<ORD>(d[i], sc, as, bs, dst[i]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(dst[i])); // keep the fold here
   };
 
+  auto uniform = [](float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); };
   // One K block: the wave's 64 rows (two halves h of two fragments) against all 128 tokens.
   v4i w[2][2][2]; // the wave's weights of the current K block
   v4f wsc[2][2];  // W4: the scales of the lane's rows 4q .. 4q+3 of each fragment
-  auto read_w = [&]() __attribute__((always_inline)) {
+  float ws_max = 0.0f; // W4: largest |row scale| so far (of row `lane` of the wave's 64)
+  auto read_w = [&](auto BIASED) __attribute__((always_inline)) {
     if constexpr (W4) {
+      if constexpr (decltype(BIASED)::value)
+        ws_max = fmaxf(ws_max, fabsf(*reinterpret_cast<const float *>(sWw + 4096 + lane * 4)));
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -346,7 +364,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
           if constexpr (!PC) {
             const int row0 = (FUSED_ACT ? 32 * rf + 16 * h : 32 * h + 16 * rf) + 4 * q;
             wsc[h][rf] = *reinterpret_cast<const v4f *>(sWw + 4096 + row0 * 4);
-            wsc[h][rf] = wsc[h][rf] * 0.0625f;
+            wsc[h][rf] = wsc[h][rf] * (decltype(BIASED)::value ? fold_weight_scale(0.0625f) : 0.0625f);
           }
         }
     } else {
@@ -368,7 +386,16 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   float s_pending;   // token scales on their way from global memory to sS
   v4i bf_first[2];   // first token fragment of the next K block
   float as_first = 0.0f;
-  auto kblock = [&](auto NST, int kb) __attribute__((always_inline)) {
+  auto put_scale = [&](auto BIASED, int stage, float s) __attribute__((always_inline)) {
+    if (tid < T) {
+      if constexpr (decltype(BIASED)::value) {
+        if (__builtin_amdgcn_ballot_w64(!fold_token_scale_ok(s))) sFlag[wave] = 1;
+        s = fold_token_scale(s);
+      }
+      sS[stage * T + tid] = s;
+    }
+  };
+  auto kblock = [&](auto BIASED, auto NST, int kb) __attribute__((always_inline)) {
     constexpr int nst_c = decltype(NST)::value; // stages of this variant: 4, 8, 12, 16 (or 20)
     constexpr int kFull = 2 * NTB;              // stages of a full tile
     constexpr int kE0 = nst_c - 2, kE1 = nst_c - 1;
@@ -388,29 +415,32 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       for (int kh = 0; kh < 2; ++kh) bf[0][kh] = *reinterpret_cast<const v4i *>(ta + alds[kh]);
       as_t[0] = ts[r];
     }
-    const float bs0 = W4 ? 0.0f : sBs0[kb], bs1 = W4 ? 0.0f : sBs1[kb];
+    const float bs0 = W4 ? 0.0f : uniform(sBs0[kb]), bs1 = W4 ? 0.0f : uniform(sBs1[kb]);
 
     // The weight stage was read into registers before the barrier, so it is free; it and the other
     // token stage are refilled with the next K block, two copies per pipeline stage so that the
     // texture path never sees a burst that this wave (or the other workgroup's) queues behind.
-    const v4i cinit = {0, 0, 0, 0};
+    constexpr int c0 = decltype(BIASED)::value ? kFoldBias : 0;
+    const v4i cinit = {c0, c0, c0, c0};
     v4i dprev[2];
     float as_p = 0.0f;
+    float as_bias = 0.0f;
     float sc0 = 0.0f, sc1 = 0.0f; // scale products of the token fragment being folded (both row halves)
     auto fold_stage = [&](int st) __attribute__((always_inline)) { // fold the fragments of stage st
       const int tb = st >> 1, h = st & 1;
       if constexpr (PC) return;
+      if (decltype(BIASED)::value && h == 0) as_bias = fold_bias(as_p);
       if constexpr (W4) {
-        fold4(dprev[0], as_p, wsc[h][0], acc[h][tb][0]);
-        fold4(dprev[1], as_p, wsc[h][1], acc[h][tb][1]);
+        fold4(BIASED, dprev[0], as_p, as_bias, wsc[h][0], acc[h][tb][0]);
+        fold4(BIASED, dprev[1], as_p, as_bias, wsc[h][1], acc[h][tb][1]);
         return;
       }
       if (ORD == kOrdFusedScale && h == 0) {
         sc0 = as_p * bs0;
         sc1 = FUSED_ACT ? as_p * bs1 : sc0;
       }
-      fold(dprev[0], sc0, as_p, bs0, acc[h][tb][0]);
-      fold(dprev[1], sc1, as_p, FUSED_ACT ? bs1 : bs0, acc[h][tb][1]);
+      fold(BIASED, dprev[0], sc0, as_p, as_bias, bs0, acc[h][tb][0]);
+      fold(BIASED, dprev[1], sc1, as_p, as_bias, FUSED_ACT ? bs1 : bs0, acc[h][tb][1]);
     };
     // pipeline stage (tb, h): its MFMAs are issued, then the previous stage's fragments are folded
     // while the matrix pipe works; the operands of token fragment tb + 1 are requested in (tb, 0)
@@ -431,7 +461,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if (st < nst_c) {
         if (kEarly && st == kE0) {
           wait_copies_barrier<0>();
-          if (tid < T) sS[(kb & 1) * T + tid] = kb + 2 < KB ? s_pending : 0.0f;
+          put_scale(BIASED, kb & 1, kb + 2 < KB ? s_pending : 0.0f);
           s_pending = load_scale(kb + 3);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -472,7 +502,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           if (nst_c >= 8 ? ((g < 2 && st < 6) || (NTB == 10 && g == 0 && st == 6)) : (g < 3 && st < 4))
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, W4 ? 7 : 5, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, decltype(BIASED)::value ? (W4 ? 5 : 4) : W4 ? 7 : 5, 0);
         }
         if (kEarly && st == kE0) __builtin_amdgcn_sched_group_barrier(0x100, 7, 0);
         if (kEarly && st == kE1) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
@@ -488,31 +518,37 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       // the next K block's weights have had a whole K block to arrive; reading them here puts the
       // LDS latency under the barrier instead of in front of the first MFMA
       wait_copies<0>();
-      read_w();
+      read_w(BIASED);
     }
   };
 
   // ---- prologue ------------------------------------------------------------------------------------------
-  float s_now = load_scale(0);
-  s_pending = load_scale(1);
-  __builtin_amdgcn_sched_barrier(0);
-  copy_a(0);
-  __builtin_amdgcn_sched_barrier(0);
-  if (tid < T) sS[tid] = s_now;
-  sBs[tid] = bs_mine;
-  wait_copies<0>();
-  read_w();
+  auto start = [&](auto BIASED) __attribute__((always_inline)) {
+    const float s_now = load_scale(0);
+    s_pending = load_scale(1);
+    __builtin_amdgcn_sched_barrier(0);
+    copy_a(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (decltype(BIASED)::value) {
+      sFlag[wave] = !W4 && __builtin_amdgcn_ballot_w64(!fold_weight_scale_ok(bs_mine)) ? 1 : 0; // one value for the wave
+      bs_mine = fold_weight_scale(bs_mine);
+    }
+    put_scale(BIASED, 0, s_now);
+    sBs[tid] = bs_mine;
+    wait_copies<0>();
+    read_w(BIASED);
+  };
 
-  auto k_loop = [&](auto NST) __attribute__((always_inline)) {
+  auto k_loop = [&](auto BIASED, auto NST) __attribute__((always_inline)) {
     if constexpr (decltype(NST)::value >= kEarlyFrom && !W4 && NTB >= 8) {
       wait_copies_barrier<0>(); // K block 0 is complete in LDS
-      if (tid < T) sS[T + tid] = 1 < KB ? s_pending : 0.0f;
+      put_scale(BIASED, 1, 1 < KB ? s_pending : 0.0f);
       s_pending = load_scale(2);
 #pragma unroll
       for (int kh = 0; kh < 2; ++kh) bf_first[kh] = *reinterpret_cast<const v4i *>(sA + alds[kh]);
       as_first = sS[r];
       __builtin_amdgcn_sched_barrier(0);
-      for (int kb = 0; kb < KB; ++kb) kblock(NST, kb);
+      for (int kb = 0; kb < KB; ++kb) kblock(BIASED, NST, kb);
       return;
     }
     for (int kb = 0; kb < KB; ++kb) {
@@ -520,48 +556,84 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       // else's token rows, and nobody still reads the token stage and the scales of K block kb-1,
       // which are refilled below
       wait_copies_barrier<0>();
-      if (tid < T) sS[((kb + 1) & 1) * T + tid] = kb + 1 < KB ? s_pending : 0.0f;
+      put_scale(BIASED, (kb + 1) & 1, kb + 1 < KB ? s_pending : 0.0f);
       s_pending = load_scale(kb + 2);
       __builtin_amdgcn_sched_barrier(0);
-      kblock(NST, kb);
+      kblock(BIASED, NST, kb);
     }
   };
+  constexpr std::integral_constant<bool, kBiased> biased{};
+  start(biased);
   // one K loop per number of token fragments that hold valid tokens (wave-uniform choice)
   // in steps of 16 tokens where the registers allow it: a 96-token block costs three quarters of a full one
   if constexpr (NTB == 10 && PC) {
-    if (nst > 18) k_loop(std::integral_constant<int, 20>{});
-    else if (nst > 16) k_loop(std::integral_constant<int, 18>{});
-    else if (nst > 14) k_loop(std::integral_constant<int, 16>{});
-    else if (nst > 12) k_loop(std::integral_constant<int, 14>{});
-    else if (nst > 10) k_loop(std::integral_constant<int, 12>{});
-    else if (nst > 8) k_loop(std::integral_constant<int, 10>{});
-    else k_loop(std::integral_constant<int, 8>{});
+    if (nst > 18) k_loop(biased, std::integral_constant<int, 20>{});
+    else if (nst > 16) k_loop(biased, std::integral_constant<int, 18>{});
+    else if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{});
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{});
+    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{});
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{});
+    else k_loop(biased, std::integral_constant<int, 8>{});
   } else if constexpr (NTB == 10) {
-    if (nst > 16) k_loop(std::integral_constant<int, 20>{});
-    else if (nst > 12) k_loop(std::integral_constant<int, 16>{});
-    else if (nst > 8) k_loop(std::integral_constant<int, 12>{});
-    else k_loop(std::integral_constant<int, 8>{});
+    if (nst > 16) k_loop(biased, std::integral_constant<int, 20>{});
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{});
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{});
+    else k_loop(biased, std::integral_constant<int, 8>{});
   } else if constexpr (NTB == 8 && W4 && !PC) {
-    if (nst > 12) k_loop(std::integral_constant<int, 16>{});
-    else if (nst > 8) k_loop(std::integral_constant<int, 12>{});
-    else if (nst > 4) k_loop(std::integral_constant<int, 8>{});
-    else k_loop(std::integral_constant<int, 4>{});
+    if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{});
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{});
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 8>{});
+    else k_loop(biased, std::integral_constant<int, 4>{});
   } else if constexpr (NTB == 8) {
-    if (nst > 14) k_loop(std::integral_constant<int, 16>{});
-    else if (nst > 12) k_loop(std::integral_constant<int, 14>{});
-    else if (nst > 10) k_loop(std::integral_constant<int, 12>{});
-    else if (nst > 8) k_loop(std::integral_constant<int, 10>{});
-    else if (nst > 6) k_loop(std::integral_constant<int, 8>{});
-    else if (nst > 4) k_loop(std::integral_constant<int, 6>{});
-    else k_loop(std::integral_constant<int, 4>{});
+    if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{});
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{});
+    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{});
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{});
+    else if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{});
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{});
+    else k_loop(biased, std::integral_constant<int, 4>{});
   } else if constexpr (NTB == 4) {
-    if (nst > 6) k_loop(std::integral_constant<int, 8>{});
-    else if (nst > 4) k_loop(std::integral_constant<int, 6>{});
-    else k_loop(std::integral_constant<int, 4>{});
+    if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{});
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{});
+    else k_loop(biased, std::integral_constant<int, 4>{});
   } else {
-    k_loop(std::integral_constant<int, 2 * NTB>{});
+    k_loop(biased, std::integral_constant<int, 2 * NTB>{});
   }
   wait_copies<0>(); // no copy may still be writing LDS when the epilogue reuses it or the wave ends
+  // Lane indexes derived afresh, so that nothing computed from them is kept through the K loop.
+  auto derive = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(tid));
+    lane = tid & 63;
+    r = lane & 15;
+    q = lane >> 4;
+  };
+  derive();
+  if constexpr (kBiased) {
+    // (the flags of the last token scales were written a barrier of the K loop ago)
+    if constexpr (W4) {
+      if (__builtin_amdgcn_ballot_w64(!fold_weight_scale_ok(ws_max))) sFlag[wave] = 1;
+      __syncthreads();
+    }
+    const v4i met = *reinterpret_cast<const v4i *>(sFlag);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(met[0] | met[1] | met[2] | met[3]) != 0, 0)) {
+      constexpr std::false_type plain{};
+      __syncthreads(); // every wave is done with the token stages and the tables
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int tb = 0; tb < NTB; ++tb)
+#pragma unroll
+          for (int rf = 0; rf < 2; ++rf)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[h][tb][rf][i] = 0.0f;
+      copy_w0();
+      bs_mine = load_bs();
+      start(plain);
+      k_loop(plain, std::integral_constant<int, 2 * NTB>{});
+      wait_copies<0>();
+      derive();
+    }
+  }
   if constexpr (!FUSED_ACT) {
     if (!wave_active) return;
     // A lane holds 4 consecutive columns of one token per fragment.  Each wave turns a 16-token x
@@ -779,7 +851,7 @@ bool gemm_rows_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
 template <int NTB>
 static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, dim3 g, int mbi, int gi, hipStream_t s) {
   constexpr int T = 16 * NTB;
-  constexpr int kLds = kTW + 2 * T * kGroup + 2 * T * 4 + 4 * T * 4 + kTBs + T * 4;
+  constexpr int kLds = kTW + 2 * T * kGroup + 2 * T * 4 + 4 * T * 4 + kTBs + T * 4 + kTFlag;
 #define LO_ROWS_LAUNCH2(ORD, FA, ST, PCV)                                                                       \
   do {                                                                                                          \
     static unsigned long long lds_done = 0; /* per instantiation: one bit per device */                         \
