@@ -6,16 +6,13 @@
 // walks several 256-row weight tiles with them: the K loop needs no barrier, no LDS
 // write and no token reload, the weight prefetch (two K blocks deep) runs on across tile boundaries, and the
 // gather of sorted_token_ids is paid once per token block instead of once per tile.
-// Wave tile, MFMA layout, scaling order and output are those of the LDS-tiled kernel
-// (gemm_tile.hip); reference: Triton fused_moe_kernel, python/lightop/_lmslim_native/
+// Each wave owns 64 rows x 64 tokens as 4 x 4 fragments of v_mfma_i32_16x16x64_i8 (weights as the A operand); reference: Triton fused_moe_kernel, python/lightop/_lmslim_native/
 // layers/fused_moe/int8.py:485-541.
 #include <type_traits>
 
 #include "gemm.h"
 
 namespace lo {
-
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 // KBT: K / 128 as a compile-time constant (a multiple of three, so that a tile starts on ring buffer 0),
 // or 0 for any K.  With it a tile's steps and its stores are straight-line code: the compiler then
@@ -33,8 +30,15 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   const int pitch = K + 16; // = 16 mod 128: ds_read_b128 of 32 consecutive rows is conflict-free
   int8_t *const sA = smem;
   float *const sS = reinterpret_cast<float *>(smem + kTileM * pitch); // [KB][64]
-  // per-wave staging of 32 output rows x 64 columns (bf16), for row-contiguous stores
+  // per-wave staging of 16 output rows x 64 columns (bf16), for row-contiguous stores
   int8_t *const sStage = smem + kTileM * pitch + KB * kTileM * 4;
+  int32_t *const sFlag = reinterpret_cast<int32_t *>(sStage + 4 * 16 * kStgPitch); // [wave]: a scale that the biased fold does not take
+  float *const sB = reinterpret_cast<float *>(sFlag + 4);                          // weight-block scales of the workgroup's tiles
+  // The contracted order folds without a conversion (fold_biased), or with one where the scales do not allow that.  In 16x16
+  // fragments, whose bias is four registers: sixteen, beside 64 accumulators, 96 registers of weights and two fragments of 32x32,
+  // spill.  With the weight-block scales in LDS, not in the ring of weights: second stage of the Qwen3-30B-A3B layer at 8192
+  // tokens 223 -> 219 us, whole layer with its router 561 -> 553.
+  constexpr bool kBiased = ORD == kOrdContract;
 
   int mb, ng;
   if (!tile_of(blockIdx.x, n_groups, m_blocks, group_m, mb, ng)) return;
@@ -51,7 +55,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
       __builtin_amdgcn_ballot_w64(a.sorted[static_cast<int64_t>(mb) * kTileM + lane] < a.num_valid) == 0)
     return;
   const int wr = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of a tile
-  const int r = lane & 31, c = lane >> 5;
+  const int r = lane & 15, q = lane >> 4;
   const int64_t N = a.N;
   const int n_tiles = static_cast<int>((N + 255) / 256);
   const int nt0 = ng * n_cnt;
@@ -59,26 +63,20 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   // N % 64 == 0 is checked on the host; in the last tile the waves past N have no rows
   if (static_cast<int64_t>(nt_end - 1) * 256 + wr * 64 >= N) --nt_end;
 
-  int64_t f[2];
-  bool valid[2];
+  int32_t f[4]; // slots of the tokens this lane holds in the accumulator layout
 #pragma unroll
-  for (int tb = 0; tb < 2; ++tb) {
-    f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 32 + r];
-    valid[tb] = f[tb] < a.num_valid;
-  }
+  for (int tb = 0; tb < 4; ++tb) f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 16 + r];
 
   if (e < 0) {
     if ((!a.skip_nonlocal || e_oob)) {
       for (int nt = nt0; nt < nt_end; ++nt)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
-          if (valid[tb])
+        for (int tb = 0; tb < 4; ++tb)
+          if (f[tb] < a.num_valid)
 #pragma unroll
-            for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<v2i *>(a.C + f[tb] * N + static_cast<int64_t>(nt) * 256 + wr * 64 + rb * 32 +
-                                         8 * q + 4 * c) = v2i{0, 0};
+            for (int rb = 0; rb < 4; ++rb)
+              *reinterpret_cast<v2i *>(a.C + f[tb] * N + static_cast<int64_t>(nt) * 256 + wr * 64 + rb * 16 + 4 * q) =
+                  v2i{0, 0};
     }
     return;
   }
@@ -100,92 +98,106 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
       for (int j = 0; j < 4; ++j)
         if (j0 + j < pieces) *reinterpret_cast<v4i *>(dst + (j0 + j) * 64) = t[j];
     }
+  }
+  // every scale the workgroup needs, once; `fit`: for the biased fold, noting one that it does not take
+  const int NB = static_cast<int>((N + kGroup - 1) / kGroup);
+  const int b_cnt = (n_cnt * 2 < NB - nt0 * 2 ? n_cnt * 2 : NB - nt0 * 2) * KB; // [tile][half][K block]
+  auto fill_scales = [&](auto FIT) __attribute__((always_inline)) {
+    constexpr bool fit = decltype(FIT)::value;
     const int st = tid & 63;
     const int64_t sf = a.sorted[static_cast<int64_t>(mb) * kTileM + st];
     const int64_t srow = token_row(a, sf);
-    for (int kb = tid >> 6; kb < KB; kb += 4) sS[kb * kTileM + st] = a.As[srow * KB + kb];
-  }
+    bool bad = false;
+    for (int kb = wr; kb < KB; kb += 4) {
+      const float v = a.As[srow * KB + kb];
+      bad |= !fold_token_scale_ok(v);
+      sS[kb * kTileM + st] = fit ? fold_token_scale(v) : v;
+    }
+    const float *const ws = a.Ws + (static_cast<int64_t>(e) * NB + nt0 * 2) * KB;
+    for (int i = tid; i < b_cnt; i += 256) {
+      const float v = ws[i];
+      bad |= !fold_weight_scale_ok(v);
+      sB[i] = fit ? fold_weight_scale(v) : v;
+    }
+    if constexpr (fit) sFlag[wr] = __builtin_amdgcn_ballot_w64(bad) ? 1 : 0; // one value for the wave
+  };
+  fill_scales(std::integral_constant<bool, kBiased>{});
 
-  const int NB = static_cast<int>((N + kGroup - 1) / kGroup);
   const brsrc rW = make_rsrc(a.W + static_cast<int64_t>(e) * N * K, static_cast<uint32_t>(N * K));
-  // the offset in 32 bits: a 64-bit multiply is a vector instruction, and a descriptor that has
-  // been through vector registers costs a readfirstlane loop at every load
-  const brsrc rWs = make_rsrc(a.Ws + e * NB * KB, static_cast<uint32_t>(NB * KB * 4));
-  // lane offsets inside tile nt0; a later tile and the K block go into the scalar offset
-  int woff[2], wsoff[2];
+  // The wave's 64 rows are four 2 KB blocks, in lane order; tile, K block and k-half go into the scalar offset.
   const int wkstride = shuf_kb_stride(static_cast<int>(N / 16));
   const int wtstride = 16 * shuf_nb_stride(KB); // 256 rows further
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const int nr = nt0 * 256 + wr * 64 + rb * 32;
-    // 2 KB blocks; k-step j of lane half c reads 16-byte chunk 2j+c
-    woff[rb] = (nr / 16 + (r >> 4)) * shuf_nb_stride(KB) + (c * 16 + (r & 15)) * 16;
-    wsoff[rb] = (nr / kGroup) * KB * 4;
-  }
+  const int woff = (nt0 * 16 + wr * 4) * shuf_nb_stride(KB) + lane * 16;
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
   using B2 = std::integral_constant<int, 2>;
-  v16i zero16;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) zero16[i] = 0;
-  float acc[2][2][16]; // [token fragment][row fragment][element]
-  // Ring of three weight buffers: a K block is short work (16 MFMAs per wave), an L2 round trip
+  float acc[4][4][4]; // [token fragment][row fragment][element]
+  // Ring of three weight buffers: a K block is short work (32 MFMAs per wave), an L2 round trip
   // under load is not, so fragments are requested two K blocks ahead.
-  v4i wreg[3][2][4];   // [buffer][row fragment][k-step]
-  float bsc[3][2];     // [buffer][row fragment] weight-block scales, fetched with the fragments
+  v4i wreg[3][4][2];   // [buffer][row fragment][k-half]
 
   auto load_w = [&](auto BUF, int nt, int kb) __attribute__((always_inline)) {
     constexpr int b = decltype(BUF)::value;
     const int so = (nt - nt0) * wtstride + kb * wkstride;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) wreg[b][rb][ks] = bld16(rW, woff[rb], so + ks * 512);
-    const int ss = ((nt - nt0) * 2 * KB + kb) * 4;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) bsc[b][rb] = bld_f32(rWs, wsoff[rb], ss);
+      for (int kh = 0; kh < 2; ++kh) wreg[b][rb][kh] = bld16(rW, woff, so + rb * shuf_nb_stride(KB) + kh * 1024);
   };
-  auto fold = [&](const v16i &d, float as, float bs, float *dst) __attribute__((always_inline)) {
+  auto fold = [&](auto BIASED, const v4i &d, float as, float as_bias, float bs, float *dst) __attribute__((always_inline)) {
     const float sc = ORD == kOrdFusedScale ? as * bs : 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dst[i] = fold_elem<ORD>(d[i], sc, as, bs, dst[i]);
+    for (int i = 0; i < 4; ++i)
+      if constexpr (decltype(BIASED)::value) dst[i] = fold_biased(d[i], as, as_bias, bs, dst[i]);
+      else dst[i] = fold_elem<ORD>(d[i], sc, as, bs, dst[i]);
     // The accumulators must be final here: an empty asm that "modifies" them stops the
     // optimiser from postponing the fold (and keeping the int32 fragment alive instead).
 #pragma unroll
-    for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(dst[i]));
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(dst[i]));
   };
-  auto compute = [&](auto BUF, int kb, bool live) __attribute__((always_inline)) {
+  auto compute = [&](auto BIASED, auto BUF, int nt, int kb, bool live) __attribute__((always_inline)) {
     constexpr int b = decltype(BUF)::value;
-    // The four 32x32 fragments are software-pipelined: the MFMAs of one fragment are
-    // issued, then the previous fragment is folded into the fp32 accumulators while the
-    // matrix pipe works.
-    v16i dprev = zero16;
-    float as_prev = 0.0f;
+    constexpr int c0 = decltype(BIASED)::value ? kFoldBias : 0;
+    const v4i cinit = {c0, c0, c0, c0};
+    // the wave's 64 rows lie in one 128-row block
+    const float bs = sB[live ? ((nt - nt0) * 2 + (wr >> 1)) * KB + kb : 0];
+    // Software pipeline over half token fragments: the MFMAs of two row fragments are issued, then the previous two are folded
+    // into the fp32 accumulators while the matrix pipe works; the next token fragment is read under the first half.
+    const int8_t *src = sA + r * pitch + kb * kGroup + q * 16;
+    const float *ts = sS + kb * kTileM + r;
+    v4i bf[2][2], dprev[2];
+    float as_t[2], as_prev = 0.0f, as_bias = 0.0f;
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) {
-      v4i bf[4];
-      // the K bytes of k-step ks must be the ones the weight operand holds for it
-      const int8_t *src = sA + (tb * 32 + r) * pitch + kb * kGroup + c * 16;
+    for (int kh = 0; kh < 2; ++kh) bf[0][kh] = *reinterpret_cast<const v4i *>(src + kh * 64);
+    as_t[0] = live ? ts[0] : 0.0f; // a step past the end adds 0
+    auto fold_pair = [&](int st) __attribute__((always_inline)) {
+      const int tb = st >> 1, h = st & 1;
+      if (h == 0) as_bias = fold_bias(as_prev);
+      fold(BIASED, dprev[0], as_prev, as_bias, bs, acc[tb][2 * h]);
+      fold(BIASED, dprev[1], as_prev, as_bias, bs, acc[tb][2 * h + 1]);
+    };
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) bf[ks] = *reinterpret_cast<const v4i *>(src + ks * 32);
-      const float as = live ? sS[kb * kTileM + tb * 32 + r] : 0.0f; // a step past the end adds 0
+    for (int st = 0; st < 8; ++st) {
+      const int tb = st >> 1, h = st & 1;
+      if (h == 0 && tb < 3) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        v16i d = zero16;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-          d = __builtin_amdgcn_mfma_i32_32x32x32_i8(wreg[b][rb][ks], bf[ks], d, 0, 0, 0);
-        if (tb + rb > 0) {
-          const int ptb = rb ? tb : tb - 1, prb = rb ? 0 : 1;
-          fold(dprev, as_prev, bsc[b][prb], acc[ptb][prb]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        dprev = d;
-        as_prev = as;
+        for (int kh = 0; kh < 2; ++kh)
+          bf[(tb + 1) & 1][kh] = *reinterpret_cast<const v4i *>(src + (tb + 1) * 16 * pitch + kh * 64);
+        as_t[(tb + 1) & 1] = live ? ts[(tb + 1) * 16] : 0.0f;
       }
+      v4i d[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[b][2 * h + j][0], bf[tb & 1][0], cinit, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[b][2 * h + j][1], bf[tb & 1][1], d[j], 0, 0, 0);
+      if (st > 0) fold_pair(st - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      dprev[0] = d[0];
+      dprev[1] = d[1];
+      as_prev = as_t[tb & 1];
     }
-    fold(dprev, as_prev, bsc[b][1], acc[1][1]);
+    fold_pair(7);
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -205,36 +217,46 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   };
   auto zero_acc = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
+      for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[tb][rb][i] = 0.0f;
+        for (int i = 0; i < 4; ++i) acc[tb][rb][i] = 0.0f;
   };
   auto store_tile = [&](int nt) __attribute__((always_inline)) {
     const int64_t nrow0 = static_cast<int64_t>(nt) * 256 + wr * 64;
-    int8_t *stg = sStage + wr * (32 * kStgPitch);
+    int8_t *stg = sStage + wr * (16 * kStgPitch);
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) {
+    for (int tb = 0; tb < 4; ++tb) {
+      const bool valid = f[tb] < a.num_valid;
       float w = 1.0f;
-      if (a.mul_routed && valid[tb]) w = a.topk_w[f[tb]];
-      v4u16 o[2][4];
+      if (a.mul_routed && valid) w = a.topk_w[f[tb]];
       with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+        for (int rb = 0; rb < 4; ++rb) {
+          v4u16 o;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[rb][q][i] = cvt(acc[tb][rb][4 * q + i] * w); // w = 1 leaves every value as it is
+          for (int i = 0; i < 4; ++i) o[i] = cvt(acc[tb][rb][i] * w); // w = 1 leaves every value as it is
+          *reinterpret_cast<v4u16 *>(stg + r * kStgPitch + (rb * 16 + 4 * q) * 2) = o;
+        }
       });
-      wave_store_32x64_bf16(stg, o, valid[tb] ? static_cast<int>(f[tb]) : -1, a.C, N, nrow0, lane);
+      __builtin_amdgcn_wave_barrier();
+      const int slot = valid ? f[tb] : -1;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) { // 128-byte row segments, eight rows an instruction
+        const int tok = (lane >> 3) + 8 * j;
+        const v4i v = *reinterpret_cast<const v4i *>(stg + tok * kStgPitch + (lane & 7) * 16);
+        const int fs = __shfl(slot, tok);
+        if (fs >= 0) *reinterpret_cast<v4i *>(a.C + static_cast<int64_t>(fs) * N + nrow0 + (lane & 7) * 8) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
   };
-  auto step = [&](auto BUF, auto NEXT) __attribute__((always_inline)) {
+  auto step = [&](auto BIASED, auto BUF, auto NEXT) __attribute__((always_inline)) {
     load_step(NEXT);
     __builtin_amdgcn_sched_barrier(0); // keep the prefetch ahead of the MFMAs
     const bool live = c_nt < nt_end;
-    compute(BUF, c_kb, live);
+    compute(BIASED, BUF, c_nt, c_kb, live);
     if (live && c_kb == KB - 1) { // a tile is complete
       store_tile(c_nt);
       zero_acc();
@@ -251,6 +273,26 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   }
   __syncthreads(); // the only barrier: the token block is complete
   zero_acc();
+  constexpr std::integral_constant<bool, kBiased> biased{};
+  if constexpr (kBiased) {
+    const v4i met = *reinterpret_cast<const v4i *>(sFlag);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(met[0] | met[1] | met[2] | met[3]) != 0, 0)) {
+      __syncthreads();
+      fill_scales(std::false_type{});
+      __syncthreads();
+#pragma unroll 1
+      for (int nt = nt0; nt < nt_end; ++nt) { // rare: one K block at a time
+#pragma unroll 1
+        for (int kb = 0; kb < KB; ++kb) {
+          load_w(B0{}, nt, kb);
+          compute(std::false_type{}, B0{}, nt, kb, true);
+        }
+        store_tile(nt);
+        zero_acc();
+      }
+      return;
+    }
+  }
   if constexpr (KBT > 0) {
     static_assert(KBT % 3 == 0, "a tile must start on ring buffer 0");
     for (int nt = nt0; nt < nt_end; ++nt) {
@@ -264,28 +306,35 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
         else if (kb % 3 == 1) load_w(B0{}, lnt, lkb);
         else load_w(B1{}, lnt, lkb);
         __builtin_amdgcn_sched_barrier(0); // keep the prefetch ahead of the MFMAs
-        if (kb % 3 == 0) compute(B0{}, kb, true);
-        else if (kb % 3 == 1) compute(B1{}, kb, true);
-        else compute(B2{}, kb, true);
+        if (kb % 3 == 0) compute(biased, B0{}, nt, kb, true);
+        else if (kb % 3 == 1) compute(biased, B1{}, nt, kb, true);
+        else compute(biased, B2{}, nt, kb, true);
       }
       store_tile(nt);
       zero_acc();
     }
   } else {
     for (int s = 0; s < total; s += 3) {
-      step(B0{}, B2{});
-      step(B1{}, B0{});
-      step(B2{}, B1{});
+      step(biased, B0{}, B2{});
+      step(biased, B1{}, B0{});
+      step(biased, B2{}, B1{});
     }
   }
 }
 
-static int64_t as_lds_bytes(int64_t K) { return 64 * (K + 16) + (K / kGroup) * 64 * 4 + 4 * 32 * kStgPitch; }
+// n_cnt: weight tiles of a workgroup
+static int as_tiles(int64_t N) {
+  const int n_tiles = static_cast<int>((N + 255) / 256);
+  return (n_tiles + 1) / 2;
+}
+static int64_t as_lds_bytes(int64_t N, int64_t K) {
+  return 64 * (K + 16) + (K / kGroup) * 64 * 4 + 4 * 16 * kStgPitch + as_tiles(N) * 2 * (K / kGroup) * 4 + 16;
+}
 
 bool gemm_as_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   if (fused_act || !a.w_shuffled || (block_size_m != 64 && block_size_m != 128)) return false;
   if (a.N % 64 != 0 || (reinterpret_cast<uintptr_t>(a.C) & 15) != 0) return false;
-  if (as_lds_bytes(a.K) > 80 * 1024) return false; // two workgroups per CU
+  if (as_lds_bytes(a.N, a.K) > 80 * 1024) return false; // two workgroups per CU
   // Pays off only when the launch is several rounds of workgroups deep even with half a
   // token block's weight tiles per workgroup; below that the per-tile kernel balances better.
   return a.num_valid / 64 + (a.experts_routed + 1) / 2 >= 1024;
@@ -299,9 +348,8 @@ int launch_gemm_as(const GemmArgs &a0, int flags, int block_size_m, int64_t m_bl
   // Weight tiles per workgroup: half of them.  Fewer workgroups than that leave the
   // launch unbalanced, more pay the token gather more often (measured on 128 experts,
   // N = 2048, K = 768: 250 us with two groups, 269 with one, 296 with eight at 8192 tokens).
-  int n_groups = n_tiles >= 2 ? 2 : 1;
-  const int n_cnt = (n_tiles + n_groups - 1) / n_groups;
-  n_groups = (n_tiles + n_cnt - 1) / n_cnt;
+  const int n_cnt = as_tiles(a.N);
+  const int n_groups = (n_tiles + n_cnt - 1) / n_cnt;
   a.n_tiles = n_groups;
   int64_t G = a.num_valid / (static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * 64);
   G = G < 2 ? 2 : (G > 16 ? 16 : G);
@@ -309,7 +357,7 @@ int launch_gemm_as(const GemmArgs &a0, int flags, int block_size_m, int64_t m_bl
   const int64_t grid = (chunks + 7) / 8 * (G * n_groups) * 8;
   LO_REQUIRE(grid < (1ll << 31), LO_EINVAL, "moe_gemm: grid too large");
   const int ord = scale_order(flags);
-  const size_t lds = static_cast<size_t>(as_lds_bytes(a.K));
+  const size_t lds = static_cast<size_t>(as_lds_bytes(a.N, a.K));
   const dim3 g(static_cast<unsigned>(grid)), b(256);
   const int mbi = static_cast<int>(m_blocks), Gi = static_cast<int>(G);
 #define LO_AS_LAUNCH(FS, KBT)                                                                         \
