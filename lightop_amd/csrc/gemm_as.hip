@@ -81,6 +81,15 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     return;
   }
 
+  // Their routed weights as well, asked for here: fetched by each tile's stores, a weight waited, operations retiring in order,
+  // for the rows stored and the fragments requested before it.
+  float wgt[4];
+#pragma unroll
+  for (int tb = 0; tb < 4; ++tb) {
+    wgt[tb] = 1.0f;
+    if (a.mul_routed) wgt[tb] = a.topk_w[f[tb] < a.num_valid ? f[tb] : 0];
+  }
+
   // ---- the token block into LDS, once ------------------------------------------------
   {
     const int lt = tid >> 2, lq = tid & 3; // thread -> (token, every fourth 16-byte piece)
@@ -229,14 +238,12 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb) {
       const bool valid = f[tb] < a.num_valid;
-      float w = 1.0f;
-      if (a.mul_routed && valid) w = a.topk_w[f[tb]];
       with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
           v4u16 o;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = cvt(acc[tb][rb][i] * w); // w = 1 leaves every value as it is
+          for (int i = 0; i < 4; ++i) o[i] = cvt(acc[tb][rb][i] * wgt[tb]); // 1 leaves every value as it is
           *reinterpret_cast<v4u16 *>(stg + r * kStgPitch + (rb * 16 + 4 * q) * 2) = o;
         }
       });

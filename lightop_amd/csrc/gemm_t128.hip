@@ -43,12 +43,13 @@ constexpr int kTMaxKB = 128;                  // K blocks whose weight-block sca
 constexpr int kTBs = 2 * kTMaxKB * 4;         // [fragment][K block] weight-block scales of the tile
 constexpr int kTIds = kT * 4;                  // the tile's sorted ids, for the epilogues
 constexpr int kTFlag = 16;                    // [wave]: it met a scale that the biased fold does not take
-constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds + kTFlag;
+constexpr int kTWgt = kT * 4;                  // routed weights of the tile's slots
+constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds + kTWgt + kTFlag;
 // NTB = 10: 160 tokens per workgroup (int8 block form, or int4 weights with per-channel scales, whose int32 accumulators need no fold registers), for layers
 // whose experts see a few tokens more than 128: a remainder block is a second pass over the expert's
 // weights, and at that size the weights are what the stage streams.
 constexpr int kT160 = 160;
-constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + kT160 * 4 + kTFlag;
+constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + 2 * kT160 * 4 + kTFlag;
 constexpr int kTPitch = 144;                  // staging pitch of the epilogues: 128 + 16
 
 // Wait until all but the newest `N` vector-memory operations of this wave are complete and its
@@ -88,7 +89,8 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   float *const sBs = reinterpret_cast<float *>(smem + kTW + 2 * AST + 2 * T * 4 + RED);
   int32_t *const sIds = reinterpret_cast<int32_t *>(smem + kTW + 2 * AST + 2 * T * 4 + RED + kTBs);
 
-  int32_t *const sFlag = sIds + T;
+  float *const sWgt = reinterpret_cast<float *>(sIds + T);
+  int32_t *const sFlag = sIds + 2 * T;
   // The contracted order folds without a conversion (fold_biased): 2 vector instructions an element and K block instead of 3,
   // where they were issued in 83 % of a SIMD's cycles.  Layer with its router, us, before / after: full DeepSeek-V3 layer, 8192
   // tokens 4828 / 4531, Qwen3-30B-A3B layer, 8192: 603.8 / 578.9, DeepSeek-V3 share, 4096: 539 / 525, int4 with K-group scales,
@@ -237,6 +239,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     nst = __builtin_amdgcn_readfirstlane(2 * ((last >> 4) + 1)); // the K loop comes in variants by the number of fragments
     if (NTB == 10 && a.coarse_fill && nst > 8 && nst < 16) nst = 16;
   }
+  float wgt_mine = 1.0f;
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
     const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
@@ -244,6 +247,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     // The epilogues take the ids from LDS: a global load in each of their exec-masked blocks is a
     // full memory round trip that nothing overlaps.
     if (tid < T) sIds[tid] = static_cast<int32_t>(lf);
+    // The routed weights too: fetched by the epilogue, each of them waited, operations retiring in order, for the rows stored
+    // before it (int4 with K-group scales, 2048 tokens 588 -> 579 us; Qwen3-30B-A3B layer, 8192: 553 -> 549).
+    if (a.mul_routed) wgt_mine = a.topk_w[lf < a.num_valid ? lf : 0];
   }
   // weight-block scales of the tile: table row 0 / 1 = gate / up block (fused), or the first / second
   // 128 rows of the tile (plain: waves 0, 1 / waves 2, 3).  Thread t fetches entry (t >> 7, t & 127).
@@ -564,6 +570,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   };
   constexpr std::integral_constant<bool, kBiased> biased{};
   start(biased);
+  if (tid < T) sWgt[tid] = wgt_mine;
   // one K loop per number of token fragments that hold valid tokens (wave-uniform choice)
   // in steps of 16 tokens where the registers allow it: a 96-token block costs three quarters of a full one
   if constexpr (NTB == 10 && PC) {
@@ -659,8 +666,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if (2 * tb >= nst) continue;
       const int64_t ft = sIds[tb * 16 + r];
       const bool valid = ft < a.num_valid;
-      float wgt = 1.0f;
-      if (a.mul_routed && valid) wgt = a.topk_w[ft];
+      const float wgt = sWgt[tb * 16 + r];
       with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -717,8 +723,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       if (2 * tb >= nst) continue;
       const int64_t ft = sIds[tb * 16 + r];
       const bool valid = ft < a.num_valid;
-      float wgt = 1.0f;
-      if (a.mul_routed && valid) wgt = a.topk_w[ft];
+      const float wgt = sWgt[tb * 16 + r];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         float gu[2][4], act[4];
@@ -752,8 +757,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (a.mul_routed) { // router weight on the first GEMM's output: rare, kept out of the main pass
 #pragma unroll
       for (int tb = 0; tb < NTB; ++tb) {
-        const int64_t ft = sIds[tb * 16 + r];
-        const float wgt = ft < a.num_valid ? a.topk_w[ft] : 1.0f;
+        const float wgt = sWgt[tb * 16 + r];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -851,7 +855,7 @@ bool gemm_rows_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
 template <int NTB>
 static int launch_rows(const GemmArgs &a, bool fused_act, int ord, bool stream, dim3 g, int mbi, int gi, hipStream_t s) {
   constexpr int T = 16 * NTB;
-  constexpr int kLds = kTW + 2 * T * kGroup + 2 * T * 4 + 4 * T * 4 + kTBs + T * 4 + kTFlag;
+  constexpr int kLds = kTW + 2 * T * kGroup + 2 * T * 4 + 4 * T * 4 + kTBs + 2 * T * 4 + kTFlag;
 #define LO_ROWS_LAUNCH2(ORD, FA, ST, PCV)                                                                       \
   do {                                                                                                          \
     static unsigned long long lds_done = 0; /* per instantiation: one bit per device */                         \
