@@ -128,7 +128,17 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   // 1024 tokens of the Qwen3-235B-A22B-shaped layer, 720 / 660 at 2048, 1227 / 1074 at 4096; equal
   // or 3 % behind up to 512 tokens, where a K block of half-size weights is shorter than the memory
   // round trip it would have to hide).
-  if (form == LO_FORM_W4) return per_expert <= 8.0 ? 16 : (per_expert < 48.0 ? 64 : 128);
+  // Around 128 slots per expert 160-token blocks of that kernel hold in one block what would spill into a second pass over the
+  // expert's weights and row scales.  64 / 128 / 160, us: the same layer at 96 slots per expert 479 / 424 / 438, at 112: 524 / 495 /
+  // 467, at 128: 611 / 592 / 516, at 144: 693 / 665 / 597, at 160: 724 / 723 / 746 (two blocks of 160 instead of three of 128 gain
+  // 2 % at 272 and 288 and lose as much beside); DeepSeek-V3 share (32 of 256 experts, 7168 x 2048) at 104: 328 / 296 / 298, at
+  // 112: 399 / 429 / 317, at 128: 407 / 433 / 352, at 144: 468 / 462 / 493; 128 experts of 2048 x 768 at 104: 171 / 158 / 164, at 112: 193 /
+  // 181 / 169, at 128: 210 / 207 / 207; 64 of 2048 x 1408, top 6, at 108: 148 / 137 / 140, at 120: 171 / 167 / 151, at 132: 196 / 192 / 202.
+  if (form == LO_FORM_W4) {
+    const bool small = H < 4096, large = !small && 3 * H * I >= (32ll << 20);
+    if (allow160 && per_expert >= (small ? 110.0 : 106.0) && per_expert < (small ? 130.0 : large ? 136.0 : 154.0)) return 160;
+    return per_expert <= 8.0 ? 16 : (per_expert < 48.0 ? 64 : 128);
+  }
   // Block form with pre-shuffled weights: the kernel that copies both operands straight into LDS
   // (gemm_t128.hip, 128-token blocks, padded parts of a block skipped in steps of 32 tokens) takes
   // over from the weight-streaming kernels as soon as an expert sees a handful of tokens - with
@@ -249,12 +259,13 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false);
   if (block_size_m == 0)
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false,
-                                !w4 && dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true),
+                                dtype == LO_BF16 && !gelu && blocks_of_160_fit(H, I, true) &&
+                                    !(w4 && (flags & LO_GEMM_FORCE_STREAMING)),
                                 !pre && !(flags & LO_GEMM_FORCE_STREAMING) && H / kGroup <= 128 && I / kGroup <= 128);
-  // 160: the 160-token form of the direct-to-LDS kernel (int8 block form, load-time layout) for both GEMMs; bf16
-  // rows with SiLU take its fused first stage, fp16 rows and GELU the plain one and the activation launch
+  // 160: the 160-token form of the direct-to-LDS kernel (load-time layout; int4 weights as the table's pick only) for both
+  // GEMMs; bf16 rows with SiLU take its fused first stage, fp16 rows and GELU the plain one and the activation launch
   const bool silu_bf16 = dtype == LO_BF16 && !gelu;
-  const bool bs160 = block_size_m == 160 && pre && !w4 && dtype != LO_F32 && blocks_of_160_fit(H, I, silu_bf16);
+  const bool bs160 = block_size_m == 160 && pre && (!w4 || block_size_m_auto) && dtype != LO_F32 && blocks_of_160_fit(H, I, silu_bf16);
   LO_REQUIRE(block_size_m == 16 || block_size_m == 32 || block_size_m == 64 || block_size_m == 128 || bs160,
              LO_EINVAL,
              "fused_experts: block_size_m %d is not one of 16, 32, 64, 128 (160: int8 weights in the load-time "
@@ -450,9 +461,9 @@ extern "C" int lo_fused_experts_block_int8(
   if (!plan.fused) {
     // rows of slots whose expert another rank holds are neither written by the first GEMM nor read by
     // the activation launch (the slot mask of the alignment says which)
-    rc = lo_moe_gemm_block_int8(a1q, a1s, w1, w1s, cache3, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
+    rc = launch_gemm_block(a1q, a1s, w1, w1s, cache3, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
                                 num_experts, 2 * I, H, top_k, block_size_m, apply_router_weight_on_input,
-                                (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), stream);
+                                (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), static_cast<hipStream_t>(stream));
     if (rc) return rc;
     rc = launch_act_mul_group_quant(cache3, dtype, gelu ? LO_ACT_GELU : LO_ACT_SILU, S, I, a2q, a2s, mask,
                                     static_cast<hipStream_t>(stream));
@@ -467,10 +478,10 @@ extern "C" int lo_fused_experts_block_int8(
                                 static_cast<hipStream_t>(stream));
   }
   if (rc) return rc;
-  rc = lo_moe_gemm_block_int8(a2q, a2s, w2, w2s, cache3, dtype, topk_w, sorted, eids, ntpp,
+  rc = launch_gemm_block(a2q, a2s, w2, w2s, cache3, dtype, topk_w, sorted, eids, ntpp,
                               L.sorted_cap, S, S, E, num_experts, H, I, 1, block_size_m,
                               !apply_router_weight_on_input,
-                              (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), stream);
+                              (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), static_cast<hipStream_t>(stream));
   if (rc) return rc;
   return lo_moe_sum(cache3, out, shared_output, mask, dtype, M, top_k, H, routed_scaling_factor,
                     nullptr, stream);

@@ -99,14 +99,12 @@ static int launch_gemm(const GemmArgs &a, bool fused_act, int bs, int flags, int
 
 } // namespace lo
 
-extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const int8_t *W,
-                                      const float *Ws, void *C, int c_dtype, const float *topk_w,
-                                      const int32_t *sorted_ids, const int32_t *expert_ids,
-                                      const int32_t *num_tokens_post_pad, int64_t sorted_cap,
-                                      int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts,
-                                      int64_t N, int64_t K, int32_t top_k, int32_t block_size_m,
-                                      int mul_routed, int flags, lo_stream_t stream) {
-  using namespace lo;
+namespace lo {
+int launch_gemm_block(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype,
+                      const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
+                      const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
+                      int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
+                      int flags, hipStream_t stream) {
   int rc = validate_common("moe_gemm", A, As, W, Ws, sorted_ids, expert_ids, num_tokens_post_pad, K,
                            top_k, E, a_rows);
   if (rc) return rc;
@@ -137,15 +135,14 @@ extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const in
              "moe_gemm: int4 weights must be in the layout of lo_preshuffle_weight_int4 (LO_GEMM_W_PRESHUFFLED)");
   a.n_tiles = static_cast<int32_t>((N + 63) / 64);
   LO_REQUIRE(block_size_m != 160 || gemm_t128_supports(a, false, 160), LO_ENOTSUP,
-             "moe_gemm: 160-token blocks need int8 weights in the load-time layout (LO_GEMM_W_PRESHUFFLED), "
+             "moe_gemm: 160-token blocks need weights in the load-time layout (LO_GEMM_W_PRESHUFFLED), "
              "N a multiple of 64 and K <= %d", kGroup * 128);
   const int64_t mblocks = grid_m_blocks(sorted_cap, num_valid, block_size_m);
   LO_REQUIRE(mblocks * a.n_tiles < (1ll << 30), LO_EINVAL, "moe_gemm: grid too large");
   if (mblocks == 0) return LO_OK;
-  return launch_gemm(a, false, block_size_m, flags, mblocks, static_cast<hipStream_t>(stream));
+  return launch_gemm(a, false, block_size_m, flags, mblocks, stream);
 }
 
-namespace lo {
 int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
                            int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,
                            const int32_t *expert_ids, const int32_t *num_tokens_post_pad, int64_t sorted_cap,
@@ -180,7 +177,7 @@ int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, co
              "(LO_GEMM_W_PRESHUFFLED)");
   a.n_tiles = static_cast<int32_t>(I / kGroup);
   LO_REQUIRE(block_size_m != 160 || (fused == kActSiluBf16 && gemm_t128_supports(a, true, 160)), LO_ENOTSUP,
-             "moe_gemm1_silu_quant: 160-token blocks need int8 weights in the load-time layout "
+             "moe_gemm1_silu_quant: 160-token blocks need weights in the load-time layout "
              "(LO_GEMM_W_PRESHUFFLED) and K <= %d", kGroup * 128);
   LO_REQUIRE(fused == kActSiluBf16 || fused_table_supports(K, block_size_m, flags), LO_ENOTSUP,
              "moe_gemm1_silu_quant: no looked-up activation at this block size or scale order");
@@ -191,6 +188,20 @@ int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, co
 }
 } // namespace lo
 
+extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const int8_t *W,
+                                      const float *Ws, void *C, int c_dtype, const float *topk_w,
+                                      const int32_t *sorted_ids, const int32_t *expert_ids,
+                                      const int32_t *num_tokens_post_pad, int64_t sorted_cap,
+                                      int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts,
+                                      int64_t N, int64_t K, int32_t top_k, int32_t block_size_m,
+                                      int mul_routed, int flags, lo_stream_t stream) {
+  using namespace lo;
+  LO_REQUIRE(block_size_m != 160 || !(flags & LO_GEMM_W4), LO_ENOTSUP, "moe_gemm: 160-token blocks need int8 weights");
+  return launch_gemm_block(A, As, W, Ws, C, c_dtype, topk_w, sorted_ids, expert_ids, num_tokens_post_pad, sorted_cap, num_valid,
+                           a_rows, E, num_experts, N, K, top_k, block_size_m, mul_routed, flags,
+                           static_cast<hipStream_t>(stream));
+}
+
 extern "C" int lo_moe_gemm1_silu_quant_block_int8(
     const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
     int c_dtype, const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
@@ -199,6 +210,8 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
     int flags, lo_stream_t stream) {
   using namespace lo;
   LO_REQUIRE(c_dtype == LO_BF16, LO_ENOTSUP, "moe_gemm1_silu_quant: only bf16 rounding is built");
+  LO_REQUIRE(block_size_m != 160 || !(flags & LO_GEMM_W4), LO_ENOTSUP,
+             "moe_gemm1_silu_quant: 160-token blocks need int8 weights");
   return launch_gemm1_act_quant(A, As, W, Ws, A2q, A2s, kActSiluBf16, false, nullptr, topk_w, sorted_ids, expert_ids,
                                 num_tokens_post_pad, sorted_cap, num_valid, a_rows, E, num_experts, I, K, top_k,
                                 block_size_m, mul_routed, flags, static_cast<hipStream_t>(stream));

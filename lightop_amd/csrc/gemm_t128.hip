@@ -45,9 +45,8 @@ constexpr int kTIds = kT * 4;                  // the tile's sorted ids, for the
 constexpr int kTFlag = 16;                    // [wave]: it met a scale that the biased fold does not take
 constexpr int kTWgt = kT * 4;                  // routed weights of the tile's slots
 constexpr int kTLds = kTW + kTA + kTS + kTRed + kTBs + kTIds + kTWgt + kTFlag;
-// NTB = 10: 160 tokens per workgroup (int8 block form, or int4 weights with per-channel scales, whose int32 accumulators need no fold registers), for layers
-// whose experts see a few tokens more than 128: a remainder block is a second pass over the expert's
-// weights, and at that size the weights are what the stage streams.
+// NTB = 10: 160 tokens per workgroup, for layers whose experts see a few tokens more than 128: a remainder block is a second
+// pass over the expert's weights, and at that size the weights are what the stage streams.
 constexpr int kT160 = 160;
 constexpr int kTLds160 = kTW + 2 * kT160 * kGroup + 2 * kT160 * 4 + 4 * kT160 * 4 + kTBs + 2 * kT160 * 4 + kTFlag;
 constexpr int kTPitch = 144;                  // staging pitch of the epilogues: 128 + 16
@@ -74,9 +73,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTB == 1 ? 
 void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   static_assert(!PC || (ORD == kOrdSeparate && (W4 || NTB == 10 || ROWS)),
                 "per-channel scales: int4 weights, 160-token tiles of int8 weights or row-major ones");
-  static_assert(NTB == 8 || (NTB == 10 && (PC || !W4)) || ((NTB == 1 || NTB == 2 || NTB == 4) && ROWS),
-                "160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales; 16, 32 and 64 tokens: "
-                "row-major weights");
+  static_assert(NTB == 8 || NTB == 10 || ((NTB == 1 || NTB == 2 || NTB == 4) && ROWS),
+                "16, 32 and 64 tokens: row-major weights");
   static_assert(!ROWS || (!W4 && NTB <= 8), "row-major weights: int8, up to 128 tokens");
   constexpr int T = 16 * NTB;        // tokens per workgroup
   constexpr int AST = T * kGroup;    // token rows of one K block
@@ -96,12 +94,30 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // tokens 4828 / 4531, Qwen3-30B-A3B layer, 8192: 603.8 / 578.9, DeepSeek-V3 share, 4096: 539 / 525, int4 with K-group scales,
   // 2048: 629 / 594.  A tile that meets a scale outside of its range is done again with the conversion.
   constexpr bool kBiased = ORD == kOrdContract && !PC;
+  // 160 tokens of int4 weights with K-group scales: 160 accumulators, unpacked weights and their row scales are more registers
+  // than there are.  The wave takes its 64 rows in two halves, one after the other, with every token fragment: half of the
+  // unpacked weights and, but for one stage, of the row scales at a time, and each token fragment read from LDS twice.  The
+  // second half is read from LDS in mid K block, so the weights have two stages, in the room that 8-bit ones take; the row
+  // scales' are in the amax exchange of the epilogue.  Qwen3-235B-A22B-shaped layer, 2048 tokens: 592 us in 128-token blocks, 516.
+  constexpr bool kHalves = W4 && !PC && NTB == 10;
 
   int mb, nt;
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
   int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of the tile
   int r = lane & 15, q = lane >> 4;
+  // Lane indexes derived afresh, so that nothing computed from them is kept through the K loop.
+  auto derive = [&]() __attribute__((always_inline)) {
+    if constexpr (kHalves) {
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+      tid = wave * 64 + lane;
+    } else {
+      asm volatile("" : "+v"(tid));
+      lane = tid & 63;
+    }
+    r = lane & 15;
+    q = lane >> 4;
+  };
   const int32_t *const sorted = a.sorted + static_cast<int64_t>(mb) * T;
   // Everything the tile's start-up reads from memory by its block index alone is requested here, in one go:
   // the number of blocks in use, the block's expert and the sorted ids this thread needs (token rows it
@@ -140,6 +156,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   if (e < 0) {
     if constexpr (!FUSED_ACT) {
       if (wave_active && (!a.skip_nonlocal || e_oob)) {
+        if constexpr (kHalves) derive(); // (the compiler moves this branch to the end)
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) {
           const int64_t ft = sorted[tb * 16 + r];
@@ -196,12 +213,16 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // The first K block's weights depend on the expert only: they are requested before the token
   // ids are read, so that the two dependent round trips of the tile's start-up overlap.
   int8_t *const sWw = smem + wave * kTWStage; // int8: [row half][fragment][k half] x 1 KB; W4: [row half][fragment] x 1 KB, row scales
+  // W4: the scales of the wave's 64 rows beside the weights of K block kb
+  auto row_scales = [&](int kb) __attribute__((always_inline)) {
+    return kHalves ? reinterpret_cast<int8_t *>(sRed) + ((kb & 1) * 4 + wave) * 256 : sWw + 4096;
+  };
   auto copy_w0 = [&]() __attribute__((always_inline)) {
     if constexpr (W4) {
 #pragma unroll
       for (int p = 0; p < 4; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff, wsoff[p >> 1][p & 1], 0, kWAux);
-      if constexpr (!PC) __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, sWw + 4096, 4, wsvoff, 0, 0, kWAux);
+      if constexpr (!PC) __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, row_scales(0), 4, wsvoff, 0, 0, kWAux);
     } else {
 #pragma unroll
       for (int p = 0; p < 8; ++p)
@@ -270,10 +291,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (p < 8) {
       if constexpr (W4) { // four weight pieces, the row scales, three empty slots
         if (p < 4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff,
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + (kHalves ? (kb & 1) * 4096 : 0) + p * 1024, 16, wvoff,
                                                    __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[p >> 1][p & 1], 0, kWAux);
         else if (p == 4 && !PC)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, sWw + 4096, 4, wsvoff,
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, row_scales(kb), 4, wsvoff,
                                                    __builtin_amdgcn_readfirstlane(kc) * static_cast<int>(N) * 4, 0, kWAux);
       } else {
         const int h = p >> 2, rf = (p >> 1) & 1, kh = p & 1;
@@ -349,29 +370,32 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   v4i w[2][2][2]; // the wave's weights of the current K block
   v4f wsc[2][2];  // W4: the scales of the lane's rows 4q .. 4q+3 of each fragment
   float ws_max = 0.0f; // W4: largest |row scale| so far (of row `lane` of the wave's 64)
-  auto read_w = [&](auto BIASED) __attribute__((always_inline)) {
+  auto unpack = [&](const v4i &pk, v4i (&to)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const uint32_t word = static_cast<uint32_t>(pk[2 * ks + x]);
+        to[ks][2 * x] = static_cast<int>((word << 4) & 0xf0f0f0f0u);
+        to[ks][2 * x + 1] = static_cast<int>(word & 0xf0f0f0f0u);
+      }
+  };
+  // scales of the lane's rows 4q .. 4q+3 of fragment (h, rf), whose rows among the wave's 64 are: fused 32*rf + 16*h, plain 32*h + 16*rf
+  auto read_scales = [&](auto BIASED, int h, int rf, int kb) __attribute__((always_inline)) {
+    const int row0 = (FUSED_ACT ? 32 * rf + 16 * h : 32 * h + 16 * rf) + 4 * q;
+    wsc[h][rf] = *reinterpret_cast<const v4f *>(row_scales(kb) + row0 * 4) * (decltype(BIASED)::value ? fold_weight_scale(0.0625f) : 0.0625f);
+  };
+  // the weights of K block kb (kHalves: of its first half)
+  auto read_w = [&](auto BIASED, int kb) __attribute__((always_inline)) {
     if constexpr (W4) {
       if constexpr (decltype(BIASED)::value)
-        ws_max = fmaxf(ws_max, fabsf(*reinterpret_cast<const float *>(sWw + 4096 + lane * 4)));
+        ws_max = fmaxf(ws_max, fabsf(*reinterpret_cast<const float *>(row_scales(kb) + lane * 4)));
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < (kHalves ? 1 : 2); ++h)
 #pragma unroll
         for (int rf = 0; rf < 2; ++rf) {
-          const v4i pk = *reinterpret_cast<const v4i *>(sWw + (h * 2 + rf) * 1024 + lane * 16);
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-              const uint32_t word = static_cast<uint32_t>(pk[2 * ks + x]);
-              w[h][rf][ks][2 * x] = static_cast<int>((word << 4) & 0xf0f0f0f0u);
-              w[h][rf][ks][2 * x + 1] = static_cast<int>(word & 0xf0f0f0f0u);
-            }
-          // rows of fragment (h, rf) among the wave's 64: fused 32*rf + 16*h, plain 32*h + 16*rf
-          if constexpr (!PC) {
-            const int row0 = (FUSED_ACT ? 32 * rf + 16 * h : 32 * h + 16 * rf) + 4 * q;
-            wsc[h][rf] = *reinterpret_cast<const v4f *>(sWw + 4096 + row0 * 4);
-            wsc[h][rf] = wsc[h][rf] * (decltype(BIASED)::value ? fold_weight_scale(0.0625f) : 0.0625f);
-          }
+          unpack(*reinterpret_cast<const v4i *>(sWw + (kHalves ? (kb & 1) * 4096 : 0) + (h * 2 + rf) * 1024 + lane * 16), w[h][rf]);
+          if constexpr (!PC) read_scales(BIASED, h, rf, kb);
         }
     } else {
 #pragma unroll
@@ -388,7 +412,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // block's token stage or scales any more, so the next block's first operands are read from LDS
   // under the last two stages and no wave stands waiting for LDS right after a barrier.
   // (From twelve stages on, that is; with ten fragments of accumulators only the full variant, the others would spill.)
-  constexpr int kEarlyFrom = NTB == 10 && !PC ? 20 : 12;
+  constexpr int kEarlyFrom = NTB == 10 && !PC ? 20 : 12; // (int4 weights: none)
   float s_pending;   // token scales on their way from global memory to sS
   v4i bf_first[2];   // first token fragment of the next K block
   float as_first = 0.0f;
@@ -401,7 +425,77 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       sS[stage * T + tid] = s;
     }
   };
+  auto kblock_halves = [&](auto BIASED, auto NST, int kb) __attribute__((always_inline)) {
+    constexpr int nst_c = decltype(NST)::value, nf = nst_c / 2; // a stage: one token fragment, two row fragments
+    constexpr int c0 = decltype(BIASED)::value ? kFoldBias : 0;
+    constexpr int kCopies = 5 + APW, per = nst_c > 12 ? 1 : 2; // copies a stage: spread out, they stand in nobody's way
+    const v4i cinit = {c0, c0, c0, c0};
+    const int off0 = (kb & 1) * AST + alds[0];
+    const int8_t *const ta[2] = {sA + off0, sA + (off0 ^ 64)}; // (the other k-half, computed here: a register less through the loop)
+    const float *ts = sS + (kb & 1) * T;
+    v4i bf[2][2], pk[2], dprev[2];
+    float as_t[2], as_p = 0.0f;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) bf[0][kh] = *reinterpret_cast<const v4i *>(ta[kh]);
+    as_t[0] = ts[r];
+    auto fold_stage = [&](int st) __attribute__((always_inline)) {
+      const int tb = st % nf, h = st / nf;
+      const float as_bias = decltype(BIASED)::value ? fold_bias(as_p) : 0.0f;
+      fold4(BIASED, dprev[0], as_p, as_bias, wsc[h][0], acc[h][tb][0]);
+      fold4(BIASED, dprev[1], as_p, as_bias, wsc[h][1], acc[h][tb][1]);
+    };
+#pragma unroll
+    for (int st = 0; st < nst_c; ++st) {
+      const int cur = st & 1, nxt = cur ^ 1, tbn = (st + 1) % nf;
+#pragma unroll
+      for (int c = st * per; c < st * per + per; ++c)
+        if (c < kCopies) copy_piece(c < 5 ? c : c + 3, kb + 1);
+      if (st + 1 < nst_c) {
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh) bf[nxt][kh] = *reinterpret_cast<const v4i *>(ta[kh] + tbn * 16 * kGroup);
+        as_t[nxt] = ts[tbn * 16 + r];
+      }
+      if (st == nf - 1) {
+#pragma unroll
+        for (int rf = 0; rf < 2; ++rf) {
+          pk[rf] = *reinterpret_cast<const v4i *>(sWw + (kb & 1) * 4096 + (2 + rf) * 1024 + lane * 16);
+          read_scales(BIASED, 1, rf, kb);
+        }
+      }
+      if (st == nf) {
+#pragma unroll
+        for (int rf = 0; rf < 2; ++rf) unpack(pk[rf], w[0][rf]);
+      }
+      v4i d[2];
+#pragma unroll
+      for (int rf = 0; rf < 2; ++rf) d[rf] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[0][rf][0], bf[cur][0], cinit, 0, 0, 0);
+#pragma unroll
+      for (int rf = 0; rf < 2; ++rf) d[rf] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[0][rf][1], bf[cur][1], d[rf], 0, 0, 0);
+      if (st > 0) fold_stage(st - 1);
+      if (st != nf && st != nf - 1) {
+        if (st + 1 < nst_c) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (st * per + g < kCopies && g < per) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, decltype(BIASED)::value ? 4 : 6, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      dprev[0] = d[0];
+      dprev[1] = d[1];
+      as_p = as_t[cur];
+    }
+    fold_stage(nst_c - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_copies<0>();
+    read_w(BIASED, kb + 1);
+  };
   auto kblock = [&](auto BIASED, auto NST, int kb) __attribute__((always_inline)) {
+    if constexpr (kHalves) {
+      kblock_halves(BIASED, NST, kb);
+      return;
+    }
     constexpr int nst_c = decltype(NST)::value; // stages of this variant: 4, 8, 12, 16 (or 20)
     constexpr int kFull = 2 * NTB;              // stages of a full tile
     constexpr int kE0 = nst_c - 2, kE1 = nst_c - 1;
@@ -524,7 +618,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       // the next K block's weights have had a whole K block to arrive; reading them here puts the
       // LDS latency under the barrier instead of in front of the first MFMA
       wait_copies<0>();
-      read_w(BIASED);
+      read_w(BIASED, kb + 1);
     }
   };
 
@@ -542,7 +636,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     put_scale(BIASED, 0, s_now);
     sBs[tid] = bs_mine;
     wait_copies<0>();
-    read_w(BIASED);
+    read_w(BIASED, 0);
   };
 
   auto k_loop = [&](auto BIASED, auto NST) __attribute__((always_inline)) {
@@ -607,13 +701,6 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     k_loop(biased, std::integral_constant<int, 2 * NTB>{});
   }
   wait_copies<0>(); // no copy may still be writing LDS when the epilogue reuses it or the wave ends
-  // Lane indexes derived afresh, so that nothing computed from them is kept through the K loop.
-  auto derive = [&]() __attribute__((always_inline)) {
-    asm volatile("" : "+v"(tid));
-    lane = tid & 63;
-    r = lane & 15;
-    q = lane >> 4;
-  };
   derive();
   if constexpr (kBiased) {
     // (the flags of the last token scales were written a barrier of the K loop ago)
@@ -823,9 +910,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
 }
 
 bool gemm_t128_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
-  if (block_size_m == kT160) { // 160-token tiles: int8 block form (plain or fused epilogue) or per-channel scales
+  if (block_size_m == kT160) {
     if (!a.w_shuffled || a.K / kGroup > kTMaxKB) return false;
-    return (a.per_channel || !a.w4) && (fused_act || a.N % 64 == 0);
+    return fused_act || a.N % 64 == 0;
   }
   if (block_size_m != 128 || !a.w_shuffled) return false;
   if (a.per_channel && !a.w4) return false; // int8 per-channel weights have gemm_pc.hip
@@ -970,14 +1057,18 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     const double rounds = static_cast<double>(a.E) * a.n_tiles / 512.0, part = rounds - static_cast<int>(rounds); // (a block an expert)
     a.coarse_fill = !a.per_channel && a.K <= 4096 && slots >= 84.0 && rounds >= 1.0 && rounds < 3.0 && part >= 0.4 && part <= 0.5;
     // chosen where an expert's tokens fill one block, so a weight byte has one reader: streaming hint
-#define LO_T160_LAUNCH(FS, FA)                                                                                  \
+#define LO_T160_LAUNCH2(FS, FA, W)                                                                              \
   do {                                                                                                          \
     static unsigned long long lds_done = 0;                                                                     \
-    const int rc_lds = reserve_lds_once(                                                                        \
-        reinterpret_cast<const void *>(&moe_gemm_t128_kernel<FA, FS, true, false, false, 10>), kTLds160,        \
-        &lds_done);                                                                                             \
+    const auto kern = &moe_gemm_t128_kernel<FA, FS, true, W, false, 10>;                                        \
+    const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), kTLds160, &lds_done);             \
     if (rc_lds) return rc_lds;                                                                                  \
-    hipLaunchKernelGGL((moe_gemm_t128_kernel<FA, FS, true, false, false, 10>), g, b, kTLds160, s, a, mbi, gi);  \
+    hipLaunchKernelGGL(kern, g, b, kTLds160, s, a, mbi, gi);                                                    \
+  } while (0)
+#define LO_T160_LAUNCH(FS, FA)                                                                                  \
+  do {                                                                                                          \
+    if (a.w4) LO_T160_LAUNCH2(FS, FA, true);                                                                    \
+    else LO_T160_LAUNCH2(FS, FA, false);                                                                        \
   } while (0)
     if (a.per_channel) {
       LO_GATED_DISPATCH(a, fused_act, LO_T160_LAUNCH_PC);
@@ -987,6 +1078,7 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
       LO_ORD_DISPATCH(ord, LO_T160_LAUNCH, 0);
     }
 #undef LO_T160_LAUNCH
+#undef LO_T160_LAUNCH2
     return check_launch(fused_act ? "moe_gemm1_silu_quant(t160)" : "moe_gemm(t160)");
   }
   // one token block per expert, by and large: the slots spread over the routed experts fill half a block

@@ -1,0 +1,63 @@
+"""160-token blocks of int4 weights with K-group scales (the tile table's pick around 128 slots per expert), whole path, bit for bit
+against the CPU oracle: every fill level of a block, one and several K blocks, the three scale orders' dispatch, an expert-parallel
+share, and scales that the fold without a conversion does not take."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def run(oracle, H, I, ids, E, Eg=None, flags=0, factor=1.0, scale=1.0):
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import fused_experts_impl_w4a8, preshuffle_moe_scale_int4, preshuffle_moe_weight_int4
+
+    dev = torch.device("cuda:0")
+    M, k = ids.shape
+    layer = wl.MoeLayer("w4-160", E=E, E_global=Eg or E, top_k=k, H=H, I=I, routing="softmax", weight_bits=4)
+    t1, t2 = _lib.LoMoeTile(), _lib.LoMoeTile()
+    assert _lib.lib().lo_moe_tile_query_path(_lib.LO_FORM_W4, flags, _lib.LO_BF16, 0, M, E, layer.E_global, k, H, I, t1, t2) == 0
+    assert t1.block_size_m == 160 == t2.block_size_m and t1.kernel == _lib.LO_KERNEL_T128 == t2.kernel
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=M)
+    x, tw, _ = wl.make_inputs(layer, M, seed=M)
+    x[::7] *= scale
+    w1s = w1s / scale
+    emap = wl.expert_map_for(layer)
+    cache13 = torch.empty(M * k * max(2 * I, H), dtype=torch.bfloat16, device=dev)
+    out = fused_experts_impl_w4a8(x.to(dev), preshuffle_moe_weight_int4(w1.to(dev)), preshuffle_moe_weight_int4(w2.to(dev)),
+                                  tw.to(dev), ids.to(dev), cache13, global_num_experts=layer.E_global,
+                                  expert_map=None if emap is None else emap.to(dev),
+                                  w1_scale=preshuffle_moe_scale_int4(w1s.to(dev)), w2_scale=preshuffle_moe_scale_int4(w2s.to(dev)),
+                                  block_shape=[1, 128], routed_scaling_factor=factor, lightop_amd_flags=flags)
+    torch.cuda.synchronize()
+    with oracle.scale_order("separate" if flags & _lib.LO_GEMM_SEPARATE_ORDER else "contract"):
+        ref = oracle.fused_experts_w4a8(x, w1, w2, w1s, w2s, tw, ids, 16, global_num_experts=layer.E_global, expert_map=emap,
+                                        routed_scaling_factor=factor)
+    return out.cpu(), ref
+
+
+@pytest.mark.parametrize("count", [1, 64, 65, 96, 97, 127, 128, 129, 144, 145, 159, 160, 161, 225])
+@pytest.mark.parametrize("H,I", [(128, 128), (384, 256)])
+def test_fill_levels(oracle, count, H, I):
+    print(f"[case] int4 160-token blocks, {count} tokens on expert 0, H={H} I={I}", flush=True)
+    ids = torch.ones(240, 1, dtype=torch.int32)
+    ids[torch.randperm(240, generator=torch.Generator().manual_seed(count))[:count]] = 0
+    out, ref = run(oracle, H, I, ids, 2)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("what", ["separate", "share", "large rows", "wide"])
+def test_forms(oracle, what):
+    from lightop_amd import _lib
+
+    print(f"[case] int4 160-token blocks, {what}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    if what == "share":  # a quarter of the experts, two slots a token
+        ids = torch.stack([torch.randperm(8, generator=g)[:2] for _ in range(480)]).to(torch.int32)
+        out, ref = run(oracle, 512, 384, ids, 2, Eg=8, factor=2.5)
+    else:
+        ids = torch.randint(0, 2, (240, 1), generator=g, dtype=torch.int32)
+        H, I = (1088 // 64 * 128, 640) if what == "wide" else (512, 384)
+        out, ref = run(oracle, H, I, ids, 2, flags=_lib.LO_GEMM_SEPARATE_ORDER if what == "separate" else 0,
+                       scale=2.0 ** 56 if what == "large rows" else 1.0)
+    assert bool(ref.float().isfinite().all())
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
