@@ -118,7 +118,8 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     const int64_t srow = token_row(a, sf);
     bool bad = false;
     for (int kb = wr; kb < KB; kb += 4) {
-      const float v = a.As[srow * KB + kb];
+      // (a padding token's is zero: row 0, which it is computed on, may be one that nobody wrote)
+      const float v = sf < a.num_valid ? a.As[srow * KB + kb] : 0.0f;
       bad |= !fold_token_scale_ok(v);
       sS[kb * kTileM + st] = fit ? fold_token_scale(v) : v;
     }

@@ -264,7 +264,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   int asoff; // thread t and thread t + T both carry the scale of token t
   {
     const int64_t lf = kEarlyIds ? lf_scale : sorted[NTB <= 8 ? (tid & (T - 1)) : (tid < T ? tid : tid - T)];
-    asoff = token_row(a, lf) * (PC ? 1 : KB) * 4;
+    // (A padding token's is read as zero, past the end of the scales: the row it is computed on, 0, may be one that nobody
+    // wrote - a slot of another rank's expert - and what it holds must not send the tile to the long fold.)
+    asoff = PC || lf < a.num_valid ? token_row(a, lf) * (PC ? 1 : KB) * 4 : 0x40000000;
     // The epilogues take the ids from LDS: a global load in each of their exec-masked blocks is a
     // full memory round trip that nothing overlaps.
     if (tid < T) sIds[tid] = static_cast<int32_t>(lf);
