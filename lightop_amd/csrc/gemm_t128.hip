@@ -1002,8 +1002,16 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
                      hipStream_t s) {
   GemmArgs a = a0;
   a.n_tiles = fused_act ? static_cast<int32_t>(a.N / 2 / kGroup) : static_cast<int32_t>((a.N + 255) / 256);
-  int64_t G = a.num_valid / (static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * block_size_m);
-  G = G < 2 ? 2 : (G > 16 ? 16 : G);
+  const int64_t experts = a.experts_routed > 0 ? a.experts_routed : 1;
+  // token blocks of a chunk: about an expert's
+  int64_t G = (a.num_valid + (block_size_m == kT160 ? experts * 64 : 0)) / (experts * block_size_m);
+  // (One block of 160 an expert, and not many experts: a chunk is one block.  What spills into a second block is a handful of
+  // workgroups after the first round, and in chunks of two they meet on a few dies.  DeepSeek-V3 share, chunks of two / of one, us:
+  // 4000 tokens 490 / 465, 4200: 492 / 469, 3500, where nothing spills: 363 / 364; second stage with 5 of 32 experts past 160:
+  // 166 / 148.  Two blocks an expert share its weights and stay together (Qwen3-30B-A3B layer, 4096 tokens 332 / 363), and 256
+  // experts of skewed routing, some with many, lose as well: 4000 tokens 2988 / 3013.)
+  const int64_t least = block_size_m == kT160 && a.E <= 128 ? 1 : 2;
+  G = G < least ? least : (G > 16 ? 16 : G);
   const int64_t chunks = (m_blocks + G - 1) / G;
   const int64_t grid = (chunks + 7) / 8 * (G * a.n_tiles) * 8;
   LO_REQUIRE(grid < (1ll << 31), LO_EINVAL, "moe_gemm: grid too large");
