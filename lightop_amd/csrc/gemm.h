@@ -31,6 +31,7 @@ struct GemmArgs {
   int32_t skip_nonlocal; // blocks of expert -1: leave the output rows untouched
   int32_t w4;            // W is packed int4 (load-time layout), Ws is [E, K/128, N]
   int32_t per_channel;   // As is [a_rows], Ws is [E, N]: scales applied once, after the whole-K int32 sum
+  int32_t stream;        // 128-token tiles: experts have about one token block
   int32_t coarse_fill;   // 160-token tiles: round the token fragments in use up to 8
   int32_t out_f16;       // C holds IEEE half instead of bf16; fused: the values between the stages are rounded to half
   int32_t out_f32;       // C holds the fp32 sums themselves (block form, weight-streaming kernel only)

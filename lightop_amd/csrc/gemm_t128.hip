@@ -58,6 +58,15 @@ template <int N>
 __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
+// 16 or 4 bytes a lane to LDS; once: with the streaming hint (a constant at each call)
+__device__ __forceinline__ void copy_weights(brsrc r, int8_t *lds, int voff, int soff, bool once) {
+  if (once) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 0, kCacheStream);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 0, kCacheDefault);
+}
+__device__ __forceinline__ void copy_row_scales(brsrc r, int8_t *lds, int voff, int soff, bool once) {
+  if (once) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 4, voff, soff, 0, kCacheStream);
+  else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 4, voff, soff, 0, kCacheDefault);
+}
 template <int N>
 __device__ __forceinline__ void wait_copies_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
@@ -127,6 +136,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   constexpr bool kEarlyIds = !(FUSED_ACT && NTB == 10);
   const int32_t blocks_end = a.ntpp[0];
   const int e_raw = a.expert_ids[mb];
+  // whether no other token block reads this one's weights (copy policy, below)
+  constexpr bool kPolicy = !W4 && !ROWS && NTB == 8;
+  const bool alone = kPolicy && (mb == 0 || a.expert_ids[mb - 1] != e_raw) &&
+                     (mb + 1 >= m_blocks || a.expert_ids[mb + 1] != e_raw);
   const int cw = NTB == 1 ? wave & 1 : wave; // 16 tokens are two pieces: the first two waves copy them
   int32_t lf_copy[APW];
   int32_t lf_v0 = 0, lf_v1 = 0, lf_v2 = 0, lf_scale = 0;
@@ -205,11 +218,12 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (row >= N) row = 0;
     wsvoff = static_cast<int>(row * 4);
   }
-  // STREAM: about one token block per expert, so a weight byte is used by one workgroup only and is
-  // requested with the streaming hint (it does not displace the token rows and scales in L2;
-  // first GEMM of the DeepSeek-V3 share at 1024 tokens 213 -> 160 us).  With several token blocks
-  // per expert the blocks share the weights through L2 and the hint costs 7 %.
-  constexpr int kWAux = STREAM ? kCacheStream : kCacheDefault;
+  // Copy policy of the weights.  A byte that one workgroup uses is requested with the streaming hint while its block has few
+  // tokens (it does not displace the token rows and scales in L2); blocks of one expert share its weights through L2, and past
+  // 64 tokens the hint costs more than it gives.  128-token int8 blocks decide for themselves: by the layer's average (STREAM:
+  // the other forms do, see the launches) skewed routing loses.
+  constexpr std::integral_constant<bool, true> once{};
+  constexpr std::integral_constant<bool, STREAM> by_launch{};
   // The first K block's weights depend on the expert only: they are requested before the token
   // ids are read, so that the two dependent round trips of the tile's start-up overlap.
   int8_t *const sWw = smem + wave * kTWStage; // int8: [row half][fragment][k half] x 1 KB; W4: [row half][fragment] x 1 KB, row scales
@@ -217,20 +231,21 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   auto row_scales = [&](int kb) __attribute__((always_inline)) {
     return kHalves ? reinterpret_cast<int8_t *>(sRed) + ((kb & 1) * 4 + wave) * 256 : sWw + 4096;
   };
-  auto copy_w0 = [&]() __attribute__((always_inline)) {
+  auto copy_w0 = [&](bool once) __attribute__((always_inline)) {
     if constexpr (W4) {
 #pragma unroll
       for (int p = 0; p < 4; ++p)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff, wsoff[p >> 1][p & 1], 0, kWAux);
-      if constexpr (!PC) __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, row_scales(0), 4, wsvoff, 0, 0, kWAux);
+        copy_weights(rW, sWw + p * 1024, wvoff, wsoff[p >> 1][p & 1], once);
+      if constexpr (!PC) copy_row_scales(rWs, row_scales(0), wsvoff, 0, once);
     } else {
 #pragma unroll
       for (int p = 0; p < 8; ++p)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff, wsoff[p >> 2][(p >> 1) & 1] + (p & 1) * wpstride, 0,
-                                                 kWAux);
+        copy_weights(rW, sWw + p * 1024, wvoff, wsoff[p >> 2][(p >> 1) & 1] + (p & 1) * wpstride, once);
     }
   };
-  copy_w0();
+  // (a block's tokens are not known yet: by the layer's average)
+  if (kPolicy && a.stream) copy_w0(true);
+  else copy_w0(STREAM);
   int avoff[5]; // 1 KB pieces wave*APW + j of a token stage, j < APW: eight token rows each
 #pragma unroll
   for (int j = 0; j < APW; ++j) {
@@ -288,20 +303,19 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   const float *const sBs1 = sBs + (FUSED_ACT ? kTMaxKB : (wave >> 1) * kTMaxKB);
 
   // piece p of the 8 + APW copies a wave issues per K block: 0..7 its weights, then its token rows
-  auto copy_piece = [&](int p, int kb) __attribute__((always_inline)) {
+  auto copy_piece = [&](bool once, int p, int kb) __attribute__((always_inline)) {
     const int kc = kb < KB ? kb : KB - 1;
     if (p < 8) {
       if constexpr (W4) { // four weight pieces, the row scales, three empty slots
         if (p < 4)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + (kHalves ? (kb & 1) * 4096 : 0) + p * 1024, 16, wvoff,
-                                                   __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[p >> 1][p & 1], 0, kWAux);
+          copy_weights(rW, sWw + (kHalves ? (kb & 1) * 4096 : 0) + p * 1024, wvoff,
+                       __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[p >> 1][p & 1], once);
         else if (p == 4 && !PC)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rWs, row_scales(kb), 4, wsvoff,
-                                                   __builtin_amdgcn_readfirstlane(kc) * static_cast<int>(N) * 4, 0, kWAux);
+          copy_row_scales(rWs, row_scales(kb), wsvoff, __builtin_amdgcn_readfirstlane(kc) * static_cast<int>(N) * 4, once);
       } else {
         const int h = p >> 2, rf = (p >> 1) & 1, kh = p & 1;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, sWw + p * 1024, 16, wvoff,
-                                                 __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[h][rf] + kh * wpstride, 0, kWAux);
+        copy_weights(rW, sWw + p * 1024, wvoff, __builtin_amdgcn_readfirstlane(kc * wkstride) + wsoff[h][rf] + kh * wpstride,
+                     once);
       }
     } else if (p - 8 < APW && (NTB > 1 || wave < 2)) {
       const int j = p - 8;
@@ -311,7 +325,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   };
   auto copy_a = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 8; p < 8 + APW; ++p) copy_piece(p, kb);
+    for (int p = 8; p < 8 + APW; ++p) copy_piece(STREAM, p, kb);
   };
   auto load_scale = [&](int kb) __attribute__((always_inline)) {
     if constexpr (PC) return 0.0f; // one scale per token, read by the epilogue
@@ -427,7 +441,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       sS[stage * T + tid] = s;
     }
   };
-  auto kblock_halves = [&](auto BIASED, auto NST, int kb) __attribute__((always_inline)) {
+  auto kblock_halves = [&](auto BIASED, auto NST, auto ONCE, int kb) __attribute__((always_inline)) {
     constexpr int nst_c = decltype(NST)::value, nf = nst_c / 2; // a stage: one token fragment, two row fragments
     constexpr int c0 = decltype(BIASED)::value ? kFoldBias : 0;
     constexpr int kCopies = 5 + APW, per = nst_c > 12 ? 1 : 2; // copies a stage: spread out, they stand in nobody's way
@@ -451,7 +465,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       const int cur = st & 1, nxt = cur ^ 1, tbn = (st + 1) % nf;
 #pragma unroll
       for (int c = st * per; c < st * per + per; ++c)
-        if (c < kCopies) copy_piece(c < 5 ? c : c + 3, kb + 1);
+        if (c < kCopies) copy_piece(decltype(ONCE)::value, c < 5 ? c : c + 3, kb + 1);
       if (st + 1 < nst_c) {
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) bf[nxt][kh] = *reinterpret_cast<const v4i *>(ta[kh] + tbn * 16 * kGroup);
@@ -493,9 +507,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     wait_copies<0>();
     read_w(BIASED, kb + 1);
   };
-  auto kblock = [&](auto BIASED, auto NST, int kb) __attribute__((always_inline)) {
+  auto kblock = [&](auto BIASED, auto NST, auto ONCE, int kb) __attribute__((always_inline)) {
     if constexpr (kHalves) {
-      kblock_halves(BIASED, NST, kb);
+      kblock_halves(BIASED, NST, ONCE, kb);
       return;
     }
     constexpr int nst_c = decltype(NST)::value; // stages of this variant: 4, 8, 12, 16 (or 20)
@@ -551,14 +565,14 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       const int tb = st >> 1, h = st & 1;
       const int cur = tb & 1, nxt = cur ^ 1;
       if (nst_c >= 8 && st < 6) {
-        copy_piece(2 * st, kb + 1);
-        copy_piece(2 * st + 1, kb + 1);
+        copy_piece(decltype(ONCE)::value, 2 * st, kb + 1);
+        copy_piece(decltype(ONCE)::value, 2 * st + 1, kb + 1);
       }
-      if (NTB == 10 && nst_c >= 8 && st == 6) copy_piece(12, kb + 1); // the fifth token piece of a 160-token stage
+      if (NTB == 10 && nst_c >= 8 && st == 6) copy_piece(decltype(ONCE)::value, 12, kb + 1); // the fifth token piece of a 160-token stage
       if (nst_c < 8 && st < 4) {
-        copy_piece(3 * st, kb + 1);
-        copy_piece(3 * st + 1, kb + 1);
-        copy_piece(3 * st + 2, kb + 1);
+        copy_piece(decltype(ONCE)::value, 3 * st, kb + 1);
+        copy_piece(decltype(ONCE)::value, 3 * st + 1, kb + 1);
+        copy_piece(decltype(ONCE)::value, 3 * st + 2, kb + 1);
       }
       if (st < nst_c) {
         if (kEarly && st == kE0) {
@@ -641,7 +655,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     read_w(BIASED, 0);
   };
 
-  auto k_loop = [&](auto BIASED, auto NST) __attribute__((always_inline)) {
+  auto k_loop = [&](auto BIASED, auto NST, auto ONCE) __attribute__((always_inline)) {
     if constexpr (decltype(NST)::value >= kEarlyFrom && !W4 && NTB >= 8) {
       wait_copies_barrier<0>(); // K block 0 is complete in LDS
       put_scale(BIASED, 1, 1 < KB ? s_pending : 0.0f);
@@ -650,7 +664,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       for (int kh = 0; kh < 2; ++kh) bf_first[kh] = *reinterpret_cast<const v4i *>(sA + alds[kh]);
       as_first = sS[r];
       __builtin_amdgcn_sched_barrier(0);
-      for (int kb = 0; kb < KB; ++kb) kblock(BIASED, NST, kb);
+      for (int kb = 0; kb < KB; ++kb) kblock(BIASED, NST, ONCE, kb);
       return;
     }
     for (int kb = 0; kb < KB; ++kb) {
@@ -661,7 +675,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       put_scale(BIASED, (kb + 1) & 1, kb + 1 < KB ? s_pending : 0.0f);
       s_pending = load_scale(kb + 2);
       __builtin_amdgcn_sched_barrier(0);
-      kblock(BIASED, NST, kb);
+      kblock(BIASED, NST, ONCE, kb);
     }
   };
   constexpr std::integral_constant<bool, kBiased> biased{};
@@ -669,38 +683,44 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   if (tid < T) sWgt[tid] = wgt_mine;
   // one K loop per number of token fragments that hold valid tokens (wave-uniform choice)
   // in steps of 16 tokens where the registers allow it: a 96-token block costs three quarters of a full one
-  if constexpr (NTB == 10 && PC) {
-    if (nst > 18) k_loop(biased, std::integral_constant<int, 20>{});
-    else if (nst > 16) k_loop(biased, std::integral_constant<int, 18>{});
-    else if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{});
-    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{});
-    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{});
-    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{});
-    else k_loop(biased, std::integral_constant<int, 8>{});
+  if (kPolicy && alone && nst <= 8) {
+    if constexpr (kPolicy) {
+      if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{}, once);
+      else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{}, once);
+      else k_loop(biased, std::integral_constant<int, 4>{}, once);
+    }
+  } else if constexpr (NTB == 10 && PC) {
+    if (nst > 18) k_loop(biased, std::integral_constant<int, 20>{}, by_launch);
+    else if (nst > 16) k_loop(biased, std::integral_constant<int, 18>{}, by_launch);
+    else if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{}, by_launch);
+    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{}, by_launch);
+    else k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
   } else if constexpr (NTB == 10) {
-    if (nst > 16) k_loop(biased, std::integral_constant<int, 20>{});
-    else if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{});
-    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{});
-    else k_loop(biased, std::integral_constant<int, 8>{});
+    if (nst > 16) k_loop(biased, std::integral_constant<int, 20>{}, by_launch);
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
+    else k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
   } else if constexpr (NTB == 8 && W4 && !PC) {
-    if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{});
-    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{});
-    else if (nst > 4) k_loop(biased, std::integral_constant<int, 8>{});
-    else k_loop(biased, std::integral_constant<int, 4>{});
+    if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
+    else k_loop(biased, std::integral_constant<int, 4>{}, by_launch);
   } else if constexpr (NTB == 8) {
-    if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{});
-    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{});
-    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{});
-    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{});
-    else if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{});
-    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{});
-    else k_loop(biased, std::integral_constant<int, 4>{});
+    if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
+    else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{}, by_launch);
+    else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
+    else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{}, by_launch);
+    else if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{}, by_launch);
+    else k_loop(biased, std::integral_constant<int, 4>{}, by_launch);
   } else if constexpr (NTB == 4) {
-    if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{});
-    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{});
-    else k_loop(biased, std::integral_constant<int, 4>{});
+    if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
+    else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{}, by_launch);
+    else k_loop(biased, std::integral_constant<int, 4>{}, by_launch);
   } else {
-    k_loop(biased, std::integral_constant<int, 2 * NTB>{});
+    k_loop(biased, std::integral_constant<int, 2 * NTB>{}, by_launch);
   }
   wait_copies<0>(); // no copy may still be writing LDS when the epilogue reuses it or the wave ends
   derive();
@@ -722,10 +742,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
           for (int rf = 0; rf < 2; ++rf)
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[h][tb][rf][i] = 0.0f;
-      copy_w0();
+      copy_w0(STREAM);
       bs_mine = load_bs();
       start(plain);
-      k_loop(plain, std::integral_constant<int, 2 * NTB>{});
+      k_loop(plain, std::integral_constant<int, 2 * NTB>{}, by_launch);
       wait_copies<0>();
       derive();
     }
@@ -1036,23 +1056,19 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   } while (0)
 #define LO_T128_LAUNCH_PC(FA)                                                                                   \
   do {                                                                                                          \
-    if (stream) LO_T128_LAUNCH_PC2(FA, true, true, 8, kTLds);                                                   \
+    if (a.stream) LO_T128_LAUNCH_PC2(FA, true, true, 8, kTLds);                                                 \
     else LO_T128_LAUNCH_PC2(FA, false, true, 8, kTLds);                                                         \
   } while (0)
 #define LO_T160_LAUNCH_PC(FA)                                                                                   \
   do {                                                                                                          \
-    if (a.w4) LO_T128_LAUNCH_PC2(FA, true, true, 10, kTLds160);                                                 \
-    else LO_T128_LAUNCH_PC2(FA, true, false, 10, kTLds160);                                                     \
+    if (a.w4 && one_block) LO_T128_LAUNCH_PC2(FA, true, true, 10, kTLds160);                                    \
+    else if (a.w4) LO_T128_LAUNCH_PC2(FA, false, true, 10, kTLds160);                                           \
+    else LO_T128_LAUNCH_PC2(FA, false, false, 10, kTLds160);                                                    \
   } while (0)
 #define LO_T128_PICK(FS, FA)                                                                                    \
   do {                                                                                                          \
-    if (a.w4) {                                                                                                 \
-      if (stream) LO_T128_LAUNCH(FA, FS, true, true);                                                           \
-      else LO_T128_LAUNCH(FA, FS, false, true);                                                                 \
-    } else {                                                                                                    \
-      if (stream) LO_T128_LAUNCH(FA, FS, true, false);                                                          \
-      else LO_T128_LAUNCH(FA, FS, false, false);                                                                \
-    }                                                                                                           \
+    if (a.w4) LO_T128_LAUNCH(FA, FS, false, true);                                                              \
+    else LO_T128_LAUNCH(FA, FS, false, false);                                                                  \
   } while (0)
   if (block_size_m == kT160) {
     // Tiles for one or two rounds of the 512 resident workgroups and almost half a round more: if they take different
@@ -1066,11 +1082,14 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     const double slots = static_cast<double>(a.num_valid) / (a.experts_routed > 0 ? a.experts_routed : 1);
     const double rounds = static_cast<double>(a.E) * a.n_tiles / 512.0, part = rounds - static_cast<int>(rounds); // (a block an expert)
     a.coarse_fill = !a.per_channel && a.K <= 4096 && slots >= 84.0 && rounds >= 1.0 && rounds < 3.0 && part >= 0.4 && part <= 0.5;
-    // chosen where an expert's tokens fill one block, so a weight byte has one reader: streaming hint
+    // Copy policy: full blocks of int8 weights run without the streaming hint (DeepSeek-V3 share at 4000 tokens 491 with it, 472
+    // without; Qwen3-30B-A3B layer at 1531: 182 / 179, at 4200: 338 / 301), int4 weights with it where an expert has one
+    // block: 128 experts of 4096 x 1536, per-channel at 2048 tokens 422 / 435, at 4300: 745 / 710; K-group scales 521 / 536.
+    const bool one_block = slots <= 160.0;
 #define LO_T160_LAUNCH2(FS, FA, W)                                                                              \
   do {                                                                                                          \
     static unsigned long long lds_done = 0;                                                                     \
-    const auto kern = &moe_gemm_t128_kernel<FA, FS, true, W, false, 10>;                                        \
+    const auto kern = &moe_gemm_t128_kernel<FA, FS, W, W, false, 10>;                                           \
     const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), kTLds160, &lds_done);             \
     if (rc_lds) return rc_lds;                                                                                  \
     hipLaunchKernelGGL(kern, g, b, kTLds160, s, a, mbi, gi);                                                    \
@@ -1091,8 +1110,12 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
 #undef LO_T160_LAUNCH2
     return check_launch(fused_act ? "moe_gemm1_silu_quant(t160)" : "moe_gemm(t160)");
   }
-  // one token block per expert, by and large: the slots spread over the routed experts fill half a block
-  const bool stream = a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * (kT / 2);
+  // Copy policy.  int8: each block's own, by the layer's average only for a block's first copy, with the hint / without at 40 /
+  // 50 / 62 / 80 slots per expert, us: DeepSeek-V3 share 288 / 298, 301 / 310, 311 / 313, 325 / 327; the full layer's skewed
+  // routing, where the average misleads, at 500 / 1000 / 2000 tokens: 1022 / 992, 1475 / 1337, 2006 / 1611.  int4, by the average, 128
+  // experts of 4096 x 1536: per-channel at 16 / 32 / 44 / 62 slots 251 / 258, 270 / 271, 285 / 283, 306 / 303; K-group scales
+  // (from 48 slots on) at 50 / 62: 340 / 334, 361 / 357.
+  a.stream = a.num_valid <= experts * (a.w4 ? 40 : kT / 2);
   if (a.per_channel) {
     LO_GATED_DISPATCH(a, fused_act, LO_T128_LAUNCH_PC);
   } else if (fused_act) {
