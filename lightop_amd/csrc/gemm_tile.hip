@@ -32,15 +32,13 @@ constexpr int kTileRow = 144;    // LDS row pitch in bytes: 128 + 16 keeps ds_re
 // workgroup per CU; 1 -> 64-token tile, 4 waves, two workgroups per CU that are not
 // synchronised with each other, so one computes while the other waits at its barrier.
 //
-// STREAM (64-token tiles): an expert's weights are read by one token block,
-// by and large, and are loaded with the streaming cache policy (first GEMM of the Qwen3-30B-A3B
-// layer at 512 tokens 132 -> 74 us).  With several token blocks per expert the blocks share the
-// weights through L2 and the default policy is the faster one.
-template <int FUSED_ACT, int ORD, int WT, bool STREAM = false>
+// Streaming hint (64-token tiles): where experts have one token block by the layer's average (a.stream: first GEMM of the
+// Qwen3-30B-A3B layer at 512 tokens 132 -> 74 us), and only for a block that reads its weights alone: the busy experts of skewed
+// routing share theirs through L2 (full DeepSeek-V3 layer with its Zipf routing, whole call, us, 200 / 500 / 1000 / 1400 tokens with
+// the hint throughout 569 / 1121 / 1669 / 1890, now 544 / 996 / 1355 / 1418; uniform routing the same to 0.5 %).
+template <int FUSED_ACT, int ORD, int WT>
 __global__ __launch_bounds__(256 * WT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
-  static_assert(!STREAM || WT == 1, "streaming policy: 64-token tiles");
-  constexpr int kWAux = STREAM ? kCacheStream : kCacheDefault;
   constexpr int kTileM = 64 * WT; // tokens per workgroup
   __shared__ __attribute__((aligned(16))) int8_t sA[2][kTileM * kTileRow];
   __shared__ float sS[2][kTileM];
@@ -51,6 +49,8 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
   const int32_t blocks_end = a.ntpp[0];
   const int e_raw = a.expert_ids[mb];
+  const bool once = WT == 1 && a.stream && (mb == 0 || a.expert_ids[mb - 1] != e_raw) &&
+                    (mb + 1 >= m_blocks || a.expert_ids[mb + 1] != e_raw);
   int32_t ids[2];
 #pragma unroll
   for (int tb = 0; tb < 2; ++tb)
@@ -167,14 +167,14 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     for (int j = 0; j < 2; ++j) *reinterpret_cast<v4i *>(d + j * 16) = areg[st][j];
     if (lq == 0) sS[st][lt] = live ? sreg[st] : 0.0f;
   };
-  auto load_w = [&](auto BUF, int kb) {
+  auto load_w = [&](auto ONCE, auto BUF, int kb) {
     constexpr int b = decltype(BUF)::value;
     const int kc = kb < KB ? kb : KB - 1;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        wreg[b][rb][ks] = bld16<kWAux>(rW, woff[rb], kc * wkstride + ks * 512);
+        wreg[b][rb][ks] = bld16<decltype(ONCE)::value ? kCacheStream : kCacheDefault>(rW, woff[rb], kc * wkstride + ks * 512);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) bsc[b][rb] = wsrow[rb][kc];
   };
@@ -224,27 +224,31 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  load_act(B0{}, 0);
-  load_act(B1{}, 1);
-  load_w(B0{}, 0);
-  store_act(B0{}, true);
-  __syncthreads();
-  for (int kb = 0; kb < KB; kb += 2) {
-    // even K block: compute from LDS stage 0 / weight buffer 0
-    load_act(B0{}, kb + 2);            // needed in two iterations
-    load_w(B1{}, kb + 1);              // needed in the next iteration
-    __builtin_amdgcn_sched_barrier(0); // keep the prefetch ahead of the MFMAs
-    compute(B0{});
-    store_act(B1{}, kb + 1 < KB);      // requested one iteration ago
+  auto k_loop = [&](auto ONCE) {
+    load_act(B0{}, 0);
+    load_act(B1{}, 1);
+    load_w(ONCE, B0{}, 0);
+    store_act(B0{}, true);
     __syncthreads();
-    // odd K block (a dead step when K/128 is odd: zero token scales)
-    load_act(B1{}, kb + 3);
-    load_w(B0{}, kb + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(B1{});
-    store_act(B0{}, kb + 2 < KB);
-    __syncthreads();
-  }
+    for (int kb = 0; kb < KB; kb += 2) {
+      // even K block: compute from LDS stage 0 / weight buffer 0
+      load_act(B0{}, kb + 2);            // needed in two iterations
+      load_w(ONCE, B1{}, kb + 1);              // needed in the next iteration
+      __builtin_amdgcn_sched_barrier(0); // keep the prefetch ahead of the MFMAs
+      compute(B0{});
+      store_act(B1{}, kb + 1 < KB);      // requested one iteration ago
+      __syncthreads();
+      // odd K block (a dead step when K/128 is odd: zero token scales)
+      load_act(B1{}, kb + 3);
+      load_w(ONCE, B0{}, kb + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(B1{});
+      store_act(B0{}, kb + 2 < KB);
+      __syncthreads();
+    }
+  };
+  if (once) k_loop(std::integral_constant<bool, WT == 1>{});
+  else k_loop(std::false_type{});
 
   if constexpr (!FUSED_ACT) {
     if (!wave_active) return;
@@ -344,12 +348,10 @@ int launch_gemm_tile(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   // one token block per expert, by and large (measured up to 48 slots per expert on average: first GEMM
   // of the Qwen3-30B-A3B layer at 768 tokens 135 -> 88 us; at 64 the second GEMM loses more than
   // the first one gains)
-  const bool stream = wt == 1 && a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * 48;
+  a.stream = a.num_valid <= static_cast<int64_t>(a.experts_routed > 0 ? a.experts_routed : 1) * 48;
 #define LO_TILE_LAUNCH(FS, FA)                         \
   do {                                                 \
-    if (stream)                                        \
-      hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 1, true>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
-    else if (wt == 2)                                  \
+    if (wt == 2)                                       \
       hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 2>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
     else                                               \
       hipLaunchKernelGGL((moe_gemm_tile_kernel<FA, FS, 1>), g, b, 0, s, a, mbi, static_cast<int>(G)); \
