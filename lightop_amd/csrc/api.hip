@@ -104,30 +104,33 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
                             int form = LO_FORM_BLOCK, bool preshuffled = true, bool int4_channel = false,
                             bool allow160 = false, bool copied_rows = false) {
   const double per_expert = static_cast<double>(M) * top_k / (num_experts > 0 ? num_experts : 1);
+  const bool small = H < 4096, large = !small && 3 * H * I >= (32ll << 20);
+  const auto within = [&](double from, double to) { return per_expert >= from && per_expert < to; };
   // Packed int4 weights with per-channel scales: the 128-token kernel has no scale arithmetic in
   // its K loop and skips the padded part of a block, so it takes over as soon as an expert sees more
   // than a dozen tokens (measured on the Qwen3-235B-A22B-shaped layer, whole path in us, 16 / 32 /
   // 64 / 128: at 128 tokens 247 / 254 / 401 / 267, at 256: 365 / 294 / 433 / 285, at 1024: 953 / 727 /
   // 842 / 382, at 2048: 1610 / 1224 / 1455 / 596).
-  // Around 128 slots per expert the 160-token form of that kernel holds an expert's tokens in one block
-  // (a remainder block is a second pass over the expert's weights): same layer, 128 / 160: at 1024
-  // tokens 345 / 358, at 1280: 394 / 386, at 1792: 488 / 422, at 2048: 541 / 444, at 2304: 629 / 517, at
-  // 2560: 658 / 620, at 3072: 686 / 754.  The same happens around 256 slots per expert, where two 160-token
-  // blocks hold what would spill into a third 128-token block (at 3840 tokens 779 / 796, at 4096: 869 / 797,
-  // at 4352: 938 / 830, at 4608: 964 / 868, at 4864: 997 / 924, at 5120: 1012 / 1030); the int8 forms,
-  // whose tiles are bound by arithmetic at that size, gain nothing there.
+  // The 160-token form of that kernel is ahead where it holds an expert's tokens in one block less (a remainder block is a
+  // second pass over the expert's weights): one instead of two, two instead of three, three instead of four.  Whole path, us,
+  // 128 / 160, the same layer at 100 slots per expert 355 / 367, at 104: 400 / 357, at 120: 413 / 375, at 164: 529 / 522, at 172:
+  // 528 / 554, at 240: 644 / 665, at 248: 688 / 672, at 270: 777 / 670, at 312: 829 / 817, at 320: 844 / 851, at 380: 1022 / 1010, at
+  // 430: 1106 / 1003, at 470: 1162 / 1132, at 490: 1201 / 1206; 128 experts of 2048 x 768 at 100: 140 / 144, at 108: 154 / 148, at 150:
+  // 200 / 183, at 160: 201 / 218, at 248: 259 / 249, at 270: 294 / 256, at 316: 318 / 313, at 380: 363 / 363, at 430: 413 / 382, at 480: 444 /
+  // 434; 32 of 256 experts of 7168 x 2048 at 100: 229 / 228, at 108: 308 / 236, at 140: 353 / 317, at 150: 356 / 363, at 240: 470 / 432, at
+  // 280: 518 / 491.
   if (form == LO_FORM_CHANNEL && int4_channel) {
     if (per_expert <= 12.0) return 16;
-    const bool one_block = per_expert >= 76.0 && per_expert < 170.0;
-    const bool two_blocks = per_expert >= 248.0 && per_expert < 312.0;
-    return (allow160 && (one_block || two_blocks)) ? 160 : 128;
+    if (allow160 && (within(103.0, small ? 156.0 : large ? 146.0 : 168.0) || within(246.0, 314.0) || (!large && within(384.0, 480.0))))
+      return 160;
+    return 128;
   }
   // W4A8: the streaming kernel re-reads the token rows per wave, which outweighs the half-size
   // weights early; the LDS-tiled kernel (64 tokens) wins above about 8 slots per expert.
-  // From 48 slots per expert on the 128-token kernel takes over (measured, 64 / 128: 475 / 394 us at
-  // 1024 tokens of the Qwen3-235B-A22B-shaped layer, 720 / 660 at 2048, 1227 / 1074 at 4096; equal
-  // or 3 % behind up to 512 tokens, where a K block of half-size weights is shorter than the memory
-  // round trip it would have to hide).
+  // From about 58 slots per expert on, 50 with large experts, the 128-token kernel takes over: below, a K block of half-size
+  // weights is shorter than the memory round trip it would have to hide (64 / 128: Qwen3-235B-A22B-shaped layer at 44 slots
+  // 284 / 309, at 54: 331 / 346, at 58: 355 / 354, at 62: 378 / 359, at 72: 473 / 373; DeepSeek-V3 share at 48: 202 / 220, at 54: 272 /
+  // 235; 128 experts of 2048 x 768 at 54: 125 / 132, at 62: 142 / 138).
   // Around 128 slots per expert 160-token blocks of that kernel hold in one block what would spill into a second pass over the
   // expert's weights and row scales.  64 / 128 / 160, us: the same layer at 96 slots per expert 479 / 424 / 438, at 112: 524 / 495 /
   // 467, at 128: 611 / 592 / 516, at 144: 693 / 665 / 597, at 160: 724 / 723 / 746 (two blocks of 160 instead of three of 128 gain
@@ -135,9 +138,8 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   // 112: 399 / 429 / 317, at 128: 407 / 433 / 352, at 144: 468 / 462 / 493; 128 experts of 2048 x 768 at 104: 171 / 158 / 164, at 112: 193 /
   // 181 / 169, at 128: 210 / 207 / 207; 64 of 2048 x 1408, top 6, at 108: 148 / 137 / 140, at 120: 171 / 167 / 151, at 132: 196 / 192 / 202.
   if (form == LO_FORM_W4) {
-    const bool small = H < 4096, large = !small && 3 * H * I >= (32ll << 20);
-    if (allow160 && per_expert >= (small ? 110.0 : 106.0) && per_expert < (small ? 130.0 : large ? 136.0 : 154.0)) return 160;
-    return per_expert <= 8.0 ? 16 : (per_expert < 48.0 ? 64 : 128);
+    if (allow160 && within(small ? 110.0 : 106.0, small ? 130.0 : large ? 136.0 : 154.0)) return 160;
+    return per_expert <= 8.0 ? 16 : (per_expert < (large ? 50.0 : 58.0) ? 64 : 128);
   }
   // Block form with pre-shuffled weights: the kernel that copies both operands straight into LDS
   // (gemm_t128.hip, 128-token blocks, padded parts of a block skipped in steps of 32 tokens) takes
@@ -152,29 +154,21 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   // - / - / 928 / 776.
   // Around 128 slots per expert a 128-token block spills a few tokens into a second block on half of
   // the experts, and that remainder block is a second pass over the expert's weights - the bytes the
-  // stage is bound by at that size.  160-token blocks (the same kernel with ten token fragments, plain
-  // epilogues, the activation in a launch of its own) hold such an expert in one block.  Measured,
-  // whole path in us, table before / 160: Qwen3-30B-A3B layer at 1280 tokens (80 slots per expert)
-  // 239 / 229, 1536: 264 / 230, 1792: 275 / 239, 2048: 302 / 265, 2304: 351 / 301, 2560: 348 / 355;
-  // DeepSeek-V3 share at 3072 (96 per expert): 435 / 451, 3584: 544 / 468, 4096: 581 / 495, 4352:
-  // 610 / 616, 4608: 620 / 660.
+  // stage is bound by at that size.  160-token blocks (the same kernel with ten token fragments) hold such an expert in one
+  // block, an expert of 280 tokens in two instead of three, one of 430 in three instead of four.  Whole path, us, 128 / 160:
+  //   Qwen3-30B-A3B layer, slots per expert 72: 170 / 174, 96: 188 / 180, 112: 212 / 187, 128: 235 / 220, 144: 256 / 227, 162: 252 / 264;
+  //   244: 311 / 320, 250: 331 / 320, 275: 361 / 321, 384: 449 / 453, 388: 456 / 450, 425: 494 / 458, 438: 510 / 476, 475: 532 / 523, 488:
+  //   531 / 546 (64 experts of 2048 x 1408, top 6, in the same places to 10);
+  //   medium experts (Qwen3-235B-A22B-shaped layer) 81: 513 / 515, 91: 523 / 525, 112: 610 / 563, 128: 713 / 598, 156: 833 / 734, 162:
+  //   772 / 778; 250: 1035 / 1044, 262: 1110 / 988, 300: 1233 / 1123, 325: 1250 / 1279; 384: 1483 / 1447, 425: 1604 / 1496, 475: 1714 /
+  //   1700 (60 experts of 4096 x 1408: 160: 366 / 368, 250: 466 / 461, 310: 552 / 533, 390: 637 / 647, 410: 678 / 669, 470: 723 / 759);
+  //   large experts (DeepSeek-V3 share) 80: 420 / 332, 100: 463 / 357, 128: 520 / 429, 138: 503 / 463, 148: 501 / 503; 253: 654 / 674, 263: 699 /
+  //   677, 288: 746 / 723 (48 of 384 experts, the same size: 260: 1004 / 870, 280: 1089 / 974, 310: 1124 / 1104).
   if (form == LO_FORM_BLOCK && preshuffled && allow160) {
-    // With the first stage's fused epilogue in the 160-token form as well (no activation launch, no [S, 2I] round
-    // trip) the window widens; whole path in us, 128 / 160: Qwen3-30B-A3B layer at 1024 tokens (64 slots per
-    // expert) 184 / 193, at 1152: 230 / 197, at 2048: 279 / 221, at 2432: 306 / 276, at 2560: 298 / 307;
-    // DeepSeek-V3 share at 2560 (80 per expert): 380 / 367, at 3072: 381 / 373, at 4096: 541 / 428, at 4352:
-    // 561 / 570.
-    // Medium experts (Qwen3-235B-A22B-shaped layer, int8): at 1280 tokens (80 per expert) 573 / 580, at 1536: 606 /
-    // 596, at 2048: 775 / 659, at 2304: 889 / 742, at 2560: 911 / 934.
-    const bool medium = H >= 4096 && 3 * H * I < (32ll << 20);
-    if (medium ? (per_expert >= 88.0 && per_expert < 152.0)
-               : H >= 4096 ? (per_expert >= 76.0 && per_expert < 134.0) : (per_expert >= 68.0 && per_expert < 156.0))
+    if (small ? within(72.0, 156.0) || within(248.0, 288.0) || within(386.0, 480.0)
+        : large ? within(76.0, 136.0) || within(260.0, 290.0)
+                : within(88.0, 158.0) || within(254.0, 314.0) || within(400.0, 460.0))
       return 160;
-    // Small experts again around 256 slots per expert, where two 160-token blocks hold what would spill into a
-    // third block of 128 (Qwen3-30B-A3B layer, 128 / 160: at 3840 tokens 365 / 381, at 4096: 391 / 376, at 4352:
-    // 415 / 382, at 4608: 429 / 427, at 5120: 445 / 491); the larger experts, whose tiles are bound by arithmetic
-    // at that size, gain nothing there (DeepSeek-V3 share at 8192 tokens 795 / 801).
-    if (H < 4096 && per_expert >= 248.0 && per_expert < 284.0) return 160;
   }
   // With about one token block per expert the 64-token kernel with register-fed weights
   // (gemm_tile.hip) streams them with the non-temporal hint as well, and its shorter start-up and
@@ -183,7 +177,7 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   // 157, at 768: - / 162 / 176, at 1024: - / 218 / 194; DeepSeek-V3 share at 512 tokens 356 / 251 / 251,
   // at 768: 508 / 264 / 264, at 1024: 638 / 276 / 283, at 1536: 847 / 292 / 303, at 2048: - / 428 / 333.
   if (form == LO_FORM_BLOCK && preshuffled) {
-    if (H < 4096) {
+    if (small) {
       if (per_expert < 6.0) return 16;
       // 96 to 152 (where 160-token blocks cannot be used): the remainder blocks' second pass costs the
       // 64-token tiles less; from 160 slots per expert on the 128-token kernel is ahead again (at 2560
@@ -191,13 +185,13 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
       if (per_expert <= 48.0 || (per_expert >= 96.0 && per_expert < 152.0)) return 64;
       return 128;
     }
-    if (3 * H * I < (32ll << 20)) {
+    if (!large) {
       // Medium experts, measured on the Qwen3-235B-A22B-shaped layer with int8 weights (us, whole path, 16 /
       // 64 / 128): at 16 tokens 253 / 246 / 256, at 64: 416 / 376 / 391, at 128: 450 / 391 / 407, at 256: 631 /
       // 414 / 427, at 512: 1022 / 444 / 461, at 768: - / 504 / 488, at 1024: - / 618 / 522, at 4096: - / 1392 /
       // 1200.
       if (per_expert < 1.0) return 16;
-      return per_expert <= 40.0 ? 64 : 128;
+      return per_expert <= 46.0 ? 64 : 128; // (at 44 slots 445 / 457, at 48: 477 / 468)
     }
     if (per_expert < 4.0) return 16;
     return (per_expert >= 28.0 && per_expert <= 48.0) ? 64 : 128; // equal within 0.2 % from 16 to 24
@@ -210,15 +204,21 @@ static int32_t pick_block_m(int64_t M, int32_t num_experts, int32_t top_k, int64
   // 130 / 132 / 127 / 130, at 256: 188 / 147 / 135 / 138, at 512: 296 / 223 / 152 / 153, at 1024:
   // 489 / 361 / 223 / 173; DeepSeek-V3 share of 32 experts at 128 tokens 252 / 251 / 253 / 253, at
   // 256: 268 / 268 / 270 / 262, at 512: 365 / 296 / 297 / 285, at 1024: 627 / 476 / 336 / 319.
-  // Around 128 slots per expert the 160-token form of the direct-to-LDS kernel (int32 sums over the whole K
-  // in its accumulators) holds an expert's tokens in one block, where a 128-token block spills into a
-  // second pass over the expert's weights.  Measured, 128 / 160: DeepSeek-V3 share at 2048 tokens 378 / 384,
-  // at 2560: 476 / 418, at 3584: 616 / 475, at 4096: 629 / 514, at 4608: 659 / 686; Qwen3-shaped layer at
-  // 1024 tokens 173 / 192, at 1280: 222 / 201, at 2048: 259 / 226, at 2304: 285 / 250, at 2560: 273 / 306.
+  // The 160-token form of the direct-to-LDS kernel (int32 sums over the whole K in its accumulators) again where it saves a
+  // block.  128 / 160, slots per expert: Qwen3-shaped layer 96: 170 / 185, 112: 192 / 193, 128: 215 / 206, 144: 231 / 216, 156: 242 / 231,
+  // 164: 228 / 255; 245: 280 / 296, 255: 305 / 299, 270: 330 / 285, 305: 342 / 326, 320: 353 / 342; 370: 381 / 386, 390: 419 / 397, 430: 455 / 408,
+  // 490: 476 / 470 (64 experts of 2048 x 1408, top 6: 140: 215 / 202, 160: 207 / 220, 260: 287 / 248, 316: 313 / 304, 324: 314 / 316, 390: 372 / 343,
+  // 490: 419 / 411); 128 experts of 4096 x 1536 72: 520 / 520, 140: 722 / 630, 160: 764 / 706, 170: 738 / 768; 240: 855 / 873, 250: 911 / 881,
+  // 260: 984 / 840, 316: 1115 / 1030; 390: 1312 / 1209, 470: 1483 / 1390; DeepSeek-V3 share 76: 325 / 324, 96: 410 / 367, 128: 480 / 445, 160:
+  // 485 / 482, 172: 496 / 498; 200: 521 / 535, 220: 585 / 546, 245: 601 / 577, 270: 686 / 641 (48 of 384 experts: 150: 696 / 606, 170: 698 / 718,
+  // 210: 731 / 779, 220: 789 / 781, 240: 853 / 793, 260: 937 / 776, 300: 1060 / 907).
   if (form == LO_FORM_CHANNEL) {
     if (per_expert <= 6.0) return 16;
-    if (allow160 && per_expert >= 72.0 && per_expert < (H >= 4096 ? 140.0 : 152.0)) return 160;
-    return (H >= 4096 || per_expert >= 48.0) ? 128 : 64;
+    if (allow160 && (small ? within(116.0, 158.0) || within(258.0, 322.0) || within(382.0, 492.0)
+                     : large ? within(72.0, 164.0) || within(222.0, 310.0)
+                             : within(72.0, 164.0) || within(246.0, 318.0) || within(384.0, 480.0)))
+      return 160;
+    return (!small || per_expert >= 48.0) ? 128 : 64;
   }
   // Row-major block-form weights, copied into LDS at every block size: 64-token tiles run three workgroups to a compute
   // unit, 128-token ones halve the passes over an expert's weights, except where its tokens spill a few rows into a second

@@ -297,3 +297,28 @@ def test_tile_query_path_follows_element_type_activation_and_block_size(lib):
     assert q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2, qwen)[0][1] == _lib.LO_KERNEL_DEC
     assert q(_lib.LO_FORM_BLOCK, _lib.LO_GEMM_W4, _lib.LO_BF16, 0, 2048, dsv3) == \
         q(_lib.LO_FORM_W4, 0, _lib.LO_BF16, 0, 2048, dsv3)
+
+
+def test_blocks_of_160_where_they_save_a_block(lib):
+    """The windows of the tile table's 160-token blocks: one block an expert instead of two of 128, two instead of three, three
+    instead of four, by shape class (small, medium, large experts) and form; 128 tokens between and past them."""
+    from lightop_amd import _lib
+
+    t1, t2 = _lib.LoMoeTile(), _lib.LoMoeTile()
+    pre = _lib.LO_GEMM_W_PRESHUFFLED
+    small, medium, large = (128, 128, 8, 2048, 768), (128, 128, 8, 4096, 1536), (32, 256, 8, 7168, 2048)
+    block, channel, w4c = (_lib.LO_FORM_BLOCK, pre), (_lib.LO_FORM_CHANNEL, pre), (_lib.LO_FORM_CHANNEL, pre | _lib.LO_GEMM_W4)
+    for (form, flags), shape, slots in (
+            (block, small, ((71, 128), (72, 160), (155, 160), (156, 128), (287, 160), (288, 128), (385, 128), (386, 160), (480, 128))),
+            (block, medium, ((87, 128), (88, 160), (157, 160), (158, 128), (254, 160), (314, 128), (399, 128), (400, 160), (460, 128))),
+            (block, large, ((75, 128), (76, 160), (135, 160), (136, 128), (259, 128), (260, 160), (290, 128))),
+            (channel, small, ((115, 128), (116, 160), (158, 128), (257, 128), (258, 160), (322, 128), (382, 160), (492, 128))),
+            (channel, medium, ((71, 128), (72, 160), (164, 128), (246, 160), (318, 128), (384, 160), (480, 128))),
+            (channel, large, ((72, 160), (164, 128), (222, 160), (310, 128))),
+            (w4c, small, ((102, 128), (103, 160), (156, 128), (246, 160), (314, 128), (384, 160), (480, 128))),
+            (w4c, medium, ((103, 160), (167, 160), (168, 128), (384, 160), (480, 128))),
+            (w4c, large, ((103, 160), (146, 128), (246, 160), (314, 128), (384, 128)))):
+        for n, want in slots:
+            M = n * (shape[1] // shape[2])
+            assert lib.lo_moe_tile_query_form(form, flags, M, *shape, t1, t2) == 0
+            assert t1.block_size_m == want, (form, flags, shape, n)
