@@ -666,10 +666,12 @@ extern "C" int lo_fused_experts_block_int8_noalloc(
   if (rc_plan) return rc_plan;
   int32_t block_size_m_arg = block_size_m;
   int64_t need = ws_layout(M, top_k, H, I, num_experts, plan.block_size_m).total;
-  // row-major weights, the table's pick of 128 and a scratch that 64-token blocks, which pad less, still fit
-  if (need > kScratchBytes && block_size_m == 0 && plan.block_size_m == 128 && !(plan.flags & LO_GEMM_W_PRESHUFFLED)) {
-    block_size_m_arg = 64;
-    need = ws_layout(M, top_k, H, I, num_experts, 64).total;
+  // the table's pick and a scratch that the next smaller blocks, which pad less, still fit: 128 tokens for 160, with row-major
+  // weights 64 for 128
+  if (need > kScratchBytes && block_size_m == 0 &&
+      (plan.block_size_m == 160 || (plan.block_size_m == 128 && !(plan.flags & LO_GEMM_W_PRESHUFFLED)))) {
+    block_size_m_arg = plan.block_size_m == 160 ? 128 : 64;
+    need = ws_layout(M, top_k, H, I, num_experts, block_size_m_arg).total;
   }
   LO_REQUIRE(need <= kScratchBytes, LO_ENOSPC,
              "fused_experts(noalloc): this problem needs %lld bytes of scratch, the built-in scratch holds %lld; "

@@ -109,3 +109,27 @@ def test_noalloc_row_major_weights_at_the_scratch_limit(dev):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     with pytest.raises(RuntimeError, match="built-in scratch holds"):
         call_both(dev, layer, M + 1, 3, (w1, w2, w1s, w2s), 0, 0)
+
+
+def test_noalloc_blocks_of_160_at_the_scratch_limit(dev):
+    """The same for the 160-token blocks of the table's pick with pre-shuffled weights: 128 tokens where only those fit."""
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import preshuffle_moe_weight
+
+    lib = _lib.lib()
+    layer = wl.MoeLayer("many-experts", E=448, E_global=448, top_k=8, H=256, I=128, routing="softmax")
+    shape = (layer.top_k, layer.H, layer.I, layer.E)
+    fits = lambda M, bs: lib.lo_fused_experts_workspace_bytes(M, *shape, bs) - 256 <= _lib.LO_NOALLOC_SCRATCH_BYTES  # noqa: E731
+    M = max(m for m in range(15000, 30000) if fits(m, 128))
+    tile = _lib.LoMoeTile()
+    assert lib.lo_moe_tile_query_form(_lib.LO_FORM_BLOCK, _lib.LO_GEMM_W_PRESHUFFLED, M, layer.E, layer.E_global, layer.top_k,
+                                      layer.H, layer.I, tile, None) == 0
+    assert tile.block_size_m == 160 and not fits(M, 160) and fits(M - 400, 160)
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=0, device=dev, gen_device="cuda")
+    weights = (preshuffle_moe_weight(w1), preshuffle_moe_weight(w2), w1s, w2s)
+    for m in (M, M - 400):
+        say(f"noalloc 160 M={m}")
+        a, b = call_both(dev, layer, m, 3, weights, 0, _lib.LO_GEMM_W_PRESHUFFLED)
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    with pytest.raises(RuntimeError, match="built-in scratch holds"):
+        call_both(dev, layer, M + 1, 3, weights, 0, _lib.LO_GEMM_W_PRESHUFFLED)
