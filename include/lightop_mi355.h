@@ -198,7 +198,7 @@ int lo_per_token_group_quant_int8(const void *x, int x_dtype, int64_t rows, int6
  *   C  [num_valid, N] c_dtype, row f;  rows of blocks whose expert id is -1 are zeroed
  *   topk_w [num_valid] f32, used when mul_routed != 0
  *   sorted_ids / expert_ids / num_tokens_post_pad as produced by lo_moe_align_block_size
- *   with block_size == block_size_m (16, 32, 64 or 128; also 160 with int8 weights in the load-time
+ *   with block_size == block_size_m (16, 32, 64 or 128; also 160 with weights in the load-time
  *   layout, N % 64 == 0 and K <= 16384); sorted_cap is the extent of sorted_ids
  *   (any extent >= the alignment's own works, e.g. one rounded up by the caller), and expert_ids
  *   holds at least sorted_cap / block_size_m entries: a kernel may read the entry and the sorted ids of
@@ -222,7 +222,7 @@ int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const int8_t *W, co
  *   W [E, 2I, K] (gate rows first, then up rows), Ws [E, 2I/128, K/128]
  *   A2q [num_valid, I] int8, A2s [num_valid, I/128] f32 (rows of -1 blocks untouched)
  * I % 128 == 0, K % 128 == 0; A, W and A2q 16-byte aligned.  block_size_m: 16, 32, 64, 128, or 160 with
- * int8 weights in the load-time layout and K <= 16384.
+ * weights in the load-time layout and K <= 16384.
  */
 int lo_moe_gemm1_silu_quant_block_int8(const int8_t *A, const float *As, const int8_t *W,
                                        const float *Ws, int8_t *A2q, float *A2s, int c_dtype,
@@ -307,7 +307,7 @@ int lo_preshuffle_weight_int8(const int8_t *src, int8_t *dst, int32_t E, int64_t
  * configs/w8a8/MOE_BLOCKINT8[128,128]_*.json.
  */
 typedef struct lo_moe_tile {
-  int32_t block_size_m; /* 16, 32, 64, 128 or 160 (160: int8 weights in the load-time layout; in the block form
+  int32_t block_size_m; /* 16, 32, 64, 128 or 160 (160: weights in the load-time layout; in the block form
                          * bf16 rows with SiLU keep the fused first stage, fp16 rows and GELU take the plain
                          * stage followed by lo_act_mul_group_quant) */
   int32_t kernel;       /* LO_KERNEL_*: the kernel the stage entry points launch for this problem */
@@ -388,7 +388,7 @@ int lo_measure_mfma_issue_rate(int valu_per_mfma, int random_operands, int iters
  *   block_size_m: 0 = take it from the tile table (lo_fused_experts_workspace_bytes(.., 0) is
  *   large enough for whatever the table picks and for every explicit block size); 16, 32, 64, 128,
  *   or 160 (int8 weights in the load-time layout: 160-token blocks of the direct-to-LDS kernel - what
- *   the table picks around 128 slots per expert, where a 128-token block would spill into a second
+ *   the table picks where they hold an expert's tokens in one block less, 128-token ones spilling into another
  *   pass over the expert's weights; with fp16 rows or GELU the first GEMM is not fused with the
  *   activation, cache3 also receives its output [M*top_k, 2I], and 2I <= H is required)
  */

@@ -196,7 +196,6 @@ extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const in
                                       int64_t N, int64_t K, int32_t top_k, int32_t block_size_m,
                                       int mul_routed, int flags, lo_stream_t stream) {
   using namespace lo;
-  LO_REQUIRE(block_size_m != 160 || !(flags & LO_GEMM_W4), LO_ENOTSUP, "moe_gemm: 160-token blocks need int8 weights");
   return launch_gemm_block(A, As, W, Ws, C, c_dtype, topk_w, sorted_ids, expert_ids, num_tokens_post_pad, sorted_cap, num_valid,
                            a_rows, E, num_experts, N, K, top_k, block_size_m, mul_routed, flags,
                            static_cast<hipStream_t>(stream));
@@ -210,8 +209,6 @@ extern "C" int lo_moe_gemm1_silu_quant_block_int8(
     int flags, lo_stream_t stream) {
   using namespace lo;
   LO_REQUIRE(c_dtype == LO_BF16, LO_ENOTSUP, "moe_gemm1_silu_quant: only bf16 rounding is built");
-  LO_REQUIRE(block_size_m != 160 || !(flags & LO_GEMM_W4), LO_ENOTSUP,
-             "moe_gemm1_silu_quant: 160-token blocks need int8 weights");
   return launch_gemm1_act_quant(A, As, W, Ws, A2q, A2s, kActSiluBf16, false, nullptr, topk_w, sorted_ids, expert_ids,
                                 num_tokens_post_pad, sorted_cap, num_valid, a_rows, E, num_experts, I, K, top_k,
                                 block_size_m, mul_routed, flags, static_cast<hipStream_t>(stream));

@@ -61,3 +61,29 @@ def test_forms(oracle, what):
                        scale=2.0 ** 56 if what == "large rows" else 1.0)
     assert bool(ref.float().isfinite().all())
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+def test_stages():
+    """The stage entry points take the size the tile table names."""
+    from lightop_amd import _lib, workloads as wl
+    from lightop_amd.moe import (invoke_fused_moe_gemm1_silu_quant, invoke_fused_moe_kernel_int8, moe_align_block_size,
+                                 preshuffle_moe_scale_int4, preshuffle_moe_weight_int4)
+    from lightop_amd.quant import per_token_group_quant_int8
+
+    dev = torch.device("cuda:0")
+    layer = wl.MoeLayer("w4-160", E=3, E_global=3, top_k=2, H=512, I=256, routing="softmax", weight_bits=4)
+    w1, w2, w1s, w2s = (t.to(dev) for t in wl.make_weights(layer, seed=1))
+    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, 300, seed=1))
+    xq, xs = per_token_group_quant_int8(x, 128)
+    got = []
+    for bs in (160, 128):
+        print(f"[case] int4 stages, block {bs}", flush=True)
+        s, e, p = moe_align_block_size(ids, bs, 3)
+        q, sc = invoke_fused_moe_gemm1_silu_quant(xq, preshuffle_moe_weight_int4(w1), xs, preshuffle_moe_scale_int4(w1s), tw, s, e, p,
+                                                  False, 2, 600, {"BLOCK_SIZE_M": bs}, flags=_lib.LO_GEMM_W4)
+        C = torch.empty(300, 2, 512, dtype=torch.bfloat16, device=dev)
+        invoke_fused_moe_kernel_int8(q, preshuffle_moe_weight_int4(w2), C, sc, preshuffle_moe_scale_int4(w2s), tw, s, e, p, True, 1,
+                                     {"BLOCK_SIZE_M": bs}, flags=_lib.LO_GEMM_W4)
+        torch.cuda.synchronize()
+        got.append((q, sc, C.view(torch.int16)))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
