@@ -1066,8 +1066,9 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   } while (0)
 #define LO_T160_LAUNCH_PC(FA)                                                                                   \
   do {                                                                                                          \
-    if (a.w4 && one_block) LO_T128_LAUNCH_PC2(FA, true, true, 10, kTLds160);                                    \
+    if (a.w4 && a.stream) LO_T128_LAUNCH_PC2(FA, true, true, 10, kTLds160);                                     \
     else if (a.w4) LO_T128_LAUNCH_PC2(FA, false, true, 10, kTLds160);                                           \
+    else if (a.stream) LO_T128_LAUNCH_PC2(FA, true, false, 10, kTLds160);                                       \
     else LO_T128_LAUNCH_PC2(FA, false, false, 10, kTLds160);                                                    \
   } while (0)
 #define LO_T128_PICK(FS, FA)                                                                                    \
@@ -1087,22 +1088,26 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     const double slots = static_cast<double>(a.num_valid) / (a.experts_routed > 0 ? a.experts_routed : 1);
     const double rounds = static_cast<double>(a.E) * a.n_tiles / 512.0, part = rounds - static_cast<int>(rounds); // (a block an expert)
     a.coarse_fill = !a.per_channel && a.K <= 4096 && slots >= 84.0 && rounds >= 1.0 && rounds < 3.0 && part >= 0.4 && part <= 0.5;
-    // Copy policy: full blocks of int8 weights run without the streaming hint (DeepSeek-V3 share at 4000 tokens 491 with it, 472
-    // without; Qwen3-30B-A3B layer at 1531: 182 / 179, at 4200: 338 / 301), int4 weights with it where an expert has one
+    // Copy policy.  int8 weights: the streaming hint while an expert has one block, with large experts while it is far from full,
+    // and not where skewed routing gives some of many experts several blocks.  With it / without, whole call with its router, us:
+    // Qwen3-30B-A3B layer at 96 slots 180 / 185, at 128: 199 / 205, per-channel 201 / 205; 128 experts of 4096 x 1536 at 94 to 128: equal;
+    // DeepSeek-V3 share at 94: 361 / 366, at 125: 502 / 481, per-channel 462 / 447; the full layer with Zipf routing at 128: 3096 / 2571;
+    // two blocks an expert, Qwen3-30B-A3B layer at 262: 338 / 301.  int4 weights, half the bytes, with it where an expert has one
     // block: 128 experts of 4096 x 1536, per-channel at 2048 tokens 422 / 435, at 4300: 745 / 710; K-group scales 521 / 536.
-    const bool one_block = slots <= 160.0;
-#define LO_T160_LAUNCH2(FS, FA, W)                                                                              \
+    a.stream = a.w4 ? slots <= 160.0 : a.E <= 128 && slots < (a.N * a.K <= (8 << 20) ? 160.0 : 112.0);
+#define LO_T160_LAUNCH2(FS, FA, ST, W)                                                                          \
   do {                                                                                                          \
     static unsigned long long lds_done = 0;                                                                     \
-    const auto kern = &moe_gemm_t128_kernel<FA, FS, W, W, false, 10>;                                           \
+    const auto kern = &moe_gemm_t128_kernel<FA, FS, ST, W, false, 10>;                                          \
     const int rc_lds = reserve_lds_once(reinterpret_cast<const void *>(kern), kTLds160, &lds_done);             \
     if (rc_lds) return rc_lds;                                                                                  \
     hipLaunchKernelGGL(kern, g, b, kTLds160, s, a, mbi, gi);                                                    \
   } while (0)
 #define LO_T160_LAUNCH(FS, FA)                                                                                  \
   do {                                                                                                          \
-    if (a.w4) LO_T160_LAUNCH2(FS, FA, true);                                                                    \
-    else LO_T160_LAUNCH2(FS, FA, false);                                                                        \
+    if (a.w4) LO_T160_LAUNCH2(FS, FA, true, true);                                                              \
+    else if (a.stream) LO_T160_LAUNCH2(FS, FA, true, false);                                                    \
+    else LO_T160_LAUNCH2(FS, FA, false, false);                                                                 \
   } while (0)
     if (a.per_channel) {
       LO_GATED_DISPATCH(a, fused_act, LO_T160_LAUNCH_PC);
