@@ -218,10 +218,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (row >= N) row = 0;
     wsvoff = static_cast<int>(row * 4);
   }
-  // Copy policy of the weights.  A byte that one workgroup uses is requested with the streaming hint while its block has few
-  // tokens (it does not displace the token rows and scales in L2); blocks of one expert share its weights through L2, and past
-  // 64 tokens the hint costs more than it gives.  128-token int8 blocks decide for themselves: by the layer's average (STREAM:
-  // the other forms do, see the launches) skewed routing loses.
+  // Copy policy of the weights.  A byte that one workgroup uses is requested with the streaming hint (it does not displace the
+  // token rows and scales in L2) while experts have half a block on average, and past that by blocks of at most 64 tokens;
+  // blocks of one expert share its weights through L2.  128-token int8 blocks look at their neighbours: by the layer's average
+  // alone (STREAM: the other forms go by it, see the launches) skewed routing loses.
   constexpr std::integral_constant<bool, true> once{};
   constexpr std::integral_constant<bool, STREAM> by_launch{};
   // The first K block's weights depend on the expert only: they are requested before the token
@@ -688,9 +688,13 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   if (tid < T) sWgt[tid] = wgt_mine;
   // one K loop per number of token fragments that hold valid tokens (wave-uniform choice)
   // in steps of 16 tokens where the registers allow it: a 96-token block costs three quarters of a full one
-  if (kPolicy && alone && nst <= 8) {
+  if (kPolicy && alone && (a.stream || nst <= 8)) {
     if constexpr (kPolicy) {
-      if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{}, once);
+      if (nst > 14) k_loop(biased, std::integral_constant<int, 16>{}, once);
+      else if (nst > 12) k_loop(biased, std::integral_constant<int, 14>{}, once);
+      else if (nst > 10) k_loop(biased, std::integral_constant<int, 12>{}, once);
+      else if (nst > 8) k_loop(biased, std::integral_constant<int, 10>{}, once);
+      else if (nst > 6) k_loop(biased, std::integral_constant<int, 8>{}, once);
       else if (nst > 4) k_loop(biased, std::integral_constant<int, 6>{}, once);
       else k_loop(biased, std::integral_constant<int, 4>{}, once);
     }
@@ -1120,9 +1124,10 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
 #undef LO_T160_LAUNCH2
     return check_launch(fused_act ? "moe_gemm1_silu_quant(t160)" : "moe_gemm(t160)");
   }
-  // Copy policy.  int8: each block's own, by the layer's average only for a block's first copy, with the hint / without at 40 /
-  // 50 / 62 / 80 slots per expert, us: DeepSeek-V3 share 288 / 298, 301 / 310, 311 / 313, 325 / 327; the full layer's skewed
-  // routing, where the average misleads, at 500 / 1000 / 2000 tokens: 1022 / 992, 1475 / 1337, 2006 / 1611.  int4, by the average, 128
+  // Copy policy.  int8: a block that shares its weights runs without the hint, one alone with it up to this average (past it up to
+  // 64 tokens).  With the hint / without at 40 / 50 / 62 / 80 slots per expert, us: DeepSeek-V3 share 288 / 298, 301 / 310, 311 / 313,
+  // 325 / 327, with inputs not seen before 50: 294 / 306, 62: 311 / 332; the full layer's skewed routing, where the average
+  // misleads, at 500 / 1000 / 2000 tokens: 1022 / 992, 1475 / 1337, 2006 / 1611.  int4, by the average, 128
   // experts of 4096 x 1536: per-channel at 16 / 32 / 44 / 62 slots 251 / 258, 270 / 271, 285 / 283, 306 / 303; K-group scales
   // (from 48 slots on) at 50 / 62: 340 / 334, 361 / 357.
   a.stream = a.num_valid <= experts * (a.w4 ? 40 : kT / 2);
