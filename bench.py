@@ -460,12 +460,13 @@ def main():
     flush = Flusher(dev, args.flush)
     order_flag = {"contract": 0, "separate": _lib.LO_GEMM_SEPARATE_ORDER, "fused": _lib.LO_GEMM_FUSED_SCALE}
     flags_default = order_flag[args.scale_order]
-    # Vector instructions the fold spends per accumulator element and K block, and the rate the matrix pipe
+    # Vector instructions the fold spends per accumulator element and K block in the direct-to-LDS kernels
+    # (default order: 2, without a conversion; the register-fed kernels spend 3), and the rate the matrix pipe
     # reaches at best under that load: measured live with a loop of nothing but int8 MFMAs, each followed by
     # its share of the fold (two elements per v_mfma_i32_16x16x64_i8) as independent v_fma_f32, two waves per
     # SIMD, on random operand bytes (the clock this chip holds depends on how many operand bits toggle; the
     # same loop on zeros and the MFMAs alone are reported next to it).
-    fold_insts = {"contract": 3, "separate": 4, "fused": 2}[args.scale_order]
+    fold_insts = {"contract": 2, "separate": 4, "fused": 2}[args.scale_order]
 
     def issue_rate(valu_per_mfma, random_operands):
         out = ctypes.c_double(0.0)

@@ -31,7 +31,7 @@ struct GemmArgs {
   int32_t skip_nonlocal; // blocks of expert -1: leave the output rows untouched
   int32_t w4;            // W is packed int4 (load-time layout), Ws is [E, K/128, N]
   int32_t per_channel;   // As is [a_rows], Ws is [E, N]: scales applied once, after the whole-K int32 sum
-  int32_t stream;        // 128-token tiles: experts have about one token block
+  int32_t stream;        // 64- and 128-token tiles: experts have about one token block
   int32_t coarse_fill;   // 160-token tiles: round the token fragments in use up to 8
   int32_t out_f16;       // C holds IEEE half instead of bf16; fused: the values between the stages are rounded to half
   int32_t out_f32;       // C holds the fp32 sums themselves (block form, weight-streaming kernel only)
@@ -155,7 +155,8 @@ __device__ __forceinline__ void with_out16(int f16, Body body) {
 // Order of the scale arithmetic per 128-wide K block (d = the block's exact int32 sum):
 //   kOrdContract   acc = fma(f32(d) * a_s, b_s, acc)    the default: what the reference's Triton line
 //                  `accumulator += tl.dot(a, b) * a_scale * b_scale` (int8.py:499-508) compiles to with
-//                  the AMD backend's default enable_fp_fusion; three vector instructions per element
+//                  the AMD backend's default enable_fp_fusion; three vector instructions per element,
+//                  two in the kernels that fold without a conversion (fold_biased)
 //   kOrdSeparate   acc = acc + (f32(d) * a_s) * b_s     the same line without fp fusion; four instructions
 //                  (LO_GEMM_SEPARATE_ORDER)
 //   kOrdFusedScale acc = fma(f32(d), a_s * b_s, acc)    two instructions, last-ulp differences in fp32

@@ -6,8 +6,8 @@
 // walks several 256-row weight tiles with them: the K loop needs no barrier, no LDS
 // write and no token reload, the weight prefetch (two K blocks deep) runs on across tile boundaries, and the
 // gather of sorted_token_ids is paid once per token block instead of once per tile.
-// Each wave owns 64 rows x 64 tokens as 4 x 4 fragments of v_mfma_i32_16x16x64_i8 (weights as the A operand); reference: Triton fused_moe_kernel, python/lightop/_lmslim_native/
-// layers/fused_moe/int8.py:485-541.
+// Each wave owns 64 rows x 64 tokens as 4 x 4 fragments of v_mfma_i32_16x16x64_i8 (weights as the A operand);
+// reference: Triton fused_moe_kernel, python/lightop/_lmslim_native/layers/fused_moe/int8.py:485-541.
 #include <type_traits>
 
 #include "gemm.h"
