@@ -109,6 +109,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // second half is read from LDS in mid K block, so the weights have two stages, in the room that 8-bit ones take; the row
   // scales' are in the amax exchange of the epilogue.  Qwen3-235B-A22B-shaped layer, 2048 tokens: 592 us in 128-token blocks, 516.
   constexpr bool kHalves = W4 && !PC && NTB == 10;
+  // So the waves have to meet between the K loop and that epilogue: until then a slower one reads its row scales, and copies of
+  // scales past the last K block land.  (The default order meets before it looks at the flags.)
+  constexpr bool kMeet = kHalves && FUSED_ACT;
 
   int mb, nt;
   if (!tile_of(blockIdx.x, a.n_tiles, m_blocks, group_m, mb, nt)) return;
@@ -733,6 +736,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   }
   wait_copies<0>(); // no copy may still be writing LDS when the epilogue reuses it or the wave ends
   derive();
+  if constexpr (kMeet && !kBiased) __syncthreads();
   if constexpr (kBiased) {
     // (the flags of the last token scales were written a barrier of the K loop ago)
     if constexpr (W4) {
@@ -757,6 +761,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
       k_loop(plain, std::integral_constant<int, 2 * NTB>{}, by_launch);
       wait_copies<0>();
       derive();
+      if constexpr (kMeet) __syncthreads();
     }
   }
   if constexpr (!FUSED_ACT) {
