@@ -309,7 +309,8 @@ int lo_preshuffle_weight_int8(const int8_t *src, int8_t *dst, int32_t E, int64_t
 typedef struct lo_moe_tile {
   int32_t block_size_m; /* 16, 32, 64, 128 or 160 (160: weights in the load-time layout; in the block form
                          * bf16 rows with SiLU keep the fused first stage, fp16 rows and GELU take the plain
-                         * stage followed by lo_act_mul_group_quant) */
+                         * stage followed by lo_act_mul_group_quant; every size the table names is accepted from
+                         * a caller with the same arguments) */
   int32_t kernel;       /* LO_KERNEL_*: the kernel the stage entry points launch for this problem */
   int32_t waves;        /* wavefronts per workgroup of that kernel */
   int32_t block_n;      /* weight rows per workgroup of that kernel */
@@ -387,10 +388,11 @@ int lo_measure_mfma_issue_rate(int valu_per_mfma, int random_operands, int iters
  *   workspace: lo_fused_experts_workspace_bytes(...) bytes of device memory, 256-byte aligned
  *   block_size_m: 0 = take it from the tile table (lo_fused_experts_workspace_bytes(.., 0) is
  *   large enough for whatever the table picks and for every explicit block size); 16, 32, 64, 128,
- *   or 160 (int8 weights in the load-time layout: 160-token blocks of the direct-to-LDS kernel - what
+ *   or 160 (weights in the load-time layout: 160-token blocks of the direct-to-LDS kernel - what
  *   the table picks where they hold an expert's tokens in one block less, 128-token ones spilling into another
- *   pass over the expert's weights; with fp16 rows or GELU the first GEMM is not fused with the
- *   activation, cache3 also receives its output [M*top_k, 2I], and 2I <= H is required)
+ *   pass over the expert's weights; int4 weights (LO_GEMM_W4) with bf16 rows and SiLU; with fp16 rows or GELU
+ *   and int8 weights the first GEMM is not fused with the activation, cache3 also receives its output
+ *   [M*top_k, 2I], and 2I <= H is required)
  */
 int64_t lo_fused_experts_workspace_bytes(int64_t M, int32_t top_k, int64_t H, int64_t I,
                                          int32_t num_experts, int32_t block_size_m);

@@ -4,7 +4,7 @@
                                [--out DIR] [--steps N]
 
 For every token count the whole path is timed with each token-block size the kernels
-offer (16, 32: weight-streaming; 64, 128: LDS-tiled), caches flushed between calls.  The
+offer (16, 32: weight-streaming; 64, 128, 160: LDS-tiled), caches flushed between calls.  The
 report shows the best size per token count next to what the compiled-in table
 (``pick_block_m`` in csrc/api.hip, ``lo_moe_tile_query``) picks and how much slower that pick
 is, so the table's thresholds (slots per expert at which the next larger block takes over) can be
@@ -26,7 +26,15 @@ import sys
 
 import torch
 
-BLOCK_SIZES = (16, 32, 64, 128)
+BLOCK_SIZES = (16, 32, 64, 128, 160)
+
+
+def block_sizes(form, flags, E, E_global, top_k, H, I):
+    """The sizes that the whole-path call takes for a layer: 160-token blocks have limits of their own."""
+    from lightop_amd import _lib
+
+    return [bs for bs in BLOCK_SIZES if not _lib.lib().lo_moe_tile_query_path(form, flags, _lib.LO_BF16, bs, 1, E, E_global, top_k, H, I,
+                                                                             None, None)]
 
 
 def time_ms(fn, steps, flush):
@@ -105,10 +113,9 @@ def main(argv=None):
 
     rows, table = [], {}
     print(f"{layer.name}: E={layer.E}/{layer.E_global} top{layer.top_k} H={layer.H} I={layer.I}")
-    # 160-token blocks exist for the block form with int8 weights (bf16 rows with SiLU keep the fused first stage)
-    # and for per-channel scales
-    has160 = (layer.weight_bits == 8 and block_shape is not None) or block_shape is None
-    sizes = BLOCK_SIZES + ((160,) if has160 else ())
+    form = _lib.LO_FORM_CHANNEL if block_shape is None else _lib.LO_FORM_W4 if layer.weight_bits == 4 else _lib.LO_FORM_BLOCK
+    flags = _lib.LO_GEMM_W_PRESHUFFLED | (_lib.LO_GEMM_W4 if layer.weight_bits == 4 else 0)
+    sizes = block_sizes(form, flags, layer.E, layer.E_global, layer.top_k, layer.H, layer.I)
     print(f"{'tokens':>7} {'slots/expert':>12} | " + " ".join(f"bs={b:<4}" for b in sizes) + " | best  table  loss")
     for M in (int(v) for v in args.tokens.split(",")):
         x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, M, seed=1))

@@ -322,3 +322,37 @@ def test_blocks_of_160_where_they_save_a_block(lib):
             M = n * (shape[1] // shape[2])
             assert lib.lo_moe_tile_query_form(form, flags, M, *shape, t1, t2) == 0
             assert t1.block_size_m == want, (form, flags, shape, n)
+
+
+def test_every_size_the_table_names_is_taken_back(lib):
+    """A caller that asks the table and passes the answer gets the launches that the table described; the tuner, whose files are
+    read back that way, times every such size."""
+    from lightop_amd import _lib, tune
+
+    t1, t2, u1, u2 = (_lib.LoMoeTile() for _ in range(4))
+    pre = _lib.LO_GEMM_W_PRESHUFFLED
+    forms = ((_lib.LO_FORM_BLOCK, 0), (_lib.LO_FORM_BLOCK, pre), (_lib.LO_FORM_W4, 0), (_lib.LO_FORM_CHANNEL, 0),
+             (_lib.LO_FORM_CHANNEL, pre), (_lib.LO_FORM_CHANNEL, pre | _lib.LO_GEMM_W4))
+    named = set()
+    for shape in ((128, 128, 8, 2048, 768), (128, 128, 8, 4096, 1536), (32, 256, 8, 7168, 2048), (8, 8, 2, 1024, 512),
+                  (64, 64, 6, 2048, 1408), (4, 4, 2, 16384, 1024), (4, 4, 2, 16512, 1024), (4, 4, 2, 1024, 16512)):
+        for form, layout in forms:
+            for extra in (0, _lib.LO_GEMM_FORCE_STREAMING, _lib.LO_FUSED_ACT_GELU, _lib.LO_GEMM_SEPARATE_ORDER):
+                for dtype in (_lib.LO_BF16, _lib.LO_F16, _lib.LO_F32):
+                    flags = layout | extra | _lib.LO_FUSED_NO_DECODE_PATH
+                    for slots in (1, 7, 30, 60, 90, 108, 120, 128, 150, 170, 270, 420, 600):
+                        case = (form, flags, dtype, slots, shape)
+                        M = max(1, slots * shape[1] // shape[2])
+                        assert lib.lo_moe_tile_query_path(form, flags, dtype, 0, M, *shape, t1, t2) == 0, case
+                        assert lib.lo_moe_tile_query_path(form, flags, dtype, t1.block_size_m, M, *shape, u1, u2) == 0, case
+                        for t, u in ((t1, u1), (t2, u2)):
+                            assert all(getattr(t, f) == getattr(u, f) for f, _ in t._fields_), case
+                        named.add((form, layout, t1.block_size_m))
+                        if layout and not extra and dtype == _lib.LO_BF16:  # (the tuner's weights are in the load-time layout)
+                            assert t1.block_size_m in tune.block_sizes(form, layout, *shape), case
+    assert {f for f, _, bs in named if bs == 160} == {_lib.LO_FORM_BLOCK, _lib.LO_FORM_W4, _lib.LO_FORM_CHANNEL}
+    # int4 weights with K-group scales: where the table may name 160, and nowhere else
+    w4 = (_lib.LO_FORM_W4, 0, _lib.LO_BF16, 160, 64, 128, 128, 8, 4096, 1536, t1, t2)
+    assert lib.lo_moe_tile_query_path(*w4) == 0 and t1.kernel == _lib.LO_KERNEL_T128 == t2.kernel
+    for i, bad in ((1, _lib.LO_GEMM_FORCE_STREAMING), (1, _lib.LO_FUSED_ACT_GELU), (2, _lib.LO_F16), (8, 16512), (9, 16512)):
+        assert lib.lo_moe_tile_query_path(*w4[:i], bad, *w4[i + 1:]) < 0

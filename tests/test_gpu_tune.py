@@ -19,7 +19,8 @@ def test_tuner_writes_the_reference_layout(tmp_path, capsys, workload, prefix):
 
     print(f"[case] tuner {workload}", flush=True)
     layer = wl.LAYERS[workload]
-    assert tune.main(["--workload", workload, "--tokens", "4,96", "--steps", "2", "--out", str(tmp_path)]) == 0
+    # (512 tokens: 128 slots per expert, where the table names 160-token blocks in either form)
+    assert tune.main(["--workload", workload, "--tokens", "4,96,512", "--steps", "2", "--out", str(tmp_path)]) == 0
     text = capsys.readouterr().out
     assert "largest loss of the compiled-in table" in text
     files = os.listdir(tmp_path)
@@ -29,7 +30,7 @@ def test_tuner_writes_the_reference_layout(tmp_path, capsys, workload, prefix):
     data = json.load(open(tmp_path / name))
     # the reader's flattening (w8a8_get_cache_json.py:166-171)
     flat = {f"{m}_{shape}": cfg for shape, per_m in data.items() for m, cfg in per_m.items()}
-    for m in (4, 96):
+    for m in (4, 96, 512):
         cfg = flat[f"{m}_{2 * layer.I}_{layer.H}_{layer.I}"]
         for part in ("config1", "config2"):
             assert cfg[part]["BLOCK_SIZE_M"] in (16, 32, 64, 128, 160)  # whichever was fastest in this run

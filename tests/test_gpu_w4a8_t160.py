@@ -7,7 +7,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def run(oracle, H, I, ids, E, Eg=None, flags=0, factor=1.0, scale=1.0):
+def run(oracle, H, I, ids, E, Eg=None, flags=0, factor=1.0, scale=1.0, dtype=torch.bfloat16, named=True, **kw):
     from lightop_amd import _lib, workloads as wl
     from lightop_amd.moe import fused_experts_impl_w4a8, preshuffle_moe_scale_int4, preshuffle_moe_weight_int4
 
@@ -16,18 +16,20 @@ def run(oracle, H, I, ids, E, Eg=None, flags=0, factor=1.0, scale=1.0):
     layer = wl.MoeLayer("w4-160", E=E, E_global=Eg or E, top_k=k, H=H, I=I, routing="softmax", weight_bits=4)
     t1, t2 = _lib.LoMoeTile(), _lib.LoMoeTile()
     assert _lib.lib().lo_moe_tile_query_path(_lib.LO_FORM_W4, flags, _lib.LO_BF16, 0, M, E, layer.E_global, k, H, I, t1, t2) == 0
-    assert t1.block_size_m == 160 == t2.block_size_m and t1.kernel == _lib.LO_KERNEL_T128 == t2.kernel
+    if named:
+        assert t1.block_size_m == 160 == t2.block_size_m and t1.kernel == _lib.LO_KERNEL_T128 == t2.kernel
     w1, w2, w1s, w2s = wl.make_weights(layer, seed=M)
     x, tw, _ = wl.make_inputs(layer, M, seed=M)
     x[::7] *= scale
+    x = x.to(dtype)
     w1s = w1s / scale
     emap = wl.expert_map_for(layer)
-    cache13 = torch.empty(M * k * max(2 * I, H), dtype=torch.bfloat16, device=dev)
+    cache13 = torch.empty(M * k * max(2 * I, H), dtype=dtype, device=dev)
     out = fused_experts_impl_w4a8(x.to(dev), preshuffle_moe_weight_int4(w1.to(dev)), preshuffle_moe_weight_int4(w2.to(dev)),
                                   tw.to(dev), ids.to(dev), cache13, global_num_experts=layer.E_global,
                                   expert_map=None if emap is None else emap.to(dev),
                                   w1_scale=preshuffle_moe_scale_int4(w1s.to(dev)), w2_scale=preshuffle_moe_scale_int4(w2s.to(dev)),
-                                  block_shape=[1, 128], routed_scaling_factor=factor, lightop_amd_flags=flags)
+                                  block_shape=[1, 128], routed_scaling_factor=factor, lightop_amd_flags=flags, **kw)
     torch.cuda.synchronize()
     with oracle.scale_order("separate" if flags & _lib.LO_GEMM_SEPARATE_ORDER else "contract"):
         ref = oracle.fused_experts_w4a8(x, w1, w2, w1s, w2s, tw, ids, 16, global_num_experts=layer.E_global, expert_map=emap,
@@ -64,6 +66,35 @@ def test_forms(oracle, what):
         err, ref = (out.float() - ref.float()).abs(), ref.float().abs()  # by a step of 1 / 127 of their group's largest: bounds of the path
         assert err.max() <= 1e-2 * ref.max() and err.sum() <= 2e-3 * ref.sum()
         return
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens", [9, 240, 700])
+def test_as_the_caller_asks(oracle, tokens):
+    """At sizes where the table names other blocks as well."""
+    print(f"[case] int4 160-token blocks on request, {tokens} tokens", flush=True)
+    ids = torch.randint(0, 2, (tokens, 1), generator=torch.Generator().manual_seed(tokens), dtype=torch.int32)
+    out, ref = run(oracle, 384, 256, ids, 2, named=False, lightop_amd_block_size_m=160)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_from_a_tuning_file(oracle, monkeypatch, tmp_path, dtype):
+    """A file's 160 is taken by a call that can, and left to the table by one that cannot."""
+    import json
+
+    from lightop_amd.moe import tile_files
+
+    print(f"[case] int4 160-token blocks from a file, {dtype}", flush=True)
+    cfg = {"BLOCK_SIZE_M": 160}
+    with open(tmp_path / tile_files.file_name(2, 512, 384, 256, 1, [1, 128], True), "w") as f:
+        json.dump({"512_384_256": {"64": {"config1": cfg, "config2": cfg}}}, f)
+    monkeypatch.setenv("TRITON_JSON_DIR", str(tmp_path))
+    tile_files.forget()
+    ids = torch.randint(0, 2, (100, 1), generator=torch.Generator().manual_seed(3), dtype=torch.int32)
+    assert tile_files.block_size_m(100, 2, 512, 384, 256, 1, [1, 128], int4=True) == 160
+    out, ref = run(oracle, 384, 256, ids, 2, dtype=dtype, named=False)
+    tile_files.forget()
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
