@@ -447,7 +447,7 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
   auto kblock_halves = [&](auto BIASED, auto NST, auto ONCE, int kb) __attribute__((always_inline)) {
     constexpr int nst_c = decltype(NST)::value, nf = nst_c / 2; // a stage: one token fragment, two row fragments
     constexpr int c0 = decltype(BIASED)::value ? kFoldBias : 0;
-    constexpr int kCopies = 5 + APW, per = nst_c > 12 ? 1 : 2; // copies a stage: spread out, they stand in nobody's way
+    constexpr int kCopies = 5 + APW, per = nst_c > 12 ? 1 : nst_c > 4 ? 2 : 3; // copies a stage: spread out, they stand in nobody's way
     const v4i cinit = {c0, c0, c0, c0};
     const int off0 = (kb & 1) * AST + alds[0];
     const int8_t *const ta[2] = {sA + off0, sA + (off0 ^ 64)}; // (the other k-half, computed here: a register less through the loop)
@@ -713,7 +713,10 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     if (nst > 16) k_loop(biased, std::integral_constant<int, 20>{}, by_launch);
     else if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
     else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
-    else k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
+    else if (!kHalves || nst > 4) k_loop(biased, std::integral_constant<int, 8>{}, by_launch);
+    // int4: skewed routing leaves many experts with a handful of tokens (128 experts of 4096 x 1536, Zipf 1.2, us, without / with
+    // this variant: 1800 tokens 601 / 589, 2048: 682 / 672; DeepSeek-V3 share, Zipf 0.6, 4096: 669 / 641)
+    else if constexpr (kHalves) k_loop(biased, std::integral_constant<int, 4>{}, by_launch);
   } else if constexpr (NTB == 8 && W4 && !PC) {
     if (nst > 12) k_loop(biased, std::integral_constant<int, 16>{}, by_launch);
     else if (nst > 8) k_loop(biased, std::integral_constant<int, 12>{}, by_launch);
@@ -1101,8 +1104,13 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
     // and not where skewed routing gives some of many experts several blocks.  With it / without, whole call with its router, us:
     // Qwen3-30B-A3B layer at 96 slots 180 / 185, at 128: 199 / 205, per-channel 201 / 205; 128 experts of 4096 x 1536 at 94 to 128: equal;
     // DeepSeek-V3 share at 94: 361 / 366, at 125: 502 / 481, per-channel 462 / 447; the full layer with Zipf routing at 128: 3096 / 2571;
-    // two blocks an expert, Qwen3-30B-A3B layer at 262: 338 / 301.  int4 weights, half the bytes, with it where an expert has one
-    // block: 128 experts of 4096 x 1536, per-channel at 2048 tokens 422 / 435, at 4300: 745 / 710; K-group scales 521 / 536.
+    // two blocks an expert, Qwen3-30B-A3B layer at 262: 338 / 301.  (The number of experts says nothing about skew: it parts the
+    // layers measured.)  int4 weights, half the bytes, with one scale per row: with it where an expert has one block, 128 experts of
+    // 4096 x 1536 at 2048 tokens 422 / 435, at 4300: 745 / 710.  int4 weights with K-group scales: in the first stage only, whose
+    // weights are twice the second's; there it costs skewed routing, whose busy experts' blocks share them, and gains uniform routing
+    // nothing.  With it in both / the first / neither: the same layer at 1800 / 2048 / 2300 tokens 483 / 484 / 484, 522 / 518 / 540, 586 /
+    // 594 / 600, Zipf 1.2 585 / 573 / 547, 674 / 656 / 627, 683 / 668 / 638; 128 experts of 2048 x 768 at 1800: 192 / 184 / 188, Zipf 1.2
+    // 226 / 216 / 208; DeepSeek-V3 share at 4096: 338 / 342 / 345, Zipf 0.6 635 / 623 / 594.
     a.stream = a.w4 ? slots <= 160.0 : a.E <= 128 && slots < (a.N * a.K <= (8 << 20) ? 160.0 : 112.0);
 #define LO_T160_LAUNCH2(FS, FA, ST, W)                                                                          \
   do {                                                                                                          \
@@ -1114,7 +1122,7 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   } while (0)
 #define LO_T160_LAUNCH(FS, FA)                                                                                  \
   do {                                                                                                          \
-    if (a.w4) LO_T160_LAUNCH2(FS, FA, true, true);                                                              \
+    if (a.w4) LO_T160_LAUNCH2(FS, FA, (FA) != 0, true);                                                         \
     else if (a.stream) LO_T160_LAUNCH2(FS, FA, true, false);                                                    \
     else LO_T160_LAUNCH2(FS, FA, false, false);                                                                 \
   } while (0)

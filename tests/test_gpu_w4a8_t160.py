@@ -37,7 +37,7 @@ def run(oracle, H, I, ids, E, Eg=None, flags=0, factor=1.0, scale=1.0, dtype=tor
     return out.cpu(), ref
 
 
-@pytest.mark.parametrize("count", [1, 64, 65, 96, 97, 127, 128, 129, 144, 145, 159, 160, 161, 225])
+@pytest.mark.parametrize("count", [1, 32, 33, 64, 65, 96, 97, 127, 128, 129, 144, 145, 159, 160, 161, 225])
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 256)])
 def test_fill_levels(oracle, count, H, I):
     print(f"[case] int4 160-token blocks, {count} tokens on expert 0, H={H} I={I}", flush=True)
