@@ -98,7 +98,7 @@ def test_from_a_tuning_file(oracle, monkeypatch, tmp_path, dtype):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
-def test_stages():
+def test_stages(oracle):
     """The stage entry points take the size the tile table names."""
     from lightop_amd import _lib, workloads as wl
     from lightop_amd.moe import (invoke_fused_moe_gemm1_silu_quant, invoke_fused_moe_kernel_int8, moe_align_block_size,
@@ -107,10 +107,16 @@ def test_stages():
 
     dev = torch.device("cuda:0")
     layer = wl.MoeLayer("w4-160", E=3, E_global=3, top_k=2, H=512, I=256, routing="softmax", weight_bits=4)
-    w1, w2, w1s, w2s = (t.to(dev) for t in wl.make_weights(layer, seed=1))
-    x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, 300, seed=1))
+    weights, inputs = wl.make_weights(layer, seed=1), wl.make_inputs(layer, 300, seed=1)
+    w1, w2, w1s, w2s = weights
+    x, tw, ids = inputs
+    rs, re, rp = oracle.moe_align_block_size(ids, 16, 3)
+    aq, asc = oracle.per_token_group_quant_int8(x)
+    rq, rsc = oracle.per_token_group_quant_int8(oracle.silu_and_mul(oracle.moe_gemm_w4a8(aq, asc, w1, w1s, rs, re, rp, tw, False, 2, 600, 16)))
+    rC = oracle.moe_gemm_w4a8(rq, rsc, w2, w2s, rs, re, rp, tw, True, 1, 600, 16)
+    w1, w2, w1s, w2s = (t.to(dev) for t in weights)
+    x, tw, ids = (t.to(dev) for t in inputs)
     xq, xs = per_token_group_quant_int8(x, 128)
-    got = []
     for bs in (160, 128):
         print(f"[case] int4 stages, block {bs}", flush=True)
         s, e, p = moe_align_block_size(ids, bs, 3)
@@ -120,5 +126,5 @@ def test_stages():
         invoke_fused_moe_kernel_int8(q, preshuffle_moe_weight_int4(w2), C, sc, preshuffle_moe_scale_int4(w2s), tw, s, e, p, True, 1,
                                      {"BLOCK_SIZE_M": bs}, flags=_lib.LO_GEMM_W4)
         torch.cuda.synchronize()
-        got.append((q, sc, C.view(torch.int16)))
-    assert all(torch.equal(a, b) for a, b in zip(*got))
+        assert torch.equal(q.cpu(), rq) and torch.equal(sc.cpu(), rsc)
+        assert torch.equal(C.view(600, 512).cpu().view(torch.int16), rC.view(torch.int16))
