@@ -461,9 +461,9 @@ extern "C" int lo_fused_experts_block_int8(
   if (!plan.fused) {
     // rows of slots whose expert another rank holds are neither written by the first GEMM nor read by
     // the activation launch (the slot mask of the alignment says which)
-    rc = launch_gemm_block(a1q, a1s, w1, w1s, cache3, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
+    rc = lo_moe_gemm_block_int8(a1q, a1s, w1, w1s, cache3, dtype, topk_w, sorted, eids, ntpp, L.sorted_cap, S, M, E,
                                 num_experts, 2 * I, H, top_k, block_size_m, apply_router_weight_on_input,
-                                (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), static_cast<hipStream_t>(stream));
+                                (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), stream);
     if (rc) return rc;
     rc = launch_act_mul_group_quant(cache3, dtype, gelu ? LO_ACT_GELU : LO_ACT_SILU, S, I, a2q, a2s, mask,
                                     static_cast<hipStream_t>(stream));
@@ -478,10 +478,10 @@ extern "C" int lo_fused_experts_block_int8(
                                 static_cast<hipStream_t>(stream));
   }
   if (rc) return rc;
-  rc = launch_gemm_block(a2q, a2s, w2, w2s, cache3, dtype, topk_w, sorted, eids, ntpp,
+  rc = lo_moe_gemm_block_int8(a2q, a2s, w2, w2s, cache3, dtype, topk_w, sorted, eids, ntpp,
                               L.sorted_cap, S, S, E, num_experts, H, I, 1, block_size_m,
                               !apply_router_weight_on_input,
-                              (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), static_cast<hipStream_t>(stream));
+                              (flags & ~LO_FUSED_ACT_GELU) | (mask ? LO_GEMM_SKIP_NONLOCAL : 0), stream);
   if (rc) return rc;
   return lo_moe_sum(cache3, out, shared_output, mask, dtype, M, top_k, H, routed_scaling_factor,
                     nullptr, stream);

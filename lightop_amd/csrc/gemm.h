@@ -321,12 +321,6 @@ int launch_gemm_w8a8(const int8_t *A, const float *As, const int8_t *W, const fl
                      const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
                      int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
                      int flags, hipStream_t stream);
-// lo_moe_gemm_block_int8, and 160-token blocks of int4 weights, which the whole path takes where the tile table says so.
-int launch_gemm_block(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype,
-                      const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
-                      const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
-                      int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
-                      int flags, hipStream_t stream);
 // The fused first stage with a given activation (lo_moe_gemm1_silu_quant_block_int8 is this with kActSiluBf16).
 int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
                            int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,

@@ -99,12 +99,14 @@ static int launch_gemm(const GemmArgs &a, bool fused_act, int bs, int flags, int
 
 } // namespace lo
 
-namespace lo {
-int launch_gemm_block(const int8_t *A, const float *As, const int8_t *W, const float *Ws, void *C, int c_dtype,
-                      const float *topk_w, const int32_t *sorted_ids, const int32_t *expert_ids,
-                      const int32_t *num_tokens_post_pad, int64_t sorted_cap, int64_t num_valid, int64_t a_rows, int32_t E,
-                      int32_t num_experts, int64_t N, int64_t K, int32_t top_k, int32_t block_size_m, int mul_routed,
-                      int flags, hipStream_t stream) {
+extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const int8_t *W,
+                                      const float *Ws, void *C, int c_dtype, const float *topk_w,
+                                      const int32_t *sorted_ids, const int32_t *expert_ids,
+                                      const int32_t *num_tokens_post_pad, int64_t sorted_cap,
+                                      int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts,
+                                      int64_t N, int64_t K, int32_t top_k, int32_t block_size_m,
+                                      int mul_routed, int flags, lo_stream_t stream) {
+  using namespace lo;
   int rc = validate_common("moe_gemm", A, As, W, Ws, sorted_ids, expert_ids, num_tokens_post_pad, K,
                            top_k, E, a_rows);
   if (rc) return rc;
@@ -140,9 +142,10 @@ int launch_gemm_block(const int8_t *A, const float *As, const int8_t *W, const f
   const int64_t mblocks = grid_m_blocks(sorted_cap, num_valid, block_size_m);
   LO_REQUIRE(mblocks * a.n_tiles < (1ll << 30), LO_EINVAL, "moe_gemm: grid too large");
   if (mblocks == 0) return LO_OK;
-  return launch_gemm(a, false, block_size_m, flags, mblocks, stream);
+  return launch_gemm(a, false, block_size_m, flags, mblocks, static_cast<hipStream_t>(stream));
 }
 
+namespace lo {
 int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,
                            int fused, bool f16, const uint16_t *act_table, const float *topk_w, const int32_t *sorted_ids,
                            const int32_t *expert_ids, const int32_t *num_tokens_post_pad, int64_t sorted_cap,
@@ -187,19 +190,6 @@ int launch_gemm1_act_quant(const int8_t *A, const float *As, const int8_t *W, co
   return launch_gemm(a, true, block_size_m, flags, mblocks, stream);
 }
 } // namespace lo
-
-extern "C" int lo_moe_gemm_block_int8(const int8_t *A, const float *As, const int8_t *W,
-                                      const float *Ws, void *C, int c_dtype, const float *topk_w,
-                                      const int32_t *sorted_ids, const int32_t *expert_ids,
-                                      const int32_t *num_tokens_post_pad, int64_t sorted_cap,
-                                      int64_t num_valid, int64_t a_rows, int32_t E, int32_t num_experts,
-                                      int64_t N, int64_t K, int32_t top_k, int32_t block_size_m,
-                                      int mul_routed, int flags, lo_stream_t stream) {
-  using namespace lo;
-  return launch_gemm_block(A, As, W, Ws, C, c_dtype, topk_w, sorted_ids, expert_ids, num_tokens_post_pad, sorted_cap, num_valid,
-                           a_rows, E, num_experts, N, K, top_k, block_size_m, mul_routed, flags,
-                           static_cast<hipStream_t>(stream));
-}
 
 extern "C" int lo_moe_gemm1_silu_quant_block_int8(
     const int8_t *A, const float *As, const int8_t *W, const float *Ws, int8_t *A2q, float *A2s,

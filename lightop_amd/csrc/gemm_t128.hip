@@ -1139,10 +1139,9 @@ int launch_gemm_t128(const GemmArgs &a0, bool fused_act, int block_size_m, int f
   }
   // Copy policy.  int8: a block that shares its weights runs without the hint, one alone with it up to this average (past it up to
   // 64 tokens).  With the hint / without at 40 / 50 / 62 / 80 slots per expert, us: DeepSeek-V3 share 288 / 298, 301 / 310, 311 / 313,
-  // 325 / 327, with inputs not seen before 50: 294 / 306, 62: 311 / 332; the full layer's skewed routing, where the average
-  // misleads, at 500 / 1000 / 2000 tokens: 1022 / 992, 1475 / 1337, 2006 / 1611.  int4, by the average, 128
-  // experts of 4096 x 1536: per-channel at 16 / 32 / 44 / 62 slots 251 / 258, 270 / 271, 285 / 283, 306 / 303; K-group scales
-  // (from 48 slots on) at 50 / 62: 340 / 334, 361 / 357.
+  // 325 / 327; the full layer's skewed routing, where the average misleads, at 500 / 1000 / 2000 tokens: 1022 / 992, 1475 / 1337,
+  // 2006 / 1611.  int4 with one scale per row, by the average, 128 experts of 4096 x 1536 at 16 / 32 / 44 / 62 slots: 251 / 258, 270 /
+  // 271, 285 / 283, 306 / 303.  int4 with K-group scales, here from 50 slots per expert on, without it: at 50 / 62 340 / 334, 361 / 357.
   a.stream = a.num_valid <= experts * (a.w4 ? 40 : kT / 2);
   if (a.per_channel) {
     LO_GATED_DISPATCH(a, fused_act, LO_T128_LAUNCH_PC);
