@@ -390,9 +390,9 @@ int lo_measure_mfma_issue_rate(int valu_per_mfma, int random_operands, int iters
  *   large enough for whatever the table picks and for every explicit block size); 16, 32, 64, 128,
  *   or 160 (weights in the load-time layout: 160-token blocks of the direct-to-LDS kernel - what
  *   the table picks where they hold an expert's tokens in one block less, 128-token ones spilling into another
- *   pass over the expert's weights; int4 weights (LO_GEMM_W4) with bf16 rows and SiLU; with fp16 rows or GELU
- *   and int8 weights the first GEMM is not fused with the activation, cache3 also receives its output
- *   [M*top_k, 2I], and 2I <= H is required)
+ *   pass over the expert's weights; int4 weights (LO_GEMM_W4) where the table names it for the same arguments; with
+ *   fp16 rows or GELU and int8 weights the first GEMM is not fused with the activation, cache3 also receives its
+ *   output [M*top_k, 2I], and 2I <= H is required)
  */
 int64_t lo_fused_experts_workspace_bytes(int64_t M, int32_t top_k, int64_t H, int64_t I,
                                          int32_t num_experts, int32_t block_size_m);

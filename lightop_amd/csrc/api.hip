@@ -256,20 +256,19 @@ static int plan_block_path(int dtype, int flags, int64_t M, int32_t num_experts,
   const bool gelu = (flags & LO_FUSED_ACT_GELU) != 0;
   const bool block_size_m_auto = block_size_m == 0;
   // 160: the 160-token form of the direct-to-LDS kernel (load-time layout) for both GEMMs; bf16 rows with SiLU take its fused first
-  // stage, with int8 weights fp16 rows and GELU the plain one and the activation launch.  Whatever the table may pick a caller may ask for.
+  // stage, with int8 weights fp16 rows and GELU the plain one and the activation launch; int4 weights where the table names it.
   const bool silu_bf16 = dtype == LO_BF16 && !gelu;
   const bool table160 = silu_bf16 && blocks_of_160_fit(H, I, true) && !(w4 && (flags & LO_GEMM_FORCE_STREAMING));
   if (block_size_m == 0 && dtype == LO_F32) // fp32 rows go through the weight-streaming kernel at every size
     block_size_m = pick_block_m(M, num_experts, top_k, H, I, LO_FORM_BLOCK, false);
-  if (block_size_m == 0)
-    block_size_m = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false,
-                                table160,
-                                !pre && !(flags & LO_GEMM_FORCE_STREAMING) && H / kGroup <= 128 && I / kGroup <= 128);
-  const bool bs160 = block_size_m == 160 && pre && (w4 ? table160 : dtype != LO_F32 && blocks_of_160_fit(H, I, silu_bf16));
+  const int32_t named = pick_block_m(M, num_experts, top_k, H, I, w4 ? LO_FORM_W4 : LO_FORM_BLOCK, pre, false, table160,
+                                     !pre && !(flags & LO_GEMM_FORCE_STREAMING) && H / kGroup <= 128 && I / kGroup <= 128);
+  if (block_size_m == 0) block_size_m = named;
+  const bool bs160 = block_size_m == 160 && pre && (w4 ? named == 160 : dtype != LO_F32 && blocks_of_160_fit(H, I, silu_bf16));
   LO_REQUIRE(block_size_m == 16 || block_size_m == 32 || block_size_m == 64 || block_size_m == 128 || bs160,
              LO_EINVAL,
              "fused_experts: block_size_m %d is not one of 16, 32, 64, 128 (160: weights in the load-time layout, H and I up to "
-             "16384 and 16-bit rows; with fp16 rows or GELU int8 weights and 2I <= H)", block_size_m);
+             "16384 and 16-bit rows; with fp16 rows or GELU 2I <= H; int4 weights where the tile table names it)", block_size_m);
   plan->flags = flags;
   plan->block_size_m = block_size_m;
   // fp32 rows have no fused epilogue; GELU and fp16 rows have one at some block sizes

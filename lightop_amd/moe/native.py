@@ -52,7 +52,7 @@ def get_w8a8moe_json(m: int, E: int, n1: int, n2: int, k: int, use_int8_w8a8: bo
         flags |= _lib.LO_FUSED_ACT_GELU
     dt = {torch.bfloat16: _lib.LO_BF16, torch.float16: _lib.LO_F16, torch.float32: _lib.LO_F32}[dtype]
     bs_file = tile_files.block_size_m(m, E, n1, n2, k, topk, block_shape, int4=int4 or form == _lib.LO_FORM_W4)
-    if bs_file == 160 and _lib.lib().lo_moe_tile_query_path(form, flags, dt, bs_file, m, E, Eg, topk, n2, k, t1, t2):
+    if form == _lib.LO_FORM_W4 and bs_file == 160 and _lib.lib().lo_moe_tile_query_path(form, flags, dt, bs_file, m, E, Eg, topk, n2, k, t1, t2):
         bs_file = 0  # as in the call (_run_fused_experts)
     _lib.check(_lib.lib().lo_moe_tile_query_path(form, flags, dt, bs_file, m, E, Eg, topk, n2, k, t1, t2))
 
@@ -697,7 +697,11 @@ def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, i
     use_files = block_size_m == 0 and tile_files.json_dir() is not None
     w4 = bool(flags & _lib.LO_GEMM_W4)
     file_shape = None if channel else ([1, 128] if w4 else [128, 128])
-    form = _lib.LO_FORM_CHANNEL if channel else _lib.LO_FORM_W4 if w4 else _lib.LO_FORM_BLOCK
+    # K-group int4 weights take 160-token blocks where the tile table names them.  A tuning file names neither the element type nor the
+    # activation and is read for token counts beside its own, and a chunk has fewer tokens than the call: the table's pick there.
+    offered = lambda m: not lib.lo_moe_tile_query_path(_lib.LO_FORM_W4, flags, _act_dtype(hidden_states), 160, m, E, global_num_experts,
+                                                       top_k_num, H, I, None, None)
+    left_to_table = w4 and not channel and (use_files or (num_tokens > CHUNK_SIZE and block_size_m == 160 and offered(num_tokens)))
     with _on_device(hidden_states):
         stream = ctypes_void(stream_handle)
         for chunk in range((num_tokens // CHUNK_SIZE) + 1):
@@ -708,10 +712,7 @@ def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, i
             x = hidden_states[begin:end]
             if use_files:  # a tuning file under TRITON_JSON_DIR wins over the compiled-in table
                 block_size_m = tile_files.block_size_m(m, E, 2 * I, H, I, top_k_num, file_shape, int4=w4)
-                # (files name no element type, activation or weight layout, which 160-token blocks depend on: the table's pick then)
-                if block_size_m == 160 and lib.lo_moe_tile_query_path(form, flags, _act_dtype(x), block_size_m, m, E, global_num_experts,
-                                                                      top_k_num, H, I, None, None):
-                    block_size_m = 0
+            chunk_size_m = 0 if block_size_m == 160 and left_to_table and not offered(m) else block_size_m
             if prequant is not None:  # the chunk's rows of the caller's quantised input
                 entry = lib.lo_fused_experts_channel_int8_prequant
                 head = (_lib.ptr(prequant[0][begin:end]), _lib.ptr(prequant[1].reshape(-1)[begin:end]))
@@ -725,7 +726,7 @@ def _run_fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, cache13, i
                 _lib.ptr(expert_map), 1 if apply_router_weight_on_input else 0,
                 float(routed_scaling_factor), _lib.ptr(None if shared_output is None else shared_output[begin:end]),
                 _lib.ptr(cache13), _lib.ptr(out_hidden_states[begin:end]),
-                ctypes_void(ws_ptr), ws_avail, block_size_m, flags, stream))
+                ctypes_void(ws_ptr), ws_avail, chunk_size_m, flags, stream))
     return out_hidden_states
 
 

@@ -29,11 +29,11 @@ import torch
 BLOCK_SIZES = (16, 32, 64, 128, 160)
 
 
-def block_sizes(form, flags, E, E_global, top_k, H, I):
-    """The sizes that the whole-path call takes for a layer: 160-token blocks have limits of their own."""
+def block_sizes(form, flags, M, E, E_global, top_k, H, I):
+    """The sizes that the whole-path call takes for a problem: 160-token blocks have limits of their own."""
     from lightop_amd import _lib
 
-    return [bs for bs in BLOCK_SIZES if not _lib.lib().lo_moe_tile_query_path(form, flags, _lib.LO_BF16, bs, 1, E, E_global, top_k, H, I,
+    return [bs for bs in BLOCK_SIZES if not _lib.lib().lo_moe_tile_query_path(form, flags, _lib.LO_BF16, bs, M, E, E_global, top_k, H, I,
                                                                              None, None)]
 
 
@@ -115,13 +115,12 @@ def main(argv=None):
     print(f"{layer.name}: E={layer.E}/{layer.E_global} top{layer.top_k} H={layer.H} I={layer.I}")
     form = _lib.LO_FORM_CHANNEL if block_shape is None else _lib.LO_FORM_W4 if layer.weight_bits == 4 else _lib.LO_FORM_BLOCK
     flags = _lib.LO_GEMM_W_PRESHUFFLED | (_lib.LO_GEMM_W4 if layer.weight_bits == 4 else 0)
-    sizes = block_sizes(form, flags, layer.E, layer.E_global, layer.top_k, layer.H, layer.I)
-    print(f"{'tokens':>7} {'slots/expert':>12} | " + " ".join(f"bs={b:<4}" for b in sizes) + " | best  table  loss")
+    print(f"{'tokens':>7} {'slots/expert':>12} | " + " ".join(f"bs={b:<4}" for b in BLOCK_SIZES) + " | best  table  loss")
     for M in (int(v) for v in args.tokens.split(",")):
         x, tw, ids = (t.to(dev) for t in wl.make_inputs(layer, M, seed=1))
         cache13 = torch.empty(M * layer.top_k * max(2 * layer.I, layer.H), dtype=torch.bfloat16, device=dev)
         ms = {}
-        for bs in sizes:
+        for bs in block_sizes(form, flags, M, layer.E, layer.E_global, layer.top_k, layer.H, layer.I):
             ms[bs] = time_ms(lambda: run(x, tw, ids, cache13, bs), args.steps, flush)
         best = min(ms, key=ms.get)
         c1, c2 = get_w8a8moe_json(M, layer.E, 2 * layer.I, layer.H, layer.I, True, block_shape, layer.top_k,
@@ -133,7 +132,7 @@ def main(argv=None):
         ms_pick = time_ms(lambda: run(x, tw, ids, cache13, 0), args.steps, flush) if two_launch else ms[pick]
         loss = ms_pick / min(ms[best], ms_pick) - 1.0
         rows.append((M, best, pick, loss))
-        print(f"{M:>7} {M * layer.top_k / layer.E_global:>12.1f} | " + " ".join(f"{ms[b]*1e3:7.1f}" for b in sizes)
+        print(f"{M:>7} {M * layer.top_k / layer.E_global:>12.1f} | " + " ".join(f"{ms[b]*1e3:7.1f}" if b in ms else f"{'-':>7}" for b in BLOCK_SIZES)
               + f" | {best:>4}  {pick:>5}  {loss*100:4.1f}%   (us)"
               + (f"   two-launch path {ms_pick*1e3:.1f}" if two_launch else ""), flush=True)
         tile = dict(c1, BLOCK_SIZE_M=best), dict(c2, BLOCK_SIZE_M=best)

@@ -349,10 +349,11 @@ def test_every_size_the_table_names_is_taken_back(lib):
                             assert all(getattr(t, f) == getattr(u, f) for f, _ in t._fields_), case
                         named.add((form, layout, t1.block_size_m))
                         if layout and not extra and dtype == _lib.LO_BF16:  # (the tuner's weights are in the load-time layout)
-                            assert t1.block_size_m in tune.block_sizes(form, layout, *shape), case
+                            assert t1.block_size_m in tune.block_sizes(form, layout, M, *shape), case
     assert {f for f, _, bs in named if bs == 160} == {_lib.LO_FORM_BLOCK, _lib.LO_FORM_W4, _lib.LO_FORM_CHANNEL}
-    # int4 weights with K-group scales: where the table may name 160, and nowhere else
-    w4 = (_lib.LO_FORM_W4, 0, _lib.LO_BF16, 160, 64, 128, 128, 8, 4096, 1536, t1, t2)
+    # int4 weights with K-group scales: where the table names 160, and nowhere else
+    w4 = (_lib.LO_FORM_W4, 0, _lib.LO_BF16, 160, 2048, 128, 128, 8, 4096, 1536, t1, t2)
     assert lib.lo_moe_tile_query_path(*w4) == 0 and t1.kernel == _lib.LO_KERNEL_T128 == t2.kernel
-    for i, bad in ((1, _lib.LO_GEMM_FORCE_STREAMING), (1, _lib.LO_FUSED_ACT_GELU), (2, _lib.LO_F16), (8, 16512), (9, 16512)):
+    for i, bad in ((1, _lib.LO_GEMM_FORCE_STREAMING), (1, _lib.LO_FUSED_ACT_GELU), (2, _lib.LO_F16), (4, 64), (4, 8192), (8, 16512),
+                   (9, 16512)):
         assert lib.lo_moe_tile_query_path(*w4[:i], bad, *w4[i + 1:]) < 0

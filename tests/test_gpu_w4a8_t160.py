@@ -71,28 +71,42 @@ def test_forms(oracle, what):
 
 @pytest.mark.parametrize("tokens", [9, 240, 700])
 def test_as_the_caller_asks(oracle, tokens):
-    """At sizes where the table names other blocks as well."""
+    """Taken where the table names it, refused beside."""
     print(f"[case] int4 160-token blocks on request, {tokens} tokens", flush=True)
     ids = torch.randint(0, 2, (tokens, 1), generator=torch.Generator().manual_seed(tokens), dtype=torch.int32)
-    out, ref = run(oracle, 384, 256, ids, 2, named=False, lightop_amd_block_size_m=160)
+    if tokens != 240:
+        with pytest.raises(RuntimeError, match="block_size_m 160"):
+            run(oracle, 384, 256, ids, 2, named=False, lightop_amd_block_size_m=160)
+        return
+    out, ref = run(oracle, 384, 256, ids, 2, lightop_amd_block_size_m=160)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
+def test_in_chunks(oracle, monkeypatch):
+    """A call that the table names 160 for, cut into chunks that it names other sizes for."""
+    print("[case] int4 160-token blocks on request, two chunks", flush=True)
+    ids = torch.randint(0, 2, (240, 1), generator=torch.Generator().manual_seed(6), dtype=torch.int32)
+    monkeypatch.setenv("LMSLIM_FUSED_MOE_CHUNK_SIZE", "200")
+    out, ref = run(oracle, 384, 256, ids, 2, lightop_amd_block_size_m=160)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens", [100, 240])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_from_a_tuning_file(oracle, monkeypatch, tmp_path, dtype):
+def test_from_a_tuning_file(oracle, monkeypatch, tmp_path, dtype, tokens):
     """A file's 160 is taken by a call that can, and left to the table by one that cannot."""
     import json
 
     from lightop_amd.moe import tile_files
 
-    print(f"[case] int4 160-token blocks from a file, {dtype}", flush=True)
+    print(f"[case] int4 160-token blocks from a file, {dtype}, {tokens} tokens", flush=True)
     cfg = {"BLOCK_SIZE_M": 160}
     with open(tmp_path / tile_files.file_name(2, 512, 384, 256, 1, [1, 128], True), "w") as f:
         json.dump({"512_384_256": {"64": {"config1": cfg, "config2": cfg}}}, f)
     monkeypatch.setenv("TRITON_JSON_DIR", str(tmp_path))
     tile_files.forget()
-    ids = torch.randint(0, 2, (100, 1), generator=torch.Generator().manual_seed(3), dtype=torch.int32)
-    assert tile_files.block_size_m(100, 2, 512, 384, 256, 1, [1, 128], int4=True) == 160
+    ids = torch.randint(0, 2, (tokens, 1), generator=torch.Generator().manual_seed(3), dtype=torch.int32)
+    assert tile_files.block_size_m(tokens, 2, 512, 384, 256, 1, [1, 128], int4=True) == 160
     out, ref = run(oracle, 384, 256, ids, 2, dtype=dtype, named=False)
     tile_files.forget()
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))

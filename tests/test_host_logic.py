@@ -404,13 +404,13 @@ def test_tuning_files_override_the_compiled_table(monkeypatch, tmp_path):
     assert tile_files.file_name(8, 1024, 1024, 512, 2, None, False).startswith("MOE_W8A8INT8_E=8_")
     assert tile_files.file_name(8, 1024, 1024, 512, 2, [1, 128], True).startswith("MOE_W4A8INT8[1,128]_E=8_")
     assert tile_files.file_name(8, 1024, 1024, 512, 2, None, True).startswith("MOE_W4A8INT8_E=8_")
-    # 160-token blocks: a file's entry is used where the call can take it, and left to the table where it cannot
+    # 160-token blocks of int4 weights: a file's entry is used where the call can take it, and left to the table where it cannot
     name = tile_files.file_name(E, 2 * I, H, I, k, [1, 128], True)
     with open(tmp_path / name, "w") as f:
-        json.dump({f"{2 * I}_{H}_{I}": {"4096": {"config1": cfg(160), "config2": cfg(160)}}}, f)
-    w4 = lambda **kw: moe.get_w8a8moe_json(4096, E, 2 * I, H, I, True, [1, 128], k, int4=True, **kw)[0]
+        json.dump({f"{2 * I}_{H}_{I}": {"1900": {"config1": cfg(160), "config2": cfg(160)}}}, f)
+    w4 = lambda m=1900, **kw: moe.get_w8a8moe_json(m, E, 2 * I, H, I, True, [1, 128], k, int4=True, **kw)[0]
     assert (w4()["BLOCK_SIZE_M"], w4()["kernel"], w4()["source"]) == (160, _lib.LO_KERNEL_T128, "file")
-    for kw in ({"dtype": torch.float16}, {"activation": "gelu"}):
+    for kw in ({"dtype": torch.float16}, {"activation": "gelu"}, {"m": 2500}):
         assert (w4(**kw)["BLOCK_SIZE_M"], w4(**kw)["source"]) == (128, "compiled")
     monkeypatch.delenv("TRITON_JSON_DIR")
     tile_files.forget()
