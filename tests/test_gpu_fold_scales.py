@@ -106,7 +106,7 @@ def test_fused(oracle, bs, form, scale):
 
 
 @pytest.mark.parametrize("name", ["as drawn", "token too large", "weight too large", "both ends"])
-@pytest.mark.parametrize("bs,K", [(64, 768), (128, 768), (64, 256)])
+@pytest.mark.parametrize("bs,K", [(64, 768), (128, 768), (64, 256), (128, 1024)])
 def test_activation_stationary(oracle, bs, K, name):
     """Several weight tiles a workgroup, the last of them 64 rows wide, with the number of K blocks known to the compiler and not."""
     from lightop_amd.moe import invoke_fused_moe_kernel_int8, moe_align_block_size, preshuffle_moe_weight
