@@ -223,13 +223,50 @@ __device__ __forceinline__ uint32_t pack4_i8(int a, int b, int c, int d) {
          __builtin_amdgcn_perm(static_cast<uint32_t>(d), static_cast<uint32_t>(c), 0x04000c0cu);
 }
 
-// four elements of one row -> four packed int8; y = 1.0f / s
+// four elements of one row -> four packed int8; y = 1.0f / s (fp32 rows)
 __device__ __forceinline__ uint32_t quant4(const float *v, float s, float y) {
   if (s < __builtin_inff()) {
     return pack4_i8(quant_one_rcp(v[0], s, y), quant_one_rcp(v[1], s, y), quant_one_rcp(v[2], s, y),
                     quant_one_rcp(v[3], s, y));
   }
   return pack4_i8(quant_one(v[0], s), quant_one(v[1], s), quant_one(v[2], s), quant_one(v[3], s));
+}
+
+// The same for a group of 16-bit values, whose quotients are one multiplication: trunc(v * y) is trunc(v / s) for every value of
+// the group if y is 1 / s to a few ulps, on the right side of it.  With the group's maximum b and a value a as integers (11 bits
+// at most), v / s is 127 a / b times a power of two and the rounding of s; a quotient that is no integer is further than
+// 1 / (127 a) of itself from one, which is more than 2^-18.  It is an integer n other than 0 where a = b, n = 127 (127 being
+// prime), or where b is a multiple of 127 and s exact.  So only which side of 127 the maximum's own quotient rounds to has to be
+// met, and an exact quotient is on the upper side.  floor: the least scale is floor / 127.  False where this does not hold - an
+// infinity, or a maximum so small that the floor, which is no 16-bit value, replaces it - and the caller divides (quant4_div).
+// 15 instead of 27 vector instructions for four values, and half of a row's: first GEMM of the Qwen3-30B-A3B layer at 8192 tokens
+// 345.7 -> 334.0 us, whole layer with its router 566.5 -> 561.3; at 1531 tokens 180.1 -> 178.1, one token 18.16 -> 17.90.
+__device__ __forceinline__ bool group_scale16(float amax, float floor, float &s, float &y) {
+  const float top = fmaxf(amax, floor), r = 1.0f / 127.0f;
+  const float q = top * r;
+  s = __builtin_fmaf(__builtin_fmaf(-127.0f, q, top), r, q); // top / 127 correctly rounded (Markstein)
+  const bool up = __builtin_fmaf(0x1p-18f, s, __builtin_fmaf(-127.0f, s, top)) >= 0.0f; // top / s rounds to 127 or above
+  y = __builtin_amdgcn_rcpf(s) * (up ? 1.0f + 0x1p-21f : 1.0f - 0x1p-21f);
+  return floor >= 1e-10f && (amax == 0.0f || (amax >= floor && amax < __builtin_inff()));
+}
+// (a NaN becomes -128 as in quant_one)
+__device__ __forceinline__ uint32_t quant4_mul(const float *v, float y) {
+  int t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i] = static_cast<int>(__builtin_amdgcn_fmed3f(v[i] * y, -128.0f, 127.0f));
+  return pack4_i8(t[0], t[1], t[2], t[3]);
+}
+__device__ __forceinline__ uint32_t quant4_div(const float *v, float s) {
+  return pack4_i8(quant_one(v[0], s), quant_one(v[1], s), quant_one(v[2], s), quant_one(v[3], s));
+}
+
+// Eight values of a group of 16-bit values whose maximum is amax, and the group's scale.
+__device__ __forceinline__ v2i group_quant8(const float (&v)[8], float amax, float floor, float &s) {
+  float y;
+  if (__builtin_expect(group_scale16(amax, floor, s, y), 1))
+    return v2i{static_cast<int>(quant4_mul(&v[0], y)), static_cast<int>(quant4_mul(&v[4], y))};
+  s = fmaxf(amax, floor) / 127.0f;
+  return v2i{static_cast<int>(quant4_div(&v[0], s)), static_cast<int>(quant4_div(&v[4], s))};
 }
 
 // per_token_group_quant_int8 for the groups g = first + i * stride (reference:
@@ -250,13 +287,8 @@ __device__ __forceinline__ void group_quant_body(const uint16_t *__restrict__ x,
     }
 #pragma unroll
     for (int d = 1; d < 16; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-    amax = fmaxf(amax, eps);
-    const float sc = amax / 127.0f;
-    // one IEEE reciprocal per group, then the correctly rounded quotient per value (quant4)
-    const float rsc = 1.0f / sc;
-    v2i packed;
-    packed[0] = static_cast<int>(quant4(&v[0], sc, rsc));
-    packed[1] = static_cast<int>(quant4(&v[4], sc, rsc));
+    float sc;
+    const v2i packed = group_quant8(v, amax, eps, sc);
     *reinterpret_cast<v2i *>(q + g * kGroup + sub * 8) = packed;
     if (sub == 0) s[g] = sc;
   }

@@ -89,13 +89,8 @@ __global__ __launch_bounds__(256) void act_mul_group_quant_kernel(const uint16_t
     }
 #pragma unroll
     for (int d = 1; d < 16; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-    amax = fmaxf(amax, eps);
-    const float sc = amax / 127.0f;
-    const float rsc = 1.0f / sc;
-    v2i packed;
-    packed[0] = static_cast<int>(quant4(&v[0], sc, rsc));
-    packed[1] = static_cast<int>(quant4(&v[4], sc, rsc));
-    *reinterpret_cast<v2i *>(q + r * I + c) = packed;
+    float sc;
+    *reinterpret_cast<v2i *>(q + r * I + c) = group_quant8(v, amax, eps, sc);
     if (sub == 0) s[g] = sc;
   }
 }

@@ -86,13 +86,7 @@ template <int DT> __device__ __forceinline__ v2i dec_quant8(const v8u16 raw, flo
   float amax = dec_widen8<DT>(raw, v);
 #pragma unroll
   for (int d = 1; d < 16; d <<= 1) amax = fmaxf(amax, __shfl_xor(amax, d));
-  amax = fmaxf(amax, 1e-10f);
-  const float sc = amax / 127.0f, rsc = 1.0f / sc;
-  scale = sc;
-  v2i packed;
-  packed[0] = static_cast<int>(quant4(&v[0], sc, rsc));
-  packed[1] = static_cast<int>(quant4(&v[4], sc, rsc));
-  return packed;
+  return group_quant8(v, amax, 1e-10f, scale);
 }
 
 // The per-token rule: round to nearest of v * (127 / amax).

@@ -912,29 +912,37 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
     // the quantised tile (128 tokens x 128 columns of int8) leaves through LDS as whole rows
     int8_t *qst = sA;
     // scales of all eight fragments first, outside the branches on nst: the reads are in bounds
-    // either way, and one batch of LDS reads and divisions replaces eight dependent chains
-    float sc_all[NTB], rsc_all[NTB];
+    // either way, and one batch of LDS reads replaces eight dependent chains
+    float sc_all[NTB], y_all[NTB];
+    bool plain = true; // one wave-uniform branch for the tile's rows
+    auto row_max = [&](int tb) __attribute__((always_inline)) {
+      const int t = tb * 16 + r;
+      return fmaxf(fmaxf(sRed[t], sRed[T + t]), fmaxf(sRed[2 * T + t], sRed[3 * T + t]));
+    };
 #pragma unroll
     for (int tb = 0; tb < NTB; ++tb) {
-      const int t = tb * 16 + r;
-      float amax = fmaxf(fmaxf(sRed[t], sRed[T + t]), fmaxf(sRed[2 * T + t], sRed[3 * T + t]));
-      amax = fmaxf(amax, 1e-10f);
-      sc_all[tb] = amax / 127.0f;
-      rsc_all[tb] = 1.0f / sc_all[tb];
+      const bool fits = group_scale16(row_max(tb), 1e-10f, sc_all[tb], y_all[tb]);
+      plain &= fits || 2 * (tb & ~1) >= nst; // (of fragments that are not in use nothing was written)
     }
+    plain = __builtin_amdgcn_ballot_w64(!plain) == 0;
+    auto put = [&](auto PLAIN) __attribute__((always_inline)) {
 #pragma unroll
-    for (int tb = 0; tb < NTB; ++tb) {
-      if (2 * (tb & ~1) >= nst) continue;
-      const int t = tb * 16 + r;
-      const float sc = sc_all[tb], rsc = rsc_all[tb];
+      for (int tb = 0; tb < NTB; ++tb) {
+        if (2 * (tb & ~1) >= nst) continue;
+        const int t = tb * 16 + r;
+        if constexpr (!decltype(PLAIN)::value) sc_all[tb] = fmaxf(row_max(tb), 1e-10f) / 127.0f;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        *reinterpret_cast<uint32_t *>(qst + t * kTPitch + wave * 32 + h * 16 + 4 * q) = quant4(actf[tb][h], sc, rsc);
-      if (wave == (tb & 3) && q == 0) { // every wave holds every token's scale: the stores are shared out
-        const int64_t ft = sIds[t];
-        if (ft < a.num_valid) a.A2s[ft * G + nt] = sc;
+        for (int h = 0; h < 2; ++h)
+          *reinterpret_cast<uint32_t *>(qst + t * kTPitch + wave * 32 + h * 16 + 4 * q) =
+              decltype(PLAIN)::value ? quant4_mul(actf[tb][h], y_all[tb]) : quant4_div(actf[tb][h], sc_all[tb]);
+        if (wave == (tb & 3) && q == 0) { // every wave holds every token's scale: the stores are shared out
+          const int64_t ft = sIds[t];
+          if (ft < a.num_valid) a.A2s[ft * G + nt] = sc_all[tb];
+        }
       }
-    }
+    };
+    if (__builtin_expect(plain, 1)) put(std::true_type{});
+    else put(std::false_type{});
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < (T * 8 + 255) / 256; ++j) {

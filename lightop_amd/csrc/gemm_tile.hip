@@ -300,19 +300,27 @@ void moe_gemm_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     // it leaves as whole 128-byte rows instead of 4-byte pieces; the token tile's LDS is free.
     constexpr int kQPitch = kGroup + 16;
     int8_t *qst = &sA[0][0];
+    bool plain = true; // one wave-uniform branch for the tile's rows
+    float sc[2], y[2];
+    auto row_max = [&](int tb) __attribute__((always_inline)) {
+      return fmaxf(fmaxf(sRed[wt][tb][0][r], sRed[wt][tb][1][r]), fmaxf(sRed[wt][tb][2][r], sRed[wt][tb][3][r]));
+    };
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) {
-      float amax = fmaxf(fmaxf(sRed[wt][tb][0][r], sRed[wt][tb][1][r]),
-                         fmaxf(sRed[wt][tb][2][r], sRed[wt][tb][3][r]));
-      amax = fmaxf(amax, 1e-10f);
-      const float sc = amax / 127.0f;
-      const float rsc = 1.0f / sc;
+    for (int tb = 0; tb < 2; ++tb) plain &= group_scale16(row_max(tb), 1e-10f, sc[tb], y[tb]);
+    plain = __builtin_amdgcn_ballot_w64(!plain) == 0;
+    auto put = [&](auto PLAIN) __attribute__((always_inline)) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<uint32_t *>(qst + (wt * 64 + tb * 32 + r) * kQPitch + wr * 32 + 8 * q + 4 * c) =
-            quant4(&actf[tb][4 * q], sc, rsc);
-      if (valid[tb] && wr == 0 && c == 0) a.A2s[f[tb] * G + nt] = sc;
-    }
+      for (int tb = 0; tb < 2; ++tb) {
+        if constexpr (!decltype(PLAIN)::value) sc[tb] = fmaxf(row_max(tb), 1e-10f) / 127.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<uint32_t *>(qst + (wt * 64 + tb * 32 + r) * kQPitch + wr * 32 + 8 * q + 4 * c) =
+              decltype(PLAIN)::value ? quant4_mul(&actf[tb][4 * q], y[tb]) : quant4_div(&actf[tb][4 * q], sc[tb]);
+        if (valid[tb] && wr == 0 && c == 0) a.A2s[f[tb] * G + nt] = sc[tb];
+      }
+    };
+    if (__builtin_expect(plain, 1)) put(std::true_type{});
+    else put(std::false_type{});
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kTileM * 8 / (256 * WT); ++j) {

@@ -333,18 +333,28 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     const int64_t G = I / kGroup;
     // the quantised tile (64 tokens x 128 columns of int8) leaves through LDS as whole rows
     int8_t *qst = &sA[0][0];
-#pragma unroll
-    for (int tf = 0; tf < 4; ++tf) {
+    bool plain = true; // one wave-uniform branch for the tile's rows
+    float sc[4], y[4];
+    auto row_max = [&](int tf) __attribute__((always_inline)) {
       const int t = tf * 16 + r;
-      float amax = fmaxf(fmaxf(sRed[0][t], sRed[1][t]), fmaxf(sRed[2][t], sRed[3][t]));
-      amax = fmaxf(amax, 1e-10f);
-      const float sc = amax / 127.0f;
-      const float rsc = 1.0f / sc;
+      return fmaxf(fmaxf(sRed[0][t], sRed[1][t]), fmaxf(sRed[2][t], sRed[3][t]));
+    };
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
-        *reinterpret_cast<uint32_t *>(qst + t * kW4Row + wr * 32 + g * 16 + 4 * q) = quant4(actf[tf][g], sc, rsc);
-      if (valid[tf] && wr == 0 && q == 0) a.A2s[f[tf] * G + nt] = sc;
-    }
+    for (int tf = 0; tf < 4; ++tf) plain &= group_scale16(row_max(tf), 1e-10f, sc[tf], y[tf]);
+    plain = __builtin_amdgcn_ballot_w64(!plain) == 0;
+    auto put = [&](auto PLAIN) __attribute__((always_inline)) {
+#pragma unroll
+      for (int tf = 0; tf < 4; ++tf) {
+        if constexpr (!decltype(PLAIN)::value) sc[tf] = fmaxf(row_max(tf), 1e-10f) / 127.0f;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          *reinterpret_cast<uint32_t *>(qst + (tf * 16 + r) * kW4Row + wr * 32 + g * 16 + 4 * q) =
+              decltype(PLAIN)::value ? quant4_mul(actf[tf][g], y[tf]) : quant4_div(actf[tf][g], sc[tf]);
+        if (valid[tf] && wr == 0 && q == 0) a.A2s[f[tf] * G + nt] = sc[tf];
+      }
+    };
+    if (__builtin_expect(plain, 1)) put(std::true_type{});
+    else put(std::false_type{});
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kTileM * 8 / 256; ++j) {

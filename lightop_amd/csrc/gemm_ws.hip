@@ -424,9 +424,10 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
       float amax = 0.0f;
 #pragma unroll
       for (int w2 = 0; w2 < NWAVES; ++w2) amax = fmaxf(amax, red[j][w2][r]);
-      amax = fmaxf(amax, 1e-10f);
-      const float sc = amax / 127.0f;
-      const uint32_t packed = quant4(actf[j], sc, 1.0f / sc);
+      float sc, y;
+      const bool plain = group_scale16(amax, 1e-10f, sc, y);
+      if (!plain) sc = fmaxf(amax, 1e-10f) / 127.0f;
+      const uint32_t packed = __builtin_expect(plain, 1) ? quant4_mul(actf[j], y) : quant4_div(actf[j], sc);
       *reinterpret_cast<uint32_t *>(a.A2q + f[j] * I + nrow[0] + 4 * c) = packed;
       if (wave == 0 && c == 0) a.A2s[f[j] * G + nt] = sc;
     }
