@@ -230,6 +230,9 @@ __device__ __forceinline__ v4i bld16(brsrc r, int voff, int soff) {
 __device__ __forceinline__ float bld_f32(brsrc r, int voff, int soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
+__device__ __forceinline__ void bst16(brsrc r, v4i v, uint32_t voff, int soff) { // nothing past the extent
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, static_cast<int>(voff), soff, 0);
+}
 
 // Consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.
 // The logical tile list is cut into chunks of (G token blocks x all weight tiles): the

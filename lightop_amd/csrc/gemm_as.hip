@@ -14,11 +14,14 @@
 
 namespace lo {
 
+constexpr uint32_t kAsMaxOut = 0xfff00000u; // bytes of an output that a descriptor addresses; an offset that none of them has
+
 // KBT: K / 128 as a compile-time constant (a multiple of three, so that a tile starts on ring buffer 0),
 // or 0 for any K.  With it a tile's steps and its stores are straight-line code: the compiler then
 // knows how many memory operations follow each weight load and waits for exactly those; in the
 // general form the stores sit in a branch, the wait counts assume they did not happen, and after
-// every tile the wave waits for loads it has only just issued.
+// every tile the wave waits for loads it has only just issued.  Straight-line stores go through a descriptor of the output
+// (< 4 GiB), padding tokens past its end.
 template <int ORD, int KBT = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
@@ -27,14 +30,13 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   constexpr int kTileM = 64;
   const int K = static_cast<int>(a.K);
   const int KB = K / kGroup;
-  // = 16 mod 128: a 16-byte column of eight consecutive rows lies on different banks.  A fragment's operand is four such columns of
-  // 16 rows, where piece q of a row and piece q - 1 of the next share theirs: SQ_LDS_BANK_CONFLICT of the Qwen3-30B-A3B layer's
-  // second stage at 8192 tokens is 1.08e7, 4.1e6 with the 32x32 fragments before.
-  const int pitch = K + 16;
+  // Tokens in operand order: K half kh of K block kb of token fragment tb is the 1 KB at ((2 kb + kh) * 4 + tb) * 1024, lane after
+  // lane.  A read of 64 consecutive pieces has no bank conflict (rows 16 bytes past a multiple of 128 had 1.08e7 on the
+  // Qwen3-30B-A3B layer's second stage at 8192 tokens) and the rows need no registers on their way here.
   int8_t *const sA = smem;
-  float *const sS = reinterpret_cast<float *>(smem + kTileM * pitch); // [KB][64]
+  float *const sS = reinterpret_cast<float *>(smem + kTileM * K); // [KB][64]
   // per-wave staging of 16 output rows x 64 columns (bf16), for row-contiguous stores
-  int8_t *const sStage = smem + kTileM * pitch + KB * kTileM * 4;
+  int8_t *const sStage = smem + kTileM * K + KB * kTileM * 4;
   int32_t *const sFlag = reinterpret_cast<int32_t *>(sStage + 4 * 16 * kStgPitch); // [wave]: a scale that the biased fold does not take
   float *const sB = reinterpret_cast<float *>(sFlag + 4);                          // weight-block scales of the workgroup's tiles
   // The contracted order folds without a conversion (fold_biased), or with one where the scales do not allow that.  In 16x16
@@ -45,30 +47,34 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
 
   int mb, ng;
   if (!tile_of(blockIdx.x, n_groups, m_blocks, group_m, mb, ng)) return;
-  if (static_cast<int64_t>(mb) * kTileM >= a.ntpp[0]) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wr = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of a tile
+  const int r = lane & 15, q = lane >> 4;
+  // The start is two round trips: the ids and the block's expert, all of them, then everything that depends on them.  One after the
+  // other they were seven.  With the tokens in operand order and the straight-line stores: Qwen3-30B-A3B layer with its router
+  // at 8192 tokens 545.4 -> 540.9 us, 12000: 740.2 -> 736.4, 24000: 1491 -> 1487 (on a slower card 583.5, 578.9 with order and
+  // stores alone, 575.4).
+  const int32_t *const ids = a.sorted + static_cast<int64_t>(mb) * kTileM;
+  const int32_t blocks_end = a.ntpp[0];
+  const int e_raw = a.expert_ids[mb >> sub_shift];
+  int32_t f[4]; // slots of the tokens this lane holds in the accumulator layout
+#pragma unroll
+  for (int tb = 0; tb < 4; ++tb) f[tb] = ids[tb * 16 + r];
+  const int32_t f_lane = ids[lane], f_row = ids[wr * 16 + r];
+  if (static_cast<int64_t>(mb) * kTileM >= blocks_end) return;
   // mb counts 64-token pieces; an alignment block of 128 tokens is two of them (sub_shift = 1), and
   // a piece that holds padding only is skipped
   // An expert_map entry outside the weight tensor is treated like an expert of another rank, but its
   // rows are always zero-filled: the slot mask of the alignment counts such a slot as local.
-  const int e_raw = a.expert_ids[mb >> sub_shift];
   const bool e_oob = e_raw >= a.E;
   const int e = e_oob ? -1 : e_raw;
-  const int tid = threadIdx.x, lane = tid & 63;
-  if (sub_shift &&
-      __builtin_amdgcn_ballot_w64(a.sorted[static_cast<int64_t>(mb) * kTileM + lane] < a.num_valid) == 0)
-    return;
-  const int wr = __builtin_amdgcn_readfirstlane(tid >> 6); // which 64 weight rows of a tile
-  const int r = lane & 15, q = lane >> 4;
+  if (sub_shift && __builtin_amdgcn_ballot_w64(f_lane < a.num_valid) == 0) return;
   const int64_t N = a.N;
   const int n_tiles = static_cast<int>((N + 255) / 256);
   const int nt0 = ng * n_cnt;
   int nt_end = nt0 + n_cnt < n_tiles ? nt0 + n_cnt : n_tiles;
   // N % 64 == 0 is checked on the host; in the last tile the waves past N have no rows
   if (static_cast<int64_t>(nt_end - 1) * 256 + wr * 64 >= N) --nt_end;
-
-  int32_t f[4]; // slots of the tokens this lane holds in the accumulator layout
-#pragma unroll
-  for (int tb = 0; tb < 4; ++tb) f[tb] = a.sorted[static_cast<int64_t>(mb) * kTileM + tb * 16 + r];
 
   if (e < 0) {
     if ((!a.skip_nonlocal || e_oob)) {
@@ -93,54 +99,62 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     if (a.mul_routed) wgt[tb] = a.topk_w[f[tb] < a.num_valid ? f[tb] : 0];
   }
 
-  // ---- the token block into LDS, once ------------------------------------------------
-  {
-    const int lt = tid >> 2, lq = tid & 3; // thread -> (token, every fourth 16-byte piece)
-    const int64_t lf = a.sorted[static_cast<int64_t>(mb) * kTileM + lt];
-    const int64_t lrow = token_row(a, lf);
-    const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
-    const int aoff = static_cast<int>(lrow * K) + lq * 16;
-    int8_t *dst = sA + lt * pitch + lq * 16;
-    const int pieces = K / 64; // per thread
-    for (int j0 = 0; j0 < pieces; j0 += 4) {
-      v4i t[4];
+  // KBT: where the lane's two pieces of a token fragment's rows go, in bytes of the output, or past its end
+  const brsrc rC = make_rsrc(a.C, static_cast<uint32_t>(a.num_valid * N * 2));
+  uint32_t coff[4][2];
+  if constexpr (KBT > 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) t[j] = bld16(rA, aoff, (j0 + j < pieces ? j0 + j : pieces - 1) * 64);
+    for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (j0 + j < pieces) *reinterpret_cast<v4i *>(dst + (j0 + j) * 64) = t[j];
-    }
+      for (int j = 0; j < 2; ++j) {
+        const int fs = __shfl(f[tb] < a.num_valid ? f[tb] : -1, (lane >> 3) + 8 * j);
+        coff[tb][j] = fs >= 0 ? fs * static_cast<uint32_t>(N) * 2 + (lane & 7) * 16 : kAsMaxOut;
+      }
   }
-  // every scale the workgroup needs, once; `fit`: for the biased fold, noting one that it does not take
-  const int NB = static_cast<int>((N + kGroup - 1) / kGroup);
-  const int b_cnt = (n_cnt * 2 < NB - nt0 * 2 ? n_cnt * 2 : NB - nt0 * 2) * KB; // [tile][half][K block]
-  auto fill_scales = [&](auto FIT) __attribute__((always_inline)) {
-    constexpr bool fit = decltype(FIT)::value;
-    const int st = tid & 63;
-    const int64_t sf = a.sorted[static_cast<int64_t>(mb) * kTileM + st];
-    const int64_t srow = token_row(a, sf);
-    bool bad = false;
-    for (int kb = wr; kb < KB; kb += 4) {
-      // (a padding token's is zero: row 0, which it is computed on, may be one that nobody wrote)
-      const float v = sf < a.num_valid ? a.As[srow * KB + kb] : 0.0f;
-      bad |= !fold_token_scale_ok(v);
-      sS[kb * kTileM + st] = fit ? fold_token_scale(v) : v;
-    }
-    const float *const ws = a.Ws + (static_cast<int64_t>(e) * NB + nt0 * 2) * KB;
-    for (int i = tid; i < b_cnt; i += 256) {
-      const float v = ws[i];
-      bad |= !fold_weight_scale_ok(v);
-      sB[i] = fit ? fold_weight_scale(v) : v;
-    }
-    if constexpr (fit) sFlag[wr] = __builtin_amdgcn_ballot_w64(bad) ? 1 : 0; // one value for the wave
-  };
-  fill_scales(std::integral_constant<bool, kBiased>{});
 
   const brsrc rW = make_rsrc(a.W + static_cast<int64_t>(e) * N * K, static_cast<uint32_t>(N * K));
   // The wave's 64 rows are four 2 KB blocks, in lane order; tile, K block and k-half go into the scalar offset.
   const int wkstride = shuf_kb_stride(static_cast<int>(N / 16));
   const int wtstride = 16 * shuf_nb_stride(KB); // 256 rows further
   const int woff = (nt0 * 16 + wr * 4) * shuf_nb_stride(KB) + lane * 16;
+
+  // ---- the token block and every scale the workgroup needs, once ----------------------
+  {
+    const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
+    const int aoff = token_row(a, f_row) * K + q * 16;
+    int8_t *const dst = sA + wr * 1024;
+#pragma unroll
+    for (int p = 0; p < (KBT ? 2 * KBT : K / 64); ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, dst + p * 4096, 16, aoff, p * 64, 0, 0);
+  }
+  const int NB = static_cast<int>((N + kGroup - 1) / kGroup);
+  const int b_cnt = (n_cnt * 2 < NB - nt0 * 2 ? n_cnt * 2 : NB - nt0 * 2) * KB; // [tile][half][K block]
+  const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * KB * 4));
+  const brsrc rWs = make_rsrc(a.Ws + (static_cast<int64_t>(e) * NB + nt0 * 2) * KB, static_cast<uint32_t>(b_cnt > 0 ? b_cnt * 4 : 0));
+  // (a padding token's is zero: row 0, which it is computed on, may be one that nobody wrote)
+  const int asoff = f_lane < a.num_valid ? token_row(a, f_lane) * KB * 4 : 0x40000000;
+  float as_mine[2]; // of token `lane`, K blocks wr and wr + 4: K <= 1024 (gemm_as_supports)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) as_mine[i] = bld_f32(rAs, asoff, (wr + 4 * i < KB ? wr + 4 * i : KB - 1) * 4);
+  const float ws_mine = bld_f32(rWs, tid * 4, 0);
+  // `fit`: for the biased fold, noting one that it does not take
+  auto fill_scales = [&](auto FIT) __attribute__((always_inline)) {
+    constexpr bool fit = decltype(FIT)::value;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int kb = wr + 4 * i;
+      const float v = as_mine[i];
+      bad |= !fold_token_scale_ok(v);
+      if (kb < KB) sS[kb * kTileM + lane] = fit ? fold_token_scale(v) : v;
+    }
+    for (int i = tid; i < b_cnt; i += 256) {
+      const float v = i < 256 ? ws_mine : bld_f32(rWs, i * 4, 0);
+      bad |= !fold_weight_scale_ok(v);
+      sB[i] = fit ? fold_weight_scale(v) : v;
+    }
+    if constexpr (fit) sFlag[wr] = __builtin_amdgcn_ballot_w64(bad) ? 1 : 0; // one value for the wave
+  };
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -177,12 +191,12 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     const float bs = sB[live ? ((nt - nt0) * 2 + (wr >> 1)) * KB + kb : 0];
     // Software pipeline over half token fragments: the MFMAs of two row fragments are issued, then the previous two are folded
     // into the fp32 accumulators while the matrix pipe works; the next token fragment is read under the first half.
-    const int8_t *src = sA + r * pitch + kb * kGroup + q * 16;
+    const int8_t *src = sA + kb * 8192 + lane * 16;
     const float *ts = sS + kb * kTileM + r;
     v4i bf[2][2], dprev[2];
     float as_t[2], as_prev = 0.0f, as_bias = 0.0f;
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh) bf[0][kh] = *reinterpret_cast<const v4i *>(src + kh * 64);
+    for (int kh = 0; kh < 2; ++kh) bf[0][kh] = *reinterpret_cast<const v4i *>(src + kh * 4096);
     as_t[0] = live ? ts[0] : 0.0f; // a step past the end adds 0
     auto fold_pair = [&](int st) __attribute__((always_inline)) {
       const int tb = st >> 1, h = st & 1;
@@ -196,7 +210,7 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
       if (h == 0 && tb < 3) {
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh)
-          bf[(tb + 1) & 1][kh] = *reinterpret_cast<const v4i *>(src + (tb + 1) * 16 * pitch + kh * 64);
+          bf[(tb + 1) & 1][kh] = *reinterpret_cast<const v4i *>(src + (tb + 1) * 1024 + kh * 4096);
         as_t[(tb + 1) & 1] = live ? ts[(tb + 1) * 16] : 0.0f;
       }
       v4i d[2];
@@ -237,11 +251,10 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
         for (int i = 0; i < 4; ++i) acc[tb][rb][i] = 0.0f;
   };
   auto store_tile = [&](int nt) __attribute__((always_inline)) {
-    const int64_t nrow0 = static_cast<int64_t>(nt) * 256 + wr * 64;
+    const int nrow0 = nt * 256 + wr * 64;
     int8_t *stg = sStage + wr * (16 * kStgPitch);
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb) {
-      const bool valid = f[tb] < a.num_valid;
       with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
@@ -252,13 +265,16 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
         }
       });
       __builtin_amdgcn_wave_barrier();
-      const int slot = valid ? f[tb] : -1;
 #pragma unroll
       for (int j = 0; j < 2; ++j) { // 128-byte row segments, eight rows an instruction
         const int tok = (lane >> 3) + 8 * j;
         const v4i v = *reinterpret_cast<const v4i *>(stg + tok * kStgPitch + (lane & 7) * 16);
-        const int fs = __shfl(slot, tok);
-        if (fs >= 0) *reinterpret_cast<v4i *>(a.C + static_cast<int64_t>(fs) * N + nrow0 + (lane & 7) * 8) = v;
+        if constexpr (KBT > 0) {
+          bst16(rC, v, coff[tb][j], nrow0 * 2);
+        } else {
+          const int fs = __shfl(f[tb] < a.num_valid ? f[tb] : -1, tok);
+          if (fs >= 0) *reinterpret_cast<v4i *>(a.C + static_cast<int64_t>(fs) * N + nrow0 + (lane & 7) * 8) = v;
+        }
       }
       __builtin_amdgcn_wave_barrier();
     }
@@ -282,6 +298,8 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
     load_step(B0{});
     load_step(B1{});
   }
+  fill_scales(std::integral_constant<bool, kBiased>{});
+  __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): the copies into LDS have landed
   __syncthreads(); // the only barrier: the token block is complete
   zero_acc();
   constexpr std::integral_constant<bool, kBiased> biased{};
@@ -333,19 +351,19 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   }
 }
 
-// n_cnt: weight tiles of a workgroup
+// weight tiles of a workgroup
 static int as_tiles(int64_t N) {
   const int n_tiles = static_cast<int>((N + 255) / 256);
   return (n_tiles + 1) / 2;
 }
 static int64_t as_lds_bytes(int64_t N, int64_t K) {
-  return 64 * (K + 16) + (K / kGroup) * 64 * 4 + 4 * 16 * kStgPitch + as_tiles(N) * 2 * (K / kGroup) * 4 + 16;
+  return 64 * K + (K / kGroup) * 64 * 4 + 4 * 16 * kStgPitch + as_tiles(N) * 2 * (K / kGroup) * 4 + 16;
 }
 
 bool gemm_as_supports(const GemmArgs &a, bool fused_act, int block_size_m) {
   if (fused_act || !a.w_shuffled || (block_size_m != 64 && block_size_m != 128)) return false;
   if (a.N % 64 != 0 || (reinterpret_cast<uintptr_t>(a.C) & 15) != 0) return false;
-  if (as_lds_bytes(a.N, a.K) > 80 * 1024) return false; // two workgroups per CU
+  if (a.K > 8 * kGroup || as_lds_bytes(a.N, a.K) > 80 * 1024) return false; // two workgroups per CU
   // Pays off only when the launch is several rounds of workgroups deep even with half a
   // token block's weight tiles per workgroup; below that the per-tile kernel balances better.
   return a.num_valid / 64 + (a.experts_routed + 1) / 2 >= 1024;
@@ -379,7 +397,7 @@ int launch_gemm_as(const GemmArgs &a0, int flags, int block_size_m, int64_t m_bl
     if (rc_lds) return rc_lds;                                                                        \
     hipLaunchKernelGGL(kern, g, b, lds, s, a, mbi, Gi, n_groups, n_cnt, sub_shift);                   \
   } while (0)
-  if (a.K == 6 * kGroup) LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, 6);
+  if (a.K == 6 * kGroup && a.num_valid * a.N * 2 <= kAsMaxOut) LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, 6);
   else LO_ORD_DISPATCH(ord, LO_AS_LAUNCH, 0);
 #undef LO_AS_LAUNCH
   return check_launch("moe_gemm(activation-stationary)");
