@@ -141,10 +141,10 @@ int lo_moe_align_block_size_mask(const void *topk_ids, int ids_dtype, int64_t nu
                                  lo_stream_t stream);
 
 /*
- * Same again with a scratch buffer that lets large inputs (numel >= 8192) be aligned by
- * many workgroups instead of one: lo_moe_align_scratch_bytes(numel, num_experts) bytes of
+ * Same again with a scratch buffer that lets large inputs (numel >= 8192) be counted in a
+ * launch of their own: lo_moe_align_scratch_bytes(numel, num_experts) bytes of
  * device memory, 4-byte aligned, contents irrelevant (0 = no scratch needed).  Without
- * scratch the single-workgroup kernel runs; the result is identical.  The reference's
+ * scratch, and where one launch is faster, it is not used; the result is identical.  The reference's
  * large-input kernels allocate a zeroed tensor themselves
  * (csrc/kernels/moe_align_sum_kernels.cu:1175).
  */

@@ -233,6 +233,144 @@ __global__ __launch_bounds__(1024) void quant_align_kernel(
   }
 }
 
+constexpr int kWideT = 1024;
+// The alignment by `nchunks` workgroups of 1024 slots each, a wave's 64 its own, in one launch: every workgroup counts the slots
+// before and behind its own for itself (from L2), so nothing has to be counted before it starts.  It is a chain of round trips, to
+// memory for the ids and in LDS, and one sweep's worth of LDS atomics; the padding and the expert ids are written by sixteen
+// lanes an expert.  Chunks, waves and lanes are in slot order: the order is the same stable one.
+template <typename IdT>
+__device__ __forceinline__ void moe_align_wide_body(
+    const IdT *__restrict__ ids, int64_t numel64, int E, int bs, const int32_t *__restrict__ expert_map,
+    int ignore_invalid, int32_t *__restrict__ sorted, int64_t sorted_cap, int32_t *__restrict__ expert_ids,
+    int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits, uint8_t *__restrict__ slot_mask,
+    const int32_t *__restrict__ num_local_tokens, int slots_per_token, int chunk, int nchunks) {
+  extern __shared__ int32_t lds[];
+  const int pad_val = static_cast<int>(numel64);
+  constexpr int T = kWideT, nw = T / kWave;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int32_t *offs = lds;            // [E + 1] padded exclusive prefix
+  int32_t *total = lds + (E + 1); // [E] slots in later chunks; then in all
+  int32_t *cbase = total + E;     // [E] slots in earlier chunks
+  int32_t *emap = cbase + E;      // [E] what expert_ids says of a block
+  int32_t *wcnt = emap + E;       // [nw][E]
+  __shared__ int32_t wave_sum[16];
+
+  const int own = chunk * T + tid;
+  const IdT own_raw = pad_val > 0 ? ids[own < pad_val ? own : 0] : IdT(0);
+  const int numel = static_cast<int>(local_slots(numel64, num_local_tokens, slots_per_token));
+  for (int i = tid; i < nw * E; i += T) wcnt[i] = 0;
+  for (int e = tid; e < E; e += T) {
+    total[e] = cbase[e] = 0;
+    emap[e] = (expert_map && !ignore_invalid) ? expert_map[e] : e;
+  }
+  auto key_of = [&](IdT id, bool in_range, bool &ok) __attribute__((always_inline)) {
+    const int64_t raw = static_cast<int64_t>(id);
+    ok = in_range && raw >= 0 && raw < E;
+    int e = ok ? static_cast<int>(raw) : 0;
+    if (ignore_invalid && expert_map) { // keys are local expert ids
+      const int m = expert_map[e];
+      ok = ok && m >= 0 && m < E;
+      e = ok ? m : 0;
+    }
+    return e;
+  };
+  bool ok;
+  const int ek = key_of(own_raw, own < numel, ok);
+  __syncthreads();
+  if (ok) atomicAdd(&wcnt[wave * E + ek], 1);
+  if (slot_mask && own < pad_val) slot_mask[own] = ok && (ignore_invalid || emap[ek] >= 0) ? 1 : 0; // is the slot's expert held by this rank?
+  constexpr int kSweep = 16; // loads in flight per thread
+  for (int u0 = 0; u0 < nchunks; u0 += kSweep) {
+    IdT raw[kSweep];
+#pragma unroll
+    for (int u = 0; u < kSweep; ++u) {
+      const int f = (u0 + u) * T + tid;
+      if (u0 + u < nchunks) raw[u] = ids[f < numel ? f : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < kSweep; ++u) {
+      const int c = u0 + u;
+      if (c >= nchunks) break;
+      bool in;
+      const int e = key_of(raw[u], c != chunk && c * T + tid < numel, in);
+      if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+    }
+  }
+  __syncthreads();
+  for (int base = 0; base < E; base += T) {
+    const int e = base + tid;
+    int t = 0;
+    if (e < E) {
+      const int before = cbase[e];
+      int c = before;
+      int v[nw];
+#pragma unroll
+      for (int w = 0; w < nw; ++w) v[w] = wcnt[w * E + e];
+#pragma unroll
+      for (int w = 0; w < nw; ++w) {
+        wcnt[w * E + e] = c; // slots of expert e before this wave's
+        c += v[w];
+      }
+      t = total[e] + c;
+      total[e] = t;
+    }
+    int incl = (t + bs - 1) / bs * bs;
+    for (int d = 1; d < kWave; d <<= 1) {
+      int up = __shfl_up(incl, d);
+      if (lane >= d) incl += up;
+    }
+    if (lane == kWave - 1) wave_sum[wave] = incl;
+    __syncthreads();
+    int carry = (base == 0) ? 0 : offs[base];
+    for (int w = 0; w < wave; ++w) carry += wave_sum[w];
+    if (e < E) offs[e + 1] = carry + incl;
+    if (base == 0 && tid == 0) offs[0] = 0;
+    __syncthreads();
+  }
+  // this wave's slots: ranks inside the 64 from a ballot match
+  {
+    const uint64_t peers = match_any(ek, key_bits, ok);
+    if (ok) sorted[offs[ek] + wcnt[wave * E + ek] + __popcll(peers & ((1ull << lane) - 1ull))] = own;
+  }
+  // padding and expert ids, shared out by expert among the chunks, sixteen lanes to an expert; what lies past the last block
+  const int P = offs[E];
+  if (chunk == 0 && tid == 0) ntpp[0] = P;
+  for (int e = chunk + (tid >> 4) * nchunks; e < E; e += nchunks * (T >> 4)) {
+    const int o0 = offs[e], o1 = offs[e + 1], v = emap[e];
+    for (int i = o0 + total[e] + (tid & 15); i < o1; i += 16) sorted[i] = pad_val;
+    for (int b = o0 / bs + (tid & 15); b < o1 / bs; b += 16) expert_ids[b] = v;
+  }
+  for (int64_t i = P + own; i < sorted_cap; i += nchunks * T) sorted[i] = pad_val;
+  for (int64_t b = P / bs + own; b < expert_ids_cap; b += nchunks * T) expert_ids[b] = -1;
+}
+
+template <typename IdT>
+__global__ __launch_bounds__(1024) void moe_align_wide_kernel(
+    const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
+    const int32_t *__restrict__ expert_map, int ignore_invalid, int32_t *__restrict__ sorted,
+    int64_t sorted_cap, int32_t *__restrict__ expert_ids, int64_t expert_ids_cap,
+    int32_t *__restrict__ ntpp, int key_bits, uint8_t *__restrict__ slot_mask,
+    const int32_t *__restrict__ num_local_tokens, int slots_per_token) {
+  moe_align_wide_body<IdT>(ids, numel, num_experts, bs, expert_map, ignore_invalid, sorted, sorted_cap, expert_ids,
+                           expert_ids_cap, ntpp, key_bits, slot_mask, num_local_tokens, slots_per_token,
+                           static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+}
+
+// The first nchunks workgroups align, the others quantise the activations: two independent stages, one launch.
+template <typename IdT, bool PER_ROW, int DT>
+__global__ __launch_bounds__(1024) void quant_align_wide_kernel(
+    const QuantJob job, const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
+    const int32_t *__restrict__ expert_map, int32_t *__restrict__ sorted, int64_t sorted_cap,
+    int32_t *__restrict__ expert_ids, int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits,
+    uint8_t *__restrict__ slot_mask, int nchunks) {
+  if (static_cast<int>(blockIdx.x) < nchunks) {
+    moe_align_wide_body<IdT>(ids, numel, num_experts, bs, expert_map, 0, sorted, sorted_cap, expert_ids, expert_ids_cap,
+                             ntpp, key_bits, slot_mask, nullptr, 1, static_cast<int>(blockIdx.x), nchunks);
+  } else {
+    quant_job<PER_ROW, DT>(job, blockIdx.x - nchunks, gridDim.x - nchunks);
+  }
+}
+
 // ---- large inputs: the same algorithm spread over many workgroups ------------------
 // Phase 1: every workgroup counts the experts of its chunk of slots into cnt[chunk][E].
 // Phase 2: every workgroup rebuilds the padded expert offsets from cnt (a few KB from
@@ -501,6 +639,23 @@ static void single_wg_shape(int64_t numel, int64_t sorted_cap, int32_t num_exper
   *lds_bytes = (static_cast<size_t>(w + 2) * num_experts + 1) * sizeof(int32_t);
 }
 
+// The one-launch form by several workgroups (moe_align_wide_body): their number, or 0 where another form is taken.  Every one of
+// them sweeps all slots, so `most` of them; below, one workgroup has nothing to share; and the counters are 4 (16 + 4) bytes of LDS
+// an expert.  Alignment alone, us, the other forms / this, at 1600, 4000, 8000, 16000, 32768 and 65536 slots: 128 experts 6.1 / 5.5,
+// 8.0 / 5.4, 10.8 / 5.8, 10.7 / 6.7, 11.7 / 9.1, 14.4 / 13.9; 256 experts 6.5 / 6.0, 8.4 / 5.9, 11.6 / 6.1, 11.7 / 6.9, 14.2 / 9.4,
+// 19.3 / 14.4; 512 experts at 1040, 1600, 2049 slots 6.8 / 7.2, 7.2 / 7.2, 7.6 / 7.3.  With the quantisation beside it, whole layer:
+// Qwen3-30B-A3B layer at 160, 333, 1000, 1531, 4000 tokens 115.5 / 115.5, 123.3 / 121.4, 165 / 160, 177.2 / 172.7, 324 / 321,
+// per-channel 700: 145.0 / 140.7; DeepSeek-V3 share at 500, 1500, 3000: 249.5 / 247.0, 351 / 345, 377 / 375.  There the sweeping
+// workgroups are slower than the two launches past 32768 slots: the share at 5000, 6000, 8192 tokens 531 / 533, 575 / 581, 710 /
+// 716; quantisation by row, past 28672: per-channel Qwen3-30B-A3B layer at 3500, 4000, 8000 276.1 / 274.6, 317.3 / 319.2, 518 / 523.
+constexpr int64_t kWideQuantSlots = 32768, kWideRowQuantSlots = 28672, kWideAlignSlots = 65536;
+static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, size_t *lds_bytes) {
+  const int64_t words = (kWideT / kWave + 4) * static_cast<int64_t>(num_experts) + 1;
+  if (numel <= kWideT || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || words > 15360) return 0;
+  *lds_bytes = static_cast<size_t>(words) * sizeof(int32_t);
+  return static_cast<int>((numel + kWideT - 1) / kWideT);
+}
+
 static void align_chunks(int64_t numel, int *nchunks, int64_t *chunk_slots) {
   int64_t n = (numel + 1023) / 1024;
   if (n > 256) n = 256;
@@ -548,6 +703,22 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
   const QuantJob job{static_cast<const uint16_t *>(x), M, H, eps, q, qs};
   const bool f16 = dtype == LO_F16;
   const int64_t groups = M * (H / kGroup);
+  {
+    size_t lds_bytes;
+    const int n = wide_shape(numel, num_experts, per_row ? kWideRowQuantSlots : kWideQuantSlots, &lds_bytes);
+    if (n > 0) {
+      int64_t qblocks = per_row ? (M + 3) / 4 : (groups + kWideT / 16 - 1) / (kWideT / 16);
+      if (qblocks > 4096) qblocks = 4096;
+      const dim3 grid(static_cast<unsigned>(n + qblocks)), block(kWideT);
+#define LO_QA_WIDE(IdT, PR, DT)                                                                                          \
+  hipLaunchKernelGGL((quant_align_wide_kernel<IdT, PR, DT>), grid, block, lds_bytes, stream, job,                        \
+                     static_cast<const IdT *>(topk_ids), numel, num_experts, block_size, expert_map, sorted_ids,         \
+                     sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, n)
+      LO_QA_DISPATCH(LO_QA_WIDE);
+#undef LO_QA_WIDE
+      return check_launch("quant_align(wide)");
+    }
+  }
   if (want > 0) { // many slots: counting, then the scatter beside the quantisation
     int nchunks;
     int64_t cs;
@@ -619,7 +790,7 @@ extern "C" int lo_moe_align_block_size_mask(const void *topk_ids, int ids_dtype,
 
 extern "C" int64_t lo_moe_align_scratch_bytes(int64_t numel, int32_t num_experts) {
   if (numel < 0 || num_experts < 1) return LO_EINVAL;
-  if (numel < 8192) return 0; // one workgroup is faster below this
+  if (numel < 8192) return 0; // one launch below this
   int nchunks;
   int64_t cs;
   lo::align_chunks(numel, &nchunks, &cs);
@@ -670,6 +841,20 @@ extern "C" int lo_moe_align_block_size_local(const void *topk_ids, int ids_dtype
   hipStream_t s = static_cast<hipStream_t>(stream);
   int key_bits = 1;
   while ((1 << key_bits) < num_experts) ++key_bits;
+  {
+    size_t lds_bytes;
+    const int n = wide_shape(numel, num_experts, kWideAlignSlots, &lds_bytes);
+    if (n > 0) {
+#define LO_WIDE(IdT)                                                                                                     \
+  hipLaunchKernelGGL(moe_align_wide_kernel<IdT>, dim3(n), dim3(kWideT), lds_bytes, s, static_cast<const IdT *>(topk_ids), \
+                     numel, num_experts, block_size, expert_map, ignore_invalid, sorted_ids, sorted_cap, expert_ids,     \
+                     expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, num_local_tokens, top_k)
+      if (ids_dtype == LO_I32) LO_WIDE(int32_t);
+      else LO_WIDE(int64_t);
+#undef LO_WIDE
+      return check_launch("moe_align_block_size(wide)");
+    }
+  }
   const int64_t want = lo_moe_align_scratch_bytes(numel, num_experts);
   if (want > 0 && scratch && scratch_bytes >= want && (reinterpret_cast<uintptr_t>(scratch) & 3) == 0) {
     int nchunks;
