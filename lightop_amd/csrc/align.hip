@@ -233,12 +233,13 @@ __global__ __launch_bounds__(1024) void quant_align_kernel(
   }
 }
 
-constexpr int kWideT = 1024;
-// The alignment by `nchunks` workgroups of 1024 slots each, a wave's 64 its own, in one launch: every workgroup counts the slots
+constexpr int kWideSlots = 1024; // of a chunk
+constexpr int kWideT = 1024, kNarrowT = 256;
+// The alignment by `nchunks` workgroups of 1024 slots each, a wave's T / 16 its own, in one launch: every workgroup counts the slots
 // before and behind its own for itself (from L2), so nothing has to be counted before it starts.  It is a chain of round trips, to
 // memory for the ids and in LDS, and one sweep's worth of LDS atomics; the padding and the expert ids are written by sixteen
 // lanes an expert.  Chunks, waves and lanes are in slot order: the order is the same stable one.
-template <typename IdT>
+template <typename IdT, int T>
 __device__ __forceinline__ void moe_align_wide_body(
     const IdT *__restrict__ ids, int64_t numel64, int E, int bs, const int32_t *__restrict__ expert_map,
     int ignore_invalid, int32_t *__restrict__ sorted, int64_t sorted_cap, int32_t *__restrict__ expert_ids,
@@ -246,7 +247,7 @@ __device__ __forceinline__ void moe_align_wide_body(
     const int32_t *__restrict__ num_local_tokens, int slots_per_token, int chunk, int nchunks) {
   extern __shared__ int32_t lds[];
   const int pad_val = static_cast<int>(numel64);
-  constexpr int T = kWideT, nw = T / kWave;
+  constexpr int nw = T / kWave, kTiles = kWideSlots / T; // waves; tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int32_t *offs = lds;            // [E + 1] padded exclusive prefix
   int32_t *total = lds + (E + 1); // [E] slots in later chunks; then in all
@@ -255,8 +256,10 @@ __device__ __forceinline__ void moe_align_wide_body(
   int32_t *wcnt = emap + E;       // [nw][E]
   __shared__ int32_t wave_sum[16];
 
-  const int own = chunk * T + tid;
-  const IdT own_raw = pad_val > 0 ? ids[own < pad_val ? own : 0] : IdT(0);
+  const int own = chunk * kWideSlots + wave * (kTiles * kWave) + lane; // the lane's slots: own, own + 64, ...
+  IdT own_raw[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) own_raw[t] = pad_val > 0 ? ids[own + t * kWave < pad_val ? own + t * kWave : 0] : IdT(0);
   const int numel = static_cast<int>(local_slots(numel64, num_local_tokens, slots_per_token));
   for (int i = tid; i < nw * E; i += T) wcnt[i] = 0;
   for (int e = tid; e < E; e += T) {
@@ -274,26 +277,70 @@ __device__ __forceinline__ void moe_align_wide_body(
     }
     return e;
   };
-  bool ok;
-  const int ek = key_of(own_raw, own < numel, ok);
+  bool ok[kTiles];
+  int ek[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) ek[t] = key_of(own_raw[t], own + t * kWave < numel, ok[t]);
   __syncthreads();
-  if (ok) atomicAdd(&wcnt[wave * E + ek], 1);
-  if (slot_mask && own < pad_val) slot_mask[own] = ok && (ignore_invalid || emap[ek] >= 0) ? 1 : 0; // is the slot's expert held by this rank?
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    if (ok[t]) atomicAdd(&wcnt[wave * E + ek[t]], 1);
+    if (slot_mask && own + t * kWave < pad_val) // is the slot's expert held by this rank?
+      slot_mask[own + t * kWave] = ok[t] && (ignore_invalid || emap[ek[t]] >= 0) ? 1 : 0;
+  }
   constexpr int kSweep = 16; // loads in flight per thread
-  for (int u0 = 0; u0 < nchunks; u0 += kSweep) {
-    IdT raw[kSweep];
+  if constexpr (T == kWideSlots) {
+    for (int u0 = 0; u0 < nchunks; u0 += kSweep) {
+      IdT raw[kSweep];
 #pragma unroll
-    for (int u = 0; u < kSweep; ++u) {
-      const int f = (u0 + u) * T + tid;
-      if (u0 + u < nchunks) raw[u] = ids[f < numel ? f : 0];
+      for (int u = 0; u < kSweep; ++u) {
+        const int f = (u0 + u) * T + tid;
+        if (u0 + u < nchunks) raw[u] = ids[f < numel ? f : 0];
+      }
+#pragma unroll
+      for (int u = 0; u < kSweep; ++u) {
+        const int c = u0 + u;
+        if (c >= nchunks) break;
+        bool in;
+        const int e = key_of(raw[u], c != chunk && c * T + tid < numel, in);
+        if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+      }
     }
+  } else { // four ids a load
+    typedef IdT v4id __attribute__((ext_vector_type(4)));
+    const bool aligned = (reinterpret_cast<uintptr_t>(ids) & (sizeof(v4id) - 1)) == 0;
+    const int full = aligned ? numel / kWideSlots : 0;
+    constexpr int kV = kSweep / (sizeof(IdT) / 4);
+    for (int c0 = 0; c0 < full; c0 += kV) {
+      v4id raw[kV];
 #pragma unroll
-    for (int u = 0; u < kSweep; ++u) {
-      const int c = u0 + u;
-      if (c >= nchunks) break;
-      bool in;
-      const int e = key_of(raw[u], c != chunk && c * T + tid < numel, in);
-      if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+      for (int u = 0; u < kV; ++u)
+        if (c0 + u < full) raw[u] = *reinterpret_cast<const v4id *>(ids + (c0 + u) * kWideSlots + tid * 4);
+#pragma unroll
+      for (int u = 0; u < kV; ++u) {
+        const int c = c0 + u;
+        if (c >= full) break;
+        if (c == chunk) continue;
+        int32_t *const to = c < chunk ? cbase : total;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          bool in;
+          const int e = key_of(raw[u][i], true, in);
+          if (in) atomicAdd(&to[e], 1);
+        }
+      }
+    }
+    for (int f0 = full * kWideSlots + tid; f0 < numel; f0 += kSweep * T) {
+      IdT raw[kSweep];
+#pragma unroll
+      for (int u = 0; u < kSweep; ++u) raw[u] = ids[f0 + u * T < numel ? f0 + u * T : 0];
+#pragma unroll
+      for (int u = 0; u < kSweep; ++u) {
+        const int f = f0 + u * T, c = f / kWideSlots;
+        bool in;
+        const int e = key_of(raw[u], c != chunk && f < numel, in);
+        if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+      }
     }
   }
   __syncthreads();
@@ -328,9 +375,19 @@ __device__ __forceinline__ void moe_align_wide_body(
     __syncthreads();
   }
   // this wave's slots: ranks inside the 64 from a ballot match
-  {
-    const uint64_t peers = match_any(ek, key_bits, ok);
-    if (ok) sorted[offs[ek] + wcnt[wave * E + ek] + __popcll(peers & ((1ull << lane) - 1ull))] = own;
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    const uint64_t peers = match_any(ek[t], key_bits, ok[t]);
+    if (ok[t]) {
+      const int run = wcnt[wave * E + ek[t]];
+      sorted[offs[ek[t]] + run + __popcll(peers & ((1ull << lane) - 1ull))] = own + t * kWave;
+      if (t + 1 < kTiles) {
+        __builtin_amdgcn_wave_barrier();
+        if (lane == __ffsll(static_cast<unsigned long long>(peers)) - 1) wcnt[wave * E + ek[t]] = run + __popcll(peers);
+      }
+    }
+    asm volatile("" ::: "memory"); // a wave's LDS operations execute in order: no wait for the global stores
+    __builtin_amdgcn_wave_barrier();
   }
   // padding and expert ids, shared out by expert among the chunks, sixteen lanes to an expert; what lies past the last block
   const int P = offs[E];
@@ -340,8 +397,9 @@ __device__ __forceinline__ void moe_align_wide_body(
     for (int i = o0 + total[e] + (tid & 15); i < o1; i += 16) sorted[i] = pad_val;
     for (int b = o0 / bs + (tid & 15); b < o1 / bs; b += 16) expert_ids[b] = v;
   }
-  for (int64_t i = P + own; i < sorted_cap; i += nchunks * T) sorted[i] = pad_val;
-  for (int64_t b = P / bs + own; b < expert_ids_cap; b += nchunks * T) expert_ids[b] = -1;
+  const int mine = chunk * T + tid;
+  for (int64_t i = P + mine; i < sorted_cap; i += nchunks * T) sorted[i] = pad_val;
+  for (int64_t b = P / bs + mine; b < expert_ids_cap; b += nchunks * T) expert_ids[b] = -1;
 }
 
 template <typename IdT>
@@ -351,20 +409,20 @@ __global__ __launch_bounds__(1024) void moe_align_wide_kernel(
     int64_t sorted_cap, int32_t *__restrict__ expert_ids, int64_t expert_ids_cap,
     int32_t *__restrict__ ntpp, int key_bits, uint8_t *__restrict__ slot_mask,
     const int32_t *__restrict__ num_local_tokens, int slots_per_token) {
-  moe_align_wide_body<IdT>(ids, numel, num_experts, bs, expert_map, ignore_invalid, sorted, sorted_cap, expert_ids,
+  moe_align_wide_body<IdT, kWideT>(ids, numel, num_experts, bs, expert_map, ignore_invalid, sorted, sorted_cap, expert_ids,
                            expert_ids_cap, ntpp, key_bits, slot_mask, num_local_tokens, slots_per_token,
                            static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
 }
 
 // The first nchunks workgroups align, the others quantise the activations: two independent stages, one launch.
-template <typename IdT, bool PER_ROW, int DT>
-__global__ __launch_bounds__(1024) void quant_align_wide_kernel(
+template <typename IdT, bool PER_ROW, int DT, int T>
+__global__ __launch_bounds__(T) void quant_align_wide_kernel(
     const QuantJob job, const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
     const int32_t *__restrict__ expert_map, int32_t *__restrict__ sorted, int64_t sorted_cap,
     int32_t *__restrict__ expert_ids, int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits,
     uint8_t *__restrict__ slot_mask, int nchunks) {
   if (static_cast<int>(blockIdx.x) < nchunks) {
-    moe_align_wide_body<IdT>(ids, numel, num_experts, bs, expert_map, 0, sorted, sorted_cap, expert_ids, expert_ids_cap,
+    moe_align_wide_body<IdT, T>(ids, numel, num_experts, bs, expert_map, 0, sorted, sorted_cap, expert_ids, expert_ids_cap,
                              ntpp, key_bits, slot_mask, nullptr, 1, static_cast<int>(blockIdx.x), nchunks);
   } else {
     quant_job<PER_ROW, DT>(job, blockIdx.x - nchunks, gridDim.x - nchunks);
@@ -649,11 +707,17 @@ static void single_wg_shape(int64_t numel, int64_t sorted_cap, int32_t num_exper
 // workgroups are slower than the two launches past 32768 slots: the share at 5000, 6000, 8192 tokens 531 / 533, 575 / 581, 710 /
 // 716; quantisation by row, past 28672: per-channel Qwen3-30B-A3B layer at 3500, 4000, 8000 276.1 / 274.6, 317.3 / 319.2, 518 / 523.
 constexpr int64_t kWideQuantSlots = 32768, kWideRowQuantSlots = 28672, kWideAlignSlots = 65536;
+// By workgroups of 256 instead: the quantisation of 29 million values takes 19.8 us beside them, 25.5 beside those of 1024, the
+// alignment of 65536 slots 23.5 instead of 21.6.  Whole layer, us, the other form / this: DeepSeek-V3 share (896 values a slot) at
+// 2100 tokens 327 / 328, 3000: 375 / 375, 4096: 470 / 466, 8192: 713 / 710, 24000: 1913 / 1907, by row 2500: 322.6 / 324.2,
+// 4096: 448 / 445, 8192: 645 / 639; int4 layer with 512 values a slot at 2048 tokens 546 / 548; Qwen3-30B-A3B layer (256) at 4000
+// 321 / 325, 8192: 561 / 563.
+constexpr int64_t kNarrowFrom = 24576, kNarrowSlots = 262144, kNarrowValues = 700;
 static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, size_t *lds_bytes) {
   const int64_t words = (kWideT / kWave + 4) * static_cast<int64_t>(num_experts) + 1;
-  if (numel <= kWideT || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || words > 15360) return 0;
+  if (numel <= kWideSlots || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || words > 15360) return 0;
   *lds_bytes = static_cast<size_t>(words) * sizeof(int32_t);
-  return static_cast<int>((numel + kWideT - 1) / kWideT);
+  return static_cast<int>((numel + kWideSlots - 1) / kWideSlots);
 }
 
 static void align_chunks(int64_t numel, int *nchunks, int64_t *chunk_slots) {
@@ -705,15 +769,25 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
   const int64_t groups = M * (H / kGroup);
   {
     size_t lds_bytes;
-    const int n = wide_shape(numel, num_experts, per_row ? kWideRowQuantSlots : kWideQuantSlots, &lds_bytes);
+    // Long rows: the quantisation, faster by small workgroups, takes longer than an alignment by small ones.
+    const bool narrow = numel > kNarrowFrom && M * H >= kNarrowValues * numel;
+    const int n = wide_shape(numel, num_experts, narrow ? kNarrowSlots : per_row ? kWideRowQuantSlots : kWideQuantSlots, &lds_bytes);
     if (n > 0) {
-      int64_t qblocks = per_row ? (M + 3) / 4 : (groups + kWideT / 16 - 1) / (kWideT / 16);
-      if (qblocks > 4096) qblocks = 4096;
-      const dim3 grid(static_cast<unsigned>(n + qblocks)), block(kWideT);
-#define LO_QA_WIDE(IdT, PR, DT)                                                                                          \
-  hipLaunchKernelGGL((quant_align_wide_kernel<IdT, PR, DT>), grid, block, lds_bytes, stream, job,                        \
+      const int T = narrow ? kNarrowT : kWideT;
+      const int64_t most = narrow ? 8192 : 4096;
+      int64_t qblocks = per_row ? (M + T / 256 - 1) / (T / 256) : (groups + T / 16 - 1) / (T / 16);
+      if (qblocks > most) qblocks = most;
+      if (narrow) lds_bytes = ((kNarrowT / kWave + 4) * static_cast<size_t>(num_experts) + 1) * sizeof(int32_t);
+      const dim3 grid(static_cast<unsigned>(n + qblocks)), block(T);
+#define LO_QA_WIDE2(IdT, PR, DT, TT)                                                                                     \
+  hipLaunchKernelGGL((quant_align_wide_kernel<IdT, PR, DT, TT>), grid, block, lds_bytes, stream, job,                    \
                      static_cast<const IdT *>(topk_ids), numel, num_experts, block_size, expert_map, sorted_ids,         \
                      sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, n)
+#define LO_QA_WIDE(IdT, PR, DT)                          \
+  do {                                                   \
+    if (narrow) LO_QA_WIDE2(IdT, PR, DT, kNarrowT);      \
+    else LO_QA_WIDE2(IdT, PR, DT, kWideT);               \
+  } while (0)
       LO_QA_DISPATCH(LO_QA_WIDE);
 #undef LO_QA_WIDE
       return check_launch("quant_align(wide)");

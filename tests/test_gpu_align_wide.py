@@ -79,3 +79,33 @@ def test_quantisation_beside_it(M, channel, share, dtype):
     got = run(slice(0, M))
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [12288, 12289, 12800, 16384])
+@pytest.mark.parametrize("channel,ids64,offset", [(False, False, 0), (False, True, 0), (False, False, 1), (True, True, 1)])
+def test_long_rows(M, channel, ids64, offset):
+    """768 values a slot: past 24576 slots by workgroups of 256 (four ids a load where their address allows it)."""
+    from lightop_amd import workloads as wl
+    from lightop_amd.moe import fused_experts_impl_int8, get_moe_cache, preshuffle_moe_weight
+
+    dev = torch.device("cuda:0")
+    print(f"[case] narrow alignment in the whole path M={M} channel={channel} ids64={ids64} offset={offset}", flush=True)
+    layer = dataclasses.replace(wl.TINY, H=1536, I=128, E_global=24, quant="channel" if channel else "block")
+    w1, w2, w1s, w2s = wl.make_weights(layer, seed=3, device=dev, gen_device="cuda")
+    w1, w2 = preshuffle_moe_weight(w1), preshuffle_moe_weight(w2)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn((M, layer.H), generator=g, device=dev).to(torch.bfloat16)
+    tw, ids = wl.route(layer, torch.randn((M + offset, layer.E_global), generator=g, device=dev))
+    ids = (ids.long() if ids64 else ids)[offset:]  # (two ids: half a 16-byte piece)
+    tw = tw[offset:]
+
+    def run(rows):
+        return fused_experts_impl_int8(
+            x[rows], w1, w2, tw[rows], ids[rows], get_moe_cache(2, 2 * layer.I, layer.H, dev, torch.bfloat16), use_int8_w8a8=True,
+            per_channel_quant=channel, global_num_experts=layer.E_global, expert_map=wl.expert_map_for(layer, dev), w1_scale=w1s,
+            w2_scale=w2s, block_shape=None if channel else [128, 128])
+
+    got = run(slice(0, M))
+    some = [slice(a, min(a + 512, M)) for a in sorted({0, M // 3 // 512 * 512, M // 2 // 512 * 512, (M - 1) // 512 * 512})]
+    for rows in some:
+        assert torch.equal(got[rows].view(torch.int16), run(rows).view(torch.int16))
