@@ -8,6 +8,11 @@
 // leaves the result open (which of several equal scores wins, the order of the fp32 sums)
 // the choice is fixed: the lower index wins, the selected weights are summed in selection
 // order, the full-row softmax sum is per-lane sequential followed by a butterfly.
+//
+// The scores of a row, and the biases, are asked for before the first is used, those past the last expert as the row's first:
+// each in a branch of its own they were two to eight round trips to memory.  Gate of 256 experts in 8 groups, us, before / now,
+// 64 rows 5.8 / 5.0, 4096: 7.6 / 7.2; without groups 4.9 / 4.5; softmax of 128 experts, 1 row 3.0 / 2.9, 256: 3.7 / 3.3, 512:
+// 4.8 / 4.0.
 #include "common.h"
 
 namespace lo {
@@ -83,7 +88,11 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const void *__restric
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int e = lane + 64 * j;
-    x[j] = e < E ? load_as_f32<DT>(gating, t * E + e) : kNeg;
+    x[j] = load_as_f32<DT>(gating, t * E + (e < E ? e : 0));
+  }
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    x[j] = lane + 64 * j < E ? x[j] : kNeg;
     mx = fmaxf(mx, x[j]);
   }
   mx = wave_max(mx);
@@ -136,6 +145,13 @@ __device__ __forceinline__ int group_of(const GateGroups &gg, int e) {
   return static_cast<int>((static_cast<uint32_t>(e) * gg.ginv) >> 20);
 }
 
+// the two largest so far
+__device__ __forceinline__ void top2(float v, float &t1, float &t2) {
+  const bool first = v > t1;
+  t2 = first ? t1 : v > t2 ? v : t2;
+  t1 = first ? v : t1;
+}
+
 template <int VPT, int DT, int BT, typename IdxT>
 __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void *__restrict__ input, const void *__restrict__ bias,
                                                              int64_t T, int E, GateGroups gg, int topk_group,
@@ -147,19 +163,24 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void *__restr
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + wv;
   if (t >= T) return;
   const int G = gg.G, gs = gg.gs, lpg = 1 << gg.lsh, kr = topk - n_share;
-  float c[VPT];
+  float xv[VPT], c[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j)
+    xv[j] = load_as_f32<DT>(input, t * E + (lane + 64 * j < E ? lane + 64 * j : 0));
+#pragma unroll
+  for (int j = 0; j < VPT; ++j)
+    c[j] = load_as_f32<BT>(bias, lane + 64 * j < E ? lane + 64 * j : 0);
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int e = lane + 64 * j;
-    if (e < E) {
-      const float xv = load_as_f32<DT>(input, t * E + e);
-      const float sg = 1.0f / (1.0f + det_expf(-xv));
-      c[j] = load_as_f32<BT>(bias, e) + sg;
-      sC[wv][e] = c[j];
-      sS[wv][e] = sg;
-    } else {
+    if (64 * j >= E) {
       c[j] = kNeg;
+      continue;
     }
+    const float sg = 1.0f / (1.0f + det_expf(-xv[j]));
+    c[j] = e < E ? c[j] + sg : kNeg;
+    sC[wv][e] = c[j];
+    sS[wv][e] = sg;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -171,16 +192,14 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void *__restr
     // order of the merges does not matter)
     const int g = lane >> gg.lsh, sub = lane & (lpg - 1);
     float t1 = kNeg, t2 = kNeg;
-    if (g < G)
-      for (int i = g * gs + sub; i < (g + 1) * gs; i += lpg) {
-        const float cv = sC[wv][i];
-        if (cv > t1) {
-          t2 = t1;
-          t1 = cv;
-        } else if (cv > t2) {
-          t2 = cv;
-        }
-      }
+    const float *const scores = sC[wv] + (g < G ? g * gs : 0);
+    for (int i0 = sub; i0 < gs + sub; i0 += 4 * lpg) { // (four LDS reads a round trip)
+      float cv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) cv[u] = scores[i0 + u * lpg < gs ? i0 + u * lpg : 0];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) top2(i0 + u * lpg < gs ? cv[u] : kNeg, t1, t2);
+    }
 #define LO_TOP2_MERGE(CTRL)                                  \
   do {                                                       \
     const float o1 = dpp_f<CTRL>(t1), o2 = dpp_f<CTRL>(t2);  \
@@ -201,13 +220,12 @@ __global__ __launch_bounds__(256) void moe_fused_gate_kernel(const void *__restr
       const float os = lane_f(gscore, o << gg.lsh);
       before += os > gscore || (os == gscore && o < g) ? 1 : 0;
     }
-    uint64_t lead = __builtin_amdgcn_ballot_w64(g < G && sub == 0 && before < topk_group);
-    for (keep = 0; lead; lead &= lead - 1) keep |= 1ull << (__builtin_ctzll(lead) >> gg.lsh);
+    keep = __builtin_amdgcn_ballot_w64(g < G && before < topk_group); // bit of group g: that of its first lane
   }
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int e = lane + 64 * j;
-    if (e < E && !((keep >> group_of(gg, e)) & 1)) c[j] = kNeg;
+    if (e < E && !((keep >> (group_of(gg, e) << gg.lsh)) & 1)) c[j] = kNeg;
   }
   float mine = 0.0f;
   int mine_idx = 0;
@@ -287,7 +305,11 @@ __global__ __launch_bounds__(256) void topk_softmax16_kernel(const void *__restr
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int e = sub + 16 * j;
-    x[j] = e < E ? load_as_f32<DT>(gating, t * E + e) : kNeg;
+    x[j] = load_as_f32<DT>(gating, t * E + (e < E ? e : 0));
+  }
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    x[j] = sub + 16 * j < E ? x[j] : kNeg;
     mx = fmaxf(mx, x[j]);
   }
   mx = row_max(mx);
@@ -344,20 +366,24 @@ __global__ __launch_bounds__(256) void moe_fused_gate16_kernel(const void *__res
   const bool active = t_raw < T;
   const int64_t t = active ? t_raw : T - 1;
   const int G = gg.G, gs = gg.gs, lpg = 1 << gg.lsh, kr = topk - n_share;
-  float s[VPT], c[VPT];
+  float xv[VPT], c[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j)
+    xv[j] = load_as_f32<DT>(input, t * E + (sub + 16 * j < E ? sub + 16 * j : 0));
+#pragma unroll
+  for (int j = 0; j < VPT; ++j)
+    c[j] = load_as_f32<BT>(bias, sub + 16 * j < E ? sub + 16 * j : 0);
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int e = sub + 16 * j;
-    if (e < E) {
-      const float xv = load_as_f32<DT>(input, t * E + e);
-      s[j] = 1.0f / (1.0f + det_expf(-xv));
-      c[j] = load_as_f32<BT>(bias, e) + s[j];
-      if (G > 1) sC[row][e] = c[j];
-      sS[row][e] = s[j];
-    } else {
-      s[j] = 0.0f;
+    if (16 * j >= E) {
       c[j] = kNeg;
+      continue;
     }
+    const float sg = 1.0f / (1.0f + det_expf(-xv[j]));
+    c[j] = e < E ? c[j] + sg : kNeg;
+    if (G > 1) sC[row][e] = c[j];
+    sS[row][e] = sg;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -366,16 +392,14 @@ __global__ __launch_bounds__(256) void moe_fused_gate16_kernel(const void *__res
   if (G > 1) { // G <= 16 (host check)
     const int g = sub >> gg.lsh, lsub = sub & (lpg - 1);
     float t1 = kNeg, t2 = kNeg;
-    if (g < G)
-      for (int i = g * gs + lsub; i < (g + 1) * gs; i += lpg) {
-        const float cv = sC[row][i];
-        if (cv > t1) {
-          t2 = t1;
-          t1 = cv;
-        } else if (cv > t2) {
-          t2 = cv;
-        }
-      }
+    const float *const scores = sC[row] + (g < G ? g * gs : 0);
+    for (int i0 = lsub; i0 < gs + lsub; i0 += 4 * lpg) {
+      float cv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) cv[u] = scores[i0 + u * lpg < gs ? i0 + u * lpg : 0];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) top2(i0 + u * lpg < gs ? cv[u] : kNeg, t1, t2);
+    }
 #define LO_TOP2_MERGE(CTRL)                                  \
   do {                                                       \
     const float o1 = dpp_f<CTRL>(t1), o2 = dpp_f<CTRL>(t2);  \
@@ -428,23 +452,21 @@ __global__ __launch_bounds__(256) void moe_fused_gate16_kernel(const void *__res
 // Rows from which the 16-lane kernels are used: below, a row per wavefront finishes sooner, since there are wavefront
 // slots to spare; above, a quarter of a wavefront per row leaves fewer instructions to issue.  The more experts, the longer
 // a quarter's chain and the later the line.  us, a wavefront / a quarter per row:
-//   softmax, 64 experts:  bf16 2048 rows 3.57 / 3.82, 2560: 3.99 / 3.83, 4096: 4.61 / 3.87
-//            128 experts: bf16 3072 rows 4.35 / 4.68, 3584: 4.87 / 4.68, 8192: 7.11 / 5.10
-//            256 experts: bf16 5120 rows 6.42 / 7.07, 5632: 7.04 / 7.10, 7168: 7.68 / 7.16; fp32 4096: 5.41 / 5.67, 4608: 6.11 / 5.96
-//   gate,    32 experts:  fp32 3072 rows 4.85 / 4.87, 4096: 5.30 / 4.88
-//            64 experts:  fp32 4096 rows 5.59 / 5.76, 5120: 6.20 / 6.00
-//            128 experts: fp32 6144 rows 7.54 / 8.21, 7168: 8.25 / 8.25, 8192: 8.94 / 8.27
-//            256 experts: fp32 8192 rows 11.5 / 13.2 (16 scores per lane): never
-template <int VPT, int DT> constexpr int64_t softmax_rows16_from() {
-  return VPT == 1 ? 2560 : VPT == 2 ? 3584 : DT == LO_F32 ? 4608 : 5632;
-}
-static int64_t gate_rows16_from(int E) { return E <= 32 ? 4096 : E <= 64 ? 4608 : 7168; }
+//   softmax, 64 experts:  bf16 2048 rows 3.50 / 3.58, 2560: 3.89 / 3.59, 4096: 4.42 / 3.60
+//            128 experts: bf16 2048 rows 3.64 / 3.77, 2560: 4.05 / 3.79, 8192: 6.83 / 4.34; fp32 the same
+//            256 experts: bf16 3072 rows 4.64 / 4.69, 3584: 5.19 / 4.70, 8192: 7.78 / 5.61; fp32 the same
+//   gate,    32 experts:  fp32 3072 rows 4.54 / 4.58, 3584: 5.10 / 4.59
+//            64 experts:  fp32 3072 rows 4.73 / 5.12, 3584: 5.34 / 5.11
+//            128 experts: fp32 5120 rows 6.57 / 7.28, 6144: 7.32 / 7.28, 8192: 8.71 / 7.30
+//            256 experts: fp32 8192 rows 10.9 / 11.4, 12288: 14.8 / 13.2, without groups 9.1 / 9.5, 12.1 / 11.3
+template <int VPT> constexpr int64_t softmax_rows16_from() { return VPT <= 2 ? 2560 : 3584; }
+static int64_t gate_rows16_from(int E) { return E <= 64 ? 3584 : E <= 128 ? 6144 : 12288; }
 
 template <int VPT, int DT> static void launch_topk_softmax(const void *g, int64_t T, int E, int k, int renorm,
                                                            float *w, void *idx, int idx_dtype, int32_t *src,
                                                            hipStream_t s) {
   if constexpr (VPT <= 4) { // up to 256 experts
-    if (T >= softmax_rows16_from<VPT, DT>() && k <= 16) {
+    if (T >= softmax_rows16_from<VPT>() && k <= 16) {
       const dim3 grid16(static_cast<unsigned>((T + 15) / 16)), block16(256);
       if (idx_dtype == LO_I64)
         hipLaunchKernelGGL((topk_softmax16_kernel<4 * VPT, DT, int64_t>), grid16, block16, 0, s, g, T, E, k, renorm, w,
@@ -469,7 +491,7 @@ static void launch_gate(const void *x, const void *b, int64_t T, int E, int G, i
                         float scale, float *w, void *idx, int idx_dtype, hipStream_t s) {
   GateGroups gg{G, E / G, 4, static_cast<uint32_t>(((1u << 20) + E / G - 1) / (E / G))};
   while ((G << gg.lsh) > 64) --gg.lsh;
-  if constexpr (VPT <= 2) { // up to 128 experts
+  if constexpr (VPT <= 4) { // up to 256 experts
     if (T >= gate_rows16_from(E) && topk <= 16 && G <= 16) {
       while ((G << gg.lsh) > 16) --gg.lsh;
       const dim3 grid16(static_cast<unsigned>((T + 15) / 16)), block16(256);
@@ -500,6 +522,7 @@ static bool float_dtype_ok(int dt) { return dt == LO_BF16 || dt == LO_F16 || dt 
     if ((E) <= 64) { CALL(1); }      \
     else if ((E) <= 128) { CALL(2); } \
     else if ((E) <= 256) { CALL(4); } \
+    else if ((E) <= 384) { CALL(6); } \
     else if ((E) <= 512) { CALL(8); } \
     else { CALL(16); }               \
   } while (0)

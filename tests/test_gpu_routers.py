@@ -205,3 +205,12 @@ def test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtyp
         w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, 2, k, 0, 2.5, False)
         rw, ridx = oracle.moe_fused_gate(x, bias, G, 2, k, 0, 2.5, False)
         assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
+
+
+@pytest.mark.parametrize("E,G,k,dtype,lines", [(64, 8, 8, torch.float32, (2560, 3584)), (128, 8, 8, torch.bfloat16, (2560, 6144)),
+                                               (256, 8, 8, torch.float32, (3584, 12288)), (200, 2, 8, torch.float16, (3584, 12288)),
+                                               (258, 3, 8, torch.float32, (64,)), (384, 12, 8, torch.float32, (64,)),
+                                               (385, 5, 8, torch.bfloat16, (64,))])
+def test_lines_with_all_scores_requested_at_once(dev, oracle, E, G, k, dtype, lines):
+    """Row counts around the lines of the kernels that request a row's scores together, and six scores a lane."""
+    test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtype, lines)
