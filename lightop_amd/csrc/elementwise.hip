@@ -296,9 +296,9 @@ static void launch_row_quant(const uint16_t *x, int64_t rows, int64_t C, const u
 // What it is bound by is memory: rows are read once, with the streaming hint (8192 tokens of the full DeepSeek-V3 layer 241 ->
 // 214 us, 5.5 TB/s, of the Qwen3-30B-A3B layer 51.9 -> 46.7, 6.5 TB/s), the mask a token ahead (DeepSeek-V3 share, 4096 tokens
 // 42.3 -> 33.3 us, of them the mask 10).
-// A workgroup takes 2048 columns of one token after the other (a flat index over all of them costs a 64-bit division in
+// A workgroup takes 2048 or 4096 columns of one token after the other (a flat index over all of them costs a 64-bit division in
 // front of the first load).
-constexpr int kSumThreads = 256;
+constexpr int kSumThreads = 512;
 template <int DT, bool HAS_BIAS, int TOPK>
 __global__ __launch_bounds__(kSumThreads) void moe_sum_kernel(const uint16_t *__restrict__ in,
                                                       uint16_t *__restrict__ out,
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(kSumThreads) void moe_sum_kernel(const uint16_t *__
     const int64_t n = num_local_tokens[0];
     M = n < M ? n : M;
   }
-  const int64_t c = (static_cast<int64_t>(blockIdx.y) * kSumThreads + threadIdx.x) * 8;
+  const int64_t c = (static_cast<int64_t>(blockIdx.y) * blockDim.x + threadIdx.x) * 8;
   if (c >= H) return;
   // The next token's mask is asked for a token ahead: behind its own it is a second memory round trip.
   uint8_t m_next[TOPK > 0 ? TOPK : 1];
@@ -659,14 +659,20 @@ extern "C" int lo_moe_sum(const void *in, void *out, const void *bias, const uin
     return launch_moe_sum_f32(static_cast<const float *>(in), static_cast<float *>(out),
                               static_cast<const float *>(bias), expert_mask, M, topk, H, factor, num_local_tokens,
                               static_cast<hipStream_t>(stream));
-  const int64_t cols = (H / 8 + kSumThreads - 1) / kSumThreads;
-  LO_REQUIRE(cols < 65536, LO_ENOTSUP, "moe_sum: rows of %lld values", (long long)H);
-  int64_t tokens = 4096 / cols; // sixteen workgroups per CU: what is resident, twice
+  // Rows of more than 4096 values: workgroups of 512 threads (7168 values in 256-thread ones: an eighth of the lanes have no
+  // column).  With a mask, once the card is full, two or more tokens a workgroup, whose masks are asked for ahead; without, one.
+  // us: DeepSeek-V3 share, 4096 tokens 34.0 -> 31.1, full layer, 8192 210.6 -> 197.1 (5.9 TB/s; 512 threads and several tokens 204).
+  // Below, the smaller ones are spread better (share, 64 tokens, whole layer 201.2, else 201.6).
+  const int threads = H > 4096 && M * ((H + 2047) / 2048) > 2048 ? kSumThreads : 256;
+  LO_REQUIRE((H + 2047) / 2048 < 65536, LO_ENOTSUP, "moe_sum: rows of %lld values", (long long)H);
+  const int64_t cols = (H / 8 + threads - 1) / threads;
+  int64_t tokens = 65536 / cols;
+  if (expert_mask && M * cols > 2048) tokens = 4096 / cols < M / 2 ? 4096 / cols : M / 2;
   tokens = tokens < 1 ? 1 : (tokens < M ? tokens : M);
   const dim3 grid(static_cast<unsigned>(tokens), static_cast<unsigned>(cols));
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define LO_SUM_LAUNCH(DTV, HB, TK)                                                                   \
-  hipLaunchKernelGGL((moe_sum_kernel<DTV, HB, TK>), grid, dim3(kSumThreads), 0, s,                  \
+  hipLaunchKernelGGL((moe_sum_kernel<DTV, HB, TK>), grid, dim3(threads), 0, s,                  \
                      static_cast<const uint16_t *>(in), static_cast<uint16_t *>(out),               \
                      static_cast<const uint16_t *>(bias), expert_mask, M, topk, H, factor, num_local_tokens)
 #define LO_SUM_PICK(TK)                                                                              \
