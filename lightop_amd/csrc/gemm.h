@@ -142,6 +142,14 @@ __device__ __forceinline__ int token_row(const GemmArgs &a, int64_t slot) {
   return slot < a.num_valid ? static_cast<int>(row) : 0;
 }
 
+// Routed weight of a slot, 1 where it is not wanted: asked for at a kernel's start, in front of the K loop's loads.  In the
+// epilogue it is a round trip to memory for every token fragment, each in a branch of its own.  Weight-streaming kernel,
+// Qwen3-30B-A3B layer at 24 / 60 tokens 96.1 -> 95.6, 110.0 -> 109.6 us, DeepSeek-V3 share at 160 234.7 -> 234.3; 64-token int4
+// tiles, 400 tokens 282.0 -> 281.1.  (The 64-token int8 kernels gain nothing: 333 tokens 121.1 / 121.3, 500: 124.7 / 125.4.)
+__device__ __forceinline__ float slot_weight(const GemmArgs &a, int64_t slot) {
+  return a.mul_routed ? a.topk_w[slot < a.num_valid ? slot : 0] : 1.0f;
+}
+
 // The 16-bit form a plain epilogue stores: bf16, or IEEE half when the caller's activations are fp16.
 // `body(cvt)` is run with the conversion of the output type; the choice is one wave-uniform branch
 // around the caller's loops, so the bf16 path pays nothing per value (a per-value select cost the

@@ -41,6 +41,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   __shared__ __attribute__((aligned(16))) int8_t sA[2][kTileM * kW4Row];
   __shared__ float sS[2][kTileM];
   __shared__ float sRed[4][kTileM];
+  __shared__ int32_t sIds[kTileM]; // the slots, for the fused epilogue's rows
   extern __shared__ __attribute__((aligned(16))) float sRowScale[]; // [K block][256 rows], already / 16
 
   int mb, nt;
@@ -67,10 +68,12 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
   // slots of the four 16-token fragments this lane sees in the accumulator layout
   int64_t f[4];
   bool valid[4];
+  float wgt[4];
 #pragma unroll
   for (int tf = 0; tf < 4; ++tf) {
     f[tf] = ids[tf];
     valid[tf] = f[tf] < a.num_valid;
+    wgt[tf] = slot_weight(a, f[tf]);
   }
 
   // weight rows of the wave: four 16-row fragments
@@ -97,6 +100,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 
   // cooperative gather role: thread -> (token, 32-byte quarter of the 128-byte K block)
   const int lt = tid >> 2, lq = tid & 3;
+  if (FUSED_ACT && lq == 0) sIds[lt] = lf;
   const int64_t lrow = token_row(a, lf);
   const brsrc rA = make_rsrc(a.A, static_cast<uint32_t>(a.a_rows * K));
   const brsrc rAs = make_rsrc(a.As, static_cast<uint32_t>(a.a_rows * KB * 4));
@@ -277,8 +281,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     int8_t *stg = &sA[0][0] + wr * (16 * kW4Row);
 #pragma unroll
     for (int tf = 0; tf < 4; ++tf) {
-      float w = 1.0f;
-      if (a.mul_routed && valid[tf]) w = a.topk_w[f[tf]];
+      const float w = wgt[tf];
       with_out16(a.out_f16, [&](auto cvt) __attribute__((always_inline)) {
 #pragma unroll
         for (int rf = 0; rf < 4; ++rf) {
@@ -310,8 +313,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
     float actf[4][2][4];
 #pragma unroll
     for (int tf = 0; tf < 4; ++tf) {
-      float w = 1.0f;
-      if (a.mul_routed && valid[tf]) w = a.topk_w[f[tf]];
+      const float w = wgt[tf];
       float amax = 0.0f;
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
@@ -359,7 +361,7 @@ void moe_gemm_w4_tile_kernel(const GemmArgs a, int m_blocks, int group_m) {
 #pragma unroll
     for (int j = 0; j < kTileM * 8 / 256; ++j) {
       const int id = tid + 256 * j, tok = id >> 3, piece = id & 7;
-      const int64_t ft = a.sorted[static_cast<int64_t>(mb) * kTileM + tok];
+      const int64_t ft = sIds[tok];
       if (ft < a.num_valid)
         *reinterpret_cast<v4i *>(a.A2q + ft * I + static_cast<int64_t>(nt) * kGroup + piece * 16) =
             *reinterpret_cast<const v4i *>(qst + tok * kW4Row + piece * 16);

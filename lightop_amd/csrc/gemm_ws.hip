@@ -80,11 +80,13 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   // tokens of this block, one per (sub-tile, r)
   int64_t f[TM];
   bool valid[TM];
+  float wgt[TM];
   int aoff[TM], asoff[TM]; // byte offsets of the token's row in A and As
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     f[j] = ids[j];
     valid[j] = f[j] < a.num_valid;
+    wgt[j] = slot_weight(a, f[j]);
     const int64_t row = token_row(a, f[j]);
     aoff[j] = static_cast<int>(row * K) + c * 16;
     asoff[j] = static_cast<int>(row * (PC ? 1 : KB) * 4);
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
     for (int j = 0; j < TM; ++j) {
       if (!valid[j]) continue;
       const float as = bld_f32(rAs, asoff[j], 0);
-      const float w = a.mul_routed ? a.topk_w[f[j]] : 1.0f;
+      const float w = wgt[j];
       const float ts = a.mul_routed ? w * as : as;
 #pragma unroll
       for (int g = 0; g < NW; ++g) {
@@ -371,8 +373,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
       if (!valid[j]) continue;
-      float w = 1.0f;
-      if (a.mul_routed) w = a.topk_w[f[j]];
+      const float w = wgt[j];
 #pragma unroll
       for (int g = 0; g < NW; ++g) {
         if (nrow[g] >= N) continue;
@@ -400,8 +401,7 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
     float actf[TM][4];
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-      float w = 1.0f;
-      if (a.mul_routed && valid[j]) w = a.topk_w[f[j]];
+      const float w = wgt[j];
       float amax = 0.0f;
       float g[4], u[4];
 #pragma unroll
