@@ -497,7 +497,11 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
         for (int g = 0; g < 4; ++g) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           if (st * per + g < kCopies && g < per) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, decltype(BIASED)::value ? 4 : 6, 0);
+          // The products close up and the folds stand behind them, as in 128-token tiles (below): four after each / this, 128 experts
+          // of 4096 x 1536 at 1800 / 2048 tokens 492 / 484, 534 / 526 us.
+          if (!decltype(BIASED)::value) __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+          else if (g < 3) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -626,15 +630,16 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           if (nst_c >= 8 ? ((g < 2 && st < 6) || (NTB == 10 && g == 0 && st == 6)) : (g < 3 && st < 4))
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-          // 128-token int8 tiles close the stage's products up and fold behind them.  Four after each / this, whole layer, us: all
-          // experts of DeepSeek-V3, skewed, 5500 tokens 3244 / 3222, 8192: 4457 / 4430, 12000: 6253 / 6204; share 7000: 650 / 647;
-          // Qwen3-235B-A22B-shaped layer 3000: 832 / 823, 6500: 1500 / 1498; Qwen3-30B-A3B layer 3000 and 8192: equal.  Tiles of
-          // 160 lose (1531 tokens 177 / 180).
-          if constexpr (decltype(BIASED)::value && !PC && !W4 && NTB == 8) {
+          // 128-token tiles close the stage's products up and fold behind them.  Four (int4: five) after each / this, whole layer,
+          // us: all experts of DeepSeek-V3, skewed, 5500 tokens 3244 / 3222, 8192: 4457 / 4430, 12000: 6253 / 6204; share 7000:
+          // 650 / 647; Qwen3-235B-A22B-shaped layer 3000: 832 / 823, 6500: 1500 / 1498; Qwen3-30B-A3B layer 3000 and 8192: equal; int4
+          // with K-group scales, 128 experts of 4096 x 1536, 1100: 375 / 366, 2800: 724 / 711, 6000: 1313 / 1291.  int8 tiles of 160
+          // lose (1531 tokens 177 / 180).
+          if constexpr (decltype(BIASED)::value && !PC && (W4 || NTB == 8)) {
             if (g < 3) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-            else __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x002, W4 ? 14 : 10, 0);
           } else {
-            __builtin_amdgcn_sched_group_barrier(0x002, decltype(BIASED)::value ? (W4 ? 5 : 4) : W4 ? 7 : 5, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, decltype(BIASED)::value ? 4 : W4 ? 7 : 5, 0);
           }
         }
         if (kEarly && st == kE0) __builtin_amdgcn_sched_group_barrier(0x100, 7, 0);
