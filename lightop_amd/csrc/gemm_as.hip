@@ -31,8 +31,8 @@ void moe_gemm_as_kernel(const GemmArgs a, int m_blocks, int group_m,
   const int K = static_cast<int>(a.K);
   const int KB = K / kGroup;
   // Tokens in operand order: K half kh of K block kb of token fragment tb is the 1 KB at ((2 kb + kh) * 4 + tb) * 1024, lane after
-  // lane.  A read of 64 consecutive pieces has no bank conflict (rows 16 bytes past a multiple of 128 had 1.08e7 on the
-  // Qwen3-30B-A3B layer's second stage at 8192 tokens) and the rows need no registers on their way here.
+  // lane.  A read of 64 consecutive pieces has no bank conflict (SQ_LDS_BANK_CONFLICT of the Qwen3-30B-A3B layer's second stage at
+  // 8192 tokens 1.08e7 -> 3.3e6, the output staging's) and the rows need no registers on their way here.
   int8_t *const sA = smem;
   float *const sS = reinterpret_cast<float *>(smem + kTileM * K); // [KB][64]
   // per-wave staging of 16 output rows x 64 columns (bf16), for row-contiguous stores
