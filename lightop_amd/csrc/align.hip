@@ -235,25 +235,29 @@ __global__ __launch_bounds__(1024) void quant_align_kernel(
 
 constexpr int kWideSlots = 1024; // of a chunk
 constexpr int kWideT = 1024, kNarrowT = 256;
+constexpr int kMostCopyBits = 2, kMostCopies = 1 << kMostCopyBits; // of the counters of a sweep
 // The alignment by `nchunks` workgroups of 1024 slots each, a wave's T / 16 its own, in one launch: every workgroup counts the slots
 // before and behind its own for itself (from L2), so nothing has to be counted before it starts.  It is a chain of round trips, to
 // memory for the ids and in LDS, and one sweep's worth of LDS atomics; the padding and the expert ids are written by sixteen
 // lanes an expert.  Chunks, waves and lanes are in slot order: the order is the same stable one.
+// An expert's counters of the sweep are 1 << copy_bits copies, a lane's by its place in the wave: lanes that add to one word take
+// turns, and rows routed alike (padding tokens, or every token to one expert) are 16 to 64 such lanes in every instruction.
 template <typename IdT, int T>
 __device__ __forceinline__ void moe_align_wide_body(
     const IdT *__restrict__ ids, int64_t numel64, int E, int bs, const int32_t *__restrict__ expert_map,
     int ignore_invalid, int32_t *__restrict__ sorted, int64_t sorted_cap, int32_t *__restrict__ expert_ids,
     int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits, uint8_t *__restrict__ slot_mask,
-    const int32_t *__restrict__ num_local_tokens, int slots_per_token, int chunk, int nchunks) {
+    const int32_t *__restrict__ num_local_tokens, int slots_per_token, int copy_bits, int chunk, int nchunks) {
   extern __shared__ int32_t lds[];
   const int pad_val = static_cast<int>(numel64);
   constexpr int nw = T / kWave, kTiles = kWideSlots / T; // waves; tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int32_t *offs = lds;            // [E + 1] padded exclusive prefix
-  int32_t *total = lds + (E + 1); // [E] slots in later chunks; then in all
-  int32_t *cbase = total + E;     // [E] slots in earlier chunks
-  int32_t *emap = cbase + E;      // [E] what expert_ids says of a block
-  int32_t *wcnt = emap + E;       // [nw][E]
+  const int copies = 1 << copy_bits, copy = lane >> (6 - copy_bits);
+  int32_t *offs = lds;                         // [E + 1] padded exclusive prefix
+  int32_t *emap = lds + (E + 1);               // [E] what expert_ids says of a block
+  int32_t *wcnt = emap + E;                    // [nw][E]
+  int32_t *later = wcnt + nw * E;              // [E][copies] slots in later chunks; then, in the first copy, in all
+  int32_t *earlier = later + (E << copy_bits); // [E][copies] slots in earlier chunks
   __shared__ int32_t wave_sum[16];
 
   const int own = chunk * kWideSlots + wave * (kTiles * kWave) + lane; // the lane's slots: own, own + 64, ...
@@ -261,11 +265,8 @@ __device__ __forceinline__ void moe_align_wide_body(
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) own_raw[t] = pad_val > 0 ? ids[own + t * kWave < pad_val ? own + t * kWave : 0] : IdT(0);
   const int numel = static_cast<int>(local_slots(numel64, num_local_tokens, slots_per_token));
-  for (int i = tid; i < nw * E; i += T) wcnt[i] = 0;
-  for (int e = tid; e < E; e += T) {
-    total[e] = cbase[e] = 0;
-    emap[e] = (expert_map && !ignore_invalid) ? expert_map[e] : e;
-  }
+  for (int i = tid; i < (nw + 2 * copies) * E; i += T) wcnt[i] = 0;
+  for (int e = tid; e < E; e += T) emap[e] = (expert_map && !ignore_invalid) ? expert_map[e] : e;
   auto key_of = [&](IdT id, bool in_range, bool &ok) __attribute__((always_inline)) {
     const int64_t raw = static_cast<int64_t>(id);
     ok = in_range && raw >= 0 && raw < E;
@@ -303,7 +304,7 @@ __device__ __forceinline__ void moe_align_wide_body(
         if (c >= nchunks) break;
         bool in;
         const int e = key_of(raw[u], c != chunk && c * T + tid < numel, in);
-        if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+        if (in) atomicAdd(&(c < chunk ? earlier : later)[(e << copy_bits) + copy], 1);
       }
     }
   } else { // four ids a load
@@ -321,12 +322,12 @@ __device__ __forceinline__ void moe_align_wide_body(
         const int c = c0 + u;
         if (c >= full) break;
         if (c == chunk) continue;
-        int32_t *const to = c < chunk ? cbase : total;
+        int32_t *const to = c < chunk ? earlier : later;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           bool in;
           const int e = key_of(raw[u][i], true, in);
-          if (in) atomicAdd(&to[e], 1);
+          if (in) atomicAdd(&to[(e << copy_bits) + copy], 1);
         }
       }
     }
@@ -339,7 +340,7 @@ __device__ __forceinline__ void moe_align_wide_body(
         const int f = f0 + u * T, c = f / kWideSlots;
         bool in;
         const int e = key_of(raw[u], c != chunk && f < numel, in);
-        if (in) atomicAdd(&(c < chunk ? cbase : total)[e], 1);
+        if (in) atomicAdd(&(c < chunk ? earlier : later)[(e << copy_bits) + copy], 1);
       }
     }
   }
@@ -348,18 +349,27 @@ __device__ __forceinline__ void moe_align_wide_body(
     const int e = base + tid;
     int t = 0;
     if (e < E) {
-      const int before = cbase[e];
-      int c = before;
-      int v[nw];
+      int c = 0;
+      int v[nw], n0[kMostCopies], n1[kMostCopies];
 #pragma unroll
       for (int w = 0; w < nw; ++w) v[w] = wcnt[w * E + e];
+#pragma unroll
+      for (int i = 0; i < kMostCopies; ++i) { // (all reads in one round trip: copies that are not there as the first)
+        n0[i] = earlier[(e << copy_bits) + (i & (copies - 1))];
+        n1[i] = later[(e << copy_bits) + (i & (copies - 1))];
+      }
+#pragma unroll
+      for (int i = 0; i < kMostCopies; ++i) {
+        c += i < copies ? n0[i] : 0;
+        t += i < copies ? n1[i] : 0;
+      }
 #pragma unroll
       for (int w = 0; w < nw; ++w) {
         wcnt[w * E + e] = c; // slots of expert e before this wave's
         c += v[w];
       }
-      t = total[e] + c;
-      total[e] = t;
+      t += c;
+      later[e << copy_bits] = t;
     }
     int incl = (t + bs - 1) / bs * bs;
     for (int d = 1; d < kWave; d <<= 1) {
@@ -394,7 +404,7 @@ __device__ __forceinline__ void moe_align_wide_body(
   if (chunk == 0 && tid == 0) ntpp[0] = P;
   for (int e = chunk + (tid >> 4) * nchunks; e < E; e += nchunks * (T >> 4)) {
     const int o0 = offs[e], o1 = offs[e + 1], v = emap[e];
-    for (int i = o0 + total[e] + (tid & 15); i < o1; i += 16) sorted[i] = pad_val;
+    for (int i = o0 + later[e << copy_bits] + (tid & 15); i < o1; i += 16) sorted[i] = pad_val;
     for (int b = o0 / bs + (tid & 15); b < o1 / bs; b += 16) expert_ids[b] = v;
   }
   const int mine = chunk * T + tid;
@@ -408,9 +418,9 @@ __global__ __launch_bounds__(1024) void moe_align_wide_kernel(
     const int32_t *__restrict__ expert_map, int ignore_invalid, int32_t *__restrict__ sorted,
     int64_t sorted_cap, int32_t *__restrict__ expert_ids, int64_t expert_ids_cap,
     int32_t *__restrict__ ntpp, int key_bits, uint8_t *__restrict__ slot_mask,
-    const int32_t *__restrict__ num_local_tokens, int slots_per_token) {
+    const int32_t *__restrict__ num_local_tokens, int slots_per_token, int copy_bits) {
   moe_align_wide_body<IdT, kWideT>(ids, numel, num_experts, bs, expert_map, ignore_invalid, sorted, sorted_cap, expert_ids,
-                           expert_ids_cap, ntpp, key_bits, slot_mask, num_local_tokens, slots_per_token,
+                           expert_ids_cap, ntpp, key_bits, slot_mask, num_local_tokens, slots_per_token, copy_bits,
                            static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
 }
 
@@ -420,10 +430,10 @@ __global__ __launch_bounds__(T) void quant_align_wide_kernel(
     const QuantJob job, const IdT *__restrict__ ids, int64_t numel, int num_experts, int bs,
     const int32_t *__restrict__ expert_map, int32_t *__restrict__ sorted, int64_t sorted_cap,
     int32_t *__restrict__ expert_ids, int64_t expert_ids_cap, int32_t *__restrict__ ntpp, int key_bits,
-    uint8_t *__restrict__ slot_mask, int nchunks) {
+    uint8_t *__restrict__ slot_mask, int copy_bits, int nchunks) {
   if (static_cast<int>(blockIdx.x) < nchunks) {
     moe_align_wide_body<IdT, T>(ids, numel, num_experts, bs, expert_map, 0, sorted, sorted_cap, expert_ids, expert_ids_cap,
-                             ntpp, key_bits, slot_mask, nullptr, 1, static_cast<int>(blockIdx.x), nchunks);
+                             ntpp, key_bits, slot_mask, nullptr, 1, copy_bits, static_cast<int>(blockIdx.x), nchunks);
   } else {
     quant_job<PER_ROW, DT>(job, blockIdx.x - nchunks, gridDim.x - nchunks);
   }
@@ -697,26 +707,40 @@ static void single_wg_shape(int64_t numel, int64_t sorted_cap, int32_t num_exper
   *lds_bytes = (static_cast<size_t>(w + 2) * num_experts + 1) * sizeof(int32_t);
 }
 
-// The one-launch form by several workgroups (moe_align_wide_body): their number, or 0 where another form is taken.  Every one of
-// them sweeps all slots, so `most` of them; below, one workgroup has nothing to share; and the counters are 4 (16 + 4) bytes of LDS
-// an expert.  Alignment alone, us, the other forms / this, at 1600, 4000, 8000, 16000, 32768 and 65536 slots: 128 experts 6.1 / 5.5,
-// 8.0 / 5.4, 10.8 / 5.8, 10.7 / 6.7, 11.7 / 9.1, 14.4 / 13.9; 256 experts 6.5 / 6.0, 8.4 / 5.9, 11.6 / 6.1, 11.7 / 6.9, 14.2 / 9.4,
-// 19.3 / 14.4; 512 experts at 1040, 1600, 2049 slots 6.8 / 7.2, 7.2 / 7.2, 7.6 / 7.3.  With the quantisation beside it, whole layer:
-// Qwen3-30B-A3B layer at 160, 333, 1000, 1531, 4000 tokens 115.5 / 115.5, 123.3 / 121.4, 165 / 160, 177.2 / 172.7, 324 / 321,
-// per-channel 700: 145.0 / 140.7; DeepSeek-V3 share at 500, 1500, 3000: 249.5 / 247.0, 351 / 345, 377 / 375.  There the sweeping
-// workgroups are slower than the two launches past 32768 slots: the share at 5000, 6000, 8192 tokens 531 / 533, 575 / 581, 710 /
-// 716; quantisation by row, past 28672: per-channel Qwen3-30B-A3B layer at 3500, 4000, 8000 276.1 / 274.6, 317.3 / 319.2, 518 / 523.
-constexpr int64_t kWideQuantSlots = 32768, kWideRowQuantSlots = 28672, kWideAlignSlots = 65536;
-// By workgroups of 256 instead: the quantisation of 29 million values takes 19.8 us beside them, 25.5 beside those of 1024, the
-// alignment of 65536 slots 23.5 instead of 21.6.  Whole layer, us, the other form / this: DeepSeek-V3 share (896 values a slot) at
-// 2100 tokens 327 / 328, 3000: 375 / 375, 4096: 470 / 466, 8192: 713 / 710, 24000: 1913 / 1907, by row 2500: 322.6 / 324.2,
-// 4096: 448 / 445, 8192: 645 / 639; int4 layer with 512 values a slot at 2048 tokens 546 / 548; Qwen3-30B-A3B layer (256) at 4000
-// 321 / 325, 8192: 561 / 563.
-constexpr int64_t kNarrowFrom = 24576, kNarrowSlots = 262144, kNarrowValues = 700;
-static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, size_t *lds_bytes) {
-  const int64_t words = (kWideT / kWave + 4) * static_cast<int64_t>(num_experts) + 1;
-  if (numel <= kWideSlots || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || words > 15360) return 0;
-  *lds_bytes = static_cast<size_t>(words) * sizeof(int32_t);
+// The one-launch form by several workgroups of T threads (moe_align_wide_body): their number, or 0 where another form is taken.
+// Every one of them sweeps all slots, so `most` of them; below, one workgroup has nothing to share.  LDS holds 4 (T / 64 + 2) bytes
+// an expert and 8 for each copy of its sweep counters: four copies up to 590 experts (T = 256: 365), fewer beyond.
+//
+// Alignment alone, us, the other forms / this, routing uniform; every slot to one expert: 2048 slots, 8 experts 6.5 / 5.6; 8.0 /
+// 5.6, 128 experts 7.5 / 6.5; 8.7 / 6.4, 8192 slots, 128 experts 10.9 / 6.7; 14.8 / 8.6, 32768 slots, 8 experts 11.4 / 9.9; 24.0 /
+// 19.1, 128 experts 12.1 / 10.2; 26.2 / 19.5 (one copy of the counters 9.8; 32.6, eight 10.4; 13.2), 65536 slots, 256 experts 19.8 /
+// 15.9; 44.5 / 34.0, 512 experts 30.4 / 16.6; 48.2 / 34.6.  There 8 and 128 experts lose (eight copies: 13.1 / 15.5, 14.8 / 15.8): the
+// line goes from 32768 slots with 128 experts to 65536 with 256.  With fewer copies than four, one expert's 24576 slots are 15 % over
+// the others (of one copy 22.2 / 25.6 us), 16384 of them 12 % under (600 experts 22.5 / 19.8), uniform ones half: the line between.
+constexpr int64_t kWideAlignSlots = 65536, kFewCopiesSlots = 20480;
+// Beside the quantisation.  Both launches, us, the other forms / this, routing uniform; all rows alike.  H = 2048, 8 of 128 experts,
+// 333, 1531, 4000 tokens: 8.0 / 6.2; 8.0 / 6.1, 11.0 / 7.3; 11.5 / 7.6, 12.5 / 10.3; 13.8 / 11.5, by row 3000, 4000: 12.2 / 11.4,
+// 12.5 / 12.6 (its line is 28672 slots).  H = 7168, 8 of 256, 1500, 2500 tokens: 13.4 / 9.1; 13.9 / 9.1, 16.0 / 14.4; 16.6 / 14.3.
+constexpr int64_t kWideQuantSlots = 32768, kWideRowQuantSlots = 28672;
+// Long rows: the quantisation is most of the time, and faster by workgroups of 256, which align as well, four ids a load.
+// H = 7168, 8 of 256 experts, at 3000, 4096, 8192 tokens 17.0 / 15.4; 17.7 / 16.5 (workgroups of 1024: 17.3; 17.1), 20.7 / 17.6;
+// 20.6 / 17.8, 33.8 / 30.3; 33.3 / 31.0, H = 6144, 8 of 128: 3100 15.6 / 14.3; 15.5 / 15.7, 8192: 30.3 / 26.5; 29.7 / 26.9; H = 16384, 8
+// of 64, 1150: 15.6 / 13.1; 15.1 / 12.9.  At 16384 tokens nothing is gained (73 / 75 us; 76 / 77), at 32768 it loses (151 / 159).
+// H = 4096 (512 values a slot) stays with the larger ones: 4096 tokens 14.9 / 14.0; 15.5 / 13.7.
+constexpr int64_t kNarrowFrom = 18000000, kNarrowValues = 700, kNarrowSlots = 65536;
+// Fewer than five slots a token: a row's ids share their lane with other rows', lanes meet on a counter (H = 3072, 4 of 60 experts,
+// 12000 tokens, by workgroups of 256: 23.1 / 29.9 with all rows alike), and the quantisation by workgroups of 1024 costs more than the
+// alignment gains (H = 4096, 2 of 8, 8192 tokens 22.2 / 23.3, by row 21.9 / 27.5; 3000 tokens 9.8 / 10.6).  Up to 2000 tokens it
+// gains: 1999 tokens H = 4096, 2 of 8 8.2 / 7.3, by row 9.7 / 9.1; H = 2816, 4 of 32 10.8 / 7.1, by row 11.0 / 9.6.
+constexpr int64_t kFewSlots = 5, kFewSlotsTokens = 2000;
+static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, int T, size_t *lds_bytes, int *copy_bits) {
+  auto words = [&](int bits) { return (T / kWave + 2 + (2 << bits)) * static_cast<int64_t>(num_experts) + 1; };
+  if (numel <= kWideSlots || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || num_experts > 767) return 0;
+  int bits = kMostCopyBits;
+  while (bits > 0 && words(bits) > (T == kNarrowT ? 5120 : 15360)) --bits;
+  if (bits < kMostCopyBits && numel > kFewCopiesSlots) return 0;
+  *lds_bytes = static_cast<size_t>(words(bits)) * sizeof(int32_t);
+  *copy_bits = bits;
   return static_cast<int>((numel + kWideSlots - 1) / kWideSlots);
 }
 
@@ -769,20 +793,21 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
   const int64_t groups = M * (H / kGroup);
   {
     size_t lds_bytes;
-    // Long rows: the quantisation, faster by small workgroups, takes longer than an alignment by small ones.
-    const bool narrow = numel > kNarrowFrom && M * H >= kNarrowValues * numel;
-    const int n = wide_shape(numel, num_experts, narrow ? kNarrowSlots : per_row ? kWideRowQuantSlots : kWideQuantSlots, &lds_bytes);
+    int copy_bits;
+    const bool few = numel < kFewSlots * M;
+    const bool narrow = !few && M * H > kNarrowFrom && M * H >= kNarrowValues * numel;
+    const int T = narrow ? kNarrowT : kWideT;
+    const int64_t most = few && M > kFewSlotsTokens ? 0 : narrow ? kNarrowSlots : per_row ? kWideRowQuantSlots : kWideQuantSlots;
+    const int n = wide_shape(numel, num_experts, most, T, &lds_bytes, &copy_bits);
     if (n > 0) {
-      const int T = narrow ? kNarrowT : kWideT;
-      const int64_t most = narrow ? 8192 : 4096;
+      const int64_t qmost = narrow ? 8192 : 4096;
       int64_t qblocks = per_row ? (M + T / 256 - 1) / (T / 256) : (groups + T / 16 - 1) / (T / 16);
-      if (qblocks > most) qblocks = most;
-      if (narrow) lds_bytes = ((kNarrowT / kWave + 4) * static_cast<size_t>(num_experts) + 1) * sizeof(int32_t);
+      if (qblocks > qmost) qblocks = qmost;
       const dim3 grid(static_cast<unsigned>(n + qblocks)), block(T);
 #define LO_QA_WIDE2(IdT, PR, DT, TT)                                                                                     \
   hipLaunchKernelGGL((quant_align_wide_kernel<IdT, PR, DT, TT>), grid, block, lds_bytes, stream, job,                    \
                      static_cast<const IdT *>(topk_ids), numel, num_experts, block_size, expert_map, sorted_ids,         \
-                     sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, n)
+                     sorted_cap, expert_ids, expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, copy_bits, n)
 #define LO_QA_WIDE(IdT, PR, DT)                          \
   do {                                                   \
     if (narrow) LO_QA_WIDE2(IdT, PR, DT, kNarrowT);      \
@@ -917,12 +942,15 @@ extern "C" int lo_moe_align_block_size_local(const void *topk_ids, int ids_dtype
   while ((1 << key_bits) < num_experts) ++key_bits;
   {
     size_t lds_bytes;
-    const int n = wide_shape(numel, num_experts, kWideAlignSlots, &lds_bytes);
+    int copy_bits;
+    int64_t most = 256ll * num_experts; // 32768 to 65536
+    most = most < kWideAlignSlots / 2 ? kWideAlignSlots / 2 : most < kWideAlignSlots ? most : kWideAlignSlots;
+    const int n = wide_shape(numel, num_experts, most, kWideT, &lds_bytes, &copy_bits);
     if (n > 0) {
 #define LO_WIDE(IdT)                                                                                                     \
   hipLaunchKernelGGL(moe_align_wide_kernel<IdT>, dim3(n), dim3(kWideT), lds_bytes, s, static_cast<const IdT *>(topk_ids), \
                      numel, num_experts, block_size, expert_map, ignore_invalid, sorted_ids, sorted_cap, expert_ids,     \
-                     expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, num_local_tokens, top_k)
+                     expert_ids_cap, num_tokens_post_pad, key_bits, slot_mask, num_local_tokens, top_k, copy_bits)
       if (ids_dtype == LO_I32) LO_WIDE(int32_t);
       else LO_WIDE(int64_t);
 #undef LO_WIDE
