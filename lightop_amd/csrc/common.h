@@ -203,7 +203,7 @@ __device__ __forceinline__ int quant_one(float v, float s) {
 // a fused multiply-add, and RN(q + rem*y) is then the correctly rounded quotient (Markstein's
 // theorem, valid for a correctly rounded reciprocal and no under/overflow).  Quotients
 // of denormal magnitude may differ in the last bit; they truncate to 0 either way.  Not
-// valid for s = inf (a row that holds an infinity): callers take quant_one then.
+// valid for s = inf (a row that holds an infinity) nor for a tiny s: callers take quant_one then.
 __device__ __forceinline__ int quant_one_rcp(float v, float s, float y) {
   const float q = v * y;
   const float rem = __builtin_fmaf(-q, s, v);
@@ -223,9 +223,10 @@ __device__ __forceinline__ uint32_t pack4_i8(int a, int b, int c, int d) {
          __builtin_amdgcn_perm(static_cast<uint32_t>(d), static_cast<uint32_t>(c), 0x04000c0cu);
 }
 
-// four elements of one row -> four packed int8; y = 1.0f / s (fp32 rows)
+// four elements of one row -> four packed int8; y = 1.0f / s.  A small scale (a floor of zero lets it be one) is divided by: its
+// reciprocal overflows below 2^-128, and the remainders lose bits before that.
 __device__ __forceinline__ uint32_t quant4(const float *v, float s, float y) {
-  if (s < __builtin_inff()) {
+  if (s >= 0x1p-100f && s < __builtin_inff()) {
     return pack4_i8(quant_one_rcp(v[0], s, y), quant_one_rcp(v[1], s, y), quant_one_rcp(v[2], s, y),
                     quant_one_rcp(v[3], s, y));
   }
