@@ -185,12 +185,13 @@ def test_rows_per_wavefront_change_over(dev, oracle, T, E, G, tg, k):
     assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
 
 
-@pytest.mark.parametrize("E,G,k,dtype,lines", [(32, 4, 4, torch.float32, (2560, 4096)), (60, 4, 8, torch.bfloat16, (2560, 4608)),
-                                               (128, 8, 8, torch.float16, (3584, 7168)), (160, 8, 6, torch.float32, (4608, 7168)),
-                                               (256, 8, 8, torch.bfloat16, (5632, 7168))])
+@pytest.mark.parametrize("E,G,k,dtype,lines", [(32, 4, 4, torch.float32, (2560, 3584)), (60, 4, 8, torch.bfloat16, (2560, 3584)),
+                                               (128, 8, 8, torch.float16, (2560, 6144)), (160, 8, 6, torch.float32, (3584, 12288)),
+                                               (256, 8, 8, torch.bfloat16, (3584, 12288)), (256, 1, 8, torch.float32, (12288,)),
+                                               (256, 16, 8, torch.float32, (12288,)), (144, 16, 4, torch.bfloat16, (12288,))])
 def test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtype, lines):
-    """Row counts around the one from which four rows share a wavefront: it differs by the number of experts, by the type
-    (softmax) and between softmax and gate."""
+    """Row counts around the one from which four rows share a wavefront: it differs by the number of experts and
+    between softmax and gate."""
     from lightop_amd.moe import moe_fused_gate
 
     for T in sorted(line + d for line in lines for d in (-1, 0, 3)):
@@ -202,8 +203,8 @@ def test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtyp
         rw, ridx, _ = oracle.topk_softmax(x, k, True)
         assert torch.equal(idx, ridx) and torch.equal(w.view(torch.int32), rw.view(torch.int32))
         bias = (torch.randint(-2, 3, (E,), generator=g).float() * 0.25).to(dtype)
-        w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, 2, k, 0, 2.5, False)
-        rw, ridx = oracle.moe_fused_gate(x, bias, G, 2, k, 0, 2.5, False)
+        w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, min(2, G), k, 0, 2.5, False)
+        rw, ridx = oracle.moe_fused_gate(x, bias, G, min(2, G), k, 0, 2.5, False)
         assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
 
 
@@ -214,3 +215,18 @@ def test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtyp
 def test_lines_with_all_scores_requested_at_once(dev, oracle, E, G, k, dtype, lines):
     """Row counts around the lines of the kernels that request a row's scores together, and six scores a lane."""
     test_either_side_of_each_line_between_the_kernels(dev, oracle, E, G, k, dtype, lines)
+
+
+@pytest.mark.parametrize("G,tg", [(1, 1), (8, 4), (16, 5)])
+@pytest.mark.parametrize("T", [12287, 12289])
+def test_shared_experts_of_many_rows(dev, oracle, T, G, tg):
+    """256 experts and two fused shared ones, by a row per wavefront and by four."""
+    from lightop_amd.moe import moe_fused_gate
+
+    say(f"gate with shared experts T={T} G={G}")
+    g = torch.Generator().manual_seed(T + G)
+    x = torch.randn(T, 256, generator=g)
+    bias = torch.randn(256, generator=g) * 0.05
+    w, idx = moe_fused_gate(x.to(dev), bias.to(dev), G, tg, 8, 2, 2.5, False)
+    rw, ridx = oracle.moe_fused_gate(x, bias, G, tg, 8, 2, 2.5, False)
+    assert torch.equal(idx.cpu(), ridx) and torch.equal(w.cpu().view(torch.int32), rw.view(torch.int32))
