@@ -251,7 +251,9 @@ __device__ __forceinline__ bool group_scale16(float amax, float floor, float &s,
   s = __builtin_fmaf(__builtin_fmaf(-127.0f, q, top), r, q); // top / 127 correctly rounded (Markstein)
   const bool up = __builtin_fmaf(0x1p-18f, s, __builtin_fmaf(-127.0f, s, top)) >= 0.0f; // top / s rounds to 127 or above
   y = __builtin_amdgcn_rcpf(s) * (up ? 1.0f + 0x1p-21f : 1.0f - 0x1p-21f);
-  return top < __builtin_inff() && (amax >= fmaxf(floor, 1e-10f) || (amax == 0.0f && floor >= 1e-10f));
+  // (with the default floor three comparisons: more of them cost the one-token kernels up to 4 %)
+  return (floor >= 1e-10f && floor < __builtin_inff() && amax == 0.0f) ||
+         (amax >= fmaxf(floor, 1e-10f) && amax < __builtin_inff());
 }
 // (a NaN becomes -128 as in quant_one)
 __device__ __forceinline__ uint32_t quant4_mul(const float *v, float y) {
@@ -263,12 +265,14 @@ __device__ __forceinline__ uint32_t quant4_mul(const float *v, float y) {
 
 // Eight values of a group of 16-bit values whose maximum is amax, and the group's scale.  A group that the multiplication does not
 // hold for is quantised by one reciprocal where that holds: 8192 rows of 7168 with a floor above their maxima 30.5 us, with a
-// division a value 38.5, without the attempt at the multiplication 29.1.
+// division a value 38.5, without the attempt at the multiplication 29.1.  ONLY_DIV: at the default floor, below which next to no
+// group's maximum lies, the division alone, which is less code (one token of the Qwen3-30B-A3B layer 18.06 -> 17.56 us).
+template <bool ONLY_DIV = false>
 __device__ __forceinline__ v2i group_quant8(const float (&v)[8], float amax, float floor, float &s) {
   float y;
   if (__builtin_expect(group_scale16(amax, floor, s, y), 1))
     return v2i{static_cast<int>(quant4_mul(&v[0], y)), static_cast<int>(quant4_mul(&v[4], y))};
-  if (s >= 0x1p-100f) { // a finite maximum: s is what the division gives
+  if (!ONLY_DIV && s >= 0x1p-100f) { // a finite maximum: s is what the division gives
     y = 1.0f / s;
     return v2i{static_cast<int>(quant4_rcp(&v[0], s, y)), static_cast<int>(quant4_rcp(&v[4], s, y))};
   }
@@ -373,9 +377,9 @@ __device__ __forceinline__ void quant_job(const QuantJob &j, int64_t block, int6
 
 // The quantisation of x [M, H] (per group, or per row) and the routing alignment with the quantisation riding in the
 // alignment's (second) launch: they are independent, and at decode sizes a launch costs as much
-// as either.  scratch: the multi-workgroup alignment's counters (lo_moe_align_scratch_bytes);
-// returns LO_ENOTSUP when they are needed and missing - the caller then launches the two stages
-// separately.
+// as either.  scratch: the counters of the form with a launch for them (lo_moe_align_scratch_bytes);
+// returns LO_ENOTSUP when that form is the one to take and they are missing - the caller then launches
+// the two stages separately.
 int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_t H, float eps, int8_t *q, float *s,
                        const void *topk_ids, int ids_dtype, int64_t numel, int32_t num_experts,
                        int32_t block_size, const int32_t *expert_map, int32_t *sorted_ids, int64_t sorted_cap,
