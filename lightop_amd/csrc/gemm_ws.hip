@@ -80,13 +80,13 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
   // tokens of this block, one per (sub-tile, r)
   int64_t f[TM];
   bool valid[TM];
-  float wgt[TM];
+  float wgt[FUSED_ACT ? 1 : TM]; // (the first stage seldom wants them, and has no registers for them)
   int aoff[TM], asoff[TM]; // byte offsets of the token's row in A and As
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     f[j] = ids[j];
     valid[j] = f[j] < a.num_valid;
-    wgt[j] = slot_weight(a, f[j]);
+    if constexpr (!FUSED_ACT) wgt[j] = slot_weight(a, f[j]);
     const int64_t row = token_row(a, f[j]);
     aoff[j] = static_cast<int>(row * K) + c * 16;
     asoff[j] = static_cast<int>(row * (PC ? 1 : KB) * 4);
@@ -401,7 +401,8 @@ __global__ __launch_bounds__(NWAVES * 64) void moe_gemm_ws_kernel(const GemmArgs
     float actf[TM][4];
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-      const float w = wgt[j];
+      float w = 1.0f;
+      if (a.mul_routed && valid[j]) w = a.topk_w[f[j]];
       float amax = 0.0f;
       float g[4], u[4];
 #pragma unroll

@@ -46,3 +46,7 @@ def test_registers_and_spills(tmp_path):
     # first kernel of few tokens, int4 weights with K-group scales: one token 27.5 us with 20 bytes, 28.5 with 36
     dec = {n: k for n, k in kernels.items() if re.match(r"_ZN2lo16dec_gemm1_kernelILi4ELb1ELb0E", n)}
     assert dec and all(spilled <= 20 for _, spilled in dec.values()), dec
+    # weight-streaming first stage of 16-token blocks, int8 in its load-time layout: past 128 registers one workgroup to a CU instead
+    # of two (24 tokens of the DeepSeek-V3 share in the separate order 120.0 -> 123.0 us)
+    ws = {n: k for n, k in kernels.items() if re.match(r"_ZN2lo18moe_gemm_ws_kernelILi1ELi1ELi[012]ELb1ELi8ELi4ELi2ELb0ELb0E", n)}
+    assert len(ws) >= 3 and all(v <= 128 and not spilled for v, spilled in ws.values()), ws
