@@ -1,6 +1,8 @@
 // moe_align_block_size for gfx950: expert histogram, padded prefix sum and a stable
-// (ascending slot id) counting sort, in one workgroup, with wavefront ballots and
-// LDS counters and no atomics on the ranking path, so the result is deterministic.
+// (ascending slot id) counting sort, with wavefront ballots and LDS counters and no
+// atomics on the ranking path, so the result is deterministic.  Three forms of the same
+// algorithm: one workgroup; several in one launch, each of which counts all slots; and a
+// counting launch with a scattering one behind it.
 //
 // Semantics follow python/lightop/_lmslim_native/vllm_compat/moe_align_block_size.py:17-120
 // and csrc/kernels/moe_align_sum_kernels.cu:1034-1115 of the reference; the order
@@ -696,7 +698,6 @@ __global__ __launch_bounds__(256) void quant_align_scatter_kernel(
   }
 }
 
-// chunks for the multi-workgroup path: about 1024 slots each, at most 256 chunks
 static void single_wg_shape(int64_t numel, int64_t sorted_cap, int32_t num_experts, int *nw, size_t *lds_bytes) {
   // waves per workgroup: as many as the per-wave LDS counters allow (<= 60 KB)
   int w = 16;
@@ -744,6 +745,7 @@ static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, int T, s
   return static_cast<int>((numel + kWideSlots - 1) / kWideSlots);
 }
 
+// chunks of the counting and the scattering launch: about 1024 slots each, at most 256 chunks
 static void align_chunks(int64_t numel, int *nchunks, int64_t *chunk_slots) {
   int64_t n = (numel + 1023) / 1024;
   if (n > 256) n = 256;
@@ -772,9 +774,6 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
                        int32_t block_size, const int32_t *expert_map, int32_t *sorted_ids, int64_t sorted_cap,
                        int32_t *expert_ids, int64_t expert_ids_cap, int32_t *num_tokens_post_pad,
                        uint8_t *slot_mask, void *scratch, int64_t scratch_bytes, hipStream_t stream) {
-  const int64_t want = lo_moe_align_scratch_bytes(numel, num_experts);
-  if (want > 0 && !(scratch && scratch_bytes >= want && (reinterpret_cast<uintptr_t>(scratch) & 3) == 0))
-    return LO_ENOTSUP; // the multi-workgroup form needs its counters
   LO_REQUIRE(x && q && qs && topk_ids && sorted_ids && expert_ids && num_tokens_post_pad, LO_EINVAL,
              "quant_align: null pointer");
   LO_REQUIRE((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(q) & 7) == 0, LO_EINVAL,
@@ -818,7 +817,9 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
       return check_launch("quant_align(wide)");
     }
   }
+  const int64_t want = lo_moe_align_scratch_bytes(numel, num_experts);
   if (want > 0) { // many slots: counting, then the scatter beside the quantisation
+    if (!(scratch && scratch_bytes >= want && (reinterpret_cast<uintptr_t>(scratch) & 3) == 0)) return LO_ENOTSUP;
     int nchunks;
     int64_t cs;
     align_chunks(numel, &nchunks, &cs);

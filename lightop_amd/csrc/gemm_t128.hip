@@ -635,8 +635,9 @@ void moe_gemm_t128_kernel(const GemmArgs a, int m_blocks, int group_m) {
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
           // 128-token tiles close the stage's products up and fold behind them.  Four (int4: five) after each / this, whole layer,
           // us: all experts of DeepSeek-V3, skewed, 5500 tokens 3244 / 3222, 8192: 4457 / 4430, 12000: 6253 / 6204; share 7000:
-          // 650 / 647; Qwen3-235B-A22B-shaped layer 3000: 832 / 823, 6500: 1500 / 1498; Qwen3-30B-A3B layer 3000 and 8192: equal; int4
-          // with K-group scales, 128 experts of 4096 x 1536, 1100: 375 / 366, 2800: 724 / 711, 6000: 1313 / 1291.  int8 tiles of 160
+          // 650 / 647; Qwen3-235B-A22B-shaped layer 3000: 832 / 823, 6500: 1500 / 1498; Qwen3-30B-A3B layer 3000 and 8192: equal; row-major
+          // weights, Qwen3-235B-A22B-shaped 4096: 1062 / 1049, 8192: 1834 / 1802, Qwen3-30B-A3B 8192: 554 / 546 (with the other steps
+          // that are in the layer since); int4 with K-group scales, 128 experts of 4096 x 1536, 1100: 375 / 366, 2800: 724 / 711, 6000: 1313 / 1291.  int8 tiles of 160
           // lose (1531 tokens 177 / 180).
           if constexpr (decltype(BIASED)::value && !PC && (W4 || NTB == 8)) {
             if (g < 3) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);

@@ -70,7 +70,7 @@ def _align(topk_ids, num_experts, block_size, sorted_token_ids, experts_ids, num
             raise RuntimeError("lightop_amd: num_local_tokens needs topk_ids of shape [num_tokens, topk]")
         top_k = topk_ids.shape[1]
     lib = _lib.lib()
-    # large inputs are aligned by many workgroups; their per-chunk counters live in a
+    # the largest inputs are counted in a launch of their own; its per-chunk counters live in a
     # scratch tensor (the reference allocates one too, moe_align_sum_kernels.cu:1175)
     nscratch = int(lib.lo_moe_align_scratch_bytes(topk_ids.numel(), int(num_experts)))
     scratch = torch.empty(nscratch, dtype=torch.uint8, device=topk_ids.device) if nscratch > 0 else None
