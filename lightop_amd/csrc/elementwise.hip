@@ -661,16 +661,16 @@ extern "C" int lo_moe_sum(const void *in, void *out, const void *bias, const uin
                               static_cast<hipStream_t>(stream));
   // Without a mask, where there is much to read: a token a workgroup.  With one: several, whose masks are asked for ahead.  Rows of
   // more than 4096 values that fill as much of workgroups of 512 threads as of 256: those, once they are several to a CU.
-  // us, 256 threads and 4096 workgroups at the most / this, 8 slots a token: 8192 tokens of 7168 values 194.6 / 182.0 (6.2 TB/s), an
-  // eighth of the slots held 64.4 / 60.6, nine tenths 199.4 / 193.0; 4096 tokens 97.3 / 92.4, 34.4 / 32.4, 100.0 / 97.0; 16384 of 1024
-  // 55.7 / 52.2, of 4096 224 / 200; 8192 of 5120 138.4 / 131.4.  What is left to the smaller grid loses: below 45 million values 4096
-  // tokens of 4096 with two slots 18.1 / 18.9, 3000 of 7168 23.4 / 23.9; rows of 256 with four 31.0 / 34.0 at 65536 tokens; masked
-  // rows of 4096, 1300 tokens 16.9 / 18.3, of 5120 21.9 / 22.8 (512 threads: three fifths of the lanes have a column), 1300 tokens of
-  // 8192, two slots 15.0 / 15.7.
+  // us, 256 threads and 4096 workgroups at the most / this, 8 slots a token: 8192 tokens of 7168 values 194.6 / 182.0 (6.2 TB/s), with
+  // a bias and an eighth of the slots held 64.4 / 60.6, nine tenths 199.4 / 193.0; 4096 tokens 97.3 / 92.4, 34.4 / 32.4, 100.0 / 97.0
+  // (without the bias an eighth 26.0 / 27.9: left as it was); 16384 of 1024 55.7 / 52.2, of 4096 224 / 200; 8192 of 5120 138.4 /
+  // 131.4.  What is left to the smaller grid loses: below 45 million values 4096 tokens of 4096 with two slots 18.1 / 18.9, 3000 of
+  // 7168 23.4 / 23.9; rows of 256 with four 31.0 / 34.0 at 65536 tokens; masked rows of 4096, 1300 tokens 16.9 / 18.3, of 5120 21.9 /
+  // 22.8 (512 threads: three fifths of the lanes have a column), 1300 tokens of 8192, two slots 15.0 / 15.7.
   const int64_t pieces = (H + 2047) / 2048, values = M * topk * H;
   LO_REQUIRE(pieces < 65536, LO_ENOTSUP, "moe_sum: rows of %lld values", (long long)H);
   const bool singly = !expert_mask && values > 45000000 && H >= 512 && (H >= 1024 || topk >= 4);
-  const bool wide = H > 4096 && pieces % 2 == 0 && (singly || (expert_mask && M * pieces > 10240));
+  const bool wide = H > 4096 && pieces % 2 == 0 && (singly || (expert_mask && bias && M * pieces > 10240));
   const int threads = wide ? kSumThreads : 256;
   const int64_t cols = (H / 8 + threads - 1) / threads;
   int64_t tokens = (singly ? 65536 : 4096) / cols;
