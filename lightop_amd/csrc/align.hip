@@ -734,12 +734,13 @@ constexpr int64_t kNarrowFrom = 18000000, kNarrowValues = 700, kNarrowSlots = 65
 // alignment gains (H = 4096, 2 of 8, 8192 tokens 22.2 / 23.3, by row 21.9 / 27.5; 3000 tokens 9.8 / 10.6).  Up to 2000 tokens it
 // gains: 1999 tokens H = 4096, 2 of 8 8.2 / 7.3, by row 9.7 / 9.1; H = 2816, 4 of 32 10.8 / 7.1, by row 11.0 / 9.6.
 constexpr int64_t kFewSlots = 5, kFewSlotsTokens = 2000;
-static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, int T, size_t *lds_bytes, int *copy_bits) {
+// (few_copies: `most` of the form with fewer copies)
+static int wide_shape(int64_t numel, int32_t num_experts, int64_t most, int64_t few_copies, int T, size_t *lds_bytes, int *copy_bits) {
   auto words = [&](int bits) { return (T / kWave + 2 + (2 << bits)) * static_cast<int64_t>(num_experts) + 1; };
   if (numel <= kWideSlots || numel < 4 * static_cast<int64_t>(num_experts) || numel > most || num_experts > 767) return 0;
   int bits = kMostCopyBits;
   while (bits > 0 && words(bits) > (T == kNarrowT ? 5120 : 15360)) --bits;
-  if (bits < kMostCopyBits && numel > kFewCopiesSlots) return 0;
+  if (bits < kMostCopyBits && numel > few_copies) return 0;
   *lds_bytes = static_cast<size_t>(words(bits)) * sizeof(int32_t);
   *copy_bits = bits;
   return static_cast<int>((numel + kWideSlots - 1) / kWideSlots);
@@ -797,7 +798,7 @@ int launch_quant_align(const void *x, int dtype, bool per_row, int64_t M, int64_
     const bool narrow = !few && M * H > kNarrowFrom && M * H >= kNarrowValues * numel;
     const int T = narrow ? kNarrowT : kWideT;
     const int64_t most = few && M > kFewSlotsTokens ? 0 : narrow ? kNarrowSlots : per_row ? kWideRowQuantSlots : kWideQuantSlots;
-    const int n = wide_shape(numel, num_experts, most, T, &lds_bytes, &copy_bits);
+    const int n = wide_shape(numel, num_experts, most, kFewCopiesSlots, T, &lds_bytes, &copy_bits);
     if (n > 0) {
       const int64_t qmost = narrow ? 8192 : 4096;
       int64_t qblocks = per_row ? (M + T / 256 - 1) / (T / 256) : (groups + T / 16 - 1) / (T / 16);
@@ -941,12 +942,15 @@ extern "C" int lo_moe_align_block_size_local(const void *topk_ids, int ids_dtype
   hipStream_t s = static_cast<hipStream_t>(stream);
   int key_bits = 1;
   while ((1 << key_bits) < num_experts) ++key_bits;
+  const int64_t want = lo_moe_align_scratch_bytes(numel, num_experts);
+  const bool counted = want > 0 && scratch && scratch_bytes >= want && (reinterpret_cast<uintptr_t>(scratch) & 3) == 0;
   {
     size_t lds_bytes;
     int copy_bits;
-    int64_t most = 256ll * num_experts; // 32768 to 65536
-    most = most < kWideAlignSlots / 2 ? kWideAlignSlots / 2 : most < kWideAlignSlots ? most : kWideAlignSlots;
-    const int n = wide_shape(numel, num_experts, most, kWideT, &lds_bytes, &copy_bits);
+    int64_t most = 256ll * num_experts; // 32768 to 65536; without the counters' launch one workgroup is all there is past that
+    most = most < kWideAlignSlots / 2 ? kWideAlignSlots / 2 : most;
+    if (most > kWideAlignSlots || !counted) most = kWideAlignSlots;
+    const int n = wide_shape(numel, num_experts, most, counted ? kFewCopiesSlots : most, kWideT, &lds_bytes, &copy_bits);
     if (n > 0) {
 #define LO_WIDE(IdT)                                                                                                     \
   hipLaunchKernelGGL(moe_align_wide_kernel<IdT>, dim3(n), dim3(kWideT), lds_bytes, s, static_cast<const IdT *>(topk_ids), \
@@ -958,8 +962,7 @@ extern "C" int lo_moe_align_block_size_local(const void *topk_ids, int ids_dtype
       return check_launch("moe_align_block_size(wide)");
     }
   }
-  const int64_t want = lo_moe_align_scratch_bytes(numel, num_experts);
-  if (want > 0 && scratch && scratch_bytes >= want && (reinterpret_cast<uintptr_t>(scratch) & 3) == 0) {
+  if (counted) {
     int nchunks;
     int64_t cs;
     align_chunks(numel, &nchunks, &cs);
